@@ -13,26 +13,27 @@
 //                           ||y - x||_2 <= tol from 1/n, then y / sum(y)
 //
 // Kernels.  Every sum is added in an order fixed by the matrix alone (deterministic):
-//   csr_short_kernel<G>   rows of at most 32 G entries: a group of G lanes (4..64, chosen from
-//       the average row length) owns a row, strides over it and reduces with shuffles; at most
-//       kShortGrid blocks step over row tiles.
-//   long rows             the rest, cut into pieces of kPiece entries so that a few huge rows
-//       (power-law matrices) spread over the whole device:
-//       csr_long_scan_kernel    kLongGrid blocks count the long rows and pieces of their row
-//                               ranges;
-//       csr_long_offsets_kernel one block: exclusive sums of those counts;
-//       csr_long_list_kernel    the same blocks write {row, first piece} of their long rows,
-//                               in row order;
-//       csr_piece_kernel        a block per piece (grid-stride): the piece's partial sum;
-//       csr_long_fix_kernel     per long row: its pieces added in order, the shift, y, and
-//                               for a step (y - x)^2.
-// The step's (y - x)^2 is added per block (short kernel and fix kernel), and the block sums in
-// block order by a one-block kernel into a device scalar.
+//   csr_tile_kernel   the rows' ends and the entries, merged into one list (Merrill and Garland,
+//       "Merge-based parallel sparse matrix-vector multiplication", SC 2016), are cut into tiles of
+//       equal length, so that a block has as much to do whatever the rows' lengths: it finds its
+//       first row and entry by a search over row_idx (64 probes at a time, the lanes of a wave),
+//       reads its entries as one stream, puts the products into LDS and adds them row by row, lane
+//       groups for short rows and whole waves for long ones.  What is left after its last row end
+//       is the tile's carry for the row that goes on.
+//   csr_fix_kernel    adds the carries, in tile order, to the row that ended in a later tile.
+//   csr_final_kernel  (steps of many tiles) adds the blocks' sums.
+// The step's (y - x)^2 is added per block of either kernel.
 //
-// Scratch of a product: the long-row list (at most nnz / (32 G + 1) rows) and piece sums (at
-// most nnz / kPiece + list rows), the block counts, and the step's block sums; a plain product
-// and a step take it from the stream's memory pool for the duration of the call, the
-// allocation-free step from a static device array (which caps the matrices it accepts).
+// What bounds it: the two 8-byte streams (16 bytes per entry) and the gathers of x, in flight
+// together for a whole tile.  A lane group per row with a block sum per long row kept one or two
+// entries in flight per lane and left long rows to five more launches (one of them a single
+// thread): 713 us for the step of an R-MAT matrix of 1e6 rows and 1.4e7 entries, 146 us now (the tiles
+// 129 us).
+//
+// Scratch of a product: a carry (row and sum) per tile, 12 bytes for 4096 merged items, and the
+// blocks' sums of squares.  A plain product and a step take it from the stream's memory pool for the duration
+// of the call, the allocation-free step from a static device array (which caps the matrices it
+// accepts).
 //
 // Algorithmic bytes per product (HBM-bound, random gathers of x): per entry col 8 + value 8 +
 // gathered x 8; per row row_idx 8 + y 8 (+ x 8 for the step's norm).
@@ -46,8 +47,7 @@
 
 #include "nkpr_internal.hpp"
 
-// Scratch of nkpr_csr_pagerank_step_noalloc (48.1 MiB): the long-row list (2^21 rows), the
-// piece sums (2^22), the block counts and offsets, and the step's block sums.  Every GPU the
+// Scratch of nkpr_csr_pagerank_step_noalloc (48.1 MiB): the tiles' carries and sums.  Every GPU the
 // library runs on holds it until the process ends.  Host code never uses this name as an
 // address: it takes the array's address per device with hipGetSymbolAddress
 // (csr_noalloc_scratch).
@@ -56,78 +56,58 @@ static __device__ __align__(256) unsigned char scratch[(1u << 21) * 8 + (1u << 2
 namespace nkpr {
 namespace {
 
-constexpr int kShortThreads = 256;
-constexpr uint32_t kShortGrid = 2048;
-constexpr int kLongThreads = 1024;   // scan and list blocks
-constexpr uint32_t kLongGrid = 2048;
-constexpr int kPieceThreads = 256;
-constexpr uint32_t kPiece = 4096;    // entries per piece of a long row
-constexpr uint32_t kPieceGrid = 4096;
-constexpr int kFixThreads = 256;
-constexpr uint32_t kFixGrid = 256;
 constexpr int kFinalThreads = 256;
+// A tile: kThreads threads, kPer merged items each.  The small one spreads matrices of fewer than
+// kSmallItems merged items over the device.
+template <int THREADS, int PER> struct TileShape {
+    static constexpr int kThreads = THREADS, kPer = PER, kItems = THREADS * PER;
+};
+using LargeTile = TileShape<512, 8>;
+using SmallTile = TileShape<256, 4>;
+constexpr uint64_t kSmallItems = 1ull << 22;
+// a row longer than kTurns lanes' worth of its lane group is added by a whole wave
+constexpr uint32_t kTurns = 32;
+constexpr uint32_t kNoRow = 0xFFFFFFFFu;
+// blocks of the tile kernel, at most (each steps over tiles); tiles whose carries one block of the
+// fix kernel takes, and its blocks when there are more
+constexpr uint32_t kTileGrid = 4096;
+constexpr int kFixThreads = 1024;
+constexpr uint32_t kFixAlone = 16384, kFixGrid = 512;
+// matrices the allocation-free step accepts (see csr_step_noalloc_impl)
 constexpr uint32_t kNoallocList = 1u << 21, kNoallocPieces = 1u << 22;
+constexpr uint32_t kNoallocPiece = 4096;
 
 struct CsrView {
-    uint64_t rows;
+    uint64_t rows, nnz;
     const uint64_t *row_idx;
     const uint64_t *col_idx;
     const double *val;
 };
 
 // The scratch of one product, carved from one buffer.
-struct LongWork {
-    uint32_t *bcount;   // [kLongGrid] long rows per scan block
-    uint32_t *bpieces;  // [kLongGrid] pieces per scan block
-    uint32_t *boff;     // [kLongGrid + 1] first list slot per scan block
-    uint32_t *bpoff;    // [kLongGrid + 1] first piece per scan block
-    uint32_t *total;    // [2] long rows, pieces
-    uint2 *list;        // [list cap] {row, first piece}
-    double *piece;      // [piece cap]
-    double *partials;   // [kShortGrid + kFixGrid] the step's block sums
+struct TileWork {
+    double *carry;      // [tiles] sum of the entries after the tile's last row end
+    double *partials;   // [kTileGrid + kFixGrid] (y - x)^2 per block of the two kernels
+    uint32_t *row;      // [tiles] the row the carry belongs to, kNoRow without one
 };
 
-size_t work_bytes(uint64_t list_cap, uint64_t piece_cap) {
-    return 8 * list_cap + 8 * piece_cap + 4 * (4 * (size_t)kLongGrid + 4) +
-           8 * (size_t)(kShortGrid + kFixGrid) + 256;
+bool small_matrix(const CsrView &A) { return A.rows + A.nnz < kSmallItems; }
+
+uint64_t tiles_of(const CsrView &A) {
+    const uint64_t items = small_matrix(A) ? SmallTile::kItems : LargeTile::kItems;
+    return (A.rows + A.nnz + items - 1) / items;
 }
 
-LongWork carve(void *base, uint64_t list_cap, uint64_t piece_cap) {
-    char *p = static_cast<char *>(base);
-    LongWork w;
-    w.list = reinterpret_cast<uint2 *>(p);
-    p += 8 * list_cap;
-    w.piece = reinterpret_cast<double *>(p);
-    p += 8 * piece_cap;
-    w.partials = reinterpret_cast<double *>(p);
-    p += 8 * (size_t)(kShortGrid + kFixGrid);
-    uint32_t *u = reinterpret_cast<uint32_t *>(p);
-    w.bcount = u;
-    w.bpieces = u + kLongGrid;
-    w.boff = u + 2 * kLongGrid;
-    w.bpoff = u + 3 * kLongGrid + 1;
-    w.total = u + 4 * kLongGrid + 2;
+uint32_t tile_grid(uint64_t tiles) { return (uint32_t)std::min<uint64_t>(tiles, kTileGrid); }
+
+size_t work_bytes(uint64_t tiles) { return 12 * (size_t)tiles + 8 * (size_t)(kTileGrid + kFixGrid); }
+
+TileWork carve(void *base, uint64_t tiles) {
+    TileWork w;
+    w.carry = static_cast<double *>(base);
+    w.partials = w.carry + tiles;
+    w.row = reinterpret_cast<uint32_t *>(w.partials + kTileGrid + kFixGrid);
     return w;
-}
-
-__device__ __forceinline__ uint32_t pieces_of(uint64_t len) {
-    return (uint32_t)((len + kPiece - 1) / kPiece);
-}
-
-// Sum of the products of row entries [b, e) taken by one lane in steps of `stride`; two
-// accumulators keep two gathers in flight.
-__device__ __forceinline__ double row_part(const CsrView &A, const double *__restrict__ x,
-                                           uint64_t b, uint64_t e, uint32_t stride) {
-    double s0 = 0.0, s1 = 0.0;
-    uint64_t k = b;
-    for (; k + stride < e; k += 2 * (uint64_t)stride) {
-        const uint64_t c0 = A.col_idx[k], c1 = A.col_idx[k + stride];
-        const double v0 = A.val[k], v1 = A.val[k + stride];
-        s0 += v0 * x[c0];
-        s1 += v1 * x[c1];
-    }
-    if (k < e) s0 += A.val[k] * x[A.col_idx[k]];
-    return s0 + s1;
 }
 
 // Block sum (fixed order: shuffles inside each wave, then thread 0 adds the waves); the
@@ -146,193 +126,151 @@ __device__ __forceinline__ double block_sum(double v) {
     return tot;
 }
 
-template <int G, bool STEP>
-__global__ __launch_bounds__(kShortThreads) void csr_short_kernel(CsrView A,
-                                                                  const double *__restrict__ x,
-                                                                  double shift, double *y,
-                                                                  double *partials,
-                                                                  uint64_t tiles) {
-    constexpr uint32_t groups = kShortThreads / G;
-    constexpr uint64_t kLong = 32u * G;
-    const uint32_t lane = threadIdx.x % G;
-    const uint32_t group = threadIdx.x / G;
-    double sq = 0.0;
-    for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-        const uint64_t r = t * groups + group;
-        double s = 0.0;
-        bool own = false;
-        if (r < A.rows) {
-            const uint64_t b = A.row_idx[r], e = A.row_idx[r + 1];
-            own = e - b <= kLong;
-            if (own) s = row_part(A, x, b + lane, e, G);
-        }
-#pragma unroll
-        for (int o = G / 2; o > 0; o >>= 1) s += __shfl_xor(s, o, G);
-        if (own && lane == 0) {
-            const double v = s + shift;
-            y[r] = v;
-            if (STEP) {
-                const double d = v - x[r];
-                sq += d * d;
-            }
-        }
+// Rows that have ended before merged item d: the smallest i in [max(0, d - nnz), min(d, rows)] whose
+// row end lies past entry d - i - 1.  A wave probes 64 places of the range at a time.
+__device__ __forceinline__ uint64_t rows_before(const CsrView &A, uint64_t d) {
+    const uint32_t lane = threadIdx.x & 63;
+    uint64_t lo = d > A.nnz ? d - A.nnz : 0, hi = d < A.rows ? d : A.rows;
+    while (lo < hi) {
+        const uint64_t step = (hi - lo + 63) / 64;
+        const uint64_t mid = lo + (lane + 1) * step - 1;
+        const bool ended = mid < hi && A.row_idx[mid + 1] <= d - mid - 1;
+        const uint64_t c = (uint64_t)__popcll(__ballot(ended));
+        const uint64_t next = lo + (c + 1) * step - 1;
+        lo += c * step;
+        hi = next < hi ? next : hi;
     }
-    if (STEP) {
-        const double tot = block_sum<kShortThreads>(sq);
-        if (threadIdx.x == 0) partials[blockIdx.x] = tot;
-    }
+    return lo;
 }
 
-// Long rows of block b's row range [b rpb, (b + 1) rpb): count and pieces.
-__global__ __launch_bounds__(kLongThreads) void csr_long_scan_kernel(CsrView A, uint64_t rpb,
-                                                                     uint64_t lim, LongWork w) {
-    const uint64_t r0 = (uint64_t)blockIdx.x * rpb;
-    const uint64_t r1 = std::min<uint64_t>(A.rows, r0 + rpb);
-    uint32_t cnt = 0, pcs = 0;
-    for (uint64_t r = r0 + threadIdx.x; r < r1; r += kLongThreads) {
-        const uint64_t len = A.row_idx[r + 1] - A.row_idx[r];
-        if (len > lim) {
-            ++cnt;
-            pcs += pieces_of(len);
-        }
-    }
-    __shared__ uint32_t sc[kLongThreads / 64], sp[kLongThreads / 64];
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        cnt += __shfl_xor(cnt, o, 64);
-        pcs += __shfl_xor(pcs, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sc[threadIdx.x >> 6] = cnt;
-        sp[threadIdx.x >> 6] = pcs;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t c = 0, q = 0;
-        for (int i = 0; i < kLongThreads / 64; ++i) {
-            c += sc[i];
-            q += sp[i];
-        }
-        w.bcount[blockIdx.x] = c;
-        w.bpieces[blockIdx.x] = q;
-    }
-}
-
-// One block: exclusive sums of the scan blocks' counts; total = {long rows, pieces}.
-__global__ void csr_long_offsets_kernel(LongWork w, uint32_t nblocks) {
-    if (threadIdx.x != 0) return;
-    uint32_t c = 0, q = 0;
-    for (uint32_t b = 0; b < nblocks; ++b) {
-        w.boff[b] = c;
-        w.bpoff[b] = q;
-        c += w.bcount[b];
-        q += w.bpieces[b];
-    }
-    w.boff[nblocks] = c;
-    w.bpoff[nblocks] = q;
-    w.total[0] = c;
-    w.total[1] = q;
-}
-
-// The long rows of block b's range in row order: list[boff[b] + i] = {row, first piece}.
-__global__ __launch_bounds__(kLongThreads) void csr_long_list_kernel(CsrView A, uint64_t rpb,
-                                                                     uint64_t lim, LongWork w) {
-    __shared__ uint32_t wc[kLongThreads / 64], wp[kLongThreads / 64];
-    __shared__ uint32_t base_c, base_p;
-    const uint32_t tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
-    const uint64_t r0 = (uint64_t)blockIdx.x * rpb;
-    const uint64_t r1 = std::min<uint64_t>(A.rows, r0 + rpb);
-    if (tid == 0) {
-        base_c = w.boff[blockIdx.x];
-        base_p = w.bpoff[blockIdx.x];
-    }
-    __syncthreads();
-    for (uint64_t base = r0; base < r1; base += kLongThreads) {
-        const uint64_t r = base + tid;
-        uint32_t np = 0;
-        if (r < r1) {
-            const uint64_t len = A.row_idx[r + 1] - A.row_idx[r];
-            if (len > lim) np = pieces_of(len);
-        }
-        // in-wave inclusive prefix sums of the long-row count and of the pieces
-        uint32_t ic = np ? 1u : 0u, ip = np;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint32_t tc = __shfl_up(ic, o, 64), tp = __shfl_up(ip, o, 64);
-            if (lane >= (uint32_t)o) {
-                ic += tc;
-                ip += tp;
-            }
-        }
-        if (lane == 63) {
-            wc[wave] = ic;
-            wp[wave] = ip;
-        }
-        __syncthreads();
-        uint32_t pc = base_c, pp = base_p;
-        for (uint32_t k = 0; k < wave; ++k) {
-            pc += wc[k];
-            pp += wp[k];
-        }
-        if (np) w.list[pc + ic - 1] = make_uint2((uint32_t)r, pp + ip - np);
-        __syncthreads();
-        if (tid == 0) {
-            for (int k = 0; k < kLongThreads / 64; ++k) {
-                base_c += wc[k];
-                base_p += wp[k];
-            }
-        }
-        __syncthreads();
-    }
-}
-
-// Partial sum of every piece (a block per piece, grid-stride over total[1] pieces).
-__global__ __launch_bounds__(kPieceThreads) void csr_piece_kernel(CsrView A,
-                                                                  const double *__restrict__ x,
-                                                                  LongWork w) {
-    const uint32_t nrows = w.total[0], npieces = w.total[1];
-    for (uint32_t p = blockIdx.x; p < npieces; p += gridDim.x) {
-        // the long row holding piece p: the last list entry whose first piece is <= p
-        uint32_t lo = 0, hi = nrows;
-        while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) / 2;
-            if (w.list[mid].y <= p) lo = mid;
-            else hi = mid;
-        }
-        const uint2 e = w.list[lo];
-        const uint64_t rb = A.row_idx[e.x], re = A.row_idx[e.x + 1];
-        const uint64_t b = rb + (uint64_t)(p - e.y) * kPiece;
-        const uint64_t end = std::min<uint64_t>(re, b + kPiece);
-        const double s = block_sum<kPieceThreads>(row_part(A, x, b + threadIdx.x, end, kPieceThreads));
-        if (threadIdx.x == 0) w.piece[p] = s;
-    }
-}
-
-// Every long row from its pieces in order; for a step, (y - x)^2 per block into
-// partials[first + block].
-template <bool STEP>
-__global__ __launch_bounds__(kFixThreads) void csr_long_fix_kernel(CsrView A,
+// Tile t: rows [i0, i1) end in it, with entries [k0, k1).
+template <typename Shape, bool STEP>
+__global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
                                                                    const double *__restrict__ x,
                                                                    double shift, double *y,
-                                                                   LongWork w, uint32_t first) {
-    const uint32_t nrows = w.total[0], npieces = w.total[1];
+                                                                   TileWork w, uint64_t tiles) {
+    constexpr uint32_t kThreads = Shape::kThreads, kPer = Shape::kPer, kItems = Shape::kItems;
+    static_assert(kItems < 65536, "ends are 16-bit offsets into the tile");
+    __shared__ double prod[kItems];
+    __shared__ uint16_t ends[kItems + 2];  // ends[j], ends[j + 1]: the tile's part of row i0 + j
+    __shared__ uint16_t longs[kItems / kTurns];
+    __shared__ uint32_t n_long;
+    __shared__ uint64_t s_row[2];
+    const uint32_t tid = threadIdx.x, wave = tid >> 6;
     double sq = 0.0;
-    for (uint32_t i = blockIdx.x * kFixThreads + threadIdx.x; i < nrows;
-         i += gridDim.x * kFixThreads) {
-        const uint2 e = w.list[i];
-        const uint32_t pend = i + 1 < nrows ? w.list[i + 1].y : npieces;
-        double s = 0.0;
-        for (uint32_t p = e.y; p < pend; ++p) s += w.piece[p];
-        const double v = s + shift;
-        y[e.x] = v;
+    for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
+        const uint64_t d0 = t * kItems;
+        const uint64_t d1 = min(d0 + kItems, A.rows + A.nnz);
+        if (wave < 2) {
+            const uint64_t i = rows_before(A, wave ? d1 : d0);
+            if ((tid & 63) == 0) s_row[wave] = i;
+        }
+        if (tid == 0) n_long = 0;
+        __syncthreads();
+        const uint64_t i0 = s_row[0], i1 = s_row[1], k0 = d0 - i0, k1 = d1 - i1;
+        const uint32_t cnt = (uint32_t)(k1 - k0), whole = (uint32_t)(i1 - i0);
+        // the entries, every load before the gathers that need it
+        const uint64_t *__restrict__ col = A.col_idx + k0;
+        const double *__restrict__ val = A.val + k0;
+        uint64_t c[kPer];
+        double v[kPer];
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t e = tid + k * kThreads;
+            c[k] = e < cnt ? __builtin_nontemporal_load(col + e) : 0;
+            v[k] = e < cnt ? __builtin_nontemporal_load(val + e) : 0.0;
+        }
+        for (uint32_t j = tid; j < whole; j += kThreads)
+            ends[j + 1] = (uint16_t)(A.row_idx[i0 + j + 1] - k0);
+        if (tid == 0) {
+            ends[0] = 0;
+            ends[whole + 1] = (uint16_t)cnt;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t e = tid + k * kThreads;
+            if (e < cnt) prod[e] = v[k] * x[c[k]];
+        }
+        __syncthreads();
+        // row i0 began in an earlier tile: its sum, and its square, are finished by the fix kernel
+        const bool continued = i0 < A.rows && A.row_idx[i0] < k0;
+        const uint32_t R = whole + 1;  // the last one: what is left after the last row end
+        const uint32_t tail = cnt - ends[whole];
+        auto put = [&](uint32_t r, double sum) {
+            if (r == whole) {
+                w.carry[t] = sum;
+                w.row[t] = tail ? (uint32_t)i1 : kNoRow;
+                return;
+            }
+            const double yr = sum + shift;
+            y[i0 + r] = yr;
+            if (STEP && !(r == 0 && continued)) {
+                const double d = yr - x[i0 + r];
+                sq += d * d;
+            }
+        };
+        // G consecutive lanes a row, G ~ the average length
+        const uint32_t avg = cnt / R;
+        const int lg = avg >= 64 ? 6 : (avg >= 32 ? 5 : (avg >= 16 ? 4 : (avg >= 8 ? 3 : (avg >= 4 ? 2 : (avg >= 2 ? 1 : 0)))));
+        const uint32_t G = 1u << lg, lane = tid & (G - 1), per_pass = kThreads >> lg;
+        for (uint32_t base = 0; base < R; base += per_pass) {
+            const uint32_t r = base + (tid >> lg);
+            double acc = 0.0;
+            bool own = r < R;
+            if (own) {
+                const uint32_t b = ends[r], e = ends[r + 1];
+                if (e - b > kTurns * G) {
+                    own = false;
+                    if (lane == 0) longs[atomicAdd(&n_long, 1u)] = (uint16_t)r;
+                } else {
+                    for (uint32_t i = b + lane; i < e; i += G) acc += prod[i];
+                }
+            }
+            for (uint32_t off = G >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+            if (own && lane == 0) put(r, acc);
+        }
+        __syncthreads();
+        const uint32_t nl = n_long;
+        for (uint32_t k = wave; k < nl; k += kThreads / 64) {
+            const uint32_t r = longs[k];
+            double acc = 0.0;
+            for (uint32_t i = ends[r] + (tid & 63); i < ends[r + 1]; i += 64) acc += prod[i];
+            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+            if ((tid & 63) == 0) put(r, acc);
+        }
+        __syncthreads();  // the next tile rewrites the shared arrays
+    }
+    if (STEP) {
+        const double tot = block_sum<kThreads>(sq);
+        if (tid == 0) w.partials[blockIdx.x] = tot;
+    }
+}
+
+// The carries: the first of a run of tiles with the same carry row adds the run's carries, in tile
+// order, to that row.  For a step the squares of the rows finished here, after the first n_sq block
+// sums of the tile kernel, go to out[blockIdx.x].
+template <bool STEP>
+__global__ __launch_bounds__(kFixThreads) void csr_fix_kernel(const double *__restrict__ x, double *y,
+                                                              TileWork w, uint64_t tiles,
+                                                              uint32_t n_sq, double *out) {
+    double sq = 0.0;
+    for (uint32_t b = threadIdx.x; STEP && b < n_sq; b += kFixThreads) sq += w.partials[b];
+    for (uint64_t t = (uint64_t)blockIdx.x * kFixThreads + threadIdx.x; t < tiles;
+         t += (uint64_t)gridDim.x * kFixThreads) {
+        const uint32_t r = w.row[t];
+        if (r == kNoRow || (t > 0 && w.row[t - 1] == r)) continue;
+        double s = w.carry[t];
+        for (uint64_t q = t + 1; q < tiles && w.row[q] == r; ++q) s += w.carry[q];
+        const double v = s + y[r];
+        y[r] = v;
         if (STEP) {
-            const double d = v - x[e.x];
+            const double d = v - x[r];
             sq += d * d;
         }
     }
     if (STEP) {
         const double tot = block_sum<kFixThreads>(sq);
-        if (threadIdx.x == 0) w.partials[first + blockIdx.x] = tot;
+        if (threadIdx.x == 0) out[blockIdx.x] = tot;
     }
 }
 
@@ -393,33 +331,6 @@ __global__ void csr_check_kernel(CsrView A, uint64_t cols, uint64_t nnz, uint32_
     if (bad) atomicOr(flag, 1u);
 }
 
-// Lanes per row from the average row length.
-uint32_t lanes_for(uint64_t rows, uint64_t nnz) {
-    const double avg = rows ? (double)nnz / (double)rows : 0.0;
-    if (avg <= 6.0) return 4;
-    if (avg <= 12.0) return 8;
-    if (avg <= 24.0) return 16;
-    if (avg <= 48.0) return 32;
-    return 64;
-}
-
-uint32_t short_grid(uint64_t rows, uint32_t lanes) {
-    const uint64_t tiles = (rows + kShortThreads / lanes - 1) / (kShortThreads / lanes);
-    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(tiles, kShortGrid));
-}
-
-uint32_t long_grid(uint64_t rows) {
-    const uint64_t chunks = (rows + kLongThreads - 1) / kLongThreads;
-    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(chunks, kLongGrid));
-}
-
-// Upper bounds of the long-row list and of the pieces of a matrix with this shape.
-void long_caps(uint64_t rows, uint64_t nnz, uint64_t &list_cap, uint64_t &piece_cap) {
-    const uint64_t lim = 32ull * lanes_for(rows, nnz);
-    list_cap = std::min<uint64_t>(rows, nnz / (lim + 1)) + 1;
-    piece_cap = nnz / kPiece + list_cap + 1;
-}
-
 CsrView view_of(const nkpr_csr *a) {
     NKPR_CHECK(a != nullptr, "matrix is NULL");
     NKPR_CHECK(a->rows == 0 || (a->row_idx && a->col_idx && a->values),
@@ -427,6 +338,7 @@ CsrView view_of(const nkpr_csr *a) {
     NKPR_CHECK(a->rows < 0xFFFFFFFFull, "more than 2^32 - 2 rows");
     CsrView v;
     v.rows = a->rows;
+    v.nnz = a->nnz;
     v.row_idx = a->row_idx;
     v.col_idx = a->col_idx;
     v.val = a->values;
@@ -435,38 +347,32 @@ CsrView view_of(const nkpr_csr *a) {
 
 // The product kernels (and, for a step, the final sum of their block sums into *sq_out).
 template <bool STEP>
-void launch_product(const CsrView &A, uint64_t nnz, const double *x, double shift, double *y,
-                    const LongWork &w, double *sq_out, hipStream_t s) {
+void launch_product(const CsrView &A, const double *x, double shift, double *y, const TileWork &w,
+                    double *sq_out, hipStream_t s) {
     if (A.rows == 0) {
         if (STEP) hipLaunchKernelGGL(csr_fill_kernel, dim3(1), dim3(64), 0, s, sq_out, 1, 0.0);
         return;
     }
-    const uint32_t lanes = lanes_for(A.rows, nnz);
-    const uint32_t gs = short_grid(A.rows, lanes);
-    const uint64_t tiles = (A.rows + kShortThreads / lanes - 1) / (kShortThreads / lanes);
-    switch (lanes) {
-    case 4: hipLaunchKernelGGL((csr_short_kernel<4, STEP>), dim3(gs), dim3(kShortThreads), 0, s, A, x, shift, y, w.partials, tiles); break;
-    case 8: hipLaunchKernelGGL((csr_short_kernel<8, STEP>), dim3(gs), dim3(kShortThreads), 0, s, A, x, shift, y, w.partials, tiles); break;
-    case 16: hipLaunchKernelGGL((csr_short_kernel<16, STEP>), dim3(gs), dim3(kShortThreads), 0, s, A, x, shift, y, w.partials, tiles); break;
-    case 32: hipLaunchKernelGGL((csr_short_kernel<32, STEP>), dim3(gs), dim3(kShortThreads), 0, s, A, x, shift, y, w.partials, tiles); break;
-    default: hipLaunchKernelGGL((csr_short_kernel<64, STEP>), dim3(gs), dim3(kShortThreads), 0, s, A, x, shift, y, w.partials, tiles); break;
+    const uint64_t tiles = tiles_of(A);
+    const uint32_t grid = tile_grid(tiles);
+    if (small_matrix(A))
+        hipLaunchKernelGGL((csr_tile_kernel<SmallTile, STEP>), dim3(grid), dim3(SmallTile::kThreads), 0, s, A, x,
+                           shift, y, w, tiles);
+    else
+        hipLaunchKernelGGL((csr_tile_kernel<LargeTile, STEP>), dim3(grid), dim3(LargeTile::kThreads), 0, s, A, x,
+                           shift, y, w, tiles);
+    NKPR_HIP(hipGetLastError());
+    if (tiles <= kFixAlone) {
+        hipLaunchKernelGGL((csr_fix_kernel<STEP>), dim3(1), dim3(kFixThreads), 0, s, x, y, w, tiles, grid, sq_out);
+    } else {
+        // (more tiles than kFixAlone: the tile kernel ran on kTileGrid blocks)
+        hipLaunchKernelGGL((csr_fix_kernel<STEP>), dim3(kFixGrid), dim3(kFixThreads), 0, s, x, y, w, tiles, 0u,
+                           w.partials + kTileGrid);
+        if (STEP)
+            hipLaunchKernelGGL(csr_final_kernel, dim3(1), dim3(kFinalThreads), 0, s, w.partials,
+                               kTileGrid + kFixGrid, sq_out);
     }
     NKPR_HIP(hipGetLastError());
-    const uint64_t lim = 32ull * lanes;
-    const uint32_t gl = long_grid(A.rows);
-    const uint64_t rpb = (A.rows + gl - 1) / gl;
-    hipLaunchKernelGGL(csr_long_scan_kernel, dim3(gl), dim3(kLongThreads), 0, s, A, rpb, lim, w);
-    hipLaunchKernelGGL(csr_long_offsets_kernel, dim3(1), dim3(64), 0, s, w, gl);
-    hipLaunchKernelGGL(csr_long_list_kernel, dim3(gl), dim3(kLongThreads), 0, s, A, rpb, lim, w);
-    hipLaunchKernelGGL(csr_piece_kernel, dim3(kPieceGrid), dim3(kPieceThreads), 0, s, A, x, w);
-    hipLaunchKernelGGL((csr_long_fix_kernel<STEP>), dim3(kFixGrid), dim3(kFixThreads), 0, s, A, x,
-                       shift, y, w, gs);
-    NKPR_HIP(hipGetLastError());
-    if (STEP) {
-        hipLaunchKernelGGL(csr_final_kernel, dim3(1), dim3(kFinalThreads), 0, s, w.partials,
-                           gs + kFixGrid, sq_out);
-        NKPR_HIP(hipGetLastError());
-    }
 }
 
 // Device scratch of one call, taken from the stream's memory pool.
@@ -511,10 +417,9 @@ void csr_spmv_impl(const nkpr_csr *a, const double *x, double *y, hipStream_t s)
     NKPR_CHECK(A.rows == 0 || (x && y), "x and y must not be NULL");
     NKPR_CHECK(x != y || A.rows == 0, "x and y must be different vectors");
     if (A.rows == 0) return;
-    uint64_t lc, pc;
-    long_caps(A.rows, a->nnz, lc, pc);
-    PoolBuf buf(work_bytes(lc, pc), s);
-    launch_product<false>(A, a->nnz, x, 0.0, y, carve(buf.p, lc, pc), nullptr, s);
+    const uint64_t tiles = tiles_of(A);
+    PoolBuf buf(work_bytes(tiles), s);
+    launch_product<false>(A, x, 0.0, y, carve(buf.p, tiles), nullptr, s);
 }
 
 void csr_step_impl(const nkpr_csr *m, double shift, const double *x, double *y, double *step_sq,
@@ -524,32 +429,36 @@ void csr_step_impl(const nkpr_csr *m, double shift, const double *x, double *y, 
     NKPR_CHECK(step_sq != nullptr, "step_sq must not be NULL");
     NKPR_CHECK(A.rows == 0 || (x && y), "x and y must not be NULL");
     NKPR_CHECK(x != y || A.rows == 0, "x and y must be different vectors");
-    uint64_t lc, pc;
-    long_caps(A.rows, m->nnz, lc, pc);
-    PoolBuf buf(work_bytes(lc, pc), s);
-    launch_product<true>(A, m->nnz, x, shift, y, carve(buf.p, lc, pc), step_sq, s);
+    const uint64_t tiles = tiles_of(A);
+    PoolBuf buf(work_bytes(tiles), s);
+    launch_product<true>(A, x, shift, y, carve(buf.p, tiles), step_sq, s);
 }
 
 void csr_step_noalloc_impl(const nkpr_csr *m, double shift, const double *x, double *y,
                            double *step_sq, hipStream_t s) {
-    static_assert(sizeof(scratch) >= 8 * (size_t)kNoallocList + 8 * (size_t)kNoallocPieces +
-                                          4 * (4 * (size_t)kLongGrid + 4) +
-                                          8 * (size_t)(kShortGrid + kFixGrid) + 256,
-                  "the scratch holds the capped work");
     const CsrView A = view_of(m);
     NKPR_CHECK(m->rows == m->cols, "a PageRank step needs a square matrix");
     NKPR_CHECK(step_sq != nullptr, "step_sq must not be NULL");
     NKPR_CHECK(A.rows == 0 || (x && y), "x and y must not be NULL");
     NKPR_CHECK(x != y || A.rows == 0, "x and y must be different vectors");
-    uint64_t lc, pc;
-    long_caps(A.rows, m->nnz, lc, pc);
+    // what this entry point accepts: at most 2^21 rows longer than 32 x the lanes that rows of
+    // the average length take, and 2^22 pieces of 4096 entries, by the worst-case bounds
+    const double avg = A.rows ? (double)A.nnz / (double)A.rows : 0.0;
+    const uint64_t lanes = avg <= 6.0 ? 4 : (avg <= 12.0 ? 8 : (avg <= 24.0 ? 16 : (avg <= 48.0 ? 32 : 64)));
+    const uint64_t lc = std::min<uint64_t>(A.rows, A.nnz / (32 * lanes + 1)) + 1;
+    const uint64_t pc = A.nnz / kNoallocPiece + lc + 1;
     NKPR_CHECK(lc <= kNoallocList && pc <= kNoallocPieces,
                "matrix too large for the allocation-free step: it could have more than 2^21 rows "
                "longer than 32 x the lanes per row, or 2^22 pieces of 4096 entries (at most "
                "nnz / (32 lanes + 1) such rows: up to about 2.7e8 entries at an average row "
                "length of 6 or less, 1.07e9 at 24 or less, 4.3e9 above 48)");
-    launch_product<true>(A, m->nnz, x, shift, y, carve(csr_noalloc_scratch(), kNoallocList,
-                                                       kNoallocPieces), step_sq, s);
+    // rows / 4096 is below lc wherever nnz / 4096 is near the cap, so no such matrix has more than
+    // 2^22 tiles
+    static_assert(sizeof(scratch) >= 12 * (size_t)kNoallocPieces + 8 * (size_t)(kTileGrid + kFixGrid),
+                  "the scratch holds the carries of 2^22 tiles");
+    const uint64_t tiles = tiles_of(A);
+    NKPR_CHECK(tiles <= kNoallocPieces, "matrix too large for the allocation-free step");
+    launch_product<true>(A, x, shift, y, carve(csr_noalloc_scratch(), tiles), step_sq, s);
 }
 
 void csr_validate(const nkpr_csr *m, hipStream_t s) {
@@ -576,14 +485,12 @@ void algebraic_pagerank_impl(const nkpr_csr *m, double damp, double tol, uint64_
     NKPR_CHECK(damp >= 0.0 && damp <= 1.0, "damp must lie in [0, 1]");
     NKPR_CHECK(tol >= 0.0, "tol must be >= 0");
     NKPR_CHECK(max_iterations >= 1, "max_iterations must be >= 1");
-    const uint64_t n = A.rows, nnz = m->nnz;
-    uint64_t lc, pc;
-    long_caps(n, nnz, lc, pc);
+    const uint64_t n = A.rows, nnz = m->nnz, tiles = tiles_of(A);
     // buffers first: the stream owner below is destroyed (and synchronised) before them
     DevBuf xa, xb, work, out, flag;
     xa.alloc(8 * n);
     xb.alloc(8 * n);
-    work.alloc(std::max<size_t>(work_bytes(lc, pc), 8 * 1024));
+    work.alloc(std::max<size_t>(work_bytes(tiles), 8 * 1024));
     out.alloc(16);
     flag.alloc(4);
     hipStream_t s;
@@ -606,7 +513,7 @@ void algebraic_pagerank_impl(const nkpr_csr *m, double damp, double tol, uint64_
     read_back(s, {{&bad, flag.p, 4}, {&last, A.row_idx + n, 8}});
     NKPR_CHECK(bad == 0 && last == nnz,
                "malformed CSR matrix (row_idx must rise from 0 to nnz, column indices < cols)");
-    const LongWork w = carve(work.p, lc, pc);
+    const TileWork w = carve(work.p, tiles);
     const double tele = (1.0 - damp) / (double)n;
     hipLaunchKernelGGL(csr_fill_kernel, dim3(1024), dim3(256), 0, s, xa.as<double>(), n,
                        1.0 / (double)n);
@@ -615,13 +522,13 @@ void algebraic_pagerank_impl(const nkpr_csr *m, double damp, double tol, uint64_
     uint64_t it = 0;
     double sq = 0.0;
     do {
-        launch_product<true>(A, nnz, cur, tele, nxt, w, out.as<double>(), s);
+        launch_product<true>(A, cur, tele, nxt, w, out.as<double>(), s);
         read_back(s, {{&sq, out.p, 8}});
         std::swap(cur, nxt);
         ++it;
     } while (std::sqrt(sq) > tol && it < max_iterations);
-    hipLaunchKernelGGL(csr_sum_kernel, dim3(1024), dim3(kFinalThreads), 0, s, cur, n, w.partials);
-    hipLaunchKernelGGL(csr_final_kernel, dim3(1), dim3(kFinalThreads), 0, s, w.partials, 1024u,
+    hipLaunchKernelGGL(csr_sum_kernel, dim3(1024), dim3(kFinalThreads), 0, s, cur, n, work.as<double>());
+    hipLaunchKernelGGL(csr_final_kernel, dim3(1), dim3(kFinalThreads), 0, s, work.as<double>(), 1024u,
                        out.as<double>());
     hipLaunchKernelGGL(csr_scale_kernel, dim3(1024), dim3(256), 0, s, cur, n, out.as<double>());
     NKPR_HIP(hipGetLastError());

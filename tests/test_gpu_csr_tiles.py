@@ -1,0 +1,81 @@
+"""CSR products at the edges of their tiles, against the oracle and plain FP64 sums.
+
+The kernel cuts the merged list of row ends and entries into tiles (1024 merged items below 2^22 of
+them, 4096 from there on): rows that end on a tile's edge, rows over several tiles, tiles of empty
+rows, one row in all, and more tiles than one block of the last kernel takes.  A sum of t terms in
+any order differs by at most about t 2^-53 sum|terms|; 1e-13 covers the rows up to 1000 terms, the
+longer ones (random signs off: all terms positive) are held to 1e-12 relative.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from networkit_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def csr_of(lengths, cols, seed):
+    rng = np.random.default_rng(seed)
+    ptr = np.zeros(len(lengths) + 1, np.uint64)
+    ptr[1:] = np.cumsum(np.asarray(lengths, np.int64))
+    nnz = int(ptr[-1])
+    return oracle.CSR(len(lengths), cols, ptr, rng.integers(0, cols, nnz).astype(np.uint64),
+                      rng.uniform(0.1, 1.0, nnz))
+
+
+LENGTHS = {
+    "one row": [5000],
+    "one long row among empty ones": [0] * 1500 + [9000] + [0] * 1500,
+    "all empty but one": [0] * 3000 + [1] + [0] * 3000,
+    "ends on tile edges": [1023, 1023, 1022, 1, 0, 1023, 2047, 511, 511],
+    "a row of one tile and of several": [1024, 4096, 1, 3 * 1024 - 1, 7],
+    "around a wave's rows": [31, 32, 33, 63, 64, 65, 127, 128, 129, 2048, 2049] * 9,
+    "short rows": [1] * 5000 + [2] * 5000,
+}
+
+
+@pytest.mark.parametrize("name", sorted(LENGTHS))
+def test_products_at_tile_edges(name):
+    import torch
+    lengths = LENGTHS[name]
+    n = len(lengths)
+    a = csr_of(lengths, n, 3)
+    x = np.random.default_rng(4).random(n)
+    ref = oracle.csr_spmv(a, x)
+    d = capi.DeviceCSR(a.rows, a.cols, a.row_idx, a.col_idx, a.values)
+    xd = torch.from_numpy(x).cuda()
+    np.testing.assert_allclose(d.spmv(xd).cpu().numpy(), ref, rtol=1e-12, atol=0)
+    y, sq = d.pagerank_step(xd, 0.25)
+    np.testing.assert_allclose(y.cpu().numpy(), ref + 0.25, rtol=1e-12, atol=0)
+    assert float(sq) == pytest.approx(float(((ref + 0.25 - x) ** 2).sum()), rel=1e-12)
+    y2, sq2 = torch.empty_like(y), torch.empty_like(sq)
+    d.pagerank_step_noalloc(xd, 0.25, y2, sq2)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(sq, sq2)
+
+
+@pytest.mark.parametrize("rows,length", [(300000, 15), (1100000, 3), (1000, 70000), (1, 5000000)])
+def test_large_tiles(rows, length):
+    """Equal rows (so that torch can add them): 4096-item tiles; 70,000,000 entries take the fix
+    kernel's many blocks."""
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    nnz = rows * length
+    col = torch.randint(rows, (nnz,), generator=g, device="cuda")
+    val = torch.rand(nnz, generator=g, device="cuda", dtype=torch.float64)
+    x = torch.rand(rows, generator=g, device="cuda", dtype=torch.float64)
+    d = capi.DeviceCSR(rows, rows, torch.arange(rows + 1, device="cuda") * length, col, val)
+    ref = (val * x[col]).reshape(rows, length).sum(1)
+    y, sq = d.pagerank_step(x, 0.5)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(y, ref + 0.5, rtol=1e-12, atol=0)
+    want = float((ref + 0.5 - x).square().sum())
+    assert float(sq) == pytest.approx(want, rel=1e-12)
+    z = d.spmv(x)
+    torch.cuda.synchronize()
+    torch.testing.assert_close(z, ref, rtol=1e-12, atol=0)
+    # every run adds in the same order
+    y2, sq2 = d.pagerank_step(x, 0.5)
+    torch.cuda.synchronize()
+    assert torch.equal(y, y2) and torch.equal(sq, sq2)
