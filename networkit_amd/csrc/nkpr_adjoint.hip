@@ -347,8 +347,7 @@ void adjoint_impl(nkpr_graph *g, const nkpr_params *p, const nkpr_csc *csc,
     int cus = 0;
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, a->device));
     RunCtx rc{a, &pa, st, pa.max_iterations, {}, 0};
-    rc.combine_grid = (int)std::min<uint64_t>(((uint64_t)a->n_s + kCombineThreads - 1) / kCombineThreads,
-                                              (uint64_t)std::max(cus, 1) * 8);
+    rc.combine_grid = combine_blocks(a, cus);
     const bool timing = p->timing != 0;
     Krylov kr = krylov_setup(a);
     a->op_pending = false;
@@ -387,7 +386,7 @@ void adjoint_impl(nkpr_graph *g, const nkpr_params *p, const nkpr_csc *csc,
         launch_copy_f32(a->base32.as<float>(), r, n, s);
         auto norm2 = [&](const float *v) {
             double h = 0.0;
-            launch_multidot(v, v, kr.ld, 1, n, kr.dpart, kr.dout, s);
+            launch_multidot(v, v, kr.ld, 1, n, kr.dpart, kr.dout, nullptr, s);
             read_back(s, {{&h, kr.dout, 8}});
             return std::sqrt(h);
         };

@@ -145,8 +145,7 @@ void algebraic_run_impl(nkpr_algebraic *h, double damp, double tol, uint64_t max
     pp.max_iterations = max_iterations;
     nkpr_stats st{};
     RunCtx rc{g, &pp, &st, max_iterations, {}, 0};
-    rc.combine_grid = (int)std::min<uint64_t>(((uint64_t)g->n_s + kCombineThreads - 1) / kCombineThreads,
-                                              (uint64_t)std::max(cus, 1) * 8);
+    rc.combine_grid = combine_blocks(g, cus);
     double *x0 = g->x64a.as<double>(), *x1 = g->x64b.as<double>();
     // the start 1/n is the same in every order
     hipLaunchKernelGGL(alg_fill_kernel, dim3(grid_for_n(n)), dim3(256), 0, s, x0, (uint64_t)n,

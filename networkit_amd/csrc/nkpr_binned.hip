@@ -1597,7 +1597,7 @@ void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArg
     FinalizeArgs ff = f;
     ff.n_split_rows = 0;
     ff.n_blocks = n ? L.nslots : 0;
-    launch_finalize64(fa, ff, kind, s);
+    launch_finalize64(fa, ff, s);
     if (ev1) NKPR_HIP(hipEventRecord(ev1, s));
     NKPR_HIP(hipGetLastError());
 }

@@ -120,8 +120,7 @@ SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64
     int cus = 0;
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
     RunCtx rc{g, p, st, max_it, {}, 0};
-    rc.combine_grid = (int)std::min<uint64_t>(((uint64_t)g->n_s + kCombineThreads - 1) / kCombineThreads,
-                                              (uint64_t)std::max(cus, 1) * 8);
+    rc.combine_grid = combine_blocks(g, cus);
     const bool dist = p->sink_handling == NKPR_SINK_DISTRIBUTE;
     PhaseCtl *ctl = g->ctl.as<PhaseCtl>();
     const int kind_plain = has_base ? kSweepBaseVec : kSweepPlain;
@@ -283,7 +282,7 @@ SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64
                 FinalizeArgs ff{};
                 ff.n_blocks = blocks;
                 ff.rule = rr;
-                launch_finalize64(fa, ff, kind_resid, s);
+                launch_finalize64(fa, ff, s);
                 read_back(s, {{g->ctl_host, g->ctl.p, sizeof(PhaseCtl)}});
             } else {
                 if (!folded) launch_prescale(xcur, g->inv64.as<double>(), xh, nullptr, nullptr, nullptr, n, g->sink_begin, s);
@@ -423,14 +422,7 @@ void apply_operator(RunCtx &rc, const float *v, float *w, const Krylov &kr, bool
     a.sink_begin = g->sink_begin;
     a.distribute = dist ? 1 : 0;
     // the sweep writes B v to kr.y (A v follows) or straight to w
-    Vecs<float> vv{{const_cast<float *>(v), minus ? kr.y : w}, {kr.vh, kr.yh}};
-    PhaseRule r{};
-    r.kind = kRuleStep;
-    r.norm = NKPR_L1;
-    r.tol = -1.0;
-    r.max_iterations = 1;
-    r.damp = rc.p->damp;
-    run_phase<float>(rc, a, vv, kSweepPlain, r, 1, timing, ms_acc);
+    launch_product(rc, a, folded ? v : kr.vh, v, minus ? kr.y : w, nullptr, timing, ms_acc);
     if (minus) launch_axpby(v, kr.y, w, n, 1.0f, -1.0f, s);
 }
 

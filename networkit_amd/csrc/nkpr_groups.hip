@@ -23,7 +23,14 @@
 namespace nkpr {
 namespace {
 
-constexpr uint32_t kChunkNodes = 16384;
+// Nodes per chunk: a block each, so small unions take small chunks (a union of 1.3e6 nodes in
+// chunks of 16384 kept 200 blocks busy for 18 us).
+constexpr uint32_t kChunkNodesMin = 2048, kChunkNodesMax = 16384;
+uint32_t chunk_nodes(uint32_t n) {
+    uint32_t c = kChunkNodesMin;
+    while (c < kChunkNodesMax && (uint64_t)c * 2048 < n) c *= 2;
+    return c;
+}
 constexpr int kRedThreads = 256;
 
 struct Chunk {
@@ -77,8 +84,10 @@ __global__ __launch_bounds__(kRedThreads) void group_reduce_kernel(
     }
 }
 
-// One block: every graph adds its chunk partials in order and applies the rule; the next
-// right-hand side per graph; all graphs done -> the phase stops.
+// One block: every graph adds its chunk partials in a fixed order (kRuleLanes lanes strided over
+// them, then a shuffle tree) and applies the rule; the next right-hand side per graph; all graphs
+// done -> the phase stops.
+constexpr uint32_t kRuleLanes = 8;
 __global__ __launch_bounds__(1024) void group_rule_kernel(
     const uint32_t *cfirst, const uint32_t *gn, uint32_t groups, const double *part,
     GroupCtl *gc, double *add, PhaseRule r, int dist, int base_only, PhaseCtl *ctl,
@@ -88,13 +97,19 @@ __global__ __launch_bounds__(1024) void group_rule_kernel(
     if (threadIdx.x == 0) s_active = 0;
     __syncthreads();
     uint32_t active = 0;
-    for (uint32_t q = threadIdx.x; q < groups; q += blockDim.x) {
+    const uint32_t lane = threadIdx.x % kRuleLanes;
+    for (uint32_t q = threadIdx.x / kRuleLanes; q < groups; q += blockDim.x / kRuleLanes) {
         GroupCtl &g = gc[q];
         const double nq = (double)gn[q];
+        const uint32_t c0 = cfirst[q], c1 = cfirst[q + 1];
         if (g.done || gn[q] == 0) continue;
         double t[4] = {0.0, 0.0, 0.0, 0.0};
-        for (uint32_t c = cfirst[q]; c < cfirst[q + 1]; ++c)
+        for (uint32_t c = c0 + lane; c < c1; c += kRuleLanes)
             for (int k = 0; k < 4; ++k) t[k] += part[(size_t)c * 4 + k];
+#pragma unroll
+        for (uint32_t off = kRuleLanes / 2; off > 0; off >>= 1)
+            for (int k = 0; k < 4; ++k) t[k] += __shfl_xor(t[k], off, kRuleLanes);
+        if (lane != 0) continue;
         if (!base_only) {
             const uint64_t it = g.iterations + 1;
             g.iterations = it;
@@ -282,12 +297,13 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
     // ---- chunks and per-graph tables ------------------------------------------------------
     if (!g->q_nchunks && n) {
         std::vector<Chunk> ch;
+        const uint32_t per = chunk_nodes(n);
         std::vector<uint32_t> cfirst(G + 1, 0), gn(G, 0);
         for (uint32_t q = 0; q < G; ++q) {
             cfirst[q] = (uint32_t)ch.size();
             gn[q] = g->goff[q + 1] - g->goff[q];
-            for (uint32_t b = g->goff[q]; b < g->goff[q + 1]; b += kChunkNodes)
-                ch.push_back({b, std::min(b + kChunkNodes, g->goff[q + 1]), q, g->gsink[q]});
+            for (uint32_t b = g->goff[q]; b < g->goff[q + 1]; b += per)
+                ch.push_back({b, std::min(b + per, g->goff[q + 1]), q, g->gsink[q]});
         }
         cfirst[G] = (uint32_t)ch.size();
         g->q_nchunks = (uint32_t)ch.size();
@@ -333,8 +349,7 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
         int cus = 0;
         NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, g->device));
         RunCtx rc{g, p, st, p->max_iterations, {}, 0};
-        rc.combine_grid = (int)std::min<uint64_t>(((uint64_t)g->n_s + kCombineThreads - 1) / kCombineThreads,
-                                                  (uint64_t)std::max(cus, 1) * 8);
+        rc.combine_grid = combine_blocks(g, cus);
         const bool folded = g->weighted;
         const bool timing = p->timing != 0;
         const uint64_t max_it = std::max<uint64_t>(p->max_iterations, 1);
@@ -424,8 +439,7 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
                     SweepArgs<float> a = args32();
                     a.base_vec = nullptr;
                     a.tele = 0.0;
-                    Vecs<float> vv{{const_cast<float *>(v), dist ? kr.y : w}, {kr.vh, kr.yh}};
-                    run_phase<float>(rc, a, vv, kSweepPlain, counting_rule(1), 1, timing, &st->ms_sweeps_fp32);
+                    launch_product(rc, a, folded ? v : kr.vh, v, dist ? kr.y : w, nullptr, timing, &st->ms_sweeps_fp32);
                 }
                 if (dist) {
                     PhaseRule r0{};

@@ -35,15 +35,23 @@ namespace nkpr {
 constexpr int kBlock = 512;
 constexpr int kCap = 4096;
 constexpr int kRowsMax = 512;
+constexpr uint32_t kCapMin = 512;         // in-edges of an item on graphs with few of them
+constexpr uint32_t kItemsWanted = 512;    // items that fill the 256 CUs twice
 constexpr uint32_t kVectorMax = 16384;
 constexpr uint32_t kChunk = 8192;
 constexpr uint32_t kSplitFlag = 0x80000000u;
 constexpr int kFinalizeThreads = 1024;
 constexpr int kSlices = 8;
+constexpr uint32_t kXcds = 8;
 constexpr int kSliceShift = 5;
 constexpr uint32_t kDefaultDirectMaxDeg = 8;
 constexpr uint32_t kDefaultSliceReplicate = 32768;  // top-ranked sources cached by every XCD
 constexpr int kCombineThreads = 256;
+// Counters of the blocks that have ended a launch: one on top, kArriveGroups below it, each on a
+// line of its own (kArriveStride words), behind the kSlices claim counters.
+constexpr uint32_t kArriveGroups = 32, kArriveStride = 32;
+constexpr uint32_t kArriveWords = kArriveStride * (1 + kArriveGroups);
+constexpr uint32_t kArriveAt = kArriveStride;  // words from the claim counters to the first one
 // The most gathered sources (relabelled ids [0, hub count)) are copied into LDS by every sweep
 // block: an LDS gather costs a fraction of an L2 hit.  32 KiB of FP32 values, 8 KiB of FP64.
 template <typename T> struct HubTable { static constexpr uint32_t size = 8192; };
@@ -168,6 +176,7 @@ struct Schedule {
     const uint32_t *dptr;        // [n_d + 1] absolute in-edge offsets
     const uint4 *ditems;         // {k0, k1, e0, cnt} over direct index k
     uint32_t n_d, n_ditems;
+    uint32_t local;              // 1: rows gather from entries near their own (a batch's graphs)
     // sliced rows: per-slice partial sums, epilogue in the combine kernel
     const uint32_t *srow;        // [n_s] row ids
     const uint32_t *sptr;        // [n_slices * n_s + 1] slice-major in-edge offsets
@@ -176,6 +185,7 @@ struct Schedule {
     uint32_t n_s;
     const uint8_t *split_flag;   // [n_s] 1: the finalize kernel finishes this row
     uint32_t *claim;             // [kSlices] worker claim counters (reset every sweep)
+    uint32_t *arrive;            // [kArriveWords] counters of the blocks that have ended
     uint32_t workers;            // workers per slice; the sweep grid is n_slices * workers
 };
 
@@ -212,7 +222,7 @@ struct FinalizeArgs {
     const uint32_t *split_first;  // [n_split_rows * n_slices] first chunk (count 0: partial)
     const uint32_t *split_count;  // [n_split_rows * n_slices]
     uint32_t n_split_rows;
-    uint32_t n_blocks;            // sweep grid + combine grid
+    uint32_t n_blocks;            // sweep grid + combine grid; 0: no reductions and no rule
     PhaseRule rule;
 };
 
@@ -224,7 +234,8 @@ enum SweepKind : int {
     kSweepBaseResid = 3,  // base vector + r32  (FP64 only)
 };
 
-// sweep (grid = n_slices * workers) + combine (combine_grid blocks, if n_s > 0) + finalize
+// sweep (grid = n_slices * workers) + combine (combine_grid >= 1 blocks, if n_s > 0); the last
+// block of the last launch applies the stopping rule
 template <typename T>
 void launch_sweep(const SweepArgs<T> &a, const FinalizeArgs &f, int kind, bool folded,
                   int combine_grid, hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
@@ -272,8 +283,8 @@ void launch_init_ctl(PhaseCtl *ctl, const double *sink_sum, uint32_t *claim, hip
 // FP32 Krylov vector kernels (nkpr_krylov.hip).  V holds vectors of length n at stride ld (a
 // multiple of 4 floats; every vector 16-byte aligned).
 constexpr int kDotGroup = 24;   // vectors per launch
-constexpr int kDotStride = 32;  // doubles per block in the partials buffer (>= kDotGroup + 1)
-constexpr int kDotPartials = kDotStride * 1024;
+constexpr int kDotBlocks = 1024;  // blocks of a multi-dot, at most
+constexpr int kDotPartials = (kDotGroup + 1) * kDotBlocks;  // a row of block sums for every dot
 struct Coefs {
     float c[kDotGroup];
 };
@@ -281,9 +292,10 @@ constexpr int kMaxKrylov = 64;  // largest GMRES restart length
 struct Scales {
     double s[kMaxKrylov];
 };
-// out[i] = <w, V[i]> (FP64 accumulation) for i < count; partials: kDotPartials doubles
+// out[i] = <w, V[i]> (FP64 accumulation) for i < count; partials: kDotPartials doubles.  `host`
+// (pinned, or nullptr) receives the results too, without a copy of its own.
 void launch_multidot(const float *w, const float *V, uint64_t ld, uint32_t count, uint32_t n,
-                     double *partials, double *out, hipStream_t s);
+                     double *partials, double *out, double *host, hipStream_t s);
 // assign: w = sum_i coef[i] V[i];  otherwise w -= sum_i coef[i] V[i]
 void launch_multiaxpy(float *w, const float *V, uint64_t ld, uint32_t count, uint32_t n,
                       const double *coef, bool assign, hipStream_t s);
@@ -293,7 +305,8 @@ void launch_gs_project(float *w, const float *V, uint64_t ld, uint32_t count, ui
                        const double *d, const double *sig, hipStream_t s);
 // w -= sum_i coef[i] V[i], then out[i] = <V[i], w> for i < count and out[count] = <w, w>
 void launch_axpy_dot(float *w, const float *V, uint64_t ld, uint32_t count, uint32_t n,
-                     const double *coef, double *partials, double *out, hipStream_t s);
+                     const double *coef, double *partials, double *out, double *host,
+                     hipStream_t s);
 // out = a x + b y  (y may be nullptr)
 void launch_axpby(const float *x, const float *y, float *out, uint32_t n, float a, float b,
                   hipStream_t s);
@@ -337,7 +350,7 @@ const int32_t *slot_index(nkpr_graph *g);
 void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArgs &f, int kind,
                     hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
 // The finalize step of launch_sweep<double> alone (nkpr_sweep.hip).
-void launch_finalize64(const SweepArgs<double> &a, const FinalizeArgs &f, int kind, hipStream_t s);
+void launch_finalize64(const SweepArgs<double> &a, const FinalizeArgs &f, hipStream_t s);
 void set_weights(nkpr_graph *g, const float *w, const double *w64, const double *out_wdeg,
                  int device_ptrs);
 void adjoint_impl(nkpr_graph *g, const nkpr_params *p, const nkpr_csc *csc,

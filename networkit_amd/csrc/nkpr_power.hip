@@ -179,8 +179,7 @@ void power_run_impl(nkpr_graph *g, const nkpr_power_params *p, double *scores, n
         pp.interrupt = p->interrupt;
         pp.max_iterations = p->max_iterations;
         RunCtx rc{g, &pp, st, p->max_iterations, {}, 0};
-        rc.combine_grid = (int)std::min<uint64_t>(((uint64_t)g->n_s + kCombineThreads - 1) / kCombineThreads,
-                                                  (uint64_t)std::max(cus, 1) * 8);
+        rc.combine_grid = combine_blocks(g, cus);
         double *x0 = g->x64a.as<double>(), *x1 = g->x64b.as<double>();
         double *xh0 = folded ? nullptr : g->xh64a.as<double>();
         double *xh1 = folded ? nullptr : g->xh64b.as<double>();

@@ -24,6 +24,10 @@ template <typename T> struct Vecs {
 };
 
 inline void ensure(DevBuf &b, size_t bytes) { b.alloc(bytes); }
+// With `timing`, an operator application's time reaches *ms_acc when the next application starts
+// or when collect_op_timing runs; every run that times applications calls it at its end (and
+// clears g->op_pending at its start).
+void collect_op_timing(nkpr_graph *g, double *ms_acc);
 
 constexpr int kMaxRefinements = 30;
 
@@ -51,6 +55,7 @@ inline Schedule make_schedule(nkpr_graph *g, uint32_t workers) {
     sc.ditems = g->ditems.as<uint4>();
     sc.n_d = g->n_d;
     sc.n_ditems = g->n_ditems;
+    sc.local = g->n_groups > 0 && g->n_slices == 1 && workers >= kXcds ? 1u : 0u;
     sc.srow = g->srow.as<uint32_t>();
     sc.sptr = g->sptr.as<uint32_t>();
     sc.sitems = g->sitems.as<uint4>();
@@ -58,8 +63,30 @@ inline Schedule make_schedule(nkpr_graph *g, uint32_t workers) {
     sc.n_s = g->n_s;
     sc.split_flag = g->split_flag.as<uint8_t>();
     sc.claim = g->claim.as<uint32_t>();
+    sc.arrive = sc.claim + kArriveAt;
     sc.workers = workers;
     return sc;
+}
+
+// Blocks of the combine kernel: every row a thread of its own up to eight blocks a CU.
+inline int combine_blocks(const nkpr_graph *g, int cus) {
+    return (int)std::max<uint64_t>(1, std::min<uint64_t>(((uint64_t)g->n_s + kCombineThreads - 1) / kCombineThreads,
+                                                         (uint64_t)std::max(cus, 1) * 8));
+}
+
+// Workers per slice that find an item: more blocks than items would only load the hub table and
+// add to the partials that the last block sums.
+inline int busy_workers(const nkpr_graph *g) {
+    if (g->n_slices == 1) return (int)std::max<uint32_t>(g->n_items, 1);
+    uint32_t most = (g->n_ditems + g->n_slices - 1) / g->n_slices;
+    for (uint32_t q = 0; q < g->n_slices; ++q) most = std::max(most, g->sitem_off[q + 1] - g->sitem_off[q]);
+    return (int)std::max<uint32_t>(most, 1);
+}
+
+// Workers per slice of a sweep: what the device holds at once, or what finds an item.
+inline int sweep_workers(const nkpr_graph *g, bool dbl, bool folded, int kind) {
+    return std::min(std::max(1, sweep_resident_blocks(g->device, dbl, folded, kind) / (int)g->n_slices),
+                    busy_workers(g));
 }
 
 // Launch sweeps of one phase until `done` or `max_launch` sweeps.  Returns completed sweeps.
@@ -72,7 +99,7 @@ uint64_t run_phase(RunCtx &rc, SweepArgs<T> a, Vecs<T> v, int kind, PhaseRule ru
     const bool dbl = sizeof(T) == 8;
     int &workers = rc.workers[dbl][kind][folded];
     if (workers <= 0)
-        workers = std::max(1, sweep_resident_blocks(g->device, dbl, folded, kind) / (int)g->n_slices);
+        workers = sweep_workers(g, dbl, folded, kind);
     FinalizeArgs f{};
     f.split_rows = g->split_rows.as<uint32_t>();
     f.split_first = g->split_first.as<uint32_t>();
@@ -137,6 +164,42 @@ uint64_t run_phase(RunCtx &rc, SweepArgs<T> a, Vecs<T> v, int kind, PhaseRule ru
     return done_sweeps;
 }
 
+// One FP32 sweep as a product (no reductions, no rule, no host read): the operator of a correction
+// solve on graphs without a binned copy.  The claim counters must be zero (launch_init_ctl).  With
+// `timing` its time reaches *ms_acc as a binned application's does (see collect_op_timing).
+inline void launch_product(RunCtx &rc, SweepArgs<float> a, const float *xg, const float *xold,
+                           float *xnew, float *xhat_new, bool timing, double *ms_acc) {
+    nkpr_graph *g = rc.g;
+    if (rc.p->interrupt && *rc.p->interrupt) throw Error(NKPR_ERR_INTERRUPTED, "interrupted");
+    int &workers = rc.workers[0][kSweepPlain][g->weighted];
+    if (workers <= 0) workers = sweep_workers(g, false, g->weighted, kSweepPlain);
+    FinalizeArgs f{};
+    f.split_rows = g->split_rows.as<uint32_t>();
+    f.split_first = g->split_first.as<uint32_t>();
+    f.split_count = g->split_count.as<uint32_t>();
+    f.n_split_rows = g->n_split_rows;
+    // only rows with split segments need the last block
+    if (f.n_split_rows) f.n_blocks = (uint32_t)(workers * g->n_slices + (g->n_s ? rc.combine_grid : 0));
+    f.rule.kind = kRuleStep;
+    f.rule.max_iterations = 1;
+    ensure(g->partials, 8 * 4 * (size_t)std::max<uint32_t>(f.n_blocks, 1));
+    a.sc = make_schedule(g, (uint32_t)workers);
+    a.partials = g->partials.as<double>();
+    a.ctl = g->ctl.as<PhaseCtl>();
+    a.xold = xold;
+    a.xnew = xnew;
+    a.xg = xg;
+    a.xhat_new = xhat_new;
+    if (timing) {
+        collect_op_timing(g, ms_acc);
+        for (hipEvent_t &e : g->op_ev)
+            if (!e) NKPR_HIP(hipEventCreate(&e));
+    }
+    launch_sweep<float>(a, f, kSweepPlain, g->weighted, rc.combine_grid, g->stream,
+                        timing ? g->op_ev[0] : nullptr, timing ? g->op_ev[1] : nullptr);
+    g->op_pending = timing;
+}
+
 inline double rel_error_bound(double damp, double l1, double sum) {
     return sum > 0.0 ? 2.0 * damp / (1.0 - damp) * l1 / sum : INFINITY;
 }
@@ -161,8 +224,8 @@ struct Krylov {
     float *vh, *yh; // prescaled copies (unweighted graphs)
     float *e;       // solution of the last solve
     double *dpart, *dout;
-    double *dhost;  // pinned host copy of dout (kDotResults entries)
-    hipEvent_t ev;  // recorded after a copy of dout to dhost
+    double *dhost;  // pinned host memory the dots land in too (kDotResults entries)
+    hipEvent_t ev;  // recorded after the kernel that writes them
 };
 constexpr uint32_t kDotResults = 128;
 
@@ -174,12 +237,8 @@ Krylov krylov_setup(nkpr_graph *g);
 void ensure_rowsum64(nkpr_graph *g);
 void apply_operator(RunCtx &rc, const float *v, float *w, const Krylov &kr, bool timing,
                     double *ms_acc, bool minus);
-// With `timing`, a binned application's time reaches *ms_acc when the next application starts
-// or when collect_op_timing runs; every run that times applications calls it at its end (and
-// clears g->op_pending at its start).
 bool apply_binned(nkpr_graph *g, const float *v, float *w, double damp, bool distribute,
                   bool minus, bool timing, double *ms_acc);
-void collect_op_timing(nkpr_graph *g, double *ms_acc);
 
 // GMRES(m) from e = 0 on A e = rhs, A = I - B, until ||A e - rhs||_2 <= rtol ||rhs||_2 or `cap`
 // operator applications.  `apply(v, w)` computes w = B v.  The Krylov spaces of A and B are
@@ -216,18 +275,18 @@ uint64_t gmres_f32(const Krylov &k, Apply &&apply, const float *rhs, float *e, d
     const int mres = k.m;
     const uint64_t ld = k.ld;
     float *const V = k.V;
-    // the results land in pinned memory (a direct copy, no staging through pageable memory)
+    // the kernels write the results to pinned memory themselves
     auto fetch = [&](double *host, uint32_t cnt) {
-        read_back(s, {{k.dhost, k.dout, 8 * cnt}});
+        NKPR_HIP(hipStreamSynchronize(s));
         std::memcpy(host, k.dhost, 8 * cnt);
     };
     auto dots = [&](const float *w, const float *Vb, uint32_t cnt, double *host) {
-        launch_multidot(w, Vb, ld, cnt, n, k.dpart, k.dout, s);
+        launch_multidot(w, Vb, ld, cnt, n, k.dpart, k.dout, k.dhost, s);
         fetch(host, cnt);
     };
     // w -= V c (cnt vectors), then host[i] = <u_i, w> for i < cnt and host[cnt] = <w, w>
     auto project = [&](float *w, uint32_t cnt, const double *c, double *host) {
-        launch_axpy_dot(w, V, ld, cnt, n, c, k.dpart, k.dout, s);
+        launch_axpy_dot(w, V, ld, cnt, n, c, k.dpart, k.dout, k.dhost, s);
         fetch(host, cnt + 1);
     };
     const auto in_range = [](double nrm) { return nrm >= 0x1p-50 && nrm <= 0x1p50; };
@@ -262,8 +321,7 @@ uint64_t gmres_f32(const Krylov &k, Apply &&apply, const float *rhs, float *e, d
         // <u_i, w> for i <= j and <w, w> (w is slot j + 1).  The projection w -= sum_i c_i u_i
         // with c_i = sig_i <u_i, w> sig_i is formed on the device and runs while the host reads
         // the dots, so that the device does not wait for the host between the steps.
-        launch_multidot(w, V, ld, j + 2, n, k.dpart, k.dout, s);
-        NKPR_HIP(hipMemcpyAsync(k.dhost, k.dout, 8 * (size_t)(j + 2), hipMemcpyDeviceToHost, s));
+        launch_multidot(w, V, ld, j + 2, n, k.dpart, k.dout, k.dhost, s);
         NKPR_HIP(hipEventRecord(k.ev, s));
         launch_gs_project(w, V, ld, j + 1, n, k.dout, sig.data(), s);
         NKPR_HIP(hipEventSynchronize(k.ev));

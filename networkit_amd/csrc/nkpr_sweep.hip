@@ -52,6 +52,69 @@ struct Acc4 {
     double l1 = 0.0, l2 = 0.0, sum = 0.0, sink = 0.0;
 };
 
+// The four sums over a block of BLOCK threads, waves added in order; valid in thread 0.
+template <int BLOCK>
+__device__ __forceinline__ Acc4 block_sum4(const Acc4 &v, double (*scratch)[BLOCK / 64]) {
+    const double w[4] = {wave_sum(v.l1), wave_sum(v.l2), wave_sum(v.sum), wave_sum(v.sink)};
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+        if (lane == q) scratch[q][wid] = w[q];
+    __syncthreads();
+    double r[4] = {0.0, 0.0, 0.0, 0.0};
+    if (threadIdx.x == 0) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            for (int k = 0; k < BLOCK / 64; ++k) r[q] += scratch[q][k];
+    }
+    Acc4 t;
+    t.l1 = r[0];
+    t.l2 = r[1];
+    t.sum = r[2];
+    t.sink = r[3];
+    return t;
+}
+
+// A block's four sums for another block of the same launch: agent-scope accesses, which are
+// coherent between the XCDs' L2 caches without a fence over everything the block wrote.
+__device__ __forceinline__ void put_partials(double *p, const Acc4 &v) {
+    __hip_atomic_store(p + 0, v.l1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, v.l2, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 2, v.sum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 3, v.sink, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double get_partial(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// True in exactly one block of the launch: the one that arrives when all others have.  Thread 0
+// has written the block's partials; it waits for those stores, then counts the block, first in
+// one of kArriveGroups counters (a line each), then, as its group's last, in the top one: a
+// thousand blocks on one counter would queue for longer than the sums take.  The counters are
+// zero again afterwards.
+__device__ __forceinline__ bool arrive_last(uint32_t *arrive, uint32_t block, uint32_t blocks,
+                                            uint32_t *slot) {
+    if (threadIdx.x == 0) {
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        const uint32_t grp = block % kArriveGroups;
+        const uint32_t members = (blocks - grp + kArriveGroups - 1) / kArriveGroups;
+        uint32_t *cnt = arrive + kArriveStride * (1 + grp);
+        uint32_t last = 0;
+        if (atomicAdd(cnt, 1u) + 1 == members) {
+            *cnt = 0u;
+            if (atomicAdd(arrive, 1u) + 1 == min(blocks, (uint32_t)kArriveGroups)) {
+                *arrive = 0u;
+                last = 1;
+            }
+        }
+        *slot = last;
+    }
+    __syncthreads();
+    return *slot != 0u;
+}
+
 // Stores of a finished row value y (old value xo already loaded) and its reductions: the
 // fused "pr[u] = pr[u]*damp + teleport" result plus everything the loop needs from it
 // (residual terms, score sum, sink mass, prescaled copy, FP32 residual).
@@ -139,14 +202,25 @@ __device__ __forceinline__ T block_row_sum(const SweepArgs<T> &a, uint32_t e0, u
     return block_sum<kBlock>(acc, red);
 }
 
+// Rows of a stream item that are summed by whole waves.  With G lanes per row an item has fewer
+// than 2 G R in-edges (G < 64; kCap otherwise) and R <= kRowsMax, so at most
+// 2 kRowsMax / kLongTurns of its rows are longer than kLongTurns G.
+constexpr uint32_t kLongTurns = 32;
+struct LongRows {
+    uint32_t count;
+    uint16_t row[2 * kRowsMax / kLongTurns];
+};
+static_assert(kCap / (64 * kLongTurns) <= 2 * kRowsMax / kLongTurns, "long rows of an item fit");
+
 // One stream item: rows [r0, r0+R) of a compressed list with absolute in-edge offsets `ptr`,
 // in-edges [e0, e0+cnt) (cnt <= kCap).  DIRECT rows finish with the epilogue (row ids from
 // sc.drow); sliced rows store their row sums into `out` (one slice's partial vector).
 template <typename T, bool FOLDED, bool BASEVEC, bool RESID, bool DIRECT>
 __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 item,
                                             const uint32_t *__restrict__ ptr, T *__restrict__ out,
-                                            T *s_prod, uint32_t *s_ptr, T *s_sum, const T *hub,
-                                            uint32_t nh, T damp, T c, Acc4 &st) {
+                                            T *s_prod, uint32_t *s_ptr, T *s_sum,
+                                            LongRows *s_long, const T *hub, uint32_t nh, T damp,
+                                            T c, Acc4 &st) {
     const uint32_t tid = threadIdx.x;
     const uint32_t r0 = item.x, R = item.y - item.x, e0 = item.z, cnt = item.w;
     // issue every load that does not depend on another load first
@@ -199,8 +273,11 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
         const uint32_t i = tid + k * kBlock;
         if (i < cnt) s_prod[i] = v[k];
     }
+    if (tid == 0) s_long->count = 0;
     __syncthreads();
-    // row sums: G consecutive lanes per row, G ~ average row length (power of two)
+    // row sums: G consecutive lanes per row, G ~ average row length (power of two).  A row of
+    // more than kLongTurns G in-edges is left to a whole wave: in a skewed item its group would
+    // add a few thousand products one after another while the block waits.
     const uint32_t avg = cnt / R;
     const int lg = avg >= 64 ? 6 : (avg >= 32 ? 5 : (avg >= 16 ? 4 : (avg >= 8 ? 3 : (avg >= 4 ? 2 : (avg >= 2 ? 1 : 0)))));
     const uint32_t G = 1u << lg;
@@ -209,14 +286,31 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
     for (uint32_t base = 0; base < R; base += per_pass) {
         const uint32_t r = base + (tid >> lg);
         T acc = 0;
-        if (r < R) {
+        bool own = r < R;
+        if (own) {
             const uint32_t b = s_ptr[r], e = s_ptr[r + 1];
-            for (uint32_t i = b + lane; i < e; i += G) acc += s_prod[i];
+            if (e - b > kLongTurns * G) {
+                own = false;
+                if (lane == 0) s_long->row[atomicAdd(&s_long->count, 1u)] = (uint16_t)r;
+            } else {
+                for (uint32_t i = b + lane; i < e; i += G) acc += s_prod[i];
+            }
         }
         for (uint32_t off = G >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-        if (r < R && lane == 0) s_sum[r] = acc;
+        if (own && lane == 0) s_sum[r] = acc;
     }
     __syncthreads();
+    const uint32_t n_long = s_long->count;
+    if (n_long) {
+        for (uint32_t k = tid >> 6; k < n_long; k += kBlock / 64) {
+            const uint32_t r = s_long->row[k];
+            T acc = 0;
+            for (uint32_t i = s_ptr[r] + (tid & 63); i < s_ptr[r + 1]; i += 64) acc += s_prod[i];
+            acc = wave_sum(acc);
+            if ((tid & 63) == 0) s_sum[r] = acc;
+        }
+        __syncthreads();
+    }
     // one thread per row; the LDS buffers are rewritten only after the next item's first
     // barrier, which every thread reaches after this point
     if (DIRECT) {
@@ -236,15 +330,92 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
     }
 }
 
+// One block ends a sweep: finish the rows with split segments, add all partials in a fixed order,
+// apply the stopping rule, reset the worker claim counters for the next sweep.  The block that
+// arrives last in the sweep's last launch does it (a launch of its own took 5.3 us of the 30 us
+// sweep of a 20,000-node graph).
+template <typename T, bool BASEVEC, bool RESID, int BLOCK>
+__device__ __forceinline__ void finish_sweep(const SweepArgs<T> &a, const FinalizeArgs &f,
+                                             double (*s_red)[BLOCK / 64]) {
+    PhaseCtl *ctl = a.ctl;
+    const T damp = (T)a.damp;
+    const T c = rhs_const(a);
+    const uint32_t S = a.sc.n_slices, ns = a.sc.n_s;
+    // split-row terms first (in row order), then block partials in block order
+    Acc4 st;
+    for (uint32_t t = threadIdx.x; t < f.n_split_rows; t += BLOCK) {
+        const uint32_t j = f.split_rows[t];
+        T acc = 0;
+        for (uint32_t s = 0; s < S; ++s) {
+            const uint32_t cnt = f.split_count[t * S + s];
+            if (cnt == 0) {
+                acc += a.partial[(size_t)s * ns + j];
+            } else {
+                const uint32_t first = f.split_first[t * S + s];
+                for (uint32_t k = 0; k < cnt; ++k) acc += a.split_partial[first + k];
+            }
+        }
+        row_epilogue<T, BASEVEC, RESID>(a, a.sc.srow[j], acc, damp, c, st);
+    }
+    double b1 = 0, b2 = 0, b3 = 0, b4 = 0;
+    for (uint32_t b = threadIdx.x; b < f.n_blocks; b += BLOCK) {
+        b1 += get_partial(a.partials + b * 4 + 0);
+        b2 += get_partial(a.partials + b * 4 + 1);
+        b3 += get_partial(a.partials + b * 4 + 2);
+        b4 += get_partial(a.partials + b * 4 + 3);
+    }
+    st.l1 += b1;
+    st.l2 += b2;
+    st.sum += b3;
+    st.sink += b4;
+    const Acc4 tot = block_sum4<BLOCK>(st, s_red);
+    if (threadIdx.x == 0) {
+        const PhaseRule &r = f.rule;
+        const uint64_t it = ctl->iterations + 1;
+        ctl->iterations = it;
+        const double prev = ctl->l1;
+        ctl->prev_l1 = prev;
+        ctl->l1 = tot.l1;
+        ctl->l2 = tot.l2;
+        ctl->sum = tot.sum;
+        ctl->sink_out = tot.sink;
+        ctl->sink_in = tot.sink;  // the next sweep reads the vector just written
+        const double bound = (tot.sum > 0.0) ? 2.0 * r.damp / (1.0 - r.damp) * tot.l1 / tot.sum : INFINITY;
+        ctl->bound = bound;
+        bool stop = it >= r.max_iterations;
+        if (r.kind == kRuleStep) {
+            const double step = (r.norm == NKPR_L2) ? sqrt(tot.l2) : tot.l1;
+            stop = stop || step <= r.tol;
+        } else if (r.kind == kRuleErr) {
+            stop = stop || bound <= r.tol;
+        } else {
+            stop = stop || tot.l1 <= r.tol_abs || bound <= r.tol;
+            if (it >= 4 && tot.l1 > r.stall_ratio * prev) stop = true;
+        }
+        ctl->done = stop ? 1u : 0u;
+        if (a.sc.claim)
+            for (int s = 0; s < kSlices; ++s) a.sc.claim[s] = 0u;
+    }
+}
+
+// Waves a SIMD.  Six (80 VGPRs) let three blocks share a CU, as their LDS does; at five two blocks
+// share it, and the sweep of a 1.3e6-node union of graphs takes 75 instead of 67 us.  The weighted
+// FP64 sweep gains nothing from the third block: 2.40 instead of 2.28 ms per solve of an R-MAT
+// graph of 9e5 nodes.
+template <typename T, bool FOLDED> constexpr int sweep_waves() {
+    return sizeof(T) == 8 && FOLDED ? 5 : 6;
+}
+
 template <typename T, bool FOLDED, bool BASEVEC, bool RESID>
-__global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs<T> a) {
+__global__ __launch_bounds__(kBlock, (sweep_waves<T, FOLDED>())) void sweep_kernel(SweepArgs<T> a, FinalizeArgs f) {
     if (a.ctl->done) return;  // converged earlier in this batch: no-op
 
     __shared__ T s_prod[kCap];
     __shared__ uint32_t s_ptr[kRowsMax + 1];
     __shared__ T s_sum[kRowsMax];
+    __shared__ LongRows s_long;
     __shared__ T s_redT[kBlock / 64];
-    __shared__ double s_red[kBlock / 64];
+    __shared__ double s_red[4][kBlock / 64];
     __shared__ uint32_t s_worker;
     __shared__ T s_hub[HubTable<T>::size];
 
@@ -255,8 +426,11 @@ __global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs<T> a) {
     Acc4 st;
 
     // claim a worker (slice, rank), trying the slice of this block's XCD first.  Each slice
-    // hands out exactly K ranks and the grid has S*K blocks, so every block gets one.
-    if (tid == 0) {
+    // hands out exactly K ranks and the grid has S*K blocks, so every block gets one.  Without
+    // slices any worker will do: the block's own number.
+    if (S == 1) {
+        if (tid == 0) s_worker = blockIdx.x;
+    } else if (tid == 0) {
         const uint32_t first = xcc_id() % S;
         uint32_t w = 0;
         for (uint32_t k = 0; k < S; ++k) {
@@ -296,24 +470,35 @@ __global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs<T> a) {
                 if (tid == 0) part[item.x] = p;
             } else {
                 stream_item<T, FOLDED, BASEVEC, RESID, false>(a, item, ptr, part, s_prod, s_ptr,
-                                                              s_sum, s_hub, nh, damp, c, st);
+                                                              s_sum, &s_long, s_hub, nh, damp, c,
+                                                              st);
             }
             item = next;
             it = nit;
         }
     }
-    // 2) direct rows, spread over all workers
+    // 2) direct rows, spread over all workers.  In a batch of graphs (local) the blocks of one XCD
+    // (dispatched round-robin) share an eighth of the items, so that a graph's vector entries are
+    // gathered through one L2; on a single graph, whose items differ in cost along the degrees,
+    // that split is uneven (R-MAT, 9e5 nodes: 2.92 instead of 2.28 ms per solve).
     {
-        const uint32_t nw = S * K;
-        uint32_t it = w;
+        const uint32_t nw = S * K, nd = a.sc.n_ditems;
+        uint32_t it = w, ie = nd, step = nw;
+        if (a.sc.local) {
+            const uint32_t x = w % kXcds;
+            step = (nw - x + kXcds - 1) / kXcds;  // this XCD's workers
+            it = (uint32_t)((uint64_t)nd * x / kXcds) + w / kXcds;
+            ie = (uint32_t)((uint64_t)nd * (x + 1) / kXcds);
+        }
         uint4 item = make_uint4(0, 0, 0, 0);
-        if (it < a.sc.n_ditems) item = a.sc.ditems[it];
-        while (it < a.sc.n_ditems) {
-            const uint32_t nit = it + nw;
+        if (it < ie) item = a.sc.ditems[it];
+        while (it < ie) {
+            const uint32_t nit = it + step;
             uint4 next = make_uint4(0, 0, 0, 0);
-            if (nit < a.sc.n_ditems) next = a.sc.ditems[nit];
+            if (nit < ie) next = a.sc.ditems[nit];
             stream_item<T, FOLDED, BASEVEC, RESID, true>(a, item, a.sc.dptr, nullptr, s_prod,
-                                                         s_ptr, s_sum, s_hub, nh, damp, c, st);
+                                                         s_ptr, s_sum, &s_long, s_hub, nh, damp, c,
+                                                         st);
             item = next;
             it = nit;
         }
@@ -322,24 +507,22 @@ __global__ __launch_bounds__(kBlock) void sweep_kernel(SweepArgs<T> a) {
     // per-worker partials (l1, l2, sum, sink) in FP64: indexed by the claimed worker, whose
     // rows are fixed, not by the block, whose worker depends on the order of the claims, so
     // that the finalize kernel adds the same values in the same order on every run
-    double v;
-    v = block_sum<kBlock>(st.l1, s_red);
-    if (tid == 0) a.partials[w * 4 + 0] = v;
-    v = block_sum<kBlock>(st.l2, s_red);
-    if (tid == 0) a.partials[w * 4 + 1] = v;
-    v = block_sum<kBlock>(st.sum, s_red);
-    if (tid == 0) a.partials[w * 4 + 2] = v;
-    v = block_sum<kBlock>(st.sink, s_red);
-    if (tid == 0) a.partials[w * 4 + 3] = v;
+    if (f.n_blocks == 0) return;  // a product alone: nothing to reduce, no rule
+    const Acc4 sums = block_sum4<kBlock>(st, s_red);
+    if (tid == 0) put_partials(a.partials + (size_t)w * 4, sums);
+    // without sliced rows this launch ends the sweep
+    if (a.sc.n_s == 0 && arrive_last(a.sc.arrive, blockIdx.x, gridDim.x, &s_worker))
+        finish_sweep<T, BASEVEC, RESID, kBlock>(a, f, s_red);
 }
 
 // Sliced rows: add the per-slice row sums in slice order and run the row epilogue.  Rows
 // with split segments are left to the finalize kernel.
 template <typename T, bool BASEVEC, bool RESID>
-__global__ __launch_bounds__(kCombineThreads) void combine_kernel(SweepArgs<T> a,
+__global__ __launch_bounds__(kCombineThreads) void combine_kernel(SweepArgs<T> a, FinalizeArgs f,
                                                                   uint32_t block_base) {
     if (a.ctl->done) return;
-    __shared__ double s_red[kCombineThreads / 64];
+    __shared__ double s_red[4][kCombineThreads / 64];
+    __shared__ uint32_t s_last;
     const T damp = (T)a.damp;
     const T c = rhs_const(a);
     const uint32_t S = a.sc.n_slices, ns = a.sc.n_s;
@@ -352,84 +535,20 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(SweepArgs<T> a
         const uint32_t u = ld_stream(a.sc.srow + j);
         row_epilogue<T, BASEVEC, RESID>(a, u, acc, damp, c, st);
     }
-    double v;
-    const uint32_t b = block_base + blockIdx.x;
-    v = block_sum<kCombineThreads>(st.l1, s_red);
-    if (threadIdx.x == 0) a.partials[b * 4 + 0] = v;
-    v = block_sum<kCombineThreads>(st.l2, s_red);
-    if (threadIdx.x == 0) a.partials[b * 4 + 1] = v;
-    v = block_sum<kCombineThreads>(st.sum, s_red);
-    if (threadIdx.x == 0) a.partials[b * 4 + 2] = v;
-    v = block_sum<kCombineThreads>(st.sink, s_red);
-    if (threadIdx.x == 0) a.partials[b * 4 + 3] = v;
+    if (f.n_blocks == 0) return;
+    const Acc4 sums = block_sum4<kCombineThreads>(st, s_red);
+    if (threadIdx.x == 0) put_partials(a.partials + (size_t)(block_base + blockIdx.x) * 4, sums);
+    if (arrive_last(a.sc.arrive, blockIdx.x, gridDim.x, &s_last))
+        finish_sweep<T, BASEVEC, RESID, kCombineThreads>(a, f, s_red);
 }
 
-// One block: finish rows with split segments, add all partials in a fixed order, apply the
-// stopping rule, reset the worker claim counters for the next sweep.
-template <typename T, bool BASEVEC, bool RESID>
-__global__ __launch_bounds__(kFinalizeThreads) void finalize_kernel(SweepArgs<T> a,
+// The end of a sweep whose rows were finished elsewhere (the binned FP64 sweep, the closed-form
+// first residual): one block.
+__global__ __launch_bounds__(kFinalizeThreads) void finalize_kernel(SweepArgs<double> a,
                                                                     FinalizeArgs f) {
-    PhaseCtl *ctl = a.ctl;
-    if (ctl->done) return;
-    __shared__ double s_red[kFinalizeThreads / 64];
-    const T damp = (T)a.damp;
-    const T c = rhs_const(a);
-    const uint32_t S = a.sc.n_slices, ns = a.sc.n_s;
-    Acc4 st;
-    for (uint32_t t = threadIdx.x; t < f.n_split_rows; t += kFinalizeThreads) {
-        const uint32_t j = f.split_rows[t];
-        T acc = 0;
-        for (uint32_t s = 0; s < S; ++s) {
-            const uint32_t cnt = f.split_count[t * S + s];
-            if (cnt == 0) {
-                acc += a.partial[(size_t)s * ns + j];
-            } else {
-                const uint32_t first = f.split_first[t * S + s];
-                for (uint32_t k = 0; k < cnt; ++k) acc += a.split_partial[first + k];
-            }
-        }
-        row_epilogue<T, BASEVEC, RESID>(a, a.sc.srow[j], acc, damp, c, st);
-    }
-    // split-row terms first (in row order), then block partials in block order
-    double l1 = st.l1, l2 = st.l2, sum = st.sum, sink = st.sink;
-    double b1 = 0, b2 = 0, b3 = 0, b4 = 0;
-    for (uint32_t b = threadIdx.x; b < f.n_blocks; b += kFinalizeThreads) {
-        b1 += a.partials[b * 4 + 0];
-        b2 += a.partials[b * 4 + 1];
-        b3 += a.partials[b * 4 + 2];
-        b4 += a.partials[b * 4 + 3];
-    }
-    l1 = block_sum<kFinalizeThreads>(l1 + b1, s_red);
-    l2 = block_sum<kFinalizeThreads>(l2 + b2, s_red);
-    sum = block_sum<kFinalizeThreads>(sum + b3, s_red);
-    sink = block_sum<kFinalizeThreads>(sink + b4, s_red);
-    if (threadIdx.x == 0) {
-        const PhaseRule &r = f.rule;
-        const uint64_t it = ctl->iterations + 1;
-        ctl->iterations = it;
-        const double prev = ctl->l1;
-        ctl->prev_l1 = prev;
-        ctl->l1 = l1;
-        ctl->l2 = l2;
-        ctl->sum = sum;
-        ctl->sink_out = sink;
-        ctl->sink_in = sink;  // the next sweep reads the vector just written
-        const double bound = (sum > 0.0) ? 2.0 * r.damp / (1.0 - r.damp) * l1 / sum : INFINITY;
-        ctl->bound = bound;
-        bool stop = it >= r.max_iterations;
-        if (r.kind == kRuleStep) {
-            const double step = (r.norm == NKPR_L2) ? sqrt(l2) : l1;
-            stop = stop || step <= r.tol;
-        } else if (r.kind == kRuleErr) {
-            stop = stop || bound <= r.tol;
-        } else {
-            stop = stop || l1 <= r.tol_abs || bound <= r.tol;
-            if (it >= 4 && l1 > r.stall_ratio * prev) stop = true;
-        }
-        ctl->done = stop ? 1u : 0u;
-        if (a.sc.claim)
-            for (int s = 0; s < kSlices; ++s) a.sc.claim[s] = 0u;
-    }
+    if (a.ctl->done) return;
+    __shared__ double s_red[4][kFinalizeThreads / 64];
+    finish_sweep<double, false, false, kFinalizeThreads>(a, f, s_red);
 }
 
 __global__ void init_ctl_kernel(PhaseCtl *ctl, const double *sink_sum, uint32_t *claim) {
@@ -654,17 +773,14 @@ void launch_pair(const SweepArgs<T> &a, const FinalizeArgs &f, int combine_grid,
     const unsigned grid = a.sc.n_slices * a.sc.workers;
     if (ev0) NKPR_HIP(hipEventRecord(ev0, s));
     hipLaunchKernelGGL((sweep_kernel<T, FOLDED, BASEVEC, RESID>), dim3(grid), dim3(kBlock), 0, s,
-                       a);
+                       a, f);
     NKPR_HIP(hipGetLastError());
-    if (a.sc.n_s > 0 && combine_grid > 0) {
+    if (a.sc.n_s > 0) {
         hipLaunchKernelGGL((combine_kernel<T, BASEVEC, RESID>), dim3(combine_grid),
-                           dim3(kCombineThreads), 0, s, a, grid);
+                           dim3(kCombineThreads), 0, s, a, f, grid);
         NKPR_HIP(hipGetLastError());
     }
     if (ev1) NKPR_HIP(hipEventRecord(ev1, s));
-    hipLaunchKernelGGL((finalize_kernel<T, BASEVEC, RESID>), dim3(1), dim3(kFinalizeThreads), 0,
-                       s, a, f);
-    NKPR_HIP(hipGetLastError());
 }
 
 template <typename T, bool FOLDED, bool BASEVEC, bool RESID>
@@ -697,18 +813,8 @@ template void launch_sweep<float>(const SweepArgs<float> &, const FinalizeArgs &
 template void launch_sweep<double>(const SweepArgs<double> &, const FinalizeArgs &, int, bool,
                                    int, hipStream_t, hipEvent_t, hipEvent_t);
 
-void launch_finalize64(const SweepArgs<double> &a, const FinalizeArgs &f, int kind, hipStream_t s) {
-    // the template flags only matter for split rows, which a binned sweep does not have
-    const bool basevec = kind == kSweepBaseVec || kind == kSweepBaseResid;
-    const bool resid = kind == kSweepResid || kind == kSweepBaseResid;
-    if (basevec && resid)
-        hipLaunchKernelGGL((finalize_kernel<double, true, true>), dim3(1), dim3(kFinalizeThreads), 0, s, a, f);
-    else if (basevec)
-        hipLaunchKernelGGL((finalize_kernel<double, true, false>), dim3(1), dim3(kFinalizeThreads), 0, s, a, f);
-    else if (resid)
-        hipLaunchKernelGGL((finalize_kernel<double, false, true>), dim3(1), dim3(kFinalizeThreads), 0, s, a, f);
-    else
-        hipLaunchKernelGGL((finalize_kernel<double, false, false>), dim3(1), dim3(kFinalizeThreads), 0, s, a, f);
+void launch_finalize64(const SweepArgs<double> &a, const FinalizeArgs &f, hipStream_t s) {
+    hipLaunchKernelGGL(finalize_kernel, dim3(1), dim3(kFinalizeThreads), 0, s, a, f);
     NKPR_HIP(hipGetLastError());
 }
 
