@@ -78,19 +78,16 @@ void algebraic_create_impl(const nkpr_csr *m, nkpr_algebraic **out) {
     std::unique_ptr<nkpr_algebraic> h(new nkpr_algebraic());
     NKPR_HIP(hipGetDevice(&h->device));
     h->rows = m->rows;
-    hipStream_t s;
-    NKPR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    const hipStream_t s = stream_get();
     struct StreamOwner {
         hipStream_t s;
-        ~StreamOwner() {
-            (void)hipStreamSynchronize(s);
-            (void)hipStreamDestroy(s);
-        }
+        int device;
+        ~StreamOwner() { stream_put(s, device); }
     };
     // the temporaries outlive the stream owner (it synchronises first)
     DevBuf src, w32, ones;
     {
-        StreamOwner owner{s};
+        StreamOwner owner{s, h->device};
         csr_validate(m, s);
         src.alloc(4 * std::max<uint64_t>(m->nnz, 1));
         w32.alloc(4 * std::max<uint64_t>(m->nnz, 1));

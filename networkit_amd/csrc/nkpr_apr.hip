@@ -53,10 +53,7 @@ struct nkpr_apr {
     uint64_t chunk_cap = 0;  // entries per heavy chunk list (two lists)
     bool dirty = true;  // p, r, flags hold a run that was not cleared
     ~nkpr_apr() {
-        if (stream) {
-            (void)hipStreamSynchronize(stream);
-            (void)hipStreamDestroy(stream);
-        }
+        nkpr::stream_put(stream, device);
     }
 };
 
@@ -351,7 +348,7 @@ void apr_create_impl(uint64_t z, const uint64_t *ptr, const int32_t *dst, const 
     NKPR_CHECK(ptr != nullptr, "ptr is NULL");
     std::unique_ptr<nkpr_apr> a(new nkpr_apr());
     NKPR_HIP(hipGetDevice(&a->device));
-    NKPR_HIP(hipStreamCreateWithFlags(&a->stream, hipStreamNonBlocking));
+    a->stream = stream_get();
     const hipStream_t s = a->stream;
     const hipMemcpyKind kind = device_ptrs ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
     uint64_t m = 0;

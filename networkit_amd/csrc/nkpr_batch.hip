@@ -1122,7 +1122,7 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
     br.st = st;
     ensure_buf(g->b_col, sizeof(BatchCol) * ld);
     ensure_buf(g->b_ctl, sizeof(BatchCtl));
-    if (!g->b_ctl_host) NKPR_HIP(hipHostMalloc((void **)&g->b_ctl_host, sizeof(BatchCtl), hipHostMallocDefault));
+    if (!g->b_ctl_host) g->b_ctl_host = static_cast<BatchCtl *>(pinned_alloc(sizeof(BatchCtl)));
     br.col = g->b_col.as<BatchCol>();
     br.ctl = g->b_ctl.as<BatchCtl>();
     br.ctl_host = g->b_ctl_host;

@@ -14,6 +14,8 @@
 #include <cstdio>
 #include <cstring>
 #include <limits>
+#include <map>
+#include <mutex>
 #include <numeric>
 #include <string>
 #include <vector>
@@ -67,7 +69,7 @@ namespace nkpr {
 
 void prepare_run(nkpr_graph *g) {
     ensure(g->ctl, sizeof(PhaseCtl));
-    if (!g->ctl_host) NKPR_HIP(hipHostMalloc((void **)&g->ctl_host, sizeof(PhaseCtl), hipHostMallocDefault));
+    if (!g->ctl_host) g->ctl_host = static_cast<PhaseCtl *>(pinned_alloc(sizeof(PhaseCtl)));
     ensure(g->red_partials, 8 * 1024);
     ensure(g->red_out, 8 * 4);
     ensure(g->split_part32, 4 * std::max<size_t>(g->n_split_items, 1));
@@ -360,7 +362,7 @@ Krylov krylov_setup(nkpr_graph *g) {
     k.e = k.y + 3 * ld;
     k.dpart = g->kdot.as<double>();
     k.dout = k.dpart + (size_t)kDotPartials;
-    if (!g->kdot_host) NKPR_HIP(hipHostMalloc((void **)&g->kdot_host, 8 * kDotResults, hipHostMallocDefault));
+    if (!g->kdot_host) g->kdot_host = static_cast<double *>(pinned_alloc(8 * kDotResults));
     if (!g->kdot_ev) NKPR_HIP(hipEventCreateWithFlags(&g->kdot_ev, hipEventDisableTiming));
     k.dhost = g->kdot_host;
     k.ev = g->kdot_ev;
@@ -547,6 +549,21 @@ int nkpr_params_default(nkpr_params *p) {
 }
 
 namespace {
+// The device's architecture, asked for once per device (the query takes as long as a small solve).
+void check_arch(int dev) {
+    static std::mutex mu;
+    static std::map<int, std::string> arch;
+    std::lock_guard<std::mutex> lock(mu);
+    auto it = arch.find(dev);
+    if (it == arch.end()) {
+        hipDeviceProp_t prop;
+        NKPR_HIP(hipGetDeviceProperties(&prop, dev));
+        it = arch.emplace(dev, prop.gcnArchName).first;
+    }
+    if (it->second.compare(0, 6, "gfx950") != 0)
+        throw Error(NKPR_ERR_NODEVICE, "libnkpr is built for gfx950, device is " + it->second);
+}
+
 int create_handle(const nkpr_csc *csc, nkpr_graph **out, const uint64_t *group_off,
                   uint32_t n_groups) {
     return guarded([&] {
@@ -557,14 +574,11 @@ int create_handle(const nkpr_csc *csc, nkpr_graph **out, const uint64_t *group_o
             throw Error(NKPR_ERR_NODEVICE, "no HIP device is visible");
         int dev = 0;
         NKPR_HIP(hipGetDevice(&dev));
-        hipDeviceProp_t prop;
-        NKPR_HIP(hipGetDeviceProperties(&prop, dev));
-        if (std::strncmp(prop.gcnArchName, "gfx950", 6) != 0)
-            throw Error(NKPR_ERR_NODEVICE, std::string("libnkpr is built for gfx950, device is ") + prop.gcnArchName);
+        check_arch(dev);
         auto *g = new nkpr_graph();
         g->device = dev;
         try {
-            NKPR_HIP(hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking));
+            g->stream = stream_get();
             create_graph(csc, g, group_off, n_groups);
         } catch (...) {
             nkpr_graph_destroy(g);
@@ -605,8 +619,9 @@ int nkpr_graph_destroy(nkpr_graph *g) {
     (void)hipSetDevice(g->device);
     if (g->stream) (void)hipStreamSynchronize(g->stream);
     hipStream_t s = g->stream;
-    delete g;  // frees device buffers
-    if (s) (void)hipStreamDestroy(s);
+    const int device = g->device;
+    delete g;  // gives the device buffers back
+    stream_put(s, device);
     if (prev >= 0) (void)hipSetDevice(prev);
     return NKPR_OK;
 }

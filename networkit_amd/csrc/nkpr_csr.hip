@@ -493,15 +493,14 @@ void algebraic_pagerank_impl(const nkpr_csr *m, double damp, double tol, uint64_
     work.alloc(std::max<size_t>(work_bytes(tiles), 8 * 1024));
     out.alloc(16);
     flag.alloc(4);
-    hipStream_t s;
-    NKPR_HIP(hipStreamCreateWithFlags(&s, hipStreamNonBlocking));
+    int device = 0;
+    NKPR_HIP(hipGetDevice(&device));
+    const hipStream_t s = stream_get();
     struct StreamOwner {
         hipStream_t s;
-        ~StreamOwner() {
-            (void)hipStreamSynchronize(s);
-            (void)hipStreamDestroy(s);
-        }
-    } owner{s};
+        int device;
+        ~StreamOwner() { stream_put(s, device); }
+    } owner{s, device};
     // the reference reads whatever the indices point at; here a malformed matrix is an error
     hipLaunchKernelGGL(csr_fill_kernel, dim3(1), dim3(64), 0, s, out.as<double>(), 2, 0.0);
     NKPR_HIP(hipMemsetAsync(flag.p, 0, 4, s));

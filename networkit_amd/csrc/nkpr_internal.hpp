@@ -108,6 +108,16 @@ inline void read_back(hipStream_t s, std::initializer_list<HostCopy> copies) {
     read_back(s, copies.begin(), copies.size());
 }
 
+// Device memory, small pinned buffers and streams, kept between handles (nkpr_pool.hip).  Memory
+// comes from and goes back to the current device's blocks (device_free: to the block's own device);
+// a released block is not handed out before the device has finished what was enqueued until then.
+void *device_alloc(size_t bytes);
+void device_free(void *p);
+void *pinned_alloc(size_t bytes);  // at most 4096 bytes; idle when released
+void pinned_free(void *p);
+hipStream_t stream_get();  // non-blocking, default priority
+void stream_put(hipStream_t s, int device);
+
 // Owning device allocation.
 struct DevBuf {
     void *p = nullptr;
@@ -117,7 +127,7 @@ struct DevBuf {
     DevBuf &operator=(const DevBuf &) = delete;
     ~DevBuf() { reset(); }
     void reset() {
-        if (p) (void)hipFree(p);
+        device_free(p);
         p = nullptr;
         bytes = 0;
     }
@@ -125,12 +135,7 @@ struct DevBuf {
         if (b <= bytes && p) return;
         reset();
         if (b == 0) b = 16;
-        hipError_t e = hipMalloc(&p, b);
-        if (e != hipSuccess) {
-            p = nullptr;
-            throw Error(NKPR_ERR_NOMEM, "hipMalloc(" + std::to_string(b) +
-                                            " bytes) failed: " + hipGetErrorString(e));
-        }
+        p = device_alloc(b);
         bytes = b;
     }
     template <typename T> T *as() const { return static_cast<T *>(p); }
@@ -531,9 +536,9 @@ struct nkpr_graph {
         for (hipEvent_t e : events) (void)hipEventDestroy(e);
         for (hipEvent_t e : op_ev)
             if (e) (void)hipEventDestroy(e);
-        if (ctl_host) (void)hipHostFree(ctl_host);
-        if (kdot_host) (void)hipHostFree(kdot_host);
+        nkpr::pinned_free(ctl_host);
+        nkpr::pinned_free(kdot_host);
         if (kdot_ev) (void)hipEventDestroy(kdot_ev);
-        if (b_ctl_host) (void)hipHostFree(b_ctl_host);
+        nkpr::pinned_free(b_ctl_host);
     }
 };
