@@ -22,6 +22,7 @@
 #include <cmath>
 #include <cstring>
 
+#include "nkpr_agg.hpp"
 #include "nkpr_internal.hpp"
 #include "nkpr_run.hpp"
 
@@ -132,11 +133,15 @@ __global__ void scatter2_kernel(const double *v, const int32_t *perm_a, const in
     if (i < n) out_z[perm_f[perm_a[i]]] = f * v[i];
 }
 
-__global__ void wdeg_slot_kernel(const int32_t *src, uint64_t m, const float *w,
-                                 const double *w64, double *deg) {
-    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
-         e += (uint64_t)gridDim.x * blockDim.x)
-        atomicAdd(&deg[src[e]], w64 ? w64[e] : (w ? (double)w[e] : 1.0));
+// Weighted out-degrees of the caller's lists, by slot.
+__global__ __launch_bounds__(kAggThreads) void wdeg_slot_kernel(const int32_t *src, uint64_t m, const float *w,
+                                                                const double *w64, double *deg) {
+    __shared__ AggTable agg;
+    agg.clear();
+    for (uint64_t e = (uint64_t)blockIdx.x * kAggThreads + threadIdx.x; e < m;
+         e += (uint64_t)gridDim.x * kAggThreads)
+        agg.add((uint32_t)src[e], w64 ? w64[e] : (w ? (double)w[e] : 1.0), nullptr, deg);
+    agg.flush(nullptr, deg);
 }
 
 // dL/dw for every in-edge of the caller's CSC: one wave per row.
@@ -487,7 +492,7 @@ void adjoint_impl(nkpr_graph *g, const nkpr_params *p, const nkpr_csc *csc,
             else NKPR_HIP(hipMemcpyAsync(deg, dz, 8 * z, hipMemcpyDeviceToDevice, s));
         } else {
             NKPR_HIP(hipMemsetAsync(deg, 0, 8 * z, s));
-            hipLaunchKernelGGL(wdeg_slot_kernel, dim3(nblocks(m)), dim3(256), 0, s, src, m, w32, w64, deg);
+            hipLaunchKernelGGL(wdeg_slot_kernel, dim3(agg_blocks(m)), dim3(kAggThreads), 0, s, src, m, w32, w64, deg);
         }
         DevBuf gw;
         double *gout = grad_weight;

@@ -733,14 +733,20 @@ void batch_layout(nkpr_graph *g) {
                            g->weighted ? g->b_coef64.as<double>() : nullptr);
         NKPR_HIP(hipGetLastError());
     }
-    g->b_rowptr_host.resize((size_t)n + 1);
-    g->b_perm_host.resize(n);
-    read_back(s, {{g->b_rowptr_host.data(), g->b_rowptr.p, 4 * ((size_t)n + 1)},
-                  {g->b_perm_host.data(), g->perm.p, 4 * (size_t)n}});
-    g->b_iperm_host.assign(g->z, -1);
-    for (uint32_t u = 0; u < n; ++u) g->b_iperm_host[(uint32_t)g->b_perm_host[u]] = (int32_t)u;
     g->b_ready = true;
     g->b_coef_ready = true;
+}
+
+void batch_host_lists(nkpr_graph *g) {
+    if (g->b_host_ready) return;
+    const uint32_t n = g->n;
+    std::vector<int32_t> perm(n);
+    g->b_rowptr_host.resize((size_t)n + 1);
+    read_back(g->stream, {{g->b_rowptr_host.data(), g->b_rowptr.p, 4 * ((size_t)n + 1)},
+                          {perm.data(), g->perm.p, 4 * (size_t)n}});
+    g->b_iperm_host.assign(g->z, -1);
+    for (uint32_t u = 0; u < n; ++u) g->b_iperm_host[(uint32_t)perm[u]] = (int32_t)u;
+    g->b_host_ready = true;
 }
 
 // Light-row list and heavy-row pieces for one threshold (cached per threshold).
@@ -1034,6 +1040,7 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
     NKPR_CHECK(seeds != nullptr, "seed_nodes is NULL");
     const hipStream_t s = g->stream;
     batch_layout(g);
+    batch_host_lists(g);
 
     // ---- row-sparse teleport in relabelled ids ----------------------------------------------
     // Entries (row, column, weight) in column order, sorted stably by row (so columns ascend

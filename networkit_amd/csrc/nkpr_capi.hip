@@ -257,7 +257,7 @@ SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64
             read_back(s, {{&hf, flag, 4}, {&cval, xcur, 8}});
             closed = hf == 0;
         }
-        if (closed) ensure_rowsum64(g);
+        if (closed) ensure_rowsum64(g, rc.combine_grid);
         for (int round = 0;; ++round) {
             // FP64 residual sweep: ynew = d P xcur + b, r32 = float(ynew - xcur)
             PhaseRule rr{};
@@ -326,16 +326,31 @@ SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64
     return res;
 }
 
-// The FP64 row sums of P (sum of each row's in-coefficients), kept per graph until new weights.
-void ensure_rowsum64(nkpr_graph *g) {
+// The FP64 row sums of P (sum of each row's in-coefficients), kept per graph until new weights: the
+// product with the vector of ones, one FP64 pull sweep over the lists as they are (a plain copy of
+// the lists, made for them alone, took ten times as long on 1.5e7 arcs).  Uses x64b.
+void ensure_rowsum64(nkpr_graph *g, int combine_grid) {
     if (g->rowsum_ready) return;
     const uint32_t n = g->n;
-    batch_layout(g);
+    const hipStream_t s = g->stream;
+    prepare_run(g);
     g->rowsum64.alloc(8 * std::max<uint64_t>(n, 1));
-    launch_rowsum64(g->b_rowptr.as<uint32_t>(), n, g->b_src.as<int32_t>(),
-                    g->weighted ? g->b_coef64.as<double>() : nullptr,
-                    g->weighted ? nullptr : g->inv64.as<double>(), g->rowsum64.as<double>(), g->stream);
-    NKPR_HIP(hipStreamSynchronize(g->stream));
+    const double *ones = g->inv64.as<double>();  // unweighted: the prescaled vector of ones
+    if (g->weighted) {
+        launch_fill(g->x64b.as<double>(), n, 1.0, s);
+        ones = g->x64b.as<double>();
+    }
+    launch_init_ctl(g->ctl.as<PhaseCtl>(), nullptr, g->claim.as<uint32_t>(), s);
+    SweepArgs<double> a{};
+    a.coef = g->weighted ? g->coef64.as<double>() : nullptr;
+    a.inv = g->weighted ? nullptr : g->inv64.as<double>();
+    a.partial = g->part64.as<double>();
+    a.split_partial = g->split_part64.as<double>();
+    a.damp = 1.0;
+    a.n = n;
+    a.sink_begin = g->sink_begin;
+    launch_product<double>(g, a, sweep_workers(g, true, g->weighted, kSweepPlain), combine_grid, ones, ones,
+                           g->rowsum64.as<double>(), nullptr, nullptr);
     g->rowsum_ready = true;
 }
 
@@ -424,7 +439,7 @@ void apply_operator(RunCtx &rc, const float *v, float *w, const Krylov &kr, bool
     a.sink_begin = g->sink_begin;
     a.distribute = dist ? 1 : 0;
     // the sweep writes B v to kr.y (A v follows) or straight to w
-    launch_product(rc, a, folded ? v : kr.vh, v, minus ? kr.y : w, nullptr, timing, ms_acc);
+    apply_product(rc, a, folded ? v : kr.vh, v, minus ? kr.y : w, timing, ms_acc);
     if (minus) launch_axpby(v, kr.y, w, n, 1.0f, -1.0f, s);
 }
 

@@ -24,6 +24,7 @@
 #include <cstring>
 #include <map>
 
+#include "nkpr_agg.hpp"
 #include "nkpr_internal.hpp"
 
 namespace nkpr {
@@ -52,19 +53,23 @@ __global__ void validate_ptr_kernel(const uint64_t *colptr, uint64_t z, uint64_t
     if (exists && !exists[u] && e != b) atomicOr(flags, kBadExists);
 }
 
-__global__ void out_degree_kernel(const int32_t *src, uint64_t m, uint64_t z,
-                                  const uint8_t *exists, const float *w, const double *w64,
-                                  uint32_t *outcnt, double *wdeg, uint32_t *flags) {
-    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
-         e += (uint64_t)gridDim.x * blockDim.x) {
+// Out-degrees and (wdeg given) weighted out-degrees of the arcs' sources.
+__global__ __launch_bounds__(kAggThreads) void out_degree_kernel(const int32_t *src, uint64_t m, uint64_t z,
+                                                                 const uint8_t *exists, const float *w,
+                                                                 const double *w64, uint32_t *outcnt,
+                                                                 double *wdeg, uint32_t *flags) {
+    __shared__ AggTable agg;
+    agg.clear();
+    for (uint64_t e = (uint64_t)blockIdx.x * kAggThreads + threadIdx.x; e < m;
+         e += (uint64_t)gridDim.x * kAggThreads) {
         const int32_t v = src[e];
         if (v < 0 || (uint64_t)v >= z || (exists && !exists[v])) {
             atomicOr(flags, kBadSrc);
             continue;
         }
-        atomicAdd(&outcnt[v], 1u);
-        if (wdeg) atomicAdd(&wdeg[v], w64 ? w64[e] : (w ? (double)w[e] : 1.0));
+        agg.add((uint32_t)v, wdeg ? (w64 ? w64[e] : (w ? (double)w[e] : 1.0)) : 0.0, outcnt, wdeg);
     }
+    agg.flush(outcnt, wdeg);
 }
 
 __global__ void relabel_keys_kernel(const uint32_t *outcnt, const uint8_t *exists, uint64_t z,
@@ -119,14 +124,31 @@ __global__ void group_edges_kernel(const uint64_t *colptr, const int32_t *src, c
     }
 }
 
-__global__ void count_kernel(const uint32_t *outcnt, const uint8_t *exists, uint64_t z,
-                             unsigned long long *n_exist, unsigned long long *n_nonsink) {
-    const uint64_t u = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (u >= z) return;
-    const bool ex = !exists || exists[u];
-    if (ex) {
-        atomicAdd(n_exist, 1ull);
-        if (outcnt[u] > 0) atomicAdd(n_nonsink, 1ull);
+// Existing nodes and those with out-edges: one atomic per block on either count.
+__global__ __launch_bounds__(256) void count_kernel(const uint32_t *outcnt, const uint8_t *exists, uint64_t z,
+                                                    unsigned long long *n_exist,
+                                                    unsigned long long *n_nonsink) {
+    __shared__ uint32_t s_cnt[2];
+    if (threadIdx.x < 2) s_cnt[threadIdx.x] = 0;
+    __syncthreads();
+    uint32_t ne = 0, ns = 0;
+    for (uint64_t u = (uint64_t)blockIdx.x * 256 + threadIdx.x; u < z; u += (uint64_t)gridDim.x * 256) {
+        const bool ex = !exists || exists[u];
+        ne += ex ? 1u : 0u;
+        ns += ex && outcnt[u] > 0 ? 1u : 0u;
+    }
+    for (int off = 32; off > 0; off >>= 1) {
+        ne += __shfl_xor(ne, off, 64);
+        ns += __shfl_xor(ns, off, 64);
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicAdd(&s_cnt[0], ne);
+        atomicAdd(&s_cnt[1], ns);
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        atomicAdd(n_exist, (unsigned long long)s_cnt[0]);
+        atomicAdd(n_nonsink, (unsigned long long)s_cnt[1]);
     }
 }
 
@@ -607,8 +629,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         wdeg = wdeg_own;
     }
     if (m) {
-        const unsigned gb = (unsigned)std::min<uint64_t>(blocks_for(m), 65536);
-        hipLaunchKernelGGL(out_degree_kernel, dim3(gb), dim3(256), 0, s, src_in, m, z, exists, w_in,
+        hipLaunchKernelGGL(out_degree_kernel, dim3(agg_blocks(m)), dim3(kAggThreads), 0, s, src_in, m, z, exists, w_in,
                            w64_in, outcnt_b.as<uint32_t>(), wdeg_own, flags);
     }
     if (c->out_wdeg && z)
@@ -627,7 +648,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     NKPR_HIP(hipMemsetAsync(counts_b.p, 0, 16, s));
     auto *counts = counts_b.as<unsigned long long>();
     if (z)
-        hipLaunchKernelGGL(count_kernel, dim3(blocks_for(z)), dim3(256), 0, s,
+        hipLaunchKernelGGL(count_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(z), 1024)), dim3(256), 0, s,
                            outcnt_b.as<uint32_t>(), exists, z, counts, counts + 1);
     unsigned long long hc[2] = {0, 0};
     read_back(s, {{hc, counts, 16}});
@@ -821,13 +842,17 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
 namespace {
 
 // Weighted out-degree of every compact source from the edges in sweep order.
-__global__ void sweep_wdeg_kernel(const int32_t *src, const uint32_t *emap, uint64_t m,
-                                  const float *w, const double *w64, double *wdeg) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
-         i += (uint64_t)gridDim.x * blockDim.x) {
+__global__ __launch_bounds__(kAggThreads) void sweep_wdeg_kernel(const int32_t *src, const uint32_t *emap,
+                                                                 uint64_t m, const float *w,
+                                                                 const double *w64, double *wdeg) {
+    __shared__ AggTable agg;
+    agg.clear();
+    for (uint64_t i = (uint64_t)blockIdx.x * kAggThreads + threadIdx.x; i < m;
+         i += (uint64_t)gridDim.x * kAggThreads) {
         const uint32_t o = emap[i];
-        atomicAdd(&wdeg[src[i]], w64 ? w64[o] : (double)w[o]);
+        agg.add((uint32_t)src[i], w64 ? w64[o] : (double)w[o], nullptr, wdeg);
     }
+    agg.flush(nullptr, wdeg);
 }
 
 __global__ void gather_wdeg_kernel(const double *wdeg_z, const int32_t *perm, uint32_t n,
@@ -899,8 +924,7 @@ void set_weights(nkpr_graph *g, const float *w, const double *w64, const double 
         g->unit_degrees = false;
         NKPR_HIP(hipMemsetAsync(deg.p, 0, 8 * std::max<uint32_t>(n, 1), s));
         if (m)
-            hipLaunchKernelGGL(sweep_wdeg_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(m), 65536)),
-                               dim3(256), 0, s, g->src.as<int32_t>(), g->emap.as<uint32_t>(), m, w,
+            hipLaunchKernelGGL(sweep_wdeg_kernel, dim3(agg_blocks(m)), dim3(kAggThreads), 0, s, g->src.as<int32_t>(), g->emap.as<uint32_t>(), m, w,
                                w64, deg.as<double>());
     }
     NKPR_HIP(hipGetLastError());

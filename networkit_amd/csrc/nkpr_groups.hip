@@ -439,7 +439,7 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
                     SweepArgs<float> a = args32();
                     a.base_vec = nullptr;
                     a.tele = 0.0;
-                    launch_product(rc, a, folded ? v : kr.vh, v, dist ? kr.y : w, nullptr, timing, &st->ms_sweeps_fp32);
+                    apply_product(rc, a, folded ? v : kr.vh, v, dist ? kr.y : w, timing, &st->ms_sweeps_fp32);
                 }
                 if (dist) {
                     PhaseRule r0{};
@@ -476,7 +476,7 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
                 read_back(s, {{&hf, flag, 4}});
                 closed = hf == 0;
             }
-            if (closed) ensure_rowsum64(g);
+            if (closed) ensure_rowsum64(g, rc.combine_grid);
             for (int round = 0;; ++round) {
                 const bool closed_round = closed && round == 0;
                 start_base<double>(q, xcur, g->base64.as<double>(), damp);

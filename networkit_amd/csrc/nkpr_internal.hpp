@@ -260,9 +260,7 @@ void launch_to_double(const float *x32, double *x64, uint32_t n, hipStream_t s);
 void launch_add_correction(double *x64, const float *e32, uint32_t n, hipStream_t s);
 void launch_set_correction(double *x64, double c, const float *e32, uint32_t n, hipStream_t s);
 void launch_copy_f32(const float *in, float *out, uint32_t n, hipStream_t s);
-// rowsum[u] = sum of the in-coefficients of u (FP64), from the plain CSC copy
-void launch_rowsum64(const uint32_t *rowptr, uint32_t n, const int32_t *src, const double *coef,
-                     const double *inv, double *rowsum, hipStream_t s);
+void launch_fill(double *x, uint32_t n, double v, hipStream_t s);
 // flag (device) = 1 when x[0, n) is not constant
 void launch_constant_check(const double *x, uint32_t n, uint32_t *flag, hipStream_t s);
 // residual sweep from a constant vector c in closed form (ynew, r32 and the block partials
@@ -339,6 +337,8 @@ struct BatchTune {
     uint32_t heavy;
 };
 void batch_layout(nkpr_graph *g);
+// row offsets and slot map of the plain copy on the host (b_rowptr_host, b_iperm_host)
+void batch_host_lists(nkpr_graph *g);
 void batch_split(nkpr_graph *g, uint32_t heavy);
 void ensure_buf(DevBuf &b, size_t bytes);
 // Binned FP32 operator of the GMRES corrections (nkpr_binned.hip).
@@ -495,10 +495,9 @@ struct nkpr_graph {
     bool op_pending = false;
 
     // batched personalised PageRank: plain CSC copy and its row split (built on first use)
-    bool b_ready = false, b_split_ready = false, b_coef_ready = false;
+    bool b_ready = false, b_split_ready = false, b_coef_ready = false, b_host_ready = false;
     nkpr::DevBuf b_rowptr, b_src, b_coef32, b_coef64;
     std::vector<uint32_t> b_rowptr_host;
-    std::vector<int32_t> b_perm_host;
     std::vector<int32_t> b_iperm_host;  // [z]: compact id of a slot, -1 without a node
     uint32_t b_heavy = 0, b_n_light = 0, b_n_heavy = 0, b_n_pieces = 0;
     nkpr::DevBuf b_light, b_hrow, b_hpiece, b_pieces;

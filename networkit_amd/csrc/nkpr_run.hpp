@@ -164,22 +164,18 @@ uint64_t run_phase(RunCtx &rc, SweepArgs<T> a, Vecs<T> v, int kind, PhaseRule ru
     return done_sweeps;
 }
 
-// One FP32 sweep as a product (no reductions, no rule, no host read): the operator of a correction
-// solve on graphs without a binned copy.  The claim counters must be zero (launch_init_ctl).  With
-// `timing` its time reaches *ms_acc as a binned application's does (see collect_op_timing).
-inline void launch_product(RunCtx &rc, SweepArgs<float> a, const float *xg, const float *xold,
-                           float *xnew, float *xhat_new, bool timing, double *ms_acc) {
-    nkpr_graph *g = rc.g;
-    if (rc.p->interrupt && *rc.p->interrupt) throw Error(NKPR_ERR_INTERRUPTED, "interrupted");
-    int &workers = rc.workers[0][kSweepPlain][g->weighted];
-    if (workers <= 0) workers = sweep_workers(g, false, g->weighted, kSweepPlain);
+// One sweep as a product (no reductions, no rule, no host read), `events` (two, or nullptr) around
+// it.  The claim counters must be zero (launch_init_ctl).
+template <typename T>
+void launch_product(nkpr_graph *g, SweepArgs<T> a, int workers, int combine_grid, const T *xg,
+                    const T *xold, T *xnew, T *xhat_new, const hipEvent_t *events) {
     FinalizeArgs f{};
     f.split_rows = g->split_rows.as<uint32_t>();
     f.split_first = g->split_first.as<uint32_t>();
     f.split_count = g->split_count.as<uint32_t>();
     f.n_split_rows = g->n_split_rows;
     // only rows with split segments need the last block
-    if (f.n_split_rows) f.n_blocks = (uint32_t)(workers * g->n_slices + (g->n_s ? rc.combine_grid : 0));
+    if (f.n_split_rows) f.n_blocks = (uint32_t)(workers * g->n_slices + (g->n_s ? combine_grid : 0));
     f.rule.kind = kRuleStep;
     f.rule.max_iterations = 1;
     ensure(g->partials, 8 * 4 * (size_t)std::max<uint32_t>(f.n_blocks, 1));
@@ -190,13 +186,24 @@ inline void launch_product(RunCtx &rc, SweepArgs<float> a, const float *xg, cons
     a.xnew = xnew;
     a.xg = xg;
     a.xhat_new = xhat_new;
+    launch_sweep<T>(a, f, kSweepPlain, g->weighted, combine_grid, g->stream, events ? events[0] : nullptr,
+                    events ? events[1] : nullptr);
+}
+
+// The operator of a correction solve on graphs without a binned copy: one FP32 product.  With
+// `timing` its time reaches *ms_acc as a binned application's does (see collect_op_timing).
+inline void apply_product(RunCtx &rc, const SweepArgs<float> &a, const float *xg, const float *xold,
+                          float *xnew, bool timing, double *ms_acc) {
+    nkpr_graph *g = rc.g;
+    if (rc.p->interrupt && *rc.p->interrupt) throw Error(NKPR_ERR_INTERRUPTED, "interrupted");
+    int &workers = rc.workers[0][kSweepPlain][g->weighted];
+    if (workers <= 0) workers = sweep_workers(g, false, g->weighted, kSweepPlain);
     if (timing) {
         collect_op_timing(g, ms_acc);
         for (hipEvent_t &e : g->op_ev)
             if (!e) NKPR_HIP(hipEventCreate(&e));
     }
-    launch_sweep<float>(a, f, kSweepPlain, g->weighted, rc.combine_grid, g->stream,
-                        timing ? g->op_ev[0] : nullptr, timing ? g->op_ev[1] : nullptr);
+    launch_product<float>(g, a, workers, rc.combine_grid, xg, xold, xnew, nullptr, timing ? g->op_ev : nullptr);
     g->op_pending = timing;
 }
 
@@ -234,7 +241,7 @@ bool closed_start_enabled();
 SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64,
                        const float *base32, nkpr_stats *st, const double *start_const = nullptr);
 Krylov krylov_setup(nkpr_graph *g);
-void ensure_rowsum64(nkpr_graph *g);
+void ensure_rowsum64(nkpr_graph *g, int combine_grid);
 void apply_operator(RunCtx &rc, const float *v, float *w, const Krylov &kr, bool timing,
                     double *ms_acc, bool minus);
 bool apply_binned(nkpr_graph *g, const float *v, float *w, double damp, bool distribute,

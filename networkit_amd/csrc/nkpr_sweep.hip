@@ -610,19 +610,9 @@ __global__ void set_correction_kernel(double *x64, double c, const float *e32, u
     if (i < n) x64[i] = c + (double)e32[i];
 }
 
-// rowsum[u] = the FP64 sum of row u's in-coefficients, c_vu = w_vu / deg_v (coef) or 1 / deg_v
-// (inv[v]): one wave per row, lanes strided over the row, then a fixed shuffle tree.
-__global__ void rowsum_kernel(const uint32_t *rowptr, uint32_t n, const int32_t *src,
-                              const double *coef, const double *inv, double *rowsum) {
-    const int lane = threadIdx.x & 63;
-    const uint64_t nw = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    for (uint64_t u = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; u < n; u += nw) {
-        double sum = 0.0;
-        for (uint32_t e = rowptr[u] + lane; e < rowptr[u + 1]; e += 64)
-            sum += coef ? coef[e] : inv[src[e]];
-        for (int off = 32; off > 0; off >>= 1) sum += __shfl_xor(sum, off, 64);
-        if (lane == 0) rowsum[u] = sum;
-    }
+__global__ void fill_kernel(double *x, uint32_t n, double v) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) x[i] = v;
 }
 
 // flag = 1 when some x[u], u < n, differs from x[0]
@@ -880,11 +870,9 @@ void launch_set_correction(double *x64, double c, const float *e32, uint32_t n, 
     NKPR_HIP(hipGetLastError());
 }
 
-void launch_rowsum64(const uint32_t *rowptr, uint32_t n, const int32_t *src, const double *coef,
-                     const double *inv, double *rowsum, hipStream_t s) {
+void launch_fill(double *x, uint32_t n, double v, hipStream_t s) {
     if (!n) return;
-    const unsigned grid = (unsigned)std::min<uint64_t>(((uint64_t)n * 64 + 255) / 256, 1u << 16);
-    hipLaunchKernelGGL(rowsum_kernel, dim3(grid), dim3(256), 0, s, rowptr, n, src, coef, inv, rowsum);
+    hipLaunchKernelGGL(fill_kernel, dim3(grid1d(n)), dim3(256), 0, s, x, n, v);
     NKPR_HIP(hipGetLastError());
 }
 
