@@ -6,10 +6,10 @@
 //            every neighbour v (out-list order) gets mass = (1 - alpha) res w / (2 vol) and is
 //            queued when its residual crosses eps vol(v); p[u] += alpha res;
 //            r[u] = (1 - alpha) res / 2, queued again when r[u] / vol >= eps.
-// Here all queued nodes push at once, round after round (a frontier), a wave per node:
+// Here all queued nodes push at once, round after round (a frontier):
 //   a first kernel takes every frontier node's residual (so that mass arriving during the
-//   round stays for the next one, whatever the schedule), then a wave per node adds alpha res
-//   to p, sends the masses with atomic adds and keeps (1 - alpha) res / 2; a node whose
+//   round stays for the next one, whatever the schedule), adds alpha res to p and keeps
+//   (1 - alpha) res / 2; then a lane group per node sends the masses with atomic adds; a node whose
 //   residual crosses its threshold through an add is appended to the next frontier once (a
 //   flag bit per node).
 // Residuals are 64-bit fixed point (2^-62 units; the total mass is at most 1), so the atomic
@@ -28,7 +28,7 @@
 //
 // Layout: the graph's out-lists (forNeighborsOf order) as CSR with int32 ids and optional FP64
 // weights, vol[z] computed once; p[z] (FP64), r[z] (fixed point), flags[z] (bit 0 touched, bit 1
-// queued), two frontier arrays and the taken residuals.  Only the touched entries are cleared
+// queued), two frontier arrays and what each frontier node pushes.  Only the touched entries are cleared
 // after a run, so a run costs O(z) only for the scan that lists the touched nodes.
 // Algorithmic bytes per push: 4 + 8 (id, weight) and one 8-byte atomic per out-edge, 8 + 8 + 8
 // per pushed node.
@@ -49,7 +49,7 @@ struct nkpr_apr {
     hipStream_t stream = nullptr;
     uint64_t z = 0, m = 0;
     nkpr::DevBuf ptr, dst, w, vol;
-    nkpr::DevBuf p, r, flags, f0, f1, taken, chunks, cnt, out_ids, out_p, out_r, out_cnt, seeds;
+    nkpr::DevBuf p, r, flags, f0, f1, push, chunks, cnt, out_ids, out_p, out_r, out_cnt, seeds;
     uint64_t chunk_cap = 0;  // entries per heavy chunk list (two lists)
     bool dirty = true;  // p, r, flags hold a run that was not cleared
     ~nkpr_apr() {
@@ -62,6 +62,7 @@ namespace {
 
 constexpr uint32_t kTouched = 1, kQueued = 2;
 constexpr int kPushThreads = 256;
+constexpr uint32_t kPushLanes = 32;  // lanes of the push kernel that serve one frontier node
 // rounds per host read of the counters: rounds after the frontier empties return at once, so a
 // longer batch trades a few no-op launches for fewer host reads (RHG n = 10M, 128 rounds:
 // 8.91 ms per run with 8, 8.67 ms with 16, 8.51 ms with 32)
@@ -131,8 +132,16 @@ __global__ void apr_reset_kernel(const uint32_t *ids, const uint32_t *count, dou
 // chunk lists alternate the same way (sizes cnt[kCntChunks + (k & 1)]).  [4..5] the out-edges
 // of the pushed nodes, [6..7] the pushes, [8] the rounds with a non-empty frontier.
 constexpr int kCntEdges = 4, kCntPushes = 6, kCntRounds = 8, kCntChunks = 10;
-// A node with more out-edges than kPushChunk is pushed by several waves, kPushChunk edges each.
-constexpr uint32_t kPushChunk = 256;
+// A node with more out-edges than kPushChunk is pushed by several lane groups, kPushChunk edges each.
+constexpr uint32_t kPushChunk = 64;
+
+// What the push of a frontier node needs, gathered by the take kernel: the push then starts its
+// edge loads after one read instead of three dependent ones.
+struct Push {
+    uint64_t first;  // its out-edges [first, first + count)
+    uint32_t count, node;
+    double share;    // (1 - alpha) res / (2 vol): the mass per unit of weight
+};
 
 // the seeds: residual 1/|seeds|, touched, queued, in frontier 0 (ids ascending)
 __global__ void apr_seed_kernel(const uint32_t *seeds, uint32_t k, uint64_t *r, uint32_t *flags,
@@ -159,13 +168,13 @@ __device__ __forceinline__ void append_wave(bool append, uint32_t v, uint32_t *n
     if (append) next[base + (uint32_t)__popcll(ball & ((1ull << lane) - 1))] = v;
 }
 
-// Round k, first kernel: a thread per frontier node u takes its residual res (kept in taken[]),
-// adds alpha res to p[u] and leaves (1 - alpha) res / 2 in r[u], appending u to the next
-// frontier when that alone reaches its threshold; a node with more than kPushChunk out-edges
-// lists its chunks for the push kernel.  The push kernel then only adds to residuals.
+// Round k, first kernel: a thread per frontier node u takes its residual res, adds alpha res to p[u]
+// and leaves (1 - alpha) res / 2 in r[u], appending u to the next frontier when that alone reaches
+// its threshold; a node with more than kPushChunk out-edges lists its chunks for the push kernel,
+// which then only adds to residuals.
 __global__ void apr_take_kernel(const uint64_t *ptr, const double *vol, double alpha, double eps,
                                 const uint32_t *front, uint32_t *next, uint32_t *cnt, int k3,
-                                int k2, double *p, uint64_t *r, uint32_t *flags, uint64_t *taken,
+                                int k2, double *p, uint64_t *r, uint32_t *flags, Push *push,
                                 uint2 *chunks) {
     __shared__ unsigned long long bedges;
     const uint32_t nf = cnt[k3];
@@ -189,15 +198,20 @@ __global__ void apr_take_kernel(const uint64_t *ptr, const double *vol, double a
         uint32_t u = 0;
         if (i < nf) {
             u = front[i];
-            const uint64_t res = r[u];
-            taken[i] = res;
+            const uint64_t res = r[u], b = ptr[u], deg = ptr[u + 1] - b;
+            const double vu = vol[u], pu = p[u];
             const double dres = (double)res;
-            p[u] += alpha * dres / kUnit;
+            p[u] = pu + alpha * dres / kUnit;
             const uint64_t keep = __double2ull_rn((1.0 - alpha) * dres / 2);
             r[u] = keep;
-            again = keep >= threshold_of(eps, vol[u], true);
+            again = keep >= threshold_of(eps, vu, true);
             flags[u] = again ? (kTouched | kQueued) : kTouched;
-            const uint64_t deg = ptr[u + 1] - ptr[u];
+            Push o;
+            o.first = b;
+            o.count = (uint32_t)deg;
+            o.node = u;
+            o.share = vu > 0.0 ? (1.0 - alpha) * dres / (2.0 * vu) : 0.0;
+            push[i] = o;
             atomicAdd(&bedges, (unsigned long long)deg);
             if (deg > kPushChunk) {
                 const uint32_t nc = (uint32_t)((deg + kPushChunk - 1) / kPushChunk);
@@ -212,55 +226,71 @@ __global__ void apr_take_kernel(const uint64_t *ptr, const double *vol, double a
         atomicAdd(reinterpret_cast<unsigned long long *>(cnt + kCntEdges), bedges);
 }
 
-// Round k, second kernel: a wave per frontier node with at most kPushChunk out-edges and a wave
+// Round k, second kernel: a lane group per frontier node with at most kPushChunk out-edges and one
 // per chunk of the others sends the masses (1 - alpha) res w / (2 vol).  At the start of the
 // kernel every residual lies below its threshold unless its node is already queued, and all
 // adds are positive, so the add that crosses a threshold is the one that finds the residual
 // below it and leaves it at or above it; that add sets the node's queued bit.
+//
+// Bound by latency: a round is a few thousand edges.  The returning add is issued before the
+// threshold is formed, so that it and the load of vol[v] are in flight together; only an add that
+// finds no residual marks the node touched (one that holds some was marked by an earlier add);
+// a block collects what it appends in LDS and takes its places in the next frontier with one
+// add, where a wave each queued on that counter.  13.0 us per round before, 8.0 now (hyperbolic
+// graph of 2e6 nodes, eps 1e-8).
 __global__ __launch_bounds__(kPushThreads) void apr_push_kernel(
-    const uint64_t *ptr, const int32_t *dst, const double *w, const double *vol, double alpha,
-    double eps, uint64_t *r, uint32_t *flags, const uint32_t *front, const uint64_t *taken,
-    const uint2 *chunks, uint32_t *next, uint32_t *cnt, int k3, int k2) {
+    const int32_t *dst, const double *w, const double *vol, double eps, uint64_t *r, uint32_t *flags,
+    const Push *push, const uint2 *chunks, uint32_t *next, uint32_t *cnt, int k3, int k2) {
+    constexpr uint32_t kGroups = kPushThreads / kPushLanes;
+    __shared__ uint32_t list[kGroups * kPushChunk];
+    __shared__ uint32_t n_list, base;
     const uint32_t nf = cnt[k3], nh = cnt[kCntChunks + k2];
     uint32_t *ncnt = cnt + (k3 + 1) % 3;
-    const int lane = threadIdx.x & 63;
-    const uint32_t nw = (gridDim.x * blockDim.x) >> 6;
-    for (uint32_t t = (blockIdx.x * blockDim.x + threadIdx.x) >> 6; t < nf + nh; t += nw) {
-        uint32_t i;
-        uint64_t b, end;
+    const uint32_t lane = threadIdx.x % kPushLanes;
+    if (threadIdx.x == 0) n_list = 0;
+    __syncthreads();
+    for (uint32_t t0 = blockIdx.x * kGroups; t0 < nf + nh; t0 += gridDim.x * kGroups) {
+        const uint32_t t = t0 + threadIdx.x / kPushLanes;
+        uint64_t b = 0, end = 0;
+        uint32_t u = 0;
+        double share = 0.0;
         if (t < nf) {
-            i = t;
-            const uint32_t u = front[i];
-            b = ptr[u];
-            end = ptr[u + 1];
-            if (end - b > kPushChunk) continue;  // pushed by its chunks
-        } else {
+            const Push o = push[t];
+            u = o.node;
+            share = o.share;
+            b = o.first;
+            end = o.count > kPushChunk ? b : b + o.count;  // the others are pushed by their chunks
+        } else if (t < nf + nh) {
             const uint2 c = chunks[t - nf];
-            i = c.x;
-            const uint32_t u = front[i];
-            b = ptr[u] + (uint64_t)c.y * kPushChunk;
-            end = std::min<uint64_t>(ptr[u + 1], b + kPushChunk);
+            const Push o = push[c.x];
+            u = o.node;
+            share = o.share;
+            b = o.first + (uint64_t)c.y * kPushChunk;
+            end = std::min<uint64_t>(o.first + o.count, b + kPushChunk);
         }
-        const uint32_t u = front[i];
-        const double vu = vol[u];
-        const double share = vu > 0.0 ? (1.0 - alpha) * (double)taken[i] / (2.0 * vu) : 0.0;
-        for (uint64_t e0 = b; e0 < end; e0 += 64) {
-            const uint64_t e = e0 + lane;
-            bool append = false;
-            uint32_t v = 0;
+        for (uint64_t e = b + lane; e < end; e += kPushLanes) {
+            const uint32_t v = (uint32_t)dst[e];
             // a self-loop sends nothing: the reference overwrites r[u] after its loop
-            if (e < end && (v = (uint32_t)dst[e]) != u) {
-                const uint64_t mass = __double2ull_rn(share * (w ? w[e] : 1.0));
-                const uint64_t thr = threshold_of(eps, vol[v], false);
-                const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long *>(&r[v]),
-                                               (unsigned long long)mass);
-                if (old < thr && old + mass >= thr)
-                    append = !(atomicOr(&flags[v], kQueued | kTouched) & kQueued);
-                else if (!(flags[v] & kTouched))
-                    atomicOr(&flags[v], kTouched);
+            if (v == u) continue;
+            const uint64_t mass = __double2ull_rn(share * (w ? w[e] : 1.0));
+            const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long *>(&r[v]),
+                                           (unsigned long long)mass);
+            const uint64_t thr = threshold_of(eps, vol[v], false);
+            if (old < thr && old + mass >= thr) {
+                if (!(atomicOr(&flags[v], kQueued | kTouched) & kQueued)) list[atomicAdd(&n_list, 1u)] = v;
+            } else if (old == 0) {
+                atomicOr(&flags[v], kTouched);
             }
-            append_wave(append, v, next, ncnt);
         }
+        __syncthreads();
+        const uint32_t k = n_list;
+        if (k) {
+            if (threadIdx.x == 0) base = atomicAdd(ncnt, k);
+            __syncthreads();
+            for (uint32_t i = threadIdx.x; i < k; i += kPushThreads) next[base + i] = list[i];
+            if (threadIdx.x == 0) n_list = 0;
+        }
+        __syncthreads();
     }
 }
 
@@ -371,7 +401,7 @@ void apr_create_impl(uint64_t z, const uint64_t *ptr, const int32_t *dst, const 
     a->flags.alloc(4 * z);
     a->f0.alloc(4 * z);
     a->f1.alloc(4 * z);
-    a->taken.alloc(8 * z);
+    a->push.alloc(sizeof(Push) * z);
     // chunks of the nodes with more than kPushChunk out-edges: at most 2 deg / kPushChunk per node
     a->chunk_cap = 2 * m / kPushChunk + 64;
     a->chunks.alloc(2 * 8 * a->chunk_cap);
@@ -451,11 +481,10 @@ void apr_run_impl(nkpr_apr *a, double alpha, double eps, const uint64_t *seeds, 
                                a->ptr.as<uint64_t>(), a->vol.as<double>(), alpha, eps,
                                front[k2], front[k2 ^ 1], a->cnt.as<uint32_t>(), k3, k2,
                                a->p.as<double>(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(),
-                               a->taken.as<uint64_t>(), a->chunks.as<uint2>() + (k2 ? a->chunk_cap : 0));
+                               a->push.as<Push>(), a->chunks.as<uint2>() + (k2 ? a->chunk_cap : 0));
             hipLaunchKernelGGL(apr_push_kernel, dim3(grid), dim3(kPushThreads), 0, s,
-                               a->ptr.as<uint64_t>(), a->dst.as<int32_t>(), a->w.as<double>(),
-                               a->vol.as<double>(), alpha, eps, a->r.as<uint64_t>(),
-                               a->flags.as<uint32_t>(), front[k2], a->taken.as<uint64_t>(),
+                               a->dst.as<int32_t>(), a->w.as<double>(), a->vol.as<double>(), eps,
+                               a->r.as<uint64_t>(), a->flags.as<uint32_t>(), a->push.as<Push>(),
                                a->chunks.as<uint2>() + (k2 ? a->chunk_cap : 0), front[k2 ^ 1],
                                a->cnt.as<uint32_t>(), k3, k2);
         }
