@@ -92,10 +92,20 @@ constexpr int kP2HotQuads = NKPR_P2H_QUADS;
 
 // Control words of one application: the largest |x| of the sources (the bits of a
 // non-negative double order like unsigned integers) and the queue counters of the passes.
+// Applications use two of them in turn, and pass 1 of one clears the other for the next, which
+// saves a launch of its own.
 struct BinCtl {
     unsigned long long vmax;
     uint32_t q1, q2;
 };
+
+__device__ __forceinline__ void clear_ctl(BinCtl *ctl) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        ctl->vmax = 0ull;
+        ctl->q1 = 0u;
+        ctl->q2 = 0u;
+    }
+}
 
 // The fixed-point scale is 2^e with every row sum below 2^61 units:
 // |sum| <= max|x| * max_u sum_in coef(u) = bound.  e stays within [-126, 126] so that 2^e is a
@@ -338,11 +348,8 @@ __global__ void bin_insum_kernel(const uint32_t *rowptr, uint32_t n, const int32
 }
 
 __global__ void bin_clear_kernel(BinCtl *ctl) {
-    if (threadIdx.x == 0) {
-        ctl->vmax = 0ull;
-        ctl->q1 = 0u;
-        ctl->q2 = 0u;
-    }
+    clear_ctl(ctl);
+    clear_ctl(ctl + 1);
 }
 
 // The passes run persistent blocks, as many as fit on the device; a block takes the next work
@@ -421,7 +428,8 @@ __global__ __launch_bounds__(kPassThreads) void bin_scatter_kernel(
     const uint4 *items, uint32_t nitems, const float *v, const float *inv, uint32_t n,
     const uint16_t *bsrc, const float *bcoef, const uint32_t *pos, const unsigned long long *gmask,
     const uint32_t *gfirst, const uint32_t *sdelta, uint32_t nsd, uint32_t mp, float *bval,
-    BinCtl *ctl) {
+    BinCtl *ctl, BinCtl *next) {
+    clear_ctl(next);
     constexpr uint32_t kSpan = 1u << kSpan32Shift;
     __shared__ __align__(16) float tab[kSpan + 1];
     __shared__ uint32_t slot;
@@ -725,7 +733,7 @@ struct Epi64 {
     const PhaseCtl *pctl;
     double damp, tele;
     uint32_t n, sink_begin;
-    int32_t distribute;
+    int32_t distribute, norm_only;
     int lo_shift;            // fraction bits of the low accumulator word
 };
 
@@ -746,15 +754,16 @@ __device__ __forceinline__ Row64 load_row64(const Epi64 &e, uint32_t u) {
 
 // The finished row u from its accumulated product y (the pull sweep's epilogue_store).
 __device__ __forceinline__ void finish_row64(const Epi64 &e, uint32_t u, double y, double c,
-                                             const Row64 &in, double (&s)[4]) {
-    double x = e.damp * y + c;
+                                             const Row64 &in, double damp, double (&s)[4]) {
+    double x = damp * y + c;
     if (e.base_vec) x += in.bv;
     __builtin_nontemporal_store(x, e.xnew + u);
     if (e.xhat_new != nullptr && u < e.sink_begin) __builtin_nontemporal_store(x * in.iv, e.xhat_new + u);
     const double dif = x - in.xo;
     if (e.r32) __builtin_nontemporal_store((float)dif, e.r32 + u);
+    const double t = e.norm_only ? x : dif;
     s[0] += fabs(dif);
-    s[1] += dif * dif;
+    s[1] += t * t;
     s[2] += x;
     if (u >= e.sink_begin) s[3] += x;
 }
@@ -826,8 +835,9 @@ __global__ __launch_bounds__(kPassThreads) void bin_scatter64_kernel(
     const uint4 *items, uint32_t nitems, const double *x, const double *inv, uint32_t n,
     const uint16_t *bsrc, const CT *bcoef, const uint32_t *pos, const unsigned long long *gmask,
     const uint32_t *gfirst, const uint32_t *sdelta, uint32_t nsd, double *bval, uint64_t mp,
-    BinCtl *ctl, const PhaseCtl *pctl) {
+    BinCtl *ctl, BinCtl *next, const PhaseCtl *pctl) {
     constexpr uint32_t kSpan = 1u << kSpan64Shift;
+    clear_ctl(next);
     if (pctl->done) return;
     __shared__ __align__(16) double tab[kSpan + 1];
     __shared__ uint32_t slot;
@@ -929,7 +939,7 @@ __global__ __launch_bounds__(kPassThreads) void bin_gather64_kernel(
     const int ex = fixed_exponent(ctl, insum);
     const double scale = ldexp(1.0, ex), unscale = ldexp(1.0, -ex);
     const double lscale = ldexp(1.0, e.lo_shift), lunscale = ldexp(1.0, -e.lo_shift);
-    const double c = rhs_const64(e);
+    const double c = rhs_const64(e), damp = e.damp * e.pctl->scale;
     const uint32_t n = e.n;
     for (uint32_t it = next_item(&ctl->q2, &slot); it < nitems; it = next_item(&ctl->q2, &slot)) {
         const uint4 item = items[it];
@@ -969,7 +979,7 @@ __global__ __launch_bounds__(kPassThreads) void bin_gather64_kernel(
                 const uint32_t u = base + i;
                 if (u >= n) break;
                 const double y = ((double)(long long)acc_hi[i] + (double)(long long)acc_lo[i] * lunscale) * unscale;
-                finish_row64(e, u, y, c, in[k], s);
+                finish_row64(e, u, y, c, in[k], damp, s);
             }
             block_partials<kPassThreads>(s, e.partials, item.w >> 2);
         } else {
@@ -1007,7 +1017,8 @@ __global__ __launch_bounds__(kReduce64Threads) void bin_reduce64_kernel(
             hi += p[0];
             lo += p[1];
         }
-        finish_row64(e, u, ((double)hi + (double)lo * lunscale) * unscale, c, load_row64(e, u), s);
+        finish_row64(e, u, ((double)hi + (double)lo * lunscale) * unscale, c, load_row64(e, u),
+                     e.damp * e.pctl->scale, s);
     }
     block_partials<kReduce64Threads>(s, e.partials, b.w + j);
 }
@@ -1398,7 +1409,10 @@ bool build_layout(nkpr_graph *g, BinLayout &L) {
     L.part.alloc((L.fp64 ? 16 : 8) * (size_t)std::max<uint32_t>(slots, 1) * kBin);
     if (L.fp64) L.partials.alloc(32 * (size_t)std::max<uint32_t>(pslots, 1));
     binned_insum(g, L);
-    L.ctl.alloc(sizeof(BinCtl));
+    L.ctl.alloc(2 * sizeof(BinCtl));
+    hipLaunchKernelGGL(bin_clear_kernel, dim3(1), dim3(64), 0, s, L.ctl.as<BinCtl>());
+    NKPR_HIP(hipGetLastError());
+    L.turn = 0;
     NKPR_HIP(hipStreamSynchronize(s));
     if (std::getenv("NKPR_DEBUG"))
         std::fprintf(stderr, "[nkpr] binned %s layout: %u chunks x %u bins, %llu padded edges, %llu hot entries (%u hot sources), %u + %u items (%u split)\n",
@@ -1489,8 +1503,8 @@ void binned_apply(nkpr_graph *g, const float *v, float *w, double damp, bool dis
     const auto gather = L.hot ? bin_gather_kernel<true> : bin_gather_kernel<false>;
     persistent_grids(g, L, bin_scatter_kernel<true>, gather);
     if (ev0) NKPR_HIP(hipEventRecord(ev0, s));
-    BinCtl *ctl = L.ctl.as<BinCtl>();
-    hipLaunchKernelGGL(bin_clear_kernel, dim3(1), dim3(64), 0, s, ctl);
+    BinCtl *ctl = L.ctl.as<BinCtl>() + (L.turn & 1), *next = L.ctl.as<BinCtl>() + (~L.turn & 1);
+    ++L.turn;
     const auto scatter = derived ? bin_scatter_kernel<true> : bin_scatter_kernel<false>;
     // the sources at or past sink_begin have no out-edges: pass 1 reads them as 0, so v may hold
     // anything there (GMRES keeps other data past its head) and the scale ignores it
@@ -1499,7 +1513,7 @@ void binned_apply(nkpr_graph *g, const float *v, float *w, double damp, bool dis
                        g->weighted ? nullptr : g->inv32.as<float>(), g->sink_begin, L.src.as<uint16_t>(),
                        g->weighted ? L.coef.as<float>() : nullptr, L.pos.as<uint32_t>(),
                        L.gmask.as<unsigned long long>(), L.gfirst.as<uint32_t>(), L.sdelta.as<uint32_t>(),
-                       L.nsdelta, (uint32_t)L.mp, L.val.as<float>(), ctl);
+                       L.nsdelta, (uint32_t)L.mp, L.val.as<float>(), ctl, next);
     hipLaunchKernelGGL(gather, dim3(std::min<uint32_t>(std::max<uint32_t>(L.np2, 1), L.grid2)),
                        dim3(kPassThreads), 0, s, L.p2.as<uint4>(), L.np2, L.dst.as<uint16_t>(),
                        L.val.as<float>(), L.part.as<long long>(), n, ctl, L.insum, v, minus, (float)damp,
@@ -1549,15 +1563,16 @@ void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArg
     e.n = n;
     e.sink_begin = a.sink_begin;
     e.distribute = a.distribute;
+    e.norm_only = a.norm_only;
     // fraction bits of the low word: a row's fractions (each below 2^lo_shift in magnitude)
     // must sum below 2^63
     int deg_bits = 0;
     while (deg_bits < 40 && (1ull << deg_bits) <= (uint64_t)g->max_in_degree) ++deg_bits;
     e.lo_shift = std::min(40, 62 - deg_bits);
     if (ev0) NKPR_HIP(hipEventRecord(ev0, s));
-    BinCtl *ctl = L.ctl.as<BinCtl>();
-    hipLaunchKernelGGL(bin_clear_kernel, dim3(1), dim3(64), 0, s, ctl);
+    BinCtl *ctl = L.ctl.as<BinCtl>() + (L.turn & 1), *next = L.ctl.as<BinCtl>() + (~L.turn & 1);
     if (n) {
+        ++L.turn;
         const dim3 g1(std::min<uint32_t>(std::max<uint32_t>(L.np1, 1), L.grid1));
         const dim3 g2(std::min<uint32_t>(std::max<uint32_t>(L.np2, 1), L.grid2));
         const double *inv = L.w32 ? (const double *)g->invw64.as<double>()
@@ -1567,7 +1582,7 @@ void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArg
                                L.src.as<uint16_t>(), coef, L.pos.as<uint32_t>(),
                                (const unsigned long long *)L.gmask.as<unsigned long long>(),
                                (const uint32_t *)L.gfirst.as<uint32_t>(), (const uint32_t *)L.sdelta.as<uint32_t>(),
-                               L.nsdelta, L.val.as<double>(), L.mp, ctl, (const PhaseCtl *)a.ctl);
+                               L.nsdelta, L.val.as<double>(), L.mp, ctl, next, (const PhaseCtl *)a.ctl);
         };
         const float *w32 = (const float *)L.coef.as<float>();
         const double *c64 = g->weighted ? (const double *)L.coef.as<double>() : nullptr;

@@ -152,7 +152,9 @@ struct PhaseCtl {
     double bound;     // certified L1 error bound (ERR rule)
     uint64_t iterations;
     uint32_t done;
-    uint32_t pad;
+    uint32_t bad;     // the norm is not finite (kRuleNorm)
+    double len, prev_len;  // ||x'||_2 of the last sweep and of the one before (kRuleNorm)
+    double scale;     // factor of the next sweep's product: 1, or 1 / len (kRuleNorm, rescale)
 };
 
 // Stopping rules evaluated by the finalize kernel.
@@ -160,6 +162,7 @@ enum RuleKind : int32_t {
     kRuleStep = 0,       // reference: step in `norm` <= tol
     kRuleErr = 1,        // 2 d/(1-d) l1 / sum <= tol
     kRuleAbsStall = 2,   // l1 <= tol_abs, or the step stopped shrinking (rounding floor)
+    kRuleNorm = 3,       // | ||x'||_2 - its previous value | <= tol (eigenvector, Katz)
 };
 
 struct PhaseRule {
@@ -170,6 +173,7 @@ struct PhaseRule {
     double stall_ratio;
     uint64_t max_iterations;
     double damp;
+    int32_t rescale;  // kRuleNorm: the next sweep's product is divided by the norm
 };
 
 // Device view of the sweep schedule (built once per graph).
@@ -213,6 +217,7 @@ template <typename T> struct SweepArgs {
     uint32_t n;
     uint32_t sink_begin;     // nodes [sink_begin, n) have no out-edges
     int32_t distribute;      // add damp * sink_in / n to every node
+    int32_t norm_only;       // l2 is ||x'||_2^2 instead of the step's (kRuleNorm)
     // FP64 residual sweeps through the binned copy: store each contribution in 6 bytes (an
     // FP32 head and a 16-bit tail, about 40 significant bits) instead of 8
     int32_t compact64;
@@ -422,6 +427,7 @@ struct BinLayout {
     uint32_t nsdelta = 0;
     bool derived = false;
     double insum = 0.0;         // largest in-coefficient sum of a row (fixed-point bound)
+    uint32_t turn = 0;          // application number: which of the two control blocks is in use
     uint32_t np1 = 0, np2 = 0, multi = 0, nmb = 0, nslots = 0, grid1 = 0, grid2 = 0;
     // hot sources (FP32 copy): ids [0, hot) bypass pass 1; their entries per bin, padded to
     // quads (hidx packed offsets, hcoef, horder the edge of each position), the hot range of

@@ -14,9 +14,12 @@
 // themselves as its folded coefficients, so the pull sweep with damp d and right-hand side b
 // computes y = d A x + b: d = 1, b = 0 for the eigenvector; for Katz d = alpha and
 // b[u] = alpha (sum of u's in-weights) + beta, which is alpha A (1 + x) + beta with the terms
-// grouped differently.  After every sweep a hook adds ||y||^2 in a fixed order, compares the
-// norm with the previous one on the device (it sets the phase's stop flag, so the host reads
-// back once per batch of sweeps, as in nkpr_run) and, for the eigenvector, divides y by it.
+// grouped differently.  The sweep's own reductions take ||y||^2 (in a fixed order) and its last
+// block compares the norm with the previous one (kRuleNorm: it sets the phase's stop flag, so the
+// host reads back once per batch of sweeps, as in nkpr_run).  The eigenvector's division by the
+// norm is a factor of the next sweep's product; the vectors themselves stay undivided until the
+// result is written.  As passes of their own the sum of squares and the division took 34 of the
+// 650 us of a binned sweep over 1.3e8 arcs.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -30,92 +33,6 @@
 
 namespace nkpr {
 namespace {
-
-constexpr int kSqThreads = 256;
-constexpr int kSqBlocks = 1024;
-
-// State of the norm test, kept on the device across the sweeps of a run.
-struct PowerState {
-    double len;       // ||y||_2 of the last real sweep
-    double prev;      // the norm of the sweep before
-    double inv;       // 1 / len (the eigenvector's rescaling)
-    uint64_t it;      // real sweeps
-    uint32_t apply;   // the last hook belonged to a real sweep
-    uint32_t bad;     // the norm is not finite (Katz with alpha above 1 / spectral radius)
-};
-
-__device__ __forceinline__ double wave_sum64(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
-}
-
-template <typename T>
-__global__ __launch_bounds__(kSqThreads) void sumsq_kernel(const T *y, uint32_t n,
-                                                            const PhaseCtl *ctl, double *part) {
-    if (ctl->done) return;
-    __shared__ double s_red[kSqThreads / 64];
-    double acc = 0.0;
-    for (uint64_t i = (uint64_t)blockIdx.x * kSqThreads + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * kSqThreads) {
-        const double v = (double)y[i];
-        acc += v * v;
-    }
-    acc = wave_sum64(acc);
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double t = 0.0;
-        for (int w = 0; w < kSqThreads / 64; ++w) t += s_red[w];
-        part[blockIdx.x] = t;
-    }
-}
-
-// One block: the norm of this sweep's y and the stop test |len - prev| <= tol, written in
-// the form of Aux::NumericTools::equal (len <= prev + tol and len >= prev - tol).
-__global__ __launch_bounds__(kSqThreads) void power_decide_kernel(const double *part, int np,
-                                                                   PowerState *ps, PhaseCtl *ctl,
-                                                                   double tol) {
-    if (ctl->done) {
-        if (threadIdx.x == 0) ps->apply = 0u;  // a sweep after the stop: nothing to rescale
-        return;
-    }
-    __shared__ double s_red[kSqThreads / 64];
-    double acc = 0.0;
-    for (int i = threadIdx.x; i < np; i += kSqThreads) acc += part[i];
-    acc = wave_sum64(acc);
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double ss = 0.0;
-        for (int w = 0; w < kSqThreads / 64; ++w) ss += s_red[w];
-        const double len = sqrt(ss);
-        const double prev = ps->len;
-        ps->prev = prev;
-        ps->len = len;
-        ps->inv = 1.0 / len;
-        ps->it += 1;
-        ps->apply = 1u;
-        bool stop = (len <= prev + tol) && (len >= prev - tol);
-        if (!isfinite(len)) {
-            ps->bad = 1u;
-            stop = true;
-        }
-        if (stop) ctl->done = 1u;
-    }
-}
-
-// y *= 1 / len (and the prescaled copy of an unweighted graph) after a real sweep.
-template <typename T>
-__global__ void power_scale_kernel(T *y, T *yh, uint32_t n, const PowerState *ps) {
-    if (!ps->apply) return;
-    const T f = (T)ps->inv;
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x) {
-        y[i] *= f;
-        if (yh) yh[i] *= f;
-    }
-}
 
 __global__ void fill_kernel(double *x, uint64_t count, double v) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < count;
@@ -184,12 +101,6 @@ void power_run_impl(nkpr_graph *g, const nkpr_power_params *p, double *scores, n
         double *xh0 = folded ? nullptr : g->xh64a.as<double>();
         double *xh1 = folded ? nullptr : g->xh64b.as<double>();
         ensure(g->base64, 8 * (size_t)n);
-        ensure(g->red_partials, 8 * (size_t)std::max(kSqBlocks, 1024));
-        DevBuf state;
-        state.alloc(sizeof(PowerState));
-        PowerState *ps = state.as<PowerState>();
-        NKPR_HIP(hipMemsetAsync(ps, 0, sizeof(PowerState), s));
-
         SweepArgs<double> a{};
         a.coef = folded ? g->coef64.as<double>() : nullptr;
         a.inv = folded ? nullptr : g->inv64.as<double>();
@@ -199,7 +110,7 @@ void power_run_impl(nkpr_graph *g, const nkpr_power_params *p, double *scores, n
         a.n = n;
         a.sink_begin = g->sink_begin;
         a.distribute = 0;
-        PhaseRule never{};  // the hook decides; the sweep's own rule never stops
+        PhaseRule never{};  // the sweep of the all-ones vector: no stop
         never.kind = kRuleStep;
         never.norm = NKPR_L1;
         never.tol = -1.0;
@@ -227,39 +138,26 @@ void power_run_impl(nkpr_graph *g, const nkpr_power_params *p, double *scores, n
         a.damp = katz ? p->alpha : 1.0;
         a.base_vec = katz ? g->base64.as<double>() : nullptr;
         const int kind = katz ? kSweepBaseVec : kSweepPlain;
-        double *part = g->red_partials.as<double>();
-        PhaseCtl *ctl = g->ctl.as<PhaseCtl>();
-        auto hook = [&](const double *, double *y) {
-            hipLaunchKernelGGL(sumsq_kernel<double>, dim3(std::min<unsigned>(grid_of(n), kSqBlocks)),
-                               dim3(kSqThreads), 0, s, (const double *)y, n, (const PhaseCtl *)ctl, part);
-            hipLaunchKernelGGL(power_decide_kernel, dim3(1), dim3(kSqThreads), 0, s,
-                               (const double *)part, (int)std::min<unsigned>(grid_of(n), kSqBlocks), ps, ctl,
-                               p->tol);
-            if (!katz) {
-                double *yh = folded ? nullptr : (y == x0 ? xh0 : xh1);
-                hipLaunchKernelGGL(power_scale_kernel<double>, dim3(grid_of(n)), dim3(256), 0, s, y, yh,
-                                   n, (const PowerState *)ps);
-            }
-            NKPR_HIP(hipGetLastError());
-        };
+        a.norm_only = 1;
+        PhaseRule rule = never;
+        rule.kind = kRuleNorm;
+        rule.tol = p->tol;
+        rule.rescale = katz ? 0 : 1;
         start_ones();
         Vecs<double> v{{x0, x1}, {xh0, xh1}};
-        // the sweeps are timed with HIP events (ms_sweeps_fp64), the norm hooks are not
-        const uint64_t total = run_phase<double>(rc, a, v, kind, never,
+        const uint64_t total = run_phase<double>(rc, a, v, kind, rule,
                                                  std::max<uint64_t>(p->max_iterations, 1), true,
-                                                 &st->ms_sweeps_fp64, hook);
-        PowerState hs{};
-        read_back(s, {{&hs, ps, sizeof(PowerState)}});
+                                                 &st->ms_sweeps_fp64);
+        const PhaseCtl hs = *g->ctl_host;
         NKPR_CHECK(!hs.bad, "the iteration diverged (the norm is not finite): alpha must be "
                             "below 1 / the spectral radius of the adjacency matrix");
         const double *y = v.x[total & 1];
         st->iterations = total;
         st->sweeps_fp64 = total;
-        st->last_step = std::fabs(hs.len - hs.prev);
+        st->last_step = std::fabs(hs.len - hs.prev_len);
         st->last_step_l1 = st->last_step;
         st->score_sum = hs.len;
-        // eigenvector: y is already normalised; Katz: divided by the last norm
-        launch_gather_result(y, slot_index(g), z, katz ? hs.len : 1.0, sz, s);
+        launch_gather_result(y, slot_index(g), z, hs.len, sz, s);
         if (!katz) {
             // sign correction on slot 0 (EigenvectorCentrality.cpp:58-63); deleted slots hold 1
             double s0 = 0.0;

@@ -126,8 +126,9 @@ __device__ __forceinline__ void epilogue_store(const SweepArgs<T> &a, uint32_t u
         __builtin_nontemporal_store(y * __builtin_nontemporal_load(a.inv + u), a.xhat_new + u);
     const double dif = (double)y - (double)xo;
     if (RESID) __builtin_nontemporal_store((float)dif, a.r32 + u);
+    const double t = a.norm_only ? (double)y : dif;
     s.l1 += fabs(dif);
-    s.l2 += dif * dif;
+    s.l2 += t * t;
     s.sum += (double)y;
     if (u >= a.sink_begin) s.sink += (double)y;
 }
@@ -338,7 +339,7 @@ template <typename T, bool BASEVEC, bool RESID, int BLOCK>
 __device__ __forceinline__ void finish_sweep(const SweepArgs<T> &a, const FinalizeArgs &f,
                                              double (*s_red)[BLOCK / 64]) {
     PhaseCtl *ctl = a.ctl;
-    const T damp = (T)a.damp;
+    const T damp = (T)(a.damp * a.ctl->scale);
     const T c = rhs_const(a);
     const uint32_t S = a.sc.n_slices, ns = a.sc.n_s;
     // split-row terms first (in row order), then block partials in block order
@@ -388,6 +389,17 @@ __device__ __forceinline__ void finish_sweep(const SweepArgs<T> &a, const Finali
             stop = stop || step <= r.tol;
         } else if (r.kind == kRuleErr) {
             stop = stop || bound <= r.tol;
+        } else if (r.kind == kRuleNorm) {
+            // Aux::NumericTools::equal: len <= prev + tol and len >= prev - tol
+            const double len = sqrt(tot.l2), was = ctl->len;
+            ctl->prev_len = was;
+            ctl->len = len;
+            if (r.rescale) ctl->scale = 1.0 / len;
+            stop = stop || (len <= was + r.tol && len >= was - r.tol);
+            if (!isfinite(len)) {
+                ctl->bad = 1u;
+                stop = true;
+            }
         } else {
             stop = stop || tot.l1 <= r.tol_abs || bound <= r.tol;
             if (it >= 4 && tot.l1 > r.stall_ratio * prev) stop = true;
@@ -419,7 +431,7 @@ __global__ __launch_bounds__(kBlock, (sweep_waves<T, FOLDED>())) void sweep_kern
     __shared__ uint32_t s_worker;
     __shared__ T s_hub[HubTable<T>::size];
 
-    const T damp = (T)a.damp;
+    const T damp = (T)(a.damp * a.ctl->scale);
     const T c = rhs_const(a);
     const uint32_t tid = threadIdx.x;
     const uint32_t S = a.sc.n_slices, K = a.sc.workers;
@@ -523,7 +535,7 @@ __global__ __launch_bounds__(kCombineThreads) void combine_kernel(SweepArgs<T> a
     if (a.ctl->done) return;
     __shared__ double s_red[4][kCombineThreads / 64];
     __shared__ uint32_t s_last;
-    const T damp = (T)a.damp;
+    const T damp = (T)(a.damp * a.ctl->scale);
     const T c = rhs_const(a);
     const uint32_t S = a.sc.n_slices, ns = a.sc.n_s;
     Acc4 st;
@@ -562,7 +574,10 @@ __global__ void init_ctl_kernel(PhaseCtl *ctl, const double *sink_sum, uint32_t 
         ctl->bound = INFINITY;
         ctl->iterations = 0;
         ctl->done = 0;
-        ctl->pad = 0;
+        ctl->bad = 0;
+        ctl->len = 0.0;
+        ctl->prev_len = 0.0;
+        ctl->scale = 1.0;
         for (int s = 0; s < kSlices; ++s) claim[s] = 0u;
     }
 }
