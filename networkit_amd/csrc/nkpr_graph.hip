@@ -316,55 +316,102 @@ __global__ void reorder_edges_kernel(const uint64_t *colptr, const int32_t *src,
     }
 }
 
+// ---- schedule, on the device ----------------------------------------------------------------
+
+struct DirectRow {  // rows of at most dmax in-edges (want), or the others
+    const uint64_t *colptr;
+    uint64_t dmax;
+    bool want;
+    __device__ bool operator()(uint32_t r) const { return (colptr[r + 1] - colptr[r] <= dmax) == want; }
+};
+
+__global__ void row_length_kernel(const uint64_t *colptr, const uint32_t *rows, uint32_t count, uint32_t *len) {
+    const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+    if (k < count) len[k] = (uint32_t)(colptr[rows[k] + 1] - colptr[rows[k]]);
+    else if (k == count) len[k] = 0;
+}
+
+__global__ __launch_bounds__(256) void max_length_kernel(const uint64_t *colptr, uint32_t n, unsigned long long *most) {
+    unsigned long long mine = 0;
+    for (uint64_t r = (uint64_t)blockIdx.x * 256 + threadIdx.x; r < n; r += (uint64_t)gridDim.x * 256)
+        mine = std::max<unsigned long long>(mine, colptr[r + 1] - colptr[r]);
+    for (int off = 32; off > 0; off >>= 1) mine = std::max<unsigned long long>(mine, __shfl_xor(mine, off, 64));
+    if ((threadIdx.x & 63) == 0 && mine) atomicMax(most, mine);
+}
+
+// Row segments of more than kCap in-edges, in no order: {index over all slices, first edge, length}.
+__global__ void heavy_rows_kernel(const uint32_t *ptr, uint64_t count, uint32_t *n_heavy, uint4 *heavy) {
+    for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < count;
+         j += (uint64_t)gridDim.x * blockDim.x) {
+        const uint32_t b = ptr[j], len = ptr[j + 1] - b;
+        if (len > (uint32_t)kCap) heavy[atomicAdd(n_heavy, 1u)] = make_uint4((uint32_t)j, b, len, 0u);
+    }
+}
+
+// Greedy work items over the rows of `lists` lists of nrows rows each (list q's in-edge offsets start
+// at ptr[q nrows]): runs of consecutive rows with at most `cap` in-edges and kRowsMax rows (a row with
+// more has an item of its own); rows longer than kCap are left out (see build_heavy).  A wave takes
+// kSegRows rows of a list and tries a step's kRowsMax ends at once.  Without `items` it only counts.
+constexpr uint32_t kSegRows = 32768;
+__global__ __launch_bounds__(256) void build_items_kernel(const uint32_t *ptr, uint32_t nrows, uint32_t lists,
+                                                          uint32_t segs, uint32_t cap, uint32_t *counts,
+                                                          const uint32_t *first, uint4 *items) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t seg = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (seg >= lists * segs) return;
+    const uint32_t *P = ptr + (uint64_t)(seg / segs) * nrows;
+    const uint32_t begin = (seg % segs) * kSegRows, end = min(nrows, begin + kSegRows);
+    uint32_t made = 0, r = begin;
+    while (r < end) {
+        const uint32_t p0 = P[r], most = min(end - r, (uint32_t)kRowsMax);
+        uint32_t fit = 0;
+        for (uint32_t c = 0; c < (uint32_t)kRowsMax; c += 64) {
+            const uint32_t k = c + lane + 1;
+            fit += (uint32_t)__popcll(__ballot(k <= most && P[r + min(k, most)] - p0 <= cap));
+        }
+        if (fit == 0) {
+            fit = 1;
+            if (P[r + 1] - p0 > (uint32_t)kCap) {
+                ++r;
+                continue;
+            }
+        }
+        if (items && lane == 0) items[first[seg] + made] = make_uint4(r, r + fit, p0, P[r + fit] - p0);
+        ++made;
+        r += fit;
+    }
+    if (!items && lane == 0) counts[seg] = made;
+}
+
+__global__ void split_flag_kernel(const uint32_t *rows, uint32_t count, uint8_t *flag) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < count) flag[rows[i]] = 1;
+}
+
 struct SplitRec {
     uint32_t first[kSlices];
     uint32_t count[kSlices];
 };
 
-// Greedy work items over rows [0, nrows) of a list with absolute in-edge offsets ptr[0..nrows]:
-// stream blocks of consecutive rows with at most `cap` in-edges and kRowsMax rows (a row with more
-// has a block of its own); a row segment longer than kCap becomes a vector item, or split chunks
-// (when allow_split) recorded in `splits`.
-void build_items(const uint32_t *ptr, uint32_t nrows, uint32_t slice, uint32_t cap,
-                 std::vector<uint4> &out, uint32_t &split_slots,
-                 std::map<uint32_t, SplitRec> *splits, uint64_t &maxlen) {
-    std::vector<uint4> split, vec, stream;
-    uint32_t r = 0;
-    while (r < nrows) {
-        const uint64_t len = (uint64_t)ptr[r + 1] - ptr[r];
-        maxlen = std::max(maxlen, len);
-        if (len > (uint64_t)kCap) {
-            if (len > kVectorMax && splits) {
-                const uint32_t chunks = (uint32_t)((len + kChunk - 1) / kChunk);
-                SplitRec &rec = (*splits)[r];
-                rec.first[slice] = split_slots;
-                rec.count[slice] = chunks;
-                for (uint32_t c = 0; c < chunks; ++c) {
-                    const uint64_t b = ptr[r] + (uint64_t)c * kChunk;
-                    const uint64_t e = std::min<uint64_t>(b + kChunk, ptr[r + 1]);
-                    split.push_back(make_uint4(r, split_slots++ | kSplitFlag, (uint32_t)b,
-                                               (uint32_t)(e - b)));
-                }
-            } else {
-                vec.push_back(make_uint4(r, r + 1, ptr[r], (uint32_t)len));
-            }
-            ++r;
+// Items of the rows longer than kCap of one slice: vector items, and split chunks (recorded in
+// `splits`) above kVectorMax; the chunks first.  rows: {row, first edge, length}, by row.
+void build_heavy(const std::vector<uint4> &rows, uint32_t slice, std::vector<uint4> &out, uint32_t &split_slots,
+                 std::map<uint32_t, SplitRec> &splits) {
+    std::vector<uint4> vec;
+    for (const uint4 &h : rows) {
+        if (h.z <= kVectorMax) {
+            vec.push_back(make_uint4(h.x, h.x + 1, h.y, h.z));
             continue;
         }
-        const uint32_t r0 = r;
-        uint64_t nnz = 0;
-        while (r < nrows && r - r0 < (uint32_t)kRowsMax) {
-            const uint64_t l = (uint64_t)ptr[r + 1] - ptr[r];
-            if (l > (uint64_t)kCap || (r > r0 && nnz + l > (uint64_t)cap)) break;
-            maxlen = std::max(maxlen, l);
-            nnz += l;
-            ++r;
-        }
-        stream.push_back(make_uint4(r0, r, ptr[r0], (uint32_t)nnz));
+        const uint32_t chunks = (h.z + kChunk - 1) / kChunk;
+        SplitRec &rec = splits[h.x];
+        rec.first[slice] = split_slots;
+        rec.count[slice] = chunks;
+        for (uint32_t c = 0; c < chunks; ++c)
+            out.push_back(make_uint4(h.x, split_slots++ | kSplitFlag, h.y + c * kChunk,
+                                     std::min(kChunk, h.z - c * kChunk)));
     }
-    out.insert(out.end(), split.begin(), split.end());
     out.insert(out.end(), vec.begin(), vec.end());
-    out.insert(out.end(), stream.begin(), stream.end());
 }
 
 template <typename V> void upload(nkpr_graph *g, nkpr::DevBuf &b, const std::vector<V> &h) {
@@ -382,7 +429,7 @@ uint32_t env_u32(const char *name, uint32_t dflt) {
 
 // Splits rows into direct and sliced ones, reorders the in-edges into sweep order and builds
 // the work items.  Input: g->colptr / g->src / g->coef* in (row, source) order.
-void build_schedule(nkpr_graph *g, const std::vector<uint64_t> &cp) {
+void build_schedule(nkpr_graph *g) {
     const hipStream_t s = g->stream;
     const uint32_t n = g->n;
     const uint64_t m = g->m;
@@ -404,28 +451,54 @@ void build_schedule(nkpr_graph *g, const std::vector<uint64_t> &cp) {
     g->n_slices = S;
     g->direct_max_deg = dmax;
 
-    std::vector<uint32_t> drow, srow, dptr;
-    drow.reserve(n);
-    uint64_t md = 0, maxdeg = 0;
-    for (uint32_t r = 0; r < n; ++r) {
-        const uint64_t len = cp[r + 1] - cp[r];
-        maxdeg = std::max(maxdeg, len);
-        if (len <= dmax) drow.push_back(r);
-        else srow.push_back(r);
+    // direct and sliced rows, the direct rows' offsets and the largest in-degree, without a row's
+    // length leaving the device (loops over the rows on the host and the copies they needed took
+    // half of the 18 ms of a handle over 1e6 nodes)
+    DevBuf nsel;
+    nsel.alloc(32);
+    NKPR_HIP(hipMemsetAsync(nsel.p, 0, 32, s));
+    uint32_t *sel = nsel.as<uint32_t>();  // direct rows, sliced rows, heavy segments, -, largest degree
+    {
+        DevBuf rows, tmp, lens;
+        rows.alloc(4 * std::max<size_t>(2 * (size_t)n, 1));
+        uint32_t *dr = rows.as<uint32_t>(), *sr = dr + n;
+        const hipcub::CountingInputIterator<uint32_t> ids(0);
+        const DirectRow is_d{g->colptr.as<uint64_t>(), dmax, true}, is_s{g->colptr.as<uint64_t>(), dmax, false};
+        size_t tb = 0;
+        if (n) {
+            NKPR_HIP(hipcub::DeviceSelect::If(nullptr, tb, ids, dr, sel, (int)n, is_d, s));
+            tmp.alloc(tb);
+            NKPR_HIP(hipcub::DeviceSelect::If(tmp.p, tb, ids, dr, sel, (int)n, is_d, s));
+            NKPR_HIP(hipcub::DeviceSelect::If(tmp.p, tb, ids, sr, sel + 1, (int)n, is_s, s));
+            hipLaunchKernelGGL(max_length_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(n), 1024)), dim3(256),
+                               0, s, g->colptr.as<uint64_t>(), n, reinterpret_cast<unsigned long long *>(sel + 4));
+            NKPR_HIP(hipGetLastError());
+        }
+        uint32_t got[6] = {0};
+        read_back(s, {{got, sel, sizeof(got)}});
+        g->n_d = got[0];
+        g->n_s = got[1];
+        g->max_in_degree = (uint64_t)got[4] | ((uint64_t)got[5] << 32);
+        g->drow.alloc(4 * std::max<size_t>(g->n_d, 1));
+        g->srow.alloc(4 * std::max<size_t>(g->n_s, 1));
+        g->dptr.alloc(4 * ((size_t)g->n_d + 1));
+        if (g->n_d) NKPR_HIP(hipMemcpyAsync(g->drow.p, dr, 4 * (size_t)g->n_d, hipMemcpyDeviceToDevice, s));
+        if (g->n_s) NKPR_HIP(hipMemcpyAsync(g->srow.p, sr, 4 * (size_t)g->n_s, hipMemcpyDeviceToDevice, s));
+        lens.alloc(4 * ((size_t)g->n_d + 1));
+        hipLaunchKernelGGL(row_length_kernel, dim3(blocks_for((uint64_t)g->n_d + 1)), dim3(256), 0, s,
+                           g->colptr.as<uint64_t>(), g->drow.as<uint32_t>(), g->n_d, lens.as<uint32_t>());
+        NKPR_HIP(hipGetLastError());
+        tb = 0;
+        DevBuf tmp2;
+        NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, lens.as<uint32_t>(), g->dptr.as<uint32_t>(),
+                                                  (size_t)g->n_d + 1, s));
+        tmp2.alloc(tb);
+        NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(tmp2.p, tb, lens.as<uint32_t>(), g->dptr.as<uint32_t>(),
+                                                  (size_t)g->n_d + 1, s));
     }
-    g->max_in_degree = maxdeg;
-    dptr.resize(drow.size() + 1);
-    for (size_t k = 0; k < drow.size(); ++k) {
-        dptr[k] = (uint32_t)md;
-        md += cp[drow[k] + 1] - cp[drow[k]];
-    }
-    dptr[drow.size()] = (uint32_t)md;
-    g->n_d = (uint32_t)drow.size();
-    g->n_s = (uint32_t)srow.size();
+    uint32_t md = 0;
+    read_back(s, {{&md, g->dptr.as<uint32_t>() + g->n_d, 4}});
     const uint32_t n_s = g->n_s;
-    upload(g, g->drow, drow);
-    upload(g, g->dptr, dptr);
-    upload(g, g->srow, srow);
 
     // per-slice offsets of the sliced rows: exclusive scan of the slice-major counts
     const uint64_t ns_tot = (uint64_t)S * n_s;
@@ -449,7 +522,7 @@ void build_schedule(nkpr_graph *g, const std::vector<uint64_t> &cp) {
         NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, counts.as<uint32_t>(),
                                                   g->sptr.as<uint32_t>(), (size_t)ns_tot + 1, s));
         hipLaunchKernelGGL(add_base_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(ns_tot + 1), 65536)),
-                           dim3(256), 0, s, g->sptr.as<uint32_t>(), ns_tot + 1, (uint32_t)md);
+                           dim3(256), 0, s, g->sptr.as<uint32_t>(), ns_tot + 1, md);
         NKPR_HIP(hipGetLastError());
         NKPR_HIP(hipStreamSynchronize(s));
     }
@@ -502,33 +575,85 @@ void build_schedule(nkpr_graph *g, const std::vector<uint64_t> &cp) {
         }
     }
 
-    // work items
-    std::vector<uint4> ditems, sitems;
-    uint32_t split_slots = 0;
-    uint64_t maxlen = 0;
+    // work items: the rows longer than kCap on the host (at most m / kCap), the runs of shorter rows
+    // on the device, whose counts per segment give every run its place
+    std::vector<uint4> heavy;
+    if (n_s) {
+        DevBuf hv;
+        hv.alloc(sizeof(uint4) * (m / kCap + 1));
+        hipLaunchKernelGGL(heavy_rows_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(ns_tot), 4096)), dim3(256),
+                           0, s, (const uint32_t *)g->sptr.as<uint32_t>(), ns_tot, sel + 2, hv.as<uint4>());
+        NKPR_HIP(hipGetLastError());
+        uint32_t nh = 0;
+        read_back(s, {{&nh, sel + 2, 4}});
+        heavy.resize(nh);
+        read_back(s, {{heavy.data(), hv.p, sizeof(uint4) * (size_t)nh}});
+        std::sort(heavy.begin(), heavy.end(), [](const uint4 &x, const uint4 &y) { return x.x < y.x; });
+    }
     // Items of kCap in-edges leave most CUs idle below kItemsWanted of them: a graph of 20,000
     // nodes and 1.5e5 arcs ran on 40 blocks.  Such graphs take smaller items.
     uint32_t cap = kCap;
     while (S == 1 && cap > kCapMin && m < (uint64_t)cap * kItemsWanted) cap /= 2;
-    build_items(dptr.data(), g->n_d, 0, cap, ditems, split_slots, nullptr, maxlen);
-    std::map<uint32_t, SplitRec> splits;
-    std::vector<uint32_t> hs((size_t)ns_tot + 1);
-    read_back(s, {{hs.data(), g->sptr.p, 4 * ((size_t)ns_tot + 1)}});
-    for (uint32_t q = 0; q < S; ++q) {
-        g->sitem_off[q] = (uint32_t)sitems.size();
-        build_items(hs.data() + (size_t)q * n_s, n_s, q, cap, sitems, split_slots, &splits, maxlen);
+    const uint32_t dsegs = (g->n_d + kSegRows - 1) / kSegRows, ssegs = (n_s + kSegRows - 1) / kSegRows;
+    const uint32_t nseg = dsegs + S * ssegs;
+    DevBuf cnt_b, first_b;
+    cnt_b.alloc(4 * std::max<size_t>(nseg, 1));
+    first_b.alloc(4 * std::max<size_t>(nseg, 1));
+    auto runs = [&](const uint32_t *first, uint4 *di, uint4 *si) {
+        uint32_t *cnt = cnt_b.as<uint32_t>();
+        if (dsegs)
+            hipLaunchKernelGGL(build_items_kernel, dim3((dsegs + 3) / 4), dim3(256), 0, s,
+                               (const uint32_t *)g->dptr.as<uint32_t>(), g->n_d, 1u, dsegs, cap, cnt, first, di);
+        if (ssegs)
+            hipLaunchKernelGGL(build_items_kernel, dim3((S * ssegs + 3) / 4), dim3(256), 0, s,
+                               (const uint32_t *)g->sptr.as<uint32_t>(), n_s, S, ssegs, cap, cnt + dsegs,
+                               first ? first + dsegs : nullptr, si);
+        NKPR_HIP(hipGetLastError());
+    };
+    runs(nullptr, nullptr, nullptr);
+    std::vector<uint32_t> cnt(nseg), first(nseg);
+    read_back(s, {{cnt.data(), cnt_b.p, 4 * (size_t)nseg}});
+    uint64_t at = 0;
+    for (uint32_t i = 0; i < dsegs; ++i) {
+        first[i] = (uint32_t)at;
+        at += cnt[i];
     }
-    for (uint32_t q = S; q <= (uint32_t)kSlices; ++q) g->sitem_off[q] = (uint32_t)sitems.size();
-    NKPR_CHECK(sitems.size() + ditems.size() < 0x7FFFFFFFull, "too many work items");
-    g->n_ditems = (uint32_t)ditems.size();
-    g->n_items = (uint32_t)(ditems.size() + sitems.size());
+    g->n_ditems = (uint32_t)at;
+    uint32_t split_slots = 0;
+    std::map<uint32_t, SplitRec> splits;
+    std::vector<std::vector<uint4>> hitems(S);
+    at = 0;
+    size_t h0 = 0;
+    for (uint32_t q = 0; q < S; ++q) {
+        std::vector<uint4> rows;
+        for (; h0 < heavy.size() && heavy[h0].x < (uint64_t)(q + 1) * n_s; ++h0) {
+            rows.push_back(heavy[h0]);
+            rows.back().x -= q * n_s;
+        }
+        build_heavy(rows, q, hitems[q], split_slots, splits);
+        g->sitem_off[q] = (uint32_t)at;
+        at += hitems[q].size();
+        for (uint32_t i = 0; i < ssegs; ++i) {
+            first[dsegs + q * ssegs + i] = (uint32_t)at;
+            at += cnt[dsegs + q * ssegs + i];
+        }
+    }
+    for (uint32_t q = S; q <= (uint32_t)kSlices; ++q) g->sitem_off[q] = (uint32_t)at;
+    NKPR_CHECK(at + g->n_ditems < 0x7FFFFFFFull, "too many work items");
+    g->n_items = (uint32_t)(g->n_ditems + at);
     g->n_split_items = split_slots;
-    upload(g, g->ditems, ditems);
-    upload(g, g->sitems, sitems);
-    std::vector<uint8_t> flag(std::max<uint32_t>(n_s, 1), 0);
+    g->ditems.alloc(sizeof(uint4) * std::max<size_t>(g->n_ditems, 1));
+    g->sitems.alloc(sizeof(uint4) * std::max<size_t>(at, 1));
+    if (nseg) {
+        NKPR_HIP(hipMemcpyAsync(first_b.p, first.data(), 4 * (size_t)nseg, hipMemcpyHostToDevice, s));
+        runs(first_b.as<uint32_t>(), g->ditems.as<uint4>(), g->sitems.as<uint4>());
+    }
+    for (uint32_t q = 0; q < S; ++q)
+        if (!hitems[q].empty())
+            NKPR_HIP(hipMemcpyAsync(g->sitems.as<uint4>() + g->sitem_off[q], hitems[q].data(),
+                                    sizeof(uint4) * hitems[q].size(), hipMemcpyHostToDevice, s));
     std::vector<uint32_t> srows, sfirst, scount;
     for (auto &kv : splits) {
-        flag[kv.first] = 1;
         srows.push_back(kv.first);
         for (uint32_t q = 0; q < S; ++q) {
             sfirst.push_back(kv.second.first[q]);
@@ -536,22 +661,22 @@ void build_schedule(nkpr_graph *g, const std::vector<uint64_t> &cp) {
         }
     }
     g->n_split_rows = (uint32_t)srows.size();
-    upload(g, g->split_flag, flag);
     upload(g, g->split_rows, srows);
     upload(g, g->split_first, sfirst);
     upload(g, g->split_count, scount);
+    g->split_flag.alloc(std::max<uint32_t>(n_s, 1));
+    NKPR_HIP(hipMemsetAsync(g->split_flag.p, 0, std::max<uint32_t>(n_s, 1), s));
+    if (g->n_split_rows)
+        hipLaunchKernelGGL(split_flag_kernel, dim3(blocks_for(g->n_split_rows)), dim3(256), 0, s,
+                           (const uint32_t *)g->split_rows.as<uint32_t>(), g->n_split_rows, g->split_flag.as<uint8_t>());
+    NKPR_HIP(hipGetLastError());
     g->claim.alloc(4 * (kArriveAt + kArriveWords));
     NKPR_HIP(hipMemsetAsync(g->claim.p, 0, 4 * (kArriveAt + kArriveWords), s));
     NKPR_HIP(hipStreamSynchronize(s));
-    if (env_u32("NKPR_DEBUG", 0)) {
-        std::fprintf(stderr, "[nkpr] n=%u direct rows %u (%llu edges, %u items), sliced rows %u, "
-                             "slices %u, split rows %u\n", n, g->n_d, (unsigned long long)md,
-                     g->n_ditems, n_s, S, g->n_split_rows);
-        for (uint32_t q = 0; q < S; ++q)
-            std::fprintf(stderr, "[nkpr]   slice %u: %llu edges, %u items\n", q,
-                         (unsigned long long)(hs[(size_t)(q + 1) * n_s] - hs[(size_t)q * n_s]),
-                         g->sitem_off[q + 1] - g->sitem_off[q]);
-    }
+    if (env_u32("NKPR_DEBUG", 0))
+        std::fprintf(stderr, "[nkpr] n=%u direct rows %u (%u edges, %u items), sliced rows %u (%u items), "
+                             "slices %u, split rows %u\n", n, g->n_d, md, g->n_ditems, n_s,
+                     g->n_items - g->n_ditems, S, g->n_split_rows);
 }
 
 int bits_for(uint64_t v) {
@@ -831,9 +956,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     }
 
     // --- schedule ---------------------------------------------------------------------------
-    std::vector<uint64_t> cp((size_t)n + 1);
-    read_back(s, {{cp.data(), g->colptr.p, 8 * ((size_t)n + 1)}});
-    build_schedule(g, cp);
+    build_schedule(g);
     NKPR_HIP(hipStreamSynchronize(s));
     g->prep_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
