@@ -6,7 +6,7 @@
 // and gathers, per edge, a 16-byte slice of the source's row of the iterate matrix.
 //
 // Layout (per graph, built on first use): a plain CSC in relabelled ids (uint32 row offsets,
-// int32 sources, folded FP32/FP64 coefficients for weighted graphs) copied out of the sliced
+// int32 sources, FP32 and FP64 coefficients w / deg(src) per edge) copied out of the sliced
 // sweep layout.  Iterates are node-major matrices X[n][ld] (ld = k rounded up to 16 bytes),
 // so the k values of one source are contiguous: a gather is a run of full cache lines.
 //
@@ -82,8 +82,7 @@ __device__ __forceinline__ void store16(T *p, const T (&v)[V16<T>::n]) {
 template <typename T> struct BatchArgs {
     const uint32_t *rowptr;   // [n + 1]
     const int32_t *src;       // [m]
-    const T *coef;            // [m] folded w / deg(src) (weighted) or nullptr
-    const T *inv;             // [n] 1 / deg (unweighted)
+    const T *coef;            // [m] w / deg(src)
     const T *xold;            // [n][ld]
     T *xnew;                  // [n][ld]
     const float *base;        // [n][ld] right-hand side of a correction solve (kBBase)
@@ -105,7 +104,7 @@ template <typename T> struct BatchArgs {
 };
 
 // Sum over the row's edges [e0, e1) of coef * X[src][c0 .. c0 + V) for one row group.
-template <typename T, int LPR, bool FOLDED>
+template <typename T, int LPR>
 __device__ __forceinline__ void row_dot(const BatchArgs<T> &a, uint32_t e0, uint32_t e1,
                                         uint32_t c0, bool on, int l, T (&acc)[V16<T>::n]) {
     constexpr int V = V16<T>::n;
@@ -115,7 +114,7 @@ __device__ __forceinline__ void row_dot(const BatchArgs<T> &a, uint32_t e0, uint
         T cf = T(0);
         if ((uint32_t)l < cnt) {
             s = a.src[b + l];
-            cf = FOLDED ? a.coef[b + l] : a.inv[s];
+            cf = a.coef[b + l];
         }
         uint32_t q = 0;
         for (; q + kUnroll <= cnt; q += kUnroll) {
@@ -259,7 +258,7 @@ __device__ __forceinline__ void block_partials(const BatchArgs<T> &a, uint32_t b
     }
 }
 
-template <typename T, int LPR, bool FOLDED, int KIND>
+template <typename T, int LPR, int KIND>
 __global__ __launch_bounds__(kBThreads) void spmm_kernel(BatchArgs<T> a) {
     if (a.ctl->done) return;
     constexpr int V = V16<T>::n;
@@ -285,7 +284,7 @@ __global__ __launch_bounds__(kBThreads) void spmm_kernel(BatchArgs<T> a) {
         T acc[V];
 #pragma unroll
         for (int j = 0; j < V; ++j) acc[j] = T(0);
-        row_dot<T, LPR, FOLDED>(a, pc.x, pc.x + pc.y, c0, on, l, acc);
+        row_dot<T, LPR>(a, pc.x, pc.x + pc.y, c0, on, l, acc);
         if (on) store16(a.piece_part + (size_t)p * a.ld + c0, acc);
     }
     for (uint32_t i = blockIdx.x * GROUPS + gidx; i < a.n_light; i += stride) {
@@ -293,7 +292,7 @@ __global__ __launch_bounds__(kBThreads) void spmm_kernel(BatchArgs<T> a) {
         T acc[V];
 #pragma unroll
         for (int j = 0; j < V; ++j) acc[j] = T(0);
-        row_dot<T, LPR, FOLDED>(a, a.rowptr[u], a.rowptr[u + 1], c0, on, l, acc);
+        row_dot<T, LPR>(a, a.rowptr[u], a.rowptr[u + 1], c0, on, l, acc);
         if (on) row_epilogue<T, KIND>(a, u, c0, acc, frozen, sinkterm, red);
     }
     block_partials<T, LPR>(a, blockIdx.x, tile, red);
@@ -336,83 +335,88 @@ __global__ __launch_bounds__(kBThreads) void heavy_combine_kernel(BatchArgs<T> a
     block_partials<T, LPR>(a, blk_base + blockIdx.x, tile, red);
 }
 
-// One block per real column: reduce the block partials in a fixed order and apply the rule.
+// One block per real column: reduce the block partials in a fixed order and apply the rule.  The
+// block that arrives last counts the columns still running and sets ctl->done when none is (or the
+// sweep cap is hit); a launch of its own for that cost 4 us of a 130 us sweep.
 __global__ __launch_bounds__(kFinThreads) void batch_finalize_kernel(const double *partials,
                                                                      uint32_t nblocks,
                                                                      uint32_t ld, BatchCol *col,
-                                                                     const BatchCtl *ctl,
-                                                                     PhaseRule r) {
+                                                                     BatchCtl *ctl, PhaseRule r,
+                                                                     uint64_t max_sweeps) {
     if (ctl->done) return;
-    const uint32_t c = blockIdx.x;
-    if (col[c].done) return;
+    const uint32_t c = blockIdx.x, k = gridDim.x;
     __shared__ double s_red[4][kFinThreads / 64];
-    double t[4] = {0.0, 0.0, 0.0, 0.0};
-    for (uint32_t b = threadIdx.x; b < nblocks; b += kFinThreads) {
-        const double *p = partials + ((size_t)b * ld + c) * 4;
+    __shared__ uint32_t s_last, s_cnt;
+    if (!col[c].done) {
+        double t[4] = {0.0, 0.0, 0.0, 0.0};
+        for (uint32_t b = threadIdx.x; b < nblocks; b += kFinThreads) {
+            const double *p = partials + ((size_t)b * ld + c) * 4;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) t[q] += p[q];
-    }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+            for (int q = 0; q < 4; ++q) t[q] += p[q];
+        }
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-        double v = t[q];
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-        if (lane == 0) s_red[q][wave] = v;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double tot[4];
         for (int q = 0; q < 4; ++q) {
-            double s = 0.0;
-            for (int w = 0; w < kFinThreads / 64; ++w) s += s_red[q][w];
-            tot[q] = s;
+            double v = t[q];
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+            if (lane == 0) s_red[q][wave] = v;
         }
-        BatchCol &cc = col[c];
-        const uint64_t it = cc.phase_iter + 1;
-        cc.phase_iter = it;
-        cc.iterations += 1;
-        const double prev = cc.l1;
-        cc.prev_l1 = prev;
-        cc.l1 = tot[0];
-        cc.l2 = tot[1];
-        cc.sum = tot[2];
-        cc.sink_out = tot[3];
-        cc.sink_in = tot[3];
-        const double bound =
-            (tot[2] > 0.0) ? 2.0 * r.damp / (1.0 - r.damp) * tot[0] / tot[2] : INFINITY;
-        cc.bound = bound;
-        // tolerance of a correction solve that would let the next residual certify
-        cc.target = 0.5 * r.tol * tot[2] * (1.0 - r.damp) / (2.0 * r.damp);
-        bool stop = it >= r.max_iterations;
-        if (r.kind == kRuleStep) {
-            const double step = (r.norm == NKPR_L2) ? sqrt(tot[1]) : tot[0];
-            stop = stop || step <= r.tol;
-        } else if (r.kind == kRuleErr) {
-            stop = stop || bound <= r.tol;
-        } else {
-            // correction solve (tol_abs < 0: per-column target) or FP32 phase
-            const double ta = r.tol_abs < 0.0 ? cc.solve_tol : r.tol_abs;
-            stop = stop || tot[0] <= ta || bound <= r.tol;
-            if (it >= 4 && tot[0] > r.stall_ratio * prev) stop = true;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            double tot[4];
+            for (int q = 0; q < 4; ++q) {
+                double s = 0.0;
+                for (int w = 0; w < kFinThreads / 64; ++w) s += s_red[q][w];
+                tot[q] = s;
+            }
+            BatchCol &cc = col[c];
+            const uint64_t it = cc.phase_iter + 1;
+            cc.phase_iter = it;
+            cc.iterations += 1;
+            const double prev = cc.l1;
+            cc.prev_l1 = prev;
+            cc.l1 = tot[0];
+            cc.l2 = tot[1];
+            cc.sum = tot[2];
+            cc.sink_out = tot[3];
+            cc.sink_in = tot[3];
+            const double bound =
+                (tot[2] > 0.0) ? 2.0 * r.damp / (1.0 - r.damp) * tot[0] / tot[2] : INFINITY;
+            cc.bound = bound;
+            // tolerance of a correction solve that would let the next residual certify
+            cc.target = 0.5 * r.tol * tot[2] * (1.0 - r.damp) / (2.0 * r.damp);
+            bool stop = it >= r.max_iterations;
+            if (r.kind == kRuleStep) {
+                const double step = (r.norm == NKPR_L2) ? sqrt(tot[1]) : tot[0];
+                stop = stop || step <= r.tol;
+            } else if (r.kind == kRuleErr) {
+                stop = stop || bound <= r.tol;
+            } else {
+                // correction solve (tol_abs < 0: per-column target) or FP32 phase
+                const double ta = r.tol_abs < 0.0 ? cc.solve_tol : r.tol_abs;
+                stop = stop || tot[0] <= ta || bound <= r.tol;
+                if (it >= 4 && tot[0] > r.stall_ratio * prev) stop = true;
+            }
+            // read by the block that arrives last
+            __hip_atomic_store(&cc.done, stop ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (stop && r.kind == kRuleErr && bound <= r.tol) cc.final_ = 1u;
         }
-        cc.done = stop ? 1u : 0u;
-        if (stop && r.kind == kRuleErr && bound <= r.tol) cc.final_ = 1u;
     }
-}
-
-// Counts the columns still running; sets ctl->done when none is (or the sweep cap is hit).
-__global__ void batch_count_kernel(const BatchCol *col, uint32_t k, BatchCtl *ctl,
-                                   uint64_t max_sweeps) {
-    if (ctl->done) return;
-    __shared__ uint32_t s_cnt;
-    if (threadIdx.x == 0) s_cnt = 0;
+    if (threadIdx.x == 0) {
+        s_cnt = 0;
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        s_last = atomicAdd(&ctl->arrived, 1u) + 1 == k ? 1u : 0u;
+    }
     __syncthreads();
+    if (!s_last) return;
     uint32_t cnt = 0;
-    for (uint32_t c = threadIdx.x; c < k; c += blockDim.x) cnt += col[c].done ? 0u : 1u;
+    for (uint32_t j = threadIdx.x; j < k; j += kFinThreads)
+        cnt += __hip_atomic_load(&col[j].done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) ? 0u : 1u;
     atomicAdd(&s_cnt, cnt);
     __syncthreads();
     if (threadIdx.x == 0) {
+        ctl->arrived = 0;
         ctl->sweeps += 1;
         ctl->active = s_cnt;
         ctl->done = (s_cnt == 0 || ctl->sweeps >= max_sweeps) ? 1u : 0u;
@@ -436,21 +440,55 @@ __global__ void batch_init_kernel(BatchCol *col, uint32_t k, uint32_t ld, BatchC
     }
     if (blockIdx.x == 0 && threadIdx.x == 0) {
         ctl->done = 0;
+        ctl->arrived = 0;
         ctl->active = k;
         ctl->sweeps = 0;
     }
 }
 
+// Column sums in a fixed order: a wave covers 64 columns, the waves of a block stride over the rows
+// (kInFlight of them loaded at a time), and their sums are added in wave order.  One thread per
+// column walked 586 block sums one after another before (138 us for 96 columns).
+constexpr int kSumThreads = 1024, kInFlight = 8;
+template <typename T>
+__device__ __forceinline__ double column_sum(const T *x, uint32_t ld, uint32_t c, uint32_t r0, uint32_t r1,
+                                             double (*s)[64]) {
+    constexpr uint32_t kWaves = kSumThreads / 64;
+    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    double acc = 0.0;
+    if (c < ld) {
+        for (uint32_t r = r0 + wave; r < r1; r += kWaves * kInFlight) {
+            double v[kInFlight];
+#pragma unroll
+            for (int i = 0; i < kInFlight; ++i) {
+                const uint32_t q = r + i * kWaves;
+                v[i] = q < r1 ? (double)x[(size_t)q * ld + c] : 0.0;
+            }
+#pragma unroll
+            for (int i = 0; i < kInFlight; ++i) acc += v[i];
+        }
+    }
+    __syncthreads();
+    s[wave][lane] = acc;
+    __syncthreads();
+    double t = 0.0;
+    if (wave == 0)
+        for (uint32_t w = 0; w < kWaves; ++w) t += s[w][lane];
+    return t;  // in the first wave
+}
+
 // Per-block column sums of X[begin, end) (FP64): part[b * ld + c].
 template <typename T>
-__global__ void col_range_sum_kernel(const T *x, uint32_t ld, uint32_t begin, uint32_t end,
-                                     uint32_t rows_per_block, double *part) {
+__global__ __launch_bounds__(kSumThreads) void col_range_sum_kernel(const T *x, uint32_t ld, uint32_t begin,
+                                                                    uint32_t end, uint32_t rows_per_block,
+                                                                    double *part) {
+    __shared__ double s[kSumThreads / 64][64];
     const uint32_t r0 = begin + blockIdx.x * rows_per_block;
     const uint32_t r1 = min(end, r0 + rows_per_block);
-    for (uint32_t c = threadIdx.x; c < ld; c += blockDim.x) {
-        double s = 0.0;
-        for (uint32_t r = r0; r < r1; ++r) s += (double)x[(size_t)r * ld + c];
-        part[(size_t)blockIdx.x * ld + c] = s;
+    for (uint32_t c0 = 0; c0 < ld; c0 += 64) {
+        const uint32_t c = c0 + (threadIdx.x & 63);
+        const double t = column_sum<T>(x, ld, c, r0, r1, s);
+        if (threadIdx.x < 64 && c < ld) part[(size_t)blockIdx.x * ld + c] = t;
     }
 }
 
@@ -461,10 +499,12 @@ __global__ void col_range_sum_kernel(const T *x, uint32_t ld, uint32_t begin, ui
 // (slot_u: compact id of a slot, or -1 for a slot without a node).
 constexpr uint32_t kTile = 64;
 
-// x64[u * ld + j] = scores[j * z + slot(u)] (0 for the padding columns j >= k)
+// x[u * ld + j] = scores[j * z + slot(u)] (0 for the padding columns j >= k), in the precision of
+// the first phase
+template <typename T>
 __global__ __launch_bounds__(256) void batch_gather_kernel(const double *scores, uint64_t z,
                                                            const int32_t *slot_u, uint32_t k,
-                                                           uint32_t ld, double *x64) {
+                                                           uint32_t ld, T *x) {
     __shared__ double tile[kTile][kTile + 1];
     const uint32_t lane = threadIdx.x & 63, row = threadIdx.x >> 6;
     const uint64_t st = (z + kTile - 1) / kTile, ct = (ld + kTile - 1) / kTile;
@@ -481,7 +521,7 @@ __global__ __launch_bounds__(256) void batch_gather_kernel(const double *scores,
             if (s0 + ss >= z) break;
             const int32_t u = slot_u[s0 + ss];
             const uint32_t j = j0 + lane;
-            if (u >= 0 && j < ld) x64[(uint64_t)u * ld + j] = tile[lane][ss];
+            if (u >= 0 && j < ld) x[(uint64_t)u * ld + j] = (T)tile[lane][ss];
         }
         __syncthreads();
     }
@@ -531,20 +571,20 @@ __global__ void tele_rowptr_kernel(const uint32_t *urow, const uint32_t *uoff, u
     }
 }
 
-__global__ void f64_to_f32_kernel(const double *in, float *out, uint64_t cnt) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (uint64_t)gridDim.x * blockDim.x) out[i] = (float)in[i];
-}
-
 __global__ void f32_to_f64_kernel(const float *in, double *out, uint64_t cnt) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (uint64_t)gridDim.x * blockDim.x) out[i] = (double)in[i];
 }
 
-// After a correction solve: x = y for certified columns, x += e for the others.
-__global__ void batch_update_kernel(double *x, const double *y, const float *e, uint32_t ld,
-                                    uint64_t cnt, const BatchCol *col) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (uint64_t)gridDim.x * blockDim.x) {
-        const uint32_t c = (uint32_t)(i % ld);
-        x[i] = col[c].final_ ? y[i] : x[i] + (double)e[i];
+// After a correction solve: x = y for certified columns, x += e for the others (4 columns a thread).
+__global__ void batch_update_kernel(double2 *x, const double2 *y, const float4 *e, uint32_t ld4,
+                                    uint64_t quads, const BatchCol *col) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads;
+         i += (uint64_t)gridDim.x * blockDim.x) {
+        const BatchCol *c = col + 4 * (i % ld4);
+        const double2 x0 = x[2 * i], x1 = x[2 * i + 1], y0 = y[2 * i], y1 = y[2 * i + 1];
+        const float4 f = e[i];
+        x[2 * i] = make_double2(c[0].final_ ? y0.x : x0.x + (double)f.x, c[1].final_ ? y0.y : x0.y + (double)f.y);
+        x[2 * i + 1] = make_double2(c[2].final_ ? y1.x : x1.x + (double)f.z, c[3].final_ ? y1.y : x1.y + (double)f.w);
     }
 }
 
@@ -554,29 +594,33 @@ __global__ void batch_set_solve_tol_kernel(BatchCol *col, uint32_t ld) {
     if (c < ld) col[c].solve_tol = col[c].target;
 }
 
-// Column totals of per-block column sums: out[c] = sum_b part[b * ld + c].
-__global__ void col_total_kernel(const double *part, uint32_t nblocks, uint32_t ld, double *out) {
-    const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= ld) return;
-    double t = 0.0;
-    for (uint32_t b = 0; b < nblocks; ++b) t += part[(size_t)b * ld + c];
-    out[c] = t;
+// Column totals of per-block column sums: out[c] = sum_b part[b * ld + c], 64 columns a block.
+__global__ __launch_bounds__(kSumThreads) void col_total_kernel(const double *part, uint32_t nblocks, uint32_t ld,
+                                                                double *out) {
+    __shared__ double s[kSumThreads / 64][64];
+    const uint32_t c = blockIdx.x * 64 + (threadIdx.x & 63);
+    const double t = column_sum<double>(part, ld, c, 0, nblocks, s);
+    if (threadIdx.x < 64 && c < ld) out[c] = t;
 }
 
-// e0[u][c] += shift * total[c]: with a column-stochastic operator (no sinks, or distributed
-// sinks) 1^T (I - dP) = (1-d) 1^T, so the solution of e = dPe + r sums to 1^T r / (1-d).
-// Starting there leaves no error along the eigenvalue-d mode, which would otherwise decay only
-// as d^k.
-__global__ void col_shift_kernel(float *e, uint32_t ld, uint64_t cnt, const double *total,
-                                 double shift) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        e[i] += (float)(shift * total[i % ld]);
-}
-
-// Correction solves start from e = r.
-__global__ void copy_f32_kernel(const float *in, float *out, uint64_t cnt) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (uint64_t)gridDim.x * blockDim.x) out[i] = in[i];
+// The start of a correction solve, e0 = r, plus shift * total[c] where the exact column sum is known
+// (total given): with a column-stochastic operator (no sinks, or distributed sinks)
+// 1^T (I - dP) = (1-d) 1^T, so the solution of e = dPe + r sums to 1^T r / (1-d).  Starting there
+// leaves no error along the eigenvalue-d mode, which would otherwise decay only as d^k.
+__global__ void correction_start_kernel(const float4 *r, float4 *e, uint32_t ld4, uint64_t quads,
+                                        const double *total, double shift) {
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < quads;
+         i += (uint64_t)gridDim.x * blockDim.x) {
+        float4 v = r[i];
+        if (total) {
+            const double *t = total + 4 * (i % ld4);
+            v.x += (float)(shift * t[0]);
+            v.y += (float)(shift * t[1]);
+            v.z += (float)(shift * t[2]);
+            v.w += (float)(shift * t[3]);
+        }
+        e[i] = v;
+    }
 }
 
 // Plain CSC out of the sliced sweep layout: row r's in-edges in slice order.
@@ -619,6 +663,15 @@ __global__ void plain_layout_kernel(const uint64_t *colptr, const uint32_t *drow
     }
 }
 
+__global__ void unit_coef_kernel(const int32_t *src, uint64_t m, const float *inv32, const double *inv64,
+                                 float *c32, double *c64) {
+    for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
+         e += (uint64_t)gridDim.x * blockDim.x) {
+        c32[e] = inv32[src[e]];
+        c64[e] = inv64[src[e]];
+    }
+}
+
 __global__ void rowptr32_kernel(const uint64_t *colptr, uint32_t n, uint32_t *rowptr) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i <= n) rowptr[i] = (uint32_t)colptr[i];
@@ -633,14 +686,11 @@ unsigned blocks_for(uint64_t cnt, int threads = 256) {
     return (unsigned)((cnt + threads - 1) / threads);
 }
 
-// ---- launch dispatch over (T, LPR, FOLDED, KIND) -----------------------------------------
+// ---- launch dispatch over (T, LPR, KIND) -----------------------------------------
 template <typename T, int LPR, int KIND>
-void launch_lpr(const BatchArgs<T> &a, bool folded, unsigned grid, unsigned cgrid,
+void launch_lpr(const BatchArgs<T> &a, unsigned grid, unsigned cgrid,
                 unsigned tiles, hipStream_t s) {
-    if (folded)
-        hipLaunchKernelGGL((spmm_kernel<T, LPR, true, KIND>), dim3(grid, tiles), dim3(kBThreads), 0, s, a);
-    else
-        hipLaunchKernelGGL((spmm_kernel<T, LPR, false, KIND>), dim3(grid, tiles), dim3(kBThreads), 0, s, a);
+    hipLaunchKernelGGL((spmm_kernel<T, LPR, KIND>), dim3(grid, tiles), dim3(kBThreads), 0, s, a);
     NKPR_HIP(hipGetLastError());
     if (a.n_heavy > 0) {
         hipLaunchKernelGGL((heavy_combine_kernel<T, LPR, KIND>), dim3(cgrid, tiles), dim3(kBThreads), 0, s, a, grid);
@@ -649,34 +699,34 @@ void launch_lpr(const BatchArgs<T> &a, bool folded, unsigned grid, unsigned cgri
 }
 
 template <typename T, int KIND>
-void launch_kind(const BatchArgs<T> &a, int lpr, bool folded, unsigned grid, unsigned cgrid,
+void launch_kind(const BatchArgs<T> &a, int lpr, unsigned grid, unsigned cgrid,
                  hipStream_t s) {
     constexpr int V = V16<T>::n;
     const unsigned tiles = (a.ld + (unsigned)(lpr * V) - 1) / (unsigned)(lpr * V);
     switch (lpr) {
-        case 4: launch_lpr<T, 4, KIND>(a, folded, grid, cgrid, tiles, s); break;
-        case 16: launch_lpr<T, 16, KIND>(a, folded, grid, cgrid, tiles, s); break;
-        default: launch_lpr<T, 64, KIND>(a, folded, grid, cgrid, tiles, s); break;
+        case 4: launch_lpr<T, 4, KIND>(a, grid, cgrid, tiles, s); break;
+        case 16: launch_lpr<T, 16, KIND>(a, grid, cgrid, tiles, s); break;
+        default: launch_lpr<T, 64, KIND>(a, grid, cgrid, tiles, s); break;
     }
 }
 
 template <typename T>
-void launch_spmm(const BatchArgs<T> &a, int kind, int lpr, bool folded, unsigned grid,
+void launch_spmm(const BatchArgs<T> &a, int kind, int lpr, unsigned grid,
                  unsigned cgrid, hipStream_t s) {
     if constexpr (sizeof(T) == 4) {
-        if (kind == kBBase) launch_kind<T, kBBase>(a, lpr, folded, grid, cgrid, s);
-        else launch_kind<T, kBPlain>(a, lpr, folded, grid, cgrid, s);
+        if (kind == kBBase) launch_kind<T, kBBase>(a, lpr, grid, cgrid, s);
+        else launch_kind<T, kBPlain>(a, lpr, grid, cgrid, s);
     } else {
-        if (kind == kBResid) launch_kind<T, kBResid>(a, lpr, folded, grid, cgrid, s);
-        else launch_kind<T, kBPlain>(a, lpr, folded, grid, cgrid, s);
+        if (kind == kBResid) launch_kind<T, kBResid>(a, lpr, grid, cgrid, s);
+        else launch_kind<T, kBPlain>(a, lpr, grid, cgrid, s);
     }
 }
 
-template <typename T> int occupancy_blocks(int device, int lpr, bool folded) {
+template <typename T> int occupancy_blocks(int device, int lpr) {
     const void *fn;
-    if (lpr == 4) fn = folded ? (const void *)&spmm_kernel<T, 4, true, kBPlain> : (const void *)&spmm_kernel<T, 4, false, kBPlain>;
-    else if (lpr == 16) fn = folded ? (const void *)&spmm_kernel<T, 16, true, kBPlain> : (const void *)&spmm_kernel<T, 16, false, kBPlain>;
-    else fn = folded ? (const void *)&spmm_kernel<T, 64, true, kBPlain> : (const void *)&spmm_kernel<T, 64, false, kBPlain>;
+    if (lpr == 4) fn = (const void *)&spmm_kernel<T, 4, kBPlain>;
+    else if (lpr == 16) fn = (const void *)&spmm_kernel<T, 16, kBPlain>;
+    else fn = (const void *)&spmm_kernel<T, 64, kBPlain>;
     int per_cu = 0, cus = 0;
     NKPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBThreads, 0));
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
@@ -737,9 +787,23 @@ void batch_layout(nkpr_graph *g) {
     g->b_coef_ready = true;
 }
 
+// Unweighted graphs: 1 / deg(src) per edge.  The SpMM reads it as a stream beside the source ids; a
+// gather of 1 / deg would be one more dependent access before the gather of the source's row.
+static void unit_coefficients(nkpr_graph *g) {
+    const uint64_t m = g->m;
+    g->b_coef32.alloc(4 * std::max<uint64_t>(m, 1));
+    g->b_coef64.alloc(8 * std::max<uint64_t>(m, 1));
+    if (m)
+        hipLaunchKernelGGL(unit_coef_kernel, dim3(grid_for(m)), dim3(256), 0, g->stream, g->b_src.as<int32_t>(), m,
+                           g->inv32.as<float>(), g->inv64.as<double>(), g->b_coef32.as<float>(),
+                           g->b_coef64.as<double>());
+    NKPR_HIP(hipGetLastError());
+}
+
 void batch_host_lists(nkpr_graph *g) {
     if (g->b_host_ready) return;
     const uint32_t n = g->n;
+    if (!g->weighted) unit_coefficients(g);
     std::vector<int32_t> perm(n);
     g->b_rowptr_host.resize((size_t)n + 1);
     read_back(g->stream, {{g->b_rowptr_host.data(), g->b_rowptr.p, 4 * ((size_t)n + 1)},
@@ -805,13 +869,11 @@ template <typename T> BatchArgs<T> make_args(BatchRun &br) {
     a.rowptr = g->b_rowptr.as<uint32_t>();
     a.src = g->b_src.as<int32_t>();
     if constexpr (sizeof(T) == 4) {
-        a.coef = g->weighted ? g->b_coef32.as<float>() : nullptr;
-        a.inv = g->weighted ? nullptr : g->inv32.as<float>();
+        a.coef = g->b_coef32.as<float>();
         a.tval = g->b_tval32.as<float>();
         a.piece_part = g->b_piece32.as<float>();
     } else {
-        a.coef = g->weighted ? g->b_coef64.as<double>() : nullptr;
-        a.inv = g->weighted ? nullptr : g->inv64.as<double>();
+        a.coef = g->b_coef64.as<double>();
         a.tval = g->b_tval64.as<double>();
         a.piece_part = g->b_piece64.as<double>();
     }
@@ -856,7 +918,7 @@ template <typename T> void phase_init(BatchRun &br, const T *x) {
         const uint32_t rows = n - g->sink_begin;
         const uint32_t rpb = std::max<uint32_t>(256, (rows + 1023) / 1024);
         sink_blocks = (rows + rpb - 1) / rpb;
-        hipLaunchKernelGGL(col_range_sum_kernel<T>, dim3(sink_blocks), dim3(256), 0, s, x, ld,
+        hipLaunchKernelGGL(col_range_sum_kernel<T>, dim3(sink_blocks), dim3(kSumThreads), 0, s, x, ld,
                            g->sink_begin, n, rpb, br.sink_part);
         NKPR_HIP(hipGetLastError());
     }
@@ -899,14 +961,11 @@ uint64_t batch_phase(BatchRun &br, T *x0, T *x1, int kind, PhaseRule rule, uint6
             a.xold = xs[q & 1];
             a.xnew = xs[(q & 1) ^ 1];
             if (timing) NKPR_HIP(hipEventRecord(g->events[2 * j], s));
-            launch_spmm<T>(a, kind, br.lpr[dbl], g->weighted, grid, cgrid, s);
+            launch_spmm<T>(a, kind, br.lpr[dbl], grid, cgrid, s);
             if (timing) NKPR_HIP(hipEventRecord(g->events[2 * j + 1], s));
             hipLaunchKernelGGL(batch_finalize_kernel, dim3(br.k), dim3(kFinThreads), 0, s,
                                g->b_partials.as<double>(), nblocks, br.ld, br.col,
-                               (const BatchCtl *)br.ctl, rule);
-            NKPR_HIP(hipGetLastError());
-            hipLaunchKernelGGL(batch_count_kernel, dim3(1), dim3(256), 0, s, (const BatchCol *)br.col,
-                               br.k, br.ctl, (uint64_t)max_launch);
+                               br.ctl, rule, (uint64_t)max_launch);
             NKPR_HIP(hipGetLastError());
         }
         read_back(s, {{br.ctl_host, br.ctl, sizeof(BatchCtl)}});
@@ -973,15 +1032,15 @@ void autotune(BatchRun &br, T *x0, T *x1) {
         size_pieces<T>(br);
         for (int l : lprs) {
             br.lpr[dbl] = l;
-            const unsigned grid = (unsigned)occupancy_blocks<T>(g->device, l, g->weighted);
+            const unsigned grid = (unsigned)occupancy_blocks<T>(g->device, l);
             const unsigned cgrid = std::max<unsigned>(1, std::min<unsigned>(grid, (g->b_n_heavy * l + kBThreads - 1) / kBThreads));
             size_partials(br, grid, cgrid);
             BatchArgs<T> a = make_args<T>(br);
             a.xold = x0;
             a.xnew = x1;
-            launch_spmm<T>(a, kBPlain, l, g->weighted, grid, cgrid, s);  // warm-up
+            launch_spmm<T>(a, kBPlain, l, grid, cgrid, s);  // warm-up
             NKPR_HIP(hipEventRecord(e0, s));
-            for (int r = 0; r < 2; ++r) launch_spmm<T>(a, kBPlain, l, g->weighted, grid, cgrid, s);
+            for (int r = 0; r < 2; ++r) launch_spmm<T>(a, kBPlain, l, grid, cgrid, s);
             NKPR_HIP(hipEventRecord(e1, s));
             NKPR_HIP(hipEventSynchronize(e1));
             float ms = 0.f;
@@ -1007,7 +1066,7 @@ template <typename T> void configure(BatchRun &br, T *x0, T *x1) {
     const bool dbl = sizeof(T) == 8;
     autotune<T>(br, x0, x1);
     batch_split(g, br.heavy[dbl]);
-    br.grid[dbl] = (unsigned)occupancy_blocks<T>(g->device, br.lpr[dbl], g->weighted);
+    br.grid[dbl] = (unsigned)occupancy_blocks<T>(g->device, br.lpr[dbl]);
     br.cgrid[dbl] = std::max<unsigned>(
         1, std::min<unsigned>(br.grid[dbl], (g->b_n_heavy * br.lpr[dbl] + kBThreads - 1) / kBThreads));
 }
@@ -1148,10 +1207,7 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
     }
     const int32_t *slot_u = slot_index(g);
     const uint64_t gather_tiles = ((z + kTile - 1) / kTile) * ((ld + kTile - 1) / kTile);
-    hipLaunchKernelGGL(batch_gather_kernel, dim3((unsigned)std::min<uint64_t>(std::max<uint64_t>(gather_tiles, 1), 1u << 16)),
-                       dim3(256), 0, s, (const double *)sz, z, slot_u, k, ld,
-                       x64[0]);
-    NKPR_HIP(hipGetLastError());
+    const dim3 gather_grid((unsigned)std::min<uint64_t>(std::max<uint64_t>(gather_tiles, 1), 1u << 16));
 
     const uint64_t max_it = std::max<uint64_t>(p->max_iterations, 1);
     double *result = nullptr;
@@ -1171,6 +1227,9 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
                      name, (unsigned long long)sweeps, mb, ml1, fin, k);
     };
     if (p->precision == NKPR_FP64) {
+        hipLaunchKernelGGL(batch_gather_kernel<double>, gather_grid, dim3(256), 0, s, (const double *)sz, z, slot_u,
+                           k, ld, x64[0]);
+        NKPR_HIP(hipGetLastError());
         configure<double>(br, x64[0], x64[1]);
         PhaseRule r{};
         r.kind = p->stop == NKPR_STOP_STEP ? kRuleStep : kRuleErr;
@@ -1186,8 +1245,8 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
         ensure_buf(g->b_x32a, 4 * cells);
         ensure_buf(g->b_x32b, 4 * cells);
         float *x32[2] = {g->b_x32a.as<float>(), g->b_x32b.as<float>()};
-        hipLaunchKernelGGL(f64_to_f32_kernel, dim3(grid_for(cells)), dim3(256), 0, s,
-                           (const double *)x64[0], x32[0], (uint64_t)cells);
+        hipLaunchKernelGGL(batch_gather_kernel<float>, gather_grid, dim3(256), 0, s, (const double *)sz, z, slot_u,
+                           k, ld, x32[0]);
         NKPR_HIP(hipGetLastError());
         configure<float>(br, x32[0], x32[1]);
         if (p->precision == NKPR_FP32) {
@@ -1243,23 +1302,22 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
                 for (uint32_t j = 0; j < k; ++j) open += cols[j].final_ ? 0u : 1u;
                 if (open == 0 || total >= max_it || round >= 30) break;
                 ++st->refinements;
-                // correction: e0 = r; per column stop at its own target step
-                hipLaunchKernelGGL(copy_f32_kernel, dim3(grid_for(cells)), dim3(256), 0, s,
-                                   (const float *)r32, x32[0], (uint64_t)cells);
-                NKPR_HIP(hipGetLastError());
+                // correction: e0 = r (shifted); per column stop at its own target step
+                const double *tot = nullptr;
                 if (g->sink_begin == n || p->sink_handling == NKPR_SINK_DISTRIBUTE) {
                     const uint32_t rpb = std::max<uint32_t>(256, (n + 1023) / 1024);
                     const uint32_t blocks = (n + rpb - 1) / rpb;
-                    hipLaunchKernelGGL(col_range_sum_kernel<float>, dim3(blocks), dim3(256), 0, s,
+                    hipLaunchKernelGGL(col_range_sum_kernel<float>, dim3(blocks), dim3(kSumThreads), 0, s,
                                        (const float *)r32, ld, 0u, n, rpb, br.sink_part);
-                    double *tot = br.sink_part + (size_t)1024 * ld;
-                    hipLaunchKernelGGL(col_total_kernel, dim3((ld + 255) / 256), dim3(256), 0, s,
-                                       (const double *)br.sink_part, blocks, ld, tot);
-                    hipLaunchKernelGGL(col_shift_kernel, dim3(grid_for(cells)), dim3(256), 0, s,
-                                       x32[0], ld, (uint64_t)cells, (const double *)tot,
-                                       d / (1.0 - d) / (double)n);
+                    tot = br.sink_part + (size_t)1024 * ld;
+                    hipLaunchKernelGGL(col_total_kernel, dim3((ld + 63) / 64), dim3(kSumThreads), 0, s,
+                                       (const double *)br.sink_part, blocks, ld, br.sink_part + (size_t)1024 * ld);
                     NKPR_HIP(hipGetLastError());
                 }
+                hipLaunchKernelGGL(correction_start_kernel, dim3(grid_for(cells / 4)), dim3(256), 0, s,
+                                   (const float4 *)r32, (float4 *)x32[0], ld / 4, (uint64_t)cells / 4, tot,
+                                   d / (1.0 - d) / (double)n);
+                NKPR_HIP(hipGetLastError());
                 hipLaunchKernelGGL(batch_set_solve_tol_kernel, dim3((ld + 255) / 256), dim3(256), 0, s,
                                    br.col, ld);
                 NKPR_HIP(hipGetLastError());
@@ -1275,9 +1333,9 @@ void ppr_batch_impl(nkpr_graph *g, const nkpr_params *p, uint32_t k, const uint6
                 debug_phase("fp32 correction", kc);
                 st->sweeps_fp32 += kc;
                 total += kc;
-                hipLaunchKernelGGL(batch_update_kernel, dim3(grid_for(cells)), dim3(256), 0, s,
-                                   x64[0], (const double *)x64[1], (const float *)x32[kc & 1], ld,
-                                   (uint64_t)cells, (const BatchCol *)br.col);
+                hipLaunchKernelGGL(batch_update_kernel, dim3(grid_for(cells / 4)), dim3(256), 0, s,
+                                   (double2 *)x64[0], (const double2 *)x64[1], (const float4 *)x32[kc & 1], ld / 4,
+                                   (uint64_t)cells / 4, (const BatchCol *)br.col);
                 NKPR_HIP(hipGetLastError());
             }
         }

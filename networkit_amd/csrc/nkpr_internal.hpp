@@ -335,6 +335,8 @@ struct BatchCtl {
     uint64_t sweeps;    // executed sweeps of the phase
     uint32_t active;
     uint32_t done;
+    uint32_t arrived;   // column blocks that have ended the running sweep's reduction
+    uint32_t pad;
 };
 struct BatchTune {
     uint32_t key;       // ld * 2 + (FP64)
