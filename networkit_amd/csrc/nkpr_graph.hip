@@ -168,30 +168,84 @@ __global__ void new_lengths_kernel(const int32_t *perm, uint32_t n, const uint64
     }
 }
 
-// One wave64 per old row: key = (new row << 32) | new source, value = old edge index.
-__global__ void edge_keys_kernel(const uint64_t *colptr_in, const int32_t *src_in,
-                                 const int32_t *iperm, uint64_t z, uint64_t *keys,
-                                 uint32_t *vals) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    for (uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; wave < z;
-         wave += nwaves) {
-        const int32_t r = iperm[wave];
-        const uint64_t b = colptr_in[wave], e = colptr_in[wave + 1];
-        for (uint64_t i = b + lane; i < e; i += 64) {
-            keys[i] = ((uint64_t)(uint32_t)r << 32) | (uint32_t)iperm[src_in[i]];
-            vals[i] = (uint32_t)i;
-        }
+// Row r of [lo, hi) with ptr[r] <= e < ptr[r + 1] (ptr rises; e lies in these rows).
+__device__ __forceinline__ uint64_t row_of(const uint64_t *ptr, uint64_t lo, uint64_t hi, uint64_t e) {
+    while (hi - lo > 1) {
+        const uint64_t mid = (lo + hi) / 2;
+        if (ptr[mid] <= e) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
+// Slice of an in-edge of sliced row j from source v.  Sources ranked below `rep` (the most
+// gathered ones; relabelled ids are out-degree ranks) are cached by every XCD and their edges
+// are spread over the slices by row, which keeps the slices balanced and keeps the requests
+// for the hottest lines off a single L2 channel; every other source belongs to one slice by
+// its 32-id line group.
+__device__ __forceinline__ uint32_t slice_of(uint32_t v, uint64_t j, uint32_t rep, uint32_t S) {
+    return (v < rep) ? (uint32_t)(j % S) : ((v >> kSliceShift) % S);
+}
+
+// Place of every old row in the sweep's lists: its index, with kSlicedRow set for sliced rows.
+constexpr uint32_t kSlicedRow = 0x80000000u;
+__global__ void row_place_kernel(const int32_t *perm, const uint32_t *rows, uint32_t count, uint32_t flag,
+                                 uint32_t *place) {
+    const uint32_t j = blockIdx.x * blockDim.x + threadIdx.x;
+    if (j < count) place[perm[rows[j]]] = j | flag;
+}
+
+// Sort key of every edge: (segment << vbits) | new source, value = old edge index.  A segment is a
+// direct row, or a sliced row's part in one slice; they are numbered in the order of the sweep
+// (direct rows, then slice by slice), so that one stable sort leaves the edges where the sweep reads
+// them, by source within a segment.
+//
+// A block takes kKeyTile consecutive edges and looks its rows up in the offsets: a wave per row
+// left most lanes without an edge (R-MAT, 1.5e7 arcs: 0.73 ms, and 2.8 ms more for a second
+// pair of row-wise kernels that moved the sorted edges into slices; now 0.19 ms).
+constexpr uint32_t kKeyTile = 2048;
+__global__ __launch_bounds__(256) void edge_keys_kernel(const uint64_t *colptr_in, const int32_t *src_in, uint64_t m,
+                                                        const int32_t *iperm, const uint32_t *place, uint64_t z,
+                                                        uint32_t n_d, uint32_t n_s, uint32_t S, uint32_t rep,
+                                                        int vbits, uint64_t *keys, uint32_t *vals) {
+    __shared__ uint64_t s_row[2];
+    const uint64_t e0 = (uint64_t)blockIdx.x * kKeyTile, e1 = std::min<uint64_t>(e0 + kKeyTile, m);
+    if (threadIdx.x < 2) s_row[threadIdx.x] = row_of(colptr_in, 0, z, threadIdx.x ? e1 - 1 : e0);
+    __syncthreads();
+    const uint64_t r0 = s_row[0], r1 = s_row[1] + 1;
+    for (uint64_t i = e0 + threadIdx.x; i < e1; i += 256) {
+        const uint32_t v = (uint32_t)iperm[src_in[i]];
+        const uint32_t at = place[row_of(colptr_in, r0, r1, i)], j = at & ~kSlicedRow;
+        const uint64_t seg = (at & kSlicedRow) ? n_d + (uint64_t)slice_of(v, j, rep, S) * n_s + j : j;
+        keys[i] = (seg << vbits) | v;
+        vals[i] = (uint32_t)i;
     }
 }
 
-__global__ void edge_output_kernel(const uint64_t *keys, const uint32_t *vals, uint64_t m,
+// First edge of every (slice, sliced row) segment, from the sorted keys; ptr[count] = m.
+__global__ void segment_starts_kernel(const uint64_t *keys, uint64_t m, int vbits, uint64_t first, uint64_t count,
+                                      uint32_t *ptr) {
+    for (uint64_t k = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; k <= count;
+         k += (uint64_t)gridDim.x * blockDim.x) {
+        const uint64_t key = (first + k) << vbits;
+        uint64_t lo = 0, hi = k == count ? 0 : m;
+        if (k == count) lo = m;
+        while (lo < hi) {
+            const uint64_t mid = (lo + hi) / 2;
+            if (keys[mid] < key) lo = mid + 1;
+            else hi = mid;
+        }
+        ptr[k] = (uint32_t)lo;
+    }
+}
+
+__global__ void edge_output_kernel(const uint64_t *keys, const uint32_t *vals, uint64_t m, uint64_t vmask,
                                    const float *w_in, const double *w64_in, const int32_t *src_in,
                                    const double *wdeg, int32_t *src_out, float *coef32,
                                    double *coef64) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < m;
          i += (uint64_t)gridDim.x * blockDim.x) {
-        src_out[i] = (int32_t)(uint32_t)(keys[i] & 0xFFFFFFFFull);
+        src_out[i] = (int32_t)(keys[i] & vmask);
         if (coef32) {
             const uint32_t o = vals[i];
             const double w = w64_in ? w64_in[o] : (double)w_in[o];
@@ -226,94 +280,6 @@ __global__ void fp32_exact_kernel(const float *w, const double *w64, uint64_t m,
 __global__ void inv_of_kernel(const double *deg, uint32_t n, double *invw64) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r < n) invw64[r] = deg[r] > 0.0 ? 1.0 / deg[r] : 0.0;
-}
-
-// Per sliced row j: number of in-edges whose source falls in each slice (slice-major output).
-// Slice of an in-edge of sliced row j from source v.  Sources ranked below `rep` (the most
-// gathered ones; relabelled ids are out-degree ranks) are cached by every XCD and their edges
-// are spread over the slices by row, which keeps the slices balanced and keeps the requests
-// for the hottest lines off a single L2 channel; every other source belongs to one slice by
-// its 32-id line group.
-__device__ __forceinline__ uint32_t slice_of(uint32_t v, uint64_t j, uint32_t rep, uint32_t S) {
-    return (v < rep) ? (uint32_t)(j % S) : ((v >> kSliceShift) % S);
-}
-
-__global__ void slice_count_kernel(const uint64_t *colptr, const int32_t *src,
-                                   const uint32_t *srow, uint32_t n_s, uint32_t S, uint32_t rep,
-                                   uint32_t *counts) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    for (uint64_t j = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; j < n_s;
-         j += nwaves) {
-        const uint32_t r = srow[j];
-        const uint64_t b = colptr[r], e = colptr[r + 1];
-        uint32_t cnt[kSlices] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (uint64_t i = b; i < e; i += 64) {
-            const bool valid = i + lane < e;
-            const uint32_t sl = valid ? slice_of((uint32_t)src[i + lane], j, rep, S) : 0u;
-            for (uint32_t q = 0; q < S; ++q) cnt[q] += __popcll(__ballot(valid && sl == q));
-        }
-        if (lane == 0)
-            for (uint32_t q = 0; q < S; ++q) counts[(uint64_t)q * n_s + j] = cnt[q];
-    }
-}
-
-__global__ void add_base_kernel(uint32_t *p, uint64_t n, uint32_t base) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
-         i += (uint64_t)gridDim.x * blockDim.x)
-        p[i] += base;
-}
-
-// Copy the in-edges of every row to its place in the sweep order: direct rows keep their
-// (source-sorted) order; sliced rows are split slice by slice, source order kept within a
-// slice (stable: ballot ranks).
-__global__ void reorder_edges_kernel(const uint64_t *colptr, const int32_t *src,
-                                     const float *c32, const double *c64, const uint32_t *rows,
-                                     uint32_t nrows, const uint32_t *dptr, const uint32_t *sptr,
-                                     uint32_t n_s, uint32_t S, uint32_t rep, int32_t *src2,
-                                     float *c32_2, double *c64_2, const uint32_t *em,
-                                     uint32_t *em2) {
-    const uint32_t lane = threadIdx.x & 63;
-    const uint64_t below = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint64_t nwaves = ((uint64_t)gridDim.x * blockDim.x) >> 6;
-    for (uint64_t j = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) >> 6; j < nrows;
-         j += nwaves) {
-        const uint32_t r = rows[j];
-        const uint64_t b = colptr[r], e = colptr[r + 1];
-        if (dptr) {
-            const uint32_t d = dptr[j];
-            for (uint64_t i = b + lane; i < e; i += 64) {
-                src2[d + (i - b)] = src[i];
-                if (c32) {
-                    c32_2[d + (i - b)] = c32[i];
-                    c64_2[d + (i - b)] = c64[i];
-                }
-                if (em) em2[d + (i - b)] = em[i];
-            }
-            continue;
-        }
-        uint32_t run[kSlices] = {0, 0, 0, 0, 0, 0, 0, 0};
-        for (uint64_t i = b; i < e; i += 64) {
-            const bool valid = i + lane < e;
-            const int32_t v = valid ? src[i + lane] : 0;
-            const uint32_t sl = valid ? slice_of((uint32_t)v, j, rep, S) : 0u;
-            uint32_t dest = 0;
-            for (uint32_t q = 0; q < S; ++q) {
-                const uint64_t mask = __ballot(valid && sl == q);
-                if (valid && sl == q)
-                    dest = sptr[(uint64_t)q * n_s + j] + run[q] + (uint32_t)__popcll(mask & below);
-                run[q] += (uint32_t)__popcll(mask);
-            }
-            if (valid) {
-                src2[dest] = v;
-                if (c32) {
-                    c32_2[dest] = c32[i + lane];
-                    c64_2[dest] = c64[i + lane];
-                }
-                if (em) em2[dest] = em[i + lane];
-            }
-        }
-    }
 }
 
 // ---- schedule, on the device ----------------------------------------------------------------
@@ -427,12 +393,11 @@ uint32_t env_u32(const char *name, uint32_t dflt) {
     return (uint32_t)std::strtoul(v, nullptr, 10);
 }
 
-// Splits rows into direct and sliced ones, reorders the in-edges into sweep order and builds
-// the work items.  Input: g->colptr / g->src / g->coef* in (row, source) order.
-void build_schedule(nkpr_graph *g) {
+// Splits the rows of g->colptr into direct and sliced ones, in the order in which a sweep takes
+// them; the in-edges are then sorted into that order.
+void schedule_rows(nkpr_graph *g) {
     const hipStream_t s = g->stream;
     const uint32_t n = g->n;
-    const uint64_t m = g->m;
     // slicing pays off once the gathered vector outgrows one L2; below that everything is
     // direct.  NKPR_SLICES (1 or 8) and NKPR_DIRECT_MAX_DEG override the defaults.
     // (the rows of a batch's graph gather from that graph's part of it alone: a union of 160
@@ -457,7 +422,7 @@ void build_schedule(nkpr_graph *g) {
     DevBuf nsel;
     nsel.alloc(32);
     NKPR_HIP(hipMemsetAsync(nsel.p, 0, 32, s));
-    uint32_t *sel = nsel.as<uint32_t>();  // direct rows, sliced rows, heavy segments, -, largest degree
+    uint32_t *sel = nsel.as<uint32_t>();  // direct rows, sliced rows, -, -, largest degree
     {
         DevBuf rows, tmp, lens;
         rows.alloc(4 * std::max<size_t>(2 * (size_t)n, 1));
@@ -496,96 +461,29 @@ void build_schedule(nkpr_graph *g) {
         NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(tmp2.p, tb, lens.as<uint32_t>(), g->dptr.as<uint32_t>(),
                                                   (size_t)g->n_d + 1, s));
     }
-    uint32_t md = 0;
-    read_back(s, {{&md, g->dptr.as<uint32_t>() + g->n_d, 4}});
-    const uint32_t n_s = g->n_s;
+    NKPR_CHECK((uint64_t)S * g->n_s + 1 < 0xFFFFFFFFull, "too many sliced rows");
+    NKPR_HIP(hipStreamSynchronize(s));  // the temporaries go back
+}
 
-    // per-slice offsets of the sliced rows: exclusive scan of the slice-major counts
+// The work items over the rows of schedule_rows, once g->src / g->coef* and g->sptr stand.
+void schedule_items(nkpr_graph *g) {
+    const hipStream_t s = g->stream;
+    const uint64_t m = g->m;
+    const uint32_t S = g->n_slices, n_s = g->n_s;
     const uint64_t ns_tot = (uint64_t)S * n_s;
-    NKPR_CHECK(ns_tot + 1 < 0xFFFFFFFFull, "too many sliced rows");
-    g->sptr.alloc(4 * (ns_tot + 1));
-    {
-        DevBuf counts, tmp;
-        counts.alloc(4 * (ns_tot + 1));
-        NKPR_HIP(hipMemsetAsync(counts.p, 0, 4 * (ns_tot + 1), s));
-        if (n_s) {
-            const unsigned blocks = (unsigned)std::min<uint64_t>(blocks_for((uint64_t)n_s * 64), 1u << 18);
-            hipLaunchKernelGGL(slice_count_kernel, dim3(blocks), dim3(256), 0, s,
-                               g->colptr.as<uint64_t>(), g->src.as<int32_t>(),
-                               g->srow.as<uint32_t>(), n_s, S, rep, counts.as<uint32_t>());
-            NKPR_HIP(hipGetLastError());
-        }
-        size_t tb = 0;
-        NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, tb, counts.as<uint32_t>(),
-                                                  g->sptr.as<uint32_t>(), (size_t)ns_tot + 1, s));
-        tmp.alloc(tb);
-        NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, counts.as<uint32_t>(),
-                                                  g->sptr.as<uint32_t>(), (size_t)ns_tot + 1, s));
-        hipLaunchKernelGGL(add_base_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(ns_tot + 1), 65536)),
-                           dim3(256), 0, s, g->sptr.as<uint32_t>(), ns_tot + 1, md);
-        NKPR_HIP(hipGetLastError());
-        NKPR_HIP(hipStreamSynchronize(s));
-    }
-
-    // edges into sweep order (kCap zero entries of padding after the last one)
-    {
-        DevBuf src2, c32, c64;
-        src2.alloc(4 * (m + kCap));
-        NKPR_HIP(hipMemsetAsync(src2.as<int32_t>() + m, 0, 4 * kCap, s));
-        if (g->weighted) {
-            c32.alloc(4 * (m + kCap));
-            c64.alloc(8 * (m + kCap));
-            NKPR_HIP(hipMemsetAsync(c32.as<float>() + m, 0, 4 * kCap, s));
-            NKPR_HIP(hipMemsetAsync(c64.as<double>() + m, 0, 8 * kCap, s));
-        }
-        const float *o32 = g->weighted ? g->coef32.as<float>() : nullptr;
-        const double *o64 = g->weighted ? g->coef64.as<double>() : nullptr;
-        float *n32 = g->weighted ? c32.as<float>() : nullptr;
-        double *n64 = g->weighted ? c64.as<double>() : nullptr;
-        DevBuf em2;
-        const uint32_t *em = g->weighted ? g->emap.as<uint32_t>() : nullptr;
-        if (g->weighted) em2.alloc(4 * std::max<uint64_t>(m, 1));
-        uint32_t *emo = g->weighted ? em2.as<uint32_t>() : nullptr;
-        if (g->n_d) {
-            const unsigned blocks = (unsigned)std::min<uint64_t>(blocks_for((uint64_t)g->n_d * 64), 1u << 18);
-            hipLaunchKernelGGL(reorder_edges_kernel, dim3(blocks), dim3(256), 0, s,
-                               g->colptr.as<uint64_t>(), g->src.as<int32_t>(), o32, o64,
-                               g->drow.as<uint32_t>(), g->n_d, g->dptr.as<uint32_t>(), nullptr,
-                               0u, S, rep, src2.as<int32_t>(), n32, n64, em, emo);
-            NKPR_HIP(hipGetLastError());
-        }
-        if (n_s) {
-            const unsigned blocks = (unsigned)std::min<uint64_t>(blocks_for((uint64_t)n_s * 64), 1u << 18);
-            hipLaunchKernelGGL(reorder_edges_kernel, dim3(blocks), dim3(256), 0, s,
-                               g->colptr.as<uint64_t>(), g->src.as<int32_t>(), o32, o64,
-                               g->srow.as<uint32_t>(), n_s, nullptr, g->sptr.as<uint32_t>(),
-                               n_s, S, rep, src2.as<int32_t>(), n32, n64, em, emo);
-            NKPR_HIP(hipGetLastError());
-        }
-        NKPR_HIP(hipStreamSynchronize(s));
-        std::swap(g->src.p, src2.p);
-        std::swap(g->src.bytes, src2.bytes);
-        if (g->weighted) {
-            std::swap(g->coef32.p, c32.p);
-            std::swap(g->coef32.bytes, c32.bytes);
-            std::swap(g->coef64.p, c64.p);
-            std::swap(g->coef64.bytes, c64.bytes);
-            std::swap(g->emap.p, em2.p);
-            std::swap(g->emap.bytes, em2.bytes);
-        }
-    }
-
     // work items: the rows longer than kCap on the host (at most m / kCap), the runs of shorter rows
     // on the device, whose counts per segment give every run its place
     std::vector<uint4> heavy;
     if (n_s) {
-        DevBuf hv;
+        DevBuf hv, nhv;
         hv.alloc(sizeof(uint4) * (m / kCap + 1));
+        nhv.alloc(4);
+        NKPR_HIP(hipMemsetAsync(nhv.p, 0, 4, s));
         hipLaunchKernelGGL(heavy_rows_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(ns_tot), 4096)), dim3(256),
-                           0, s, (const uint32_t *)g->sptr.as<uint32_t>(), ns_tot, sel + 2, hv.as<uint4>());
+                           0, s, (const uint32_t *)g->sptr.as<uint32_t>(), ns_tot, nhv.as<uint32_t>(), hv.as<uint4>());
         NKPR_HIP(hipGetLastError());
         uint32_t nh = 0;
-        read_back(s, {{&nh, sel + 2, 4}});
+        read_back(s, {{&nh, nhv.p, 4}});
         heavy.resize(nh);
         read_back(s, {{heavy.data(), hv.p, sizeof(uint4) * (size_t)nh}});
         std::sort(heavy.begin(), heavy.end(), [](const uint4 &x, const uint4 &y) { return x.x < y.x; });
@@ -674,8 +572,8 @@ void build_schedule(nkpr_graph *g) {
     NKPR_HIP(hipMemsetAsync(g->claim.p, 0, 4 * (kArriveAt + kArriveWords), s));
     NKPR_HIP(hipStreamSynchronize(s));
     if (env_u32("NKPR_DEBUG", 0))
-        std::fprintf(stderr, "[nkpr] n=%u direct rows %u (%u edges, %u items), sliced rows %u (%u items), "
-                             "slices %u, split rows %u\n", n, g->n_d, md, g->n_ditems, n_s,
+        std::fprintf(stderr, "[nkpr] n=%u direct rows %u (%u items), sliced rows %u (%u items), "
+                             "slices %u, split rows %u\n", g->n, g->n_d, g->n_ditems, n_s,
                      g->n_items - g->n_ditems, S, g->n_split_rows);
 }
 
@@ -887,44 +785,65 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     }
     len_b.reset();
 
-    // --- edges: sort by (new row, new source) ------------------------------------------------
-    g->src.alloc(4 * std::max<uint64_t>(m, 1));
+    // --- edges: into the order of the sweep (kCap zero entries of padding after the last one) ---
+    schedule_rows(g);
+    const uint64_t ns_tot = (uint64_t)g->n_slices * g->n_s, nseg = g->n_d + ns_tot;
+    g->sptr.alloc(4 * (ns_tot + 1));
+    g->src.alloc(4 * (m + kCap));
+    NKPR_HIP(hipMemsetAsync(g->src.as<int32_t>() + m, 0, 4 * kCap, s));
     if (g->weighted) {
-        g->coef32.alloc(4 * std::max<uint64_t>(m, 1));
-        g->coef64.alloc(8 * std::max<uint64_t>(m, 1));
+        g->coef32.alloc(4 * (m + kCap));
+        g->coef64.alloc(8 * (m + kCap));
+        NKPR_HIP(hipMemsetAsync(g->coef32.as<float>() + m, 0, 4 * kCap, s));
+        NKPR_HIP(hipMemsetAsync(g->coef64.as<double>() + m, 0, 8 * kCap, s));
     }
     if (m) {
-        DevBuf ka, kb2, va, vb2;
+        DevBuf ka, kb2, va, vb2, place;
         ka.alloc(8 * m);
         kb2.alloc(8 * m);
         va.alloc(4 * m);
         vb2.alloc(4 * m);
-        const unsigned kblocks = (unsigned)std::min<uint64_t>(blocks_for(z * 64), 1u << 18);
-        hipLaunchKernelGGL(edge_keys_kernel, dim3(kblocks), dim3(256), 0, s, colptr_in,
-                           src_in, iperm, z, ka.as<uint64_t>(), va.as<uint32_t>());
+        place.alloc(4 * z);
+        if (g->n_d)
+            hipLaunchKernelGGL(row_place_kernel, dim3(blocks_for(g->n_d)), dim3(256), 0, s, g->perm.as<int32_t>(),
+                               (const uint32_t *)g->drow.as<uint32_t>(), g->n_d, 0u, place.as<uint32_t>());
+        if (g->n_s)
+            hipLaunchKernelGGL(row_place_kernel, dim3(blocks_for(g->n_s)), dim3(256), 0, s, g->perm.as<int32_t>(),
+                               (const uint32_t *)g->srow.as<uint32_t>(), g->n_s, kSlicedRow, place.as<uint32_t>());
+        const int vbits = bits_for(n);
+        hipLaunchKernelGGL(edge_keys_kernel, dim3((unsigned)((m + kKeyTile - 1) / kKeyTile)), dim3(256), 0, s, colptr_in,
+                           src_in, m, iperm, (const uint32_t *)place.as<uint32_t>(), z, g->n_d, g->n_s, g->n_slices,
+                           env_u32("NKPR_SLICE_REPLICATE", kDefaultSliceReplicate), vbits, ka.as<uint64_t>(),
+                           va.as<uint32_t>());
         NKPR_HIP(hipGetLastError());
         hipcub::DoubleBuffer<uint64_t> kd(ka.as<uint64_t>(), kb2.as<uint64_t>());
         hipcub::DoubleBuffer<uint32_t> vd(va.as<uint32_t>(), vb2.as<uint32_t>());
-        const int end_bit = 32 + bits_for(n);
+        int end_bit = vbits;
+        while (end_bit < 64 && (1ull << (end_bit - vbits)) < nseg) ++end_bit;
         size_t tb = 0;
         NKPR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, kd, vd, (size_t)m, 0, end_bit, s));
         tmp.alloc(tb);
         NKPR_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, kd, vd, (size_t)m, 0, end_bit, s));
-        NKPR_HIP(hipStreamSynchronize(s));
-        tmp.reset();
+        hipLaunchKernelGGL(segment_starts_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(ns_tot + 1), 65536)),
+                           dim3(256), 0, s, (const uint64_t *)kd.Current(), m, vbits, (uint64_t)g->n_d, ns_tot,
+                           g->sptr.as<uint32_t>());
         const unsigned gb = (unsigned)std::min<uint64_t>(blocks_for(m), 65536);
         hipLaunchKernelGGL(edge_output_kernel, dim3(gb), dim3(256), 0, s, kd.Current(), vd.Current(),
-                           m, g->weighted ? w_in : nullptr, g->weighted ? w64_in : nullptr, src_in,
+                           m, (1ull << vbits) - 1, g->weighted ? w_in : nullptr, g->weighted ? w64_in : nullptr, src_in,
                            wdeg, g->src.as<int32_t>(),
                            g->weighted ? g->coef32.as<float>() : nullptr,
                            g->weighted ? g->coef64.as<double>() : nullptr);
         NKPR_HIP(hipGetLastError());
         if (g->weighted) {
             // input position of every edge, kept so that new weights can be folded in place
-            g->emap.alloc(4 * m);
-            NKPR_HIP(hipMemcpyAsync(g->emap.p, vd.Current(), 4 * m, hipMemcpyDeviceToDevice, s));
+            DevBuf &sorted = vd.Current() == va.as<uint32_t>() ? va : vb2;
+            std::swap(g->emap.p, sorted.p);
+            std::swap(g->emap.bytes, sorted.bytes);
         }
         NKPR_HIP(hipStreamSynchronize(s));
+        tmp.reset();
+    } else {
+        NKPR_HIP(hipMemsetAsync(g->sptr.p, 0, 4 * (ns_tot + 1), s));
     }
     if (!g->weighted) {
         g->inv32.alloc(4 * std::max<uint64_t>(n, 1));
@@ -956,7 +875,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     }
 
     // --- schedule ---------------------------------------------------------------------------
-    build_schedule(g);
+    schedule_items(g);
     NKPR_HIP(hipStreamSynchronize(s));
     g->prep_ms =
         std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
