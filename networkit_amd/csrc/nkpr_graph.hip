@@ -168,16 +168,6 @@ __global__ void new_lengths_kernel(const int32_t *perm, uint32_t n, const uint64
     }
 }
 
-// Row r of [lo, hi) with ptr[r] <= e < ptr[r + 1] (ptr rises; e lies in these rows).
-__device__ __forceinline__ uint64_t row_of(const uint64_t *ptr, uint64_t lo, uint64_t hi, uint64_t e) {
-    while (hi - lo > 1) {
-        const uint64_t mid = (lo + hi) / 2;
-        if (ptr[mid] <= e) lo = mid;
-        else hi = mid;
-    }
-    return lo;
-}
-
 // Slice of an in-edge of sliced row j from source v.  Sources ranked below `rep` (the most
 // gathered ones; relabelled ids are out-degree ranks) are cached by every XCD and their edges
 // are spread over the slices by row, which keeps the slices balanced and keeps the requests
@@ -318,7 +308,7 @@ __global__ void heavy_rows_kernel(const uint32_t *ptr, uint64_t count, uint32_t 
 // at ptr[q nrows]): runs of consecutive rows with at most `cap` in-edges and kRowsMax rows (a row with
 // more has an item of its own); rows longer than kCap are left out (see build_heavy).  A wave takes
 // kSegRows rows of a list and tries a step's kRowsMax ends at once.  Without `items` it only counts.
-constexpr uint32_t kSegRows = 32768;
+constexpr uint32_t kSegRows = 8192;
 __global__ __launch_bounds__(256) void build_items_kernel(const uint32_t *ptr, uint32_t nrows, uint32_t lists,
                                                           uint32_t segs, uint32_t cap, uint32_t *counts,
                                                           const uint32_t *first, uint4 *items) {

@@ -119,6 +119,17 @@ hipStream_t stream_get();  // non-blocking, default priority
 void stream_put(hipStream_t s, int device);
 
 // Owning device allocation.
+// Row r of [lo, hi) with ptr[r] <= e < ptr[r + 1] (ptr rises; e lies in these rows).
+template <typename P>
+__device__ __forceinline__ uint64_t row_of(const P *ptr, uint64_t lo, uint64_t hi, uint64_t e) {
+    while (hi - lo > 1) {
+        const uint64_t mid = (lo + hi) / 2;
+        if (ptr[mid] <= e) lo = mid;
+        else hi = mid;
+    }
+    return lo;
+}
+
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
