@@ -160,20 +160,23 @@ __global__ void bin_row_kernel(const uint32_t *rowptr, uint32_t n, uint32_t *row
 // by source, which spreads the destinations of a wave's atomics over the accumulator
 // (chunks of 2^ss sources, bins of kBin destinations)
 // Hot edges (source below `hot`) go to the segments of a chunk past the last one, one per bin.
+// Keys are 32 bits wide where they fit, which halves what the sort moves per pass.
+template <typename K>
 __global__ void bin_key_kernel(const int32_t *src, const uint32_t *row, uint64_t m, uint32_t nbins,
-                               int ss, uint32_t nchunks, uint32_t hot, uint64_t *key, uint32_t *val) {
+                               int ss, uint32_t nchunks, uint32_t hot, K *key, uint32_t *val) {
     for (uint64_t e = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
          e += (uint64_t)gridDim.x * blockDim.x) {
         const uint32_t v = (uint32_t)src[e];
         const uint32_t chunk = v < hot ? nchunks : (v >> ss);
         const uint64_t seg = (uint64_t)chunk * nbins + (row[e] >> kBinShift);
-        key[e] = (seg << ss) | (v & ((1u << ss) - 1));
+        key[e] = (K)((seg << ss) | (v & ((1u << ss) - 1)));
         val[e] = (uint32_t)e;
     }
 }
 
 // seg[s] = first sorted edge of segment s (binary search over the sorted keys)
-__global__ void bin_seg_kernel(const uint64_t *key, uint64_t m, uint64_t nseg, int ss, uint32_t *seg) {
+template <typename K>
+__global__ void bin_seg_kernel(const K *key, uint64_t m, uint64_t nseg, int ss, uint32_t *seg) {
     for (uint64_t sidx = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; sidx <= nseg;
          sidx += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t x = sidx << ss;
@@ -189,12 +192,13 @@ __global__ void bin_seg_kernel(const uint64_t *key, uint64_t m, uint64_t nseg, i
 
 // order[p] = edge at chunk-major padded position p: the sorted edge j of segment s goes to
 // cseg[s] + (j - rseg[s]) (rseg: unpadded segment starts, cseg: padded ones)
-__global__ void bin_place_kernel(const uint64_t *key, const uint32_t *ids, uint64_t m, int ss,
+template <typename K>
+__global__ void bin_place_kernel(const K *key, const uint32_t *ids, uint64_t m, int ss,
                                  uint64_t nseg, const uint32_t *rseg, const uint32_t *cseg,
                                  uint32_t *order) {
     for (uint64_t j = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < m;
          j += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t sidx = key[j] >> ss;
+        const uint64_t sidx = (uint64_t)key[j] >> ss;
         if (sidx >= nseg) continue;  // a hot edge
         order[cseg[sidx] + ((uint32_t)j - rseg[sidx])] = ids[j];
     }
@@ -202,12 +206,13 @@ __global__ void bin_place_kernel(const uint64_t *key, const uint32_t *ids, uint6
 
 // horder[p] = edge at padded hot position p: the sorted hot edge j of bin b (segment nseg + b)
 // goes to hseg[b] + (j - rseg[nseg + b])
-__global__ void bin_hot_place_kernel(const uint64_t *key, const uint32_t *ids, uint64_t j0,
+template <typename K>
+__global__ void bin_hot_place_kernel(const K *key, const uint32_t *ids, uint64_t j0,
                                      uint64_t m, int ss, uint64_t nseg, const uint32_t *rseg,
                                      const uint32_t *hseg, uint32_t *horder) {
     for (uint64_t j = j0 + (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; j < m;
          j += (uint64_t)gridDim.x * blockDim.x) {
-        const uint64_t sidx = key[j] >> ss;
+        const uint64_t sidx = (uint64_t)key[j] >> ss;
         horder[hseg[sidx - nseg] + ((uint32_t)j - rseg[sidx])] = ids[j];
     }
 }
@@ -1117,8 +1122,30 @@ uint32_t choose_hot(nkpr_graph *g, const BinLayout &L) {
 
 // Builds the binned copy L (once per graph; coefficients again after new weights).  Returns
 // false when the padded copy would not fit 32-bit positions.
+template <typename K> bool build_layout_keys(nkpr_graph *g, BinLayout &L, int bits);
+
+// Bits of the sort key: the source offset, then the segment (a segment more per bin for the hot
+// sources, whose number is chosen here).
+int key_bits(nkpr_graph *g, BinLayout &L) {
+    const uint32_t span = 1u << L.span_shift;
+    const uint64_t nchunks = std::max<uint32_t>(1, (g->sink_begin + span - 1) / span);
+    const uint64_t nbins = (g->n + kBin - 1) / kBin;
+    L.hot = choose_hot(g, L);
+    const uint64_t nseg = nchunks * nbins + (L.hot ? nbins : 0);
+    int bits = L.span_shift + 1;
+    while (bits < 64 && (1ull << (bits - L.span_shift)) < nseg) ++bits;
+    return bits;
+}
+
 bool build_layout(nkpr_graph *g, BinLayout &L) {
     if (L.ready && L.coef_ready) return true;
+    // new coefficients keep the order, and with it the hot sources
+    const int bits = L.ready ? 32 : key_bits(g, L);
+    // the segment search compares with the key past the last segment, one bit more
+    return bits < 32 ? build_layout_keys<uint32_t>(g, L, bits) : build_layout_keys<uint64_t>(g, L, bits);
+}
+
+template <typename K> bool build_layout_keys(nkpr_graph *g, BinLayout &L, int bits) {
     // test hook: the allocation failure of a device that is too small for the copy
     if (const char *t = std::getenv("NKPR_TEST_BINNED_NOMEM"); t && std::atoi(t) != 0)
         throw Error(NKPR_ERR_NOMEM, "binned copy: allocation refused (NKPR_TEST_BINNED_NOMEM)");
@@ -1148,37 +1175,34 @@ bool build_layout(nkpr_graph *g, BinLayout &L) {
     }
     // hot sources skip pass 1: their edges sort into one extra segment per bin (a chunk past
     // the last one)
-    L.hot = choose_hot(g, L);
     const uint64_t nseg_all = nseg + (L.hot ? nbins : 0);
     // sort the edges by key and find the unpadded segment starts (chunk-major)
     std::vector<uint32_t> seg(nseg_all + 1, 0u);
     rseg.alloc(4 * (nseg_all + 1));
     if (m) {
-        k1.alloc(8 * m);
-        k2.alloc(8 * m);
+        k1.alloc(sizeof(K) * m);
+        k2.alloc(sizeof(K) * m);
         v1.alloc(4 * m);
         v2.alloc(4 * m);
-        hipLaunchKernelGGL(bin_key_kernel, dim3(nb(m)), dim3(256), 0, s, g->b_src.as<int32_t>(),
-                           row.as<uint32_t>(), m, nbins, ss, nchunks, L.hot, k1.as<uint64_t>(),
+        hipLaunchKernelGGL(bin_key_kernel<K>, dim3(nb(m)), dim3(256), 0, s, g->b_src.as<int32_t>(),
+                           row.as<uint32_t>(), m, nbins, ss, nchunks, L.hot, k1.as<K>(),
                            v1.as<uint32_t>());
         NKPR_HIP(hipGetLastError());
-        hipcub::DoubleBuffer<uint64_t> kb(k1.as<uint64_t>(), k2.as<uint64_t>());
+        hipcub::DoubleBuffer<K> kb(k1.as<K>(), k2.as<K>());
         hipcub::DoubleBuffer<uint32_t> vb(v1.as<uint32_t>(), v2.as<uint32_t>());
-        int bits = ss + 1;
-        while (bits < 64 && (1ull << (bits - ss)) < nseg_all) ++bits;
         size_t tb = 0;
         NKPR_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, tb, kb, vb, (size_t)m, 0, bits, s));
         tmp.alloc(tb);
         NKPR_HIP(hipcub::DeviceRadixSort::SortPairs(tmp.p, tb, kb, vb, (size_t)m, 0, bits, s));
         // keep the sorted halves in k1 / v1 and free the others
-        if (kb.Current() != k1.as<uint64_t>()) std::swap(k1.p, k2.p), std::swap(k1.bytes, k2.bytes);
+        if (kb.Current() != k1.as<K>()) std::swap(k1.p, k2.p), std::swap(k1.bytes, k2.bytes);
         if (vb.Current() != v1.as<uint32_t>()) std::swap(v1.p, v2.p), std::swap(v1.bytes, v2.bytes);
         NKPR_HIP(hipStreamSynchronize(s));
         k2.reset();
         v2.reset();
         tmp.reset();
-        hipLaunchKernelGGL(bin_seg_kernel, dim3(nb(nseg_all + 1)), dim3(256), 0, s,
-                           (const uint64_t *)k1.as<uint64_t>(), m, nseg_all, ss, rseg.as<uint32_t>());
+        hipLaunchKernelGGL(bin_seg_kernel<K>, dim3(nb(nseg_all + 1)), dim3(256), 0, s,
+                           (const K *)k1.as<K>(), m, nseg_all, ss, rseg.as<uint32_t>());
         NKPR_HIP(hipGetLastError());
         read_back(s, {{seg.data(), rseg.p, 4 * (nseg_all + 1)}});
     }
@@ -1218,7 +1242,7 @@ bool build_layout(nkpr_graph *g, BinLayout &L) {
     L.order.alloc(4 * std::max<uint64_t>(mp, 1));
     NKPR_HIP(hipMemsetAsync(L.order.p, 0xFF, 4 * std::max<uint64_t>(mp, 1), s));
     if (m)
-        hipLaunchKernelGGL(bin_place_kernel, dim3(nb(m)), dim3(256), 0, s, (const uint64_t *)k1.as<uint64_t>(),
+        hipLaunchKernelGGL(bin_place_kernel<K>, dim3(nb(m)), dim3(256), 0, s, (const K *)k1.as<K>(),
                            (const uint32_t *)v1.as<uint32_t>(), m, ss, nseg, (const uint32_t *)rseg.as<uint32_t>(),
                            (const uint32_t *)cseg.as<uint32_t>(), L.order.as<uint32_t>());
     NKPR_HIP(hipGetLastError());
@@ -1239,8 +1263,8 @@ bool build_layout(nkpr_graph *g, BinLayout &L) {
         L.horder.alloc(4 * std::max<uint64_t>(h, 1));
         NKPR_HIP(hipMemsetAsync(L.horder.p, 0xFF, 4 * std::max<uint64_t>(h, 1), s));
         if (m > seg[nseg])
-            hipLaunchKernelGGL(bin_hot_place_kernel, dim3(nb(m - seg[nseg])), dim3(256), 0, s,
-                               (const uint64_t *)k1.as<uint64_t>(), (const uint32_t *)v1.as<uint32_t>(),
+            hipLaunchKernelGGL(bin_hot_place_kernel<K>, dim3(nb(m - seg[nseg])), dim3(256), 0, s,
+                               (const K *)k1.as<K>(), (const uint32_t *)v1.as<uint32_t>(),
                                (uint64_t)seg[nseg], m, ss, nseg, (const uint32_t *)rseg.as<uint32_t>(),
                                (const uint32_t *)hs.as<uint32_t>(), L.horder.as<uint32_t>());
         NKPR_HIP(hipGetLastError());
@@ -1467,17 +1491,29 @@ void persistent_grids(nkpr_graph *g, BinLayout &L, K1 k1, K2 k2) {
 // The binned copies serve graphs with at least kBinnedMinEdges edges (on R-MAT scale 26 the
 // FP32 operator takes 3.2-3.6 ms per application against 8.4 ms for the pull sweep; on graphs
 // whose gathers stay in the caches the pull sweep is as fast and needs no second copy).
+//
+// The pull sweep's gathers stay in the caches while most arcs leave a few sources (R-MAT of 2^25 arcs:
+// mixed solve 4.10 ms, binned 4.23).  Where at most one arc in kSpreadShare leaves the kHubSources
+// sources with the most, they are spread over the vector, and the copies pay once it outgrows an XCD's
+// 4 MiB of L2: uniform graphs, mixed solve, pull / binned: 2^19 nodes of 16 arcs 1.71 / 2.06 ms, 2^20
+// 3.66 / 2.71, 2^21 6.42 / 3.60; hyperbolic graphs 2^19 3.04 / 4.01, 2^20 6.87 / 6.00, 2^21 12.5 /
+// 8.5.  FP64 solves gain a doubling later: uniform 2^20 3.53 / 3.42, 2^21 6.53 / 4.58, hyperbolic 2^20
+// 12.3 / 14.2, 2^21 22.8 / 18.3.  The one or two FP64 sweeps of a mixed solve do not pay a copy of
+// their own, nor do weighted graphs (new weights re-emit the copy) and batches (rows gather near
+// their own): these keep the first bound.
 // NKPR_BINNED=0 / 1 (FP32 operator) and NKPR_BINNED64=0 / 1 (FP64 sweep) force either way.
-constexpr uint64_t kBinnedMinEdges = 1ull << 26;
+constexpr uint64_t kBinnedMinEdges = 1ull << 26, kSpreadMinEdges = 1ull << 23;
+constexpr uint64_t kSpreadShare = 6;
 
-bool policy(const nkpr_graph *g, const char *env) {
+bool policy(const nkpr_graph *g, const char *env, uint32_t spread_nodes) {
     if (const char *e = std::getenv(env); e && *e) return std::atoi(e) != 0;
-    return g->m >= kBinnedMinEdges;
+    const bool spread = !g->weighted && g->n_groups == 0 && g->n >= spread_nodes && g->hub_edges * kSpreadShare <= g->m;
+    return g->m >= (spread ? kSpreadMinEdges : kBinnedMinEdges);
 }
 
 }  // namespace
 
-bool binned_enabled(const nkpr_graph *g) { return !g->bn32.off && policy(g, "NKPR_BINNED"); }
+bool binned_enabled(const nkpr_graph *g) { return !g->bn32.off && policy(g, "NKPR_BINNED", 1u << 20); }
 
 bool binned_layout(nkpr_graph *g) {
     g->bn32.span_shift = kSpan32Shift;
@@ -1528,8 +1564,8 @@ void binned_apply(nkpr_graph *g, const float *v, float *w, double damp, bool dis
     NKPR_HIP(hipGetLastError());
 }
 
-bool binned64_active(nkpr_graph *g) {
-    if (g->bn64.off || !policy(g, "NKPR_BINNED64")) return false;
+bool binned64_active(nkpr_graph *g, bool one_sweep) {
+    if (g->bn64.off || !policy(g, "NKPR_BINNED64", one_sweep ? ~0u : 1u << 21)) return false;
     g->bn64.span_shift = kSpan64Shift;
     g->bn64.fp64 = true;
     return layout_ready(g, g->bn64);

@@ -239,7 +239,7 @@ SolveResult solve_core(nkpr_graph *g, const nkpr_params *p, const double *base64
         // d = 0.85 (1% added for the rounding of these FP64 formulas).
         // NKPR_COMPACT64=0 keeps 8-byte contributions
         const char *cenv = std::getenv("NKPR_COMPACT64");
-        const bool compact = binned64_active(g) && !(cenv && cenv[0] == '0');
+        const bool compact = binned64_active(g, true) && !(cenv && cenv[0] == '0');
         const double slack = compact ? (2.0 * damp / (1.0 - damp) + 1.0) * damp * kCompact64Rel * 1.01 : 0.0;
         // A run that starts from a constant vector x = c (every first run does: 1/n) begins
         // with y = d P x + b = d c rowsum + b in closed form, from the cached FP64 row sums of

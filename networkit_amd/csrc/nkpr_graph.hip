@@ -152,6 +152,15 @@ __global__ __launch_bounds__(256) void count_kernel(const uint32_t *outcnt, cons
     }
 }
 
+// Edges from the first `count` relabelled sources (one block).
+__global__ __launch_bounds__(1024) void hub_edges_kernel(const int32_t *perm, uint32_t count, const uint32_t *outcnt,
+                                                         unsigned long long *sum) {
+    unsigned long long mine = 0;
+    for (uint32_t r = threadIdx.x; r < count; r += 1024) mine += outcnt[perm[r]];
+    for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off, 64);
+    if ((threadIdx.x & 63) == 0) atomicAdd(sum, mine);
+}
+
 __global__ void iperm_kernel(const int32_t *perm, uint32_t n, int32_t *iperm) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r < n) iperm[perm[r]] = (int32_t)r;
@@ -754,7 +763,14 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     if (n)
         hipLaunchKernelGGL(iperm_kernel, dim3(blocks_for(n)), dim3(256), 0, s, g->perm.as<int32_t>(),
                            n, iperm);
-    NKPR_HIP(hipStreamSynchronize(s));  // the sort buffers are freed below
+    NKPR_HIP(hipMemsetAsync(counts, 0, 8, s));
+    if (n)
+        hipLaunchKernelGGL(hub_edges_kernel, dim3(1), dim3(1024), 0, s, g->perm.as<int32_t>(),
+                           std::min<uint32_t>(n, kHubSources), outcnt_b.as<uint32_t>(), counts);
+    NKPR_HIP(hipGetLastError());
+    unsigned long long hub = 0;
+    read_back(s, {{&hub, counts, 8}});  // (the sort buffers are freed below)
+    g->hub_edges = hub;
     k1.reset(); k2.reset(); v1.reset(); v2.reset(); tmp.reset();
 
     // --- new colptr -------------------------------------------------------------------------

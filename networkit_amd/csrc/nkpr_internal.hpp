@@ -46,6 +46,7 @@ constexpr uint32_t kXcds = 8;
 constexpr int kSliceShift = 5;
 constexpr uint32_t kDefaultDirectMaxDeg = 8;
 constexpr uint32_t kDefaultSliceReplicate = 32768;  // top-ranked sources cached by every XCD
+constexpr uint32_t kHubSources = 8192;
 constexpr int kCombineThreads = 256;
 // Counters of the blocks that have ended a launch: one on top, kArriveGroups below it, each on a
 // line of its own (kArriveStride words), behind the kSlices claim counters.
@@ -367,7 +368,7 @@ void binned_apply(nkpr_graph *g, const float *v, float *w, double damp, bool dis
 // Binned FP64 sweep: true when FP64 sweeps of this graph run binned (builds the copy on first
 // use); binned_sweep64 is one sweep with the epilogue, reductions and stop rule of
 // launch_sweep<double>.
-bool binned64_active(nkpr_graph *g);
+bool binned64_active(nkpr_graph *g, bool one_sweep);
 // slot -> compact id of the graph (z entries, -1 for slots without a node), built on first use
 const int32_t *slot_index(nkpr_graph *g);
 void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArgs &f, int kind,
@@ -457,6 +458,7 @@ struct nkpr_graph {
     uint64_t z = 0, m = 0;
     uint32_t n = 0, sink_begin = 0;
     uint64_t max_in_degree = 0;
+    uint64_t hub_edges = 0;  // edges from the kHubSources sources with the most out-edges
     bool weighted = false;
     double prep_ms = 0.0;
 

@@ -114,7 +114,7 @@ uint64_t run_phase(RunCtx &rc, SweepArgs<T> a, Vecs<T> v, int kind, PhaseRule ru
 
     // FP64 sweeps of large graphs run through the binned copy (per-graph hooks of a batch
     // handle run after either sweep)
-    const bool binned64 = dbl && binned64_active(g);
+    const bool binned64 = dbl && binned64_active(g, max_launch == 1);
     uint64_t launched = 0, done_sweeps = 0;
     uint64_t batch = (max_launch <= 2) ? max_launch : 4;
     const size_t need_ev = 2 * 64;
