@@ -7,8 +7,8 @@
 //            queued when its residual crosses eps vol(v); p[u] += alpha res;
 //            r[u] = (1 - alpha) res / 2, queued again when r[u] / vol >= eps.
 // Here all queued nodes push at once, round after round (a frontier):
-//   a first kernel takes every frontier node's residual (so that mass arriving during the
-//   round stays for the next one, whatever the schedule), adds alpha res to p and keeps
+//   first every frontier node's residual is taken (so that mass arriving during the
+//   round stays for the next one, whatever the schedule), adding alpha res to p and keeping
 //   (1 - alpha) res / 2; then a lane group per node sends the masses with atomic adds; a node whose
 //   residual crosses its threshold through an add is appended to the next frontier once (a
 //   flag bit per node).
@@ -61,12 +61,10 @@ namespace nkpr {
 namespace {
 
 constexpr uint32_t kTouched = 1, kQueued = 2;
-constexpr int kPushThreads = 256;
-constexpr uint32_t kPushLanes = 32;  // lanes of the push kernel that serve one frontier node
-// rounds per host read of the counters: rounds after the frontier empties return at once, so a
-// longer batch trades a few no-op launches for fewer host reads (RHG n = 10M, 128 rounds:
-// 8.91 ms per run with 8, 8.67 ms with 16, 8.51 ms with 32)
-constexpr int kBatch = 32;
+constexpr int kPushThreads = 1024;
+constexpr uint32_t kPushLanes = 32;  // lanes that push one frontier node
+// rounds per launch of the rounds kernel, after which the host looks whether the frontier is empty
+constexpr uint32_t kMaxRounds = 4096;
 constexpr double kUnit = 4611686018427387904.0;  // 2^62 fixed-point units per unit of mass
 
 // ceil(eps vol 2^62): r < thr  <=>  r 2^-62 < eps vol (the product rounded as the reference's).
@@ -126,22 +124,65 @@ __global__ void apr_reset_kernel(const uint32_t *ids, const uint32_t *count, dou
     }
 }
 
-// Counters (cnt, a 64-byte device buffer of uint32).  Round k pushes frontier k & 1 (size
-// cnt[k % 3]) and appends to the other frontier array (size cnt[(k + 1) % 3]); its take kernel
-// clears cnt[(k + 2) % 3], the size round k - 1 pushed, for round k + 1's appends.  The heavy
-// chunk lists alternate the same way (sizes cnt[kCntChunks + (k & 1)]).  [4..5] the out-edges
-// of the pushed nodes, [6..7] the pushes, [8] the rounds with a non-empty frontier.
-constexpr int kCntEdges = 4, kCntPushes = 6, kCntRounds = 8, kCntChunks = 10;
+// Counters (cnt, a device buffer of uint32).  Round k pushes frontier k & 1 (size cnt[k % 3]) and
+// appends to the other frontier array (size cnt[(k + 1) % 3]); its take clears cnt[(k + 2) % 3],
+// the size round k - 1 pushed, for round k + 1's appends.  The heavy chunk lists alternate the
+// same way (sizes cnt[kCntChunks + (k & 1)]).  [4..5] the out-edges of the pushed nodes, [6..7]
+// the pushes, [8] the rounds with a non-empty frontier, [12] set when a wait of the grid barrier
+// took too long; from kCntBarrier on the barrier's arrivals, a line per counter.
+constexpr int kCntEdges = 4, kCntPushes = 6, kCntRounds = 8, kCntChunks = 10, kCntAbort = 12;
+constexpr int kCntBarrier = 32, kBarGroups = 16, kBarStride = 32;
+constexpr int kCntWords = kCntBarrier + (kBarGroups + 1) * kBarStride;
 // A node with more out-edges than kPushChunk is pushed by several lane groups, kPushChunk edges each.
 constexpr uint32_t kPushChunk = 64;
 
-// What the push of a frontier node needs, gathered by the take kernel: the push then starts its
+// What the push of a frontier node needs, gathered by the take: the push then starts its
 // edge loads after one read instead of three dependent ones.
 struct Push {
-    uint64_t first;  // its out-edges [first, first + count)
-    uint32_t count, node;
-    double share;    // (1 - alpha) res / (2 vol): the mass per unit of weight
+    uint64_t first;       // its out-edges [first, first + count)
+    uint64_t count_node;  // count << 32 | node
+    double share;         // (1 - alpha) res / (2 vol): the mass per unit of weight
 };
+
+// Accesses to what other blocks of the launch write: coherent between the XCDs' L2 caches.
+template <typename T> __device__ __forceinline__ T ld_agent(const T *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+template <typename T> __device__ __forceinline__ void st_agent(T *p, T v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Every block arrives before any goes on; `turn` counts the barriers since the counters were
+// cleared.  Every thread waits for its own stores first.  Blocks count in kBarGroups groups, whose
+// last ones count at the top: 256 adds to one address would queue for longer than the rounds' own
+// work.  The grid has a block per CU, all of which are resident once the kernels ahead of them
+// have ended; should one still be missing after `ticks` (of 10 ns), the wait ends, every block leaves
+// (false) and the run is done again by one block, which waits for nobody.
+__device__ __forceinline__ bool grid_barrier(uint32_t *cnt, uint32_t turn, uint64_t ticks, uint32_t *ok) {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        uint32_t *bar = cnt + kCntBarrier;
+        const uint32_t grp = blockIdx.x % kBarGroups;
+        const uint32_t members = (gridDim.x - grp + kBarGroups - 1) / kBarGroups;
+        const uint32_t all = min(gridDim.x, (uint32_t)kBarGroups) * (turn + 1);
+        if (atomicAdd(bar + kBarStride * (1 + grp), 1u) + 1 == members * (turn + 1)) atomicAdd(bar, 1u);
+        const uint64_t t0 = wall_clock64();
+        uint32_t fine = 1;
+        for (uint32_t i = 1; (int32_t)(ld_agent(bar) - all) < 0; ++i) {
+            if ((i % 64 == 0 || ticks == 0) && (ld_agent(cnt + kCntAbort) || wall_clock64() - t0 > ticks)) {
+                st_agent(cnt + kCntAbort, 1u);
+                fine = 0;
+                break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+        }
+        *ok = fine;
+    }
+    __syncthreads();
+    return *ok != 0;
+}
 
 // the seeds: residual 1/|seeds|, touched, queued, in frontier 0 (ids ascending)
 __global__ void apr_seed_kernel(const uint32_t *seeds, uint32_t k, uint64_t *r, uint32_t *flags,
@@ -152,146 +193,145 @@ __global__ void apr_seed_kernel(const uint32_t *seeds, uint32_t k, uint64_t *r, 
         flags[s] = kTouched | kQueued;
         front[i] = s;
     }
-    if (blockIdx.x == 0 && threadIdx.x < 16) cnt[threadIdx.x] = threadIdx.x == 0 ? k : 0u;
+    if (blockIdx.x == 0)
+        for (int i = threadIdx.x; i < kCntWords; i += blockDim.x) cnt[i] = i == 0 ? k : 0u;
 }
 
-// Appends the nodes of the lanes with `append` set at next[*ncnt ...], one counter update per
-// wave (every lane of the wave calls it).
-__device__ __forceinline__ void append_wave(bool append, uint32_t v, uint32_t *next,
-                                            uint32_t *ncnt) {
-    const uint64_t ball = __ballot(append);
-    if (!ball) return;
-    const int lane = threadIdx.x & 63;
-    uint32_t base = 0;
-    if (lane == 0) base = atomicAdd(ncnt, (uint32_t)__popcll(ball));
-    base = __shfl(base, 0, 64);
-    if (append) next[base + (uint32_t)__popcll(ball & ((1ull << lane) - 1))] = v;
-}
-
-// Round k, first kernel: a thread per frontier node u takes its residual res, adds alpha res to p[u]
-// and leaves (1 - alpha) res / 2 in r[u], appending u to the next frontier when that alone reaches
-// its threshold; a node with more than kPushChunk out-edges lists its chunks for the push kernel,
-// which then only adds to residuals.
-__global__ void apr_take_kernel(const uint64_t *ptr, const double *vol, double alpha, double eps,
-                                const uint32_t *front, uint32_t *next, uint32_t *cnt, int k3,
-                                int k2, double *p, uint64_t *r, uint32_t *flags, Push *push,
-                                uint2 *chunks) {
-    __shared__ unsigned long long bedges;
-    const uint32_t nf = cnt[k3];
-    if (threadIdx.x == 0) bedges = 0;
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        cnt[(k3 + 2) % 3] = 0u;
-        cnt[kCntChunks + (k2 ^ 1)] = 0u;
-        if (nf) {
-            *reinterpret_cast<unsigned long long *>(cnt + kCntPushes) += nf;
-            cnt[kCntRounds] += 1u;
-        }
-    }
-    __syncthreads();
-    uint32_t *ncnt = cnt + (k3 + 1) % 3;
-    uint32_t *hcnt = cnt + kCntChunks + k2;
-    const uint32_t stride = gridDim.x * blockDim.x;
-    // whole waves step together (append_wave is a wave operation)
-    for (uint32_t i0 = blockIdx.x * blockDim.x; i0 < nf; i0 += stride) {
-        const uint32_t i = i0 + threadIdx.x;
-        bool again = false;
-        uint32_t u = 0;
-        if (i < nf) {
-            u = front[i];
-            const uint64_t res = r[u], b = ptr[u], deg = ptr[u + 1] - b;
-            const double vu = vol[u], pu = p[u];
-            const double dres = (double)res;
-            p[u] = pu + alpha * dres / kUnit;
-            const uint64_t keep = __double2ull_rn((1.0 - alpha) * dres / 2);
-            r[u] = keep;
-            again = keep >= threshold_of(eps, vu, true);
-            flags[u] = again ? (kTouched | kQueued) : kTouched;
-            Push o;
-            o.first = b;
-            o.count = (uint32_t)deg;
-            o.node = u;
-            o.share = vu > 0.0 ? (1.0 - alpha) * dres / (2.0 * vu) : 0.0;
-            push[i] = o;
-            atomicAdd(&bedges, (unsigned long long)deg);
-            if (deg > kPushChunk) {
-                const uint32_t nc = (uint32_t)((deg + kPushChunk - 1) / kPushChunk);
-                const uint32_t at = atomicAdd(hcnt, nc);
-                for (uint32_t c = 0; c < nc; ++c) chunks[at + c] = make_uint2(i, c);
-            }
-        }
-        append_wave(again, u, next, ncnt);
-    }
-    __syncthreads();
-    if (threadIdx.x == 0 && bedges)
-        atomicAdd(reinterpret_cast<unsigned long long *>(cnt + kCntEdges), bedges);
-}
-
-// Round k, second kernel: a lane group per frontier node with at most kPushChunk out-edges and one
-// per chunk of the others sends the masses (1 - alpha) res w / (2 vol).  At the start of the
-// kernel every residual lies below its threshold unless its node is already queued, and all
-// adds are positive, so the add that crosses a threshold is the one that finds the residual
-// below it and leaves it at or above it; that add sets the node's queued bit.
+// Rounds first .. first + kMaxRounds - 1, or until a frontier is empty.  A round has two parts with
+// a grid barrier after each.
 //
-// Bound by latency: a round is a few thousand edges.  The returning add is issued before the
-// threshold is formed, so that it and the load of vol[v] are in flight together; only an add that
-// finds no residual marks the node touched (one that holds some was marked by an earlier add);
-// a block collects what it appends in LDS and takes its places in the next frontier with one
-// add, where a wave each queued on that counter.  13.0 us per round before, 8.0 now (hyperbolic
-// graph of 2e6 nodes, eps 1e-8).
-__global__ __launch_bounds__(kPushThreads) void apr_push_kernel(
-    const int32_t *dst, const double *w, const double *vol, double eps, uint64_t *r, uint32_t *flags,
-    const Push *push, const uint2 *chunks, uint32_t *next, uint32_t *cnt, int k3, int k2) {
+// Take: a thread per frontier node u takes its residual res, adds alpha res to p[u] and leaves
+// (1 - alpha) res / 2 in r[u], queueing u again when that alone reaches its threshold; a node with
+// more than kPushChunk out-edges lists its chunks.
+//
+// Push: a lane group per frontier node with at most kPushChunk out-edges and one per chunk of the
+// others sends the masses (1 - alpha) res w / (2 vol).  At the start of the push every residual
+// lies below its threshold unless its node is already queued, and all adds are positive, so the
+// add that crosses a threshold is the one that finds the residual below it and leaves it at or
+// above it; that add sets the node's queued bit.  Only an add that finds no residual marks the
+// node touched (one that holds some was marked by an earlier add).
+//
+// Bound by latency: a round is a few thousand edges, some ten dependent accesses of about 1 us
+// each.  Two launches a round put some 7 us between every two kernels beside that; the rounds
+// therefore share one launch, a block per CU.  The returning add is issued
+// before the threshold is formed, so that it and the load of vol[v] are in flight together; a
+// block collects what it queues in LDS and takes its places in the next frontier with one add.
+// Hyperbolic graph of 2e6 nodes, eps 1e-8, three seeds: 3.76, 2.96 and 2.73 ms a run with two launches a
+// round, 3.24, 2.46 and 2.49 now; 64 seeds on 6e6 nodes, eps 1e-9: 18.6 and 16.3 ms (1.1e10 adds
+// a second, what the atomics give).
+__global__ __launch_bounds__(kPushThreads) void apr_rounds_kernel(
+    const uint64_t *ptr, const int32_t *dst, const double *w, const double *vol, double alpha, double eps,
+    uint32_t *f0, uint32_t *f1, uint32_t *cnt, uint32_t first, double *p, uint64_t *r, uint32_t *flags, Push *push,
+    uint64_t *chunks, uint64_t chunk_cap, uint64_t ticks) {
     constexpr uint32_t kGroups = kPushThreads / kPushLanes;
-    __shared__ uint32_t list[kGroups * kPushChunk];
-    __shared__ uint32_t n_list, base;
-    const uint32_t nf = cnt[k3], nh = cnt[kCntChunks + k2];
-    uint32_t *ncnt = cnt + (k3 + 1) % 3;
+    __shared__ uint32_t list[kPushThreads + kGroups * kPushChunk];
+    __shared__ uint32_t n_list, base, ok;
+    __shared__ unsigned long long edges;
+    if (ld_agent(cnt + kCntAbort)) return;  // (before the first barrier: set only if this block came too late)
     const uint32_t lane = threadIdx.x % kPushLanes;
-    if (threadIdx.x == 0) n_list = 0;
+    // consecutive entries go to different blocks, so that a small frontier uses every CU
+    const uint32_t group = threadIdx.x / kPushLanes * gridDim.x + blockIdx.x, ngroups = gridDim.x * kGroups;
+    const uint32_t thread = threadIdx.x * gridDim.x + blockIdx.x, nthreads = gridDim.x * kPushThreads;
+    if (threadIdx.x == 0) edges = 0, n_list = 0;
     __syncthreads();
-    for (uint32_t t0 = blockIdx.x * kGroups; t0 < nf + nh; t0 += gridDim.x * kGroups) {
-        const uint32_t t = t0 + threadIdx.x / kPushLanes;
-        uint64_t b = 0, end = 0;
-        uint32_t u = 0;
-        double share = 0.0;
-        if (t < nf) {
-            const Push o = push[t];
-            u = o.node;
-            share = o.share;
-            b = o.first;
-            end = o.count > kPushChunk ? b : b + o.count;  // the others are pushed by their chunks
-        } else if (t < nf + nh) {
-            const uint2 c = chunks[t - nf];
-            const Push o = push[c.x];
-            u = o.node;
-            share = o.share;
-            b = o.first + (uint64_t)c.y * kPushChunk;
-            end = std::min<uint64_t>(o.first + o.count, b + kPushChunk);
-        }
-        for (uint64_t e = b + lane; e < end; e += kPushLanes) {
-            const uint32_t v = (uint32_t)dst[e];
-            // a self-loop sends nothing: the reference overwrites r[u] after its loop
-            if (v == u) continue;
-            const uint64_t mass = __double2ull_rn(share * (w ? w[e] : 1.0));
-            const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long *>(&r[v]),
-                                           (unsigned long long)mass);
-            const uint64_t thr = threshold_of(eps, vol[v], false);
-            if (old < thr && old + mass >= thr) {
-                if (!(atomicOr(&flags[v], kQueued | kTouched) & kQueued)) list[atomicAdd(&n_list, 1u)] = v;
-            } else if (old == 0) {
-                atomicOr(&flags[v], kTouched);
-            }
-        }
+    // the block's list into the next frontier (every thread calls it)
+    auto flush = [&](uint32_t *next, uint32_t *ncnt) {
         __syncthreads();
         const uint32_t k = n_list;
         if (k) {
             if (threadIdx.x == 0) base = atomicAdd(ncnt, k);
             __syncthreads();
-            for (uint32_t i = threadIdx.x; i < k; i += kPushThreads) next[base + i] = list[i];
+            for (uint32_t i = threadIdx.x; i < k; i += kPushThreads) st_agent(next + base + i, list[i]);
             if (threadIdx.x == 0) n_list = 0;
         }
         __syncthreads();
+    };
+    for (uint32_t round = first; round - first < kMaxRounds; ++round) {
+        const uint32_t k2 = round & 1, k3 = round % 3;
+        const uint32_t *front = k2 ? f1 : f0;
+        uint32_t *next = k2 ? f0 : f1, *ncnt = cnt + (k3 + 1) % 3, *hcnt = cnt + kCntChunks + k2;
+        uint64_t *chunk = chunks + (k2 ? chunk_cap : 0);
+        const uint32_t nf = ld_agent(cnt + k3);
+        if (nf == 0) break;
+        if (blockIdx.x == 0 && threadIdx.x == 0) {
+            st_agent(cnt + (k3 + 2) % 3, 0u);
+            st_agent(cnt + kCntChunks + (k2 ^ 1), 0u);
+            *reinterpret_cast<unsigned long long *>(cnt + kCntPushes) += nf;
+            cnt[kCntRounds] += 1u;
+        }
+        for (uint32_t i0 = 0; i0 < nf; i0 += nthreads) {
+            const uint32_t i = i0 + thread;
+            if (i < nf) {
+                const uint32_t u = ld_agent(front + i);
+                const uint64_t res = ld_agent(r + u), b = ptr[u], deg = ptr[u + 1] - b;
+                const double vu = vol[u], pu = ld_agent(p + u);
+                const double dres = (double)res;
+                const uint64_t keep = __double2ull_rn((1.0 - alpha) * dres / 2);
+                const bool again = keep >= threshold_of(eps, vu, true);
+                st_agent(p + u, pu + alpha * dres / kUnit);
+                st_agent(r + u, keep);
+                st_agent(flags + u, again ? (kTouched | kQueued) : kTouched);
+                Push *o = push + i;
+                st_agent(&o->first, b);
+                st_agent(&o->count_node, deg << 32 | u);
+                st_agent(&o->share, vu > 0.0 ? (1.0 - alpha) * dres / (2.0 * vu) : 0.0);
+                atomicAdd(&edges, (unsigned long long)deg);
+                if (deg > kPushChunk) {
+                    const uint32_t nc = (uint32_t)((deg + kPushChunk - 1) / kPushChunk);
+                    const uint32_t at = atomicAdd(hcnt, nc);
+                    for (uint32_t c = 0; c < nc; ++c) st_agent(chunk + at + c, (uint64_t)c << 32 | i);
+                }
+                if (again) list[atomicAdd(&n_list, 1u)] = u;
+            }
+            // (the last turn's nodes wait for those of the push)
+            if (nf - i0 > nthreads) flush(next, ncnt);
+        }
+        if (!grid_barrier(cnt, 2 * round, ticks, &ok)) break;
+        // the first turn's items are on their way beside the number of chunks
+        const uint32_t nh = ld_agent(hcnt);
+        uint64_t from = 0, cn = 0;
+        double share = 0.0;
+        auto load = [&](uint32_t i) {
+            from = ld_agent(&push[i].first);
+            cn = ld_agent(&push[i].count_node);
+            share = ld_agent(&push[i].share);
+        };
+        if (group < nf) load(group);
+        for (uint32_t t0 = 0; t0 < nf + nh; t0 += ngroups) {
+            const uint32_t t = t0 + group;
+            uint64_t b = 0, end = 0;
+            if (t < nf) {
+                if (t0) load(t);
+                b = from;
+                end = cn >> 32 > kPushChunk ? b : b + (cn >> 32);  // the others are pushed by their chunks
+            } else if (t < nf + nh) {
+                const uint64_t c = ld_agent(chunk + (t - nf));
+                load((uint32_t)c);
+                b = from + (c >> 32) * kPushChunk;
+                end = std::min<uint64_t>(from + (cn >> 32), b + kPushChunk);
+            }
+            const uint32_t u = (uint32_t)cn;
+            for (uint64_t e = b + lane; e < end; e += kPushLanes) {
+                const uint32_t v = (uint32_t)dst[e];
+                // a self-loop sends nothing: the reference overwrites r[u] after its loop
+                if (v == u) continue;
+                const uint64_t mass = __double2ull_rn(share * (w ? w[e] : 1.0));
+                const uint64_t old = atomicAdd(reinterpret_cast<unsigned long long *>(&r[v]),
+                                               (unsigned long long)mass);
+                const uint64_t thr = threshold_of(eps, vol[v], false);
+                if (old < thr && old + mass >= thr) {
+                    if (!(atomicOr(&flags[v], kQueued | kTouched) & kQueued)) list[atomicAdd(&n_list, 1u)] = v;
+                } else if (old == 0) {
+                    atomicOr(&flags[v], kTouched);
+                }
+            }
+            flush(next, ncnt);
+        }
+        if (!grid_barrier(cnt, 2 * round + 1, ticks, &ok)) break;
     }
+    __syncthreads();
+    if (threadIdx.x == 0 && edges)
+        atomicAdd(reinterpret_cast<unsigned long long *>(cnt + kCntEdges), edges);
 }
 
 // touched nodes in ascending id order: per-block counts, then a one-block scan, then writes
@@ -405,7 +445,7 @@ void apr_create_impl(uint64_t z, const uint64_t *ptr, const int32_t *dst, const 
     // chunks of the nodes with more than kPushChunk out-edges: at most 2 deg / kPushChunk per node
     a->chunk_cap = 2 * m / kPushChunk + 64;
     a->chunks.alloc(2 * 8 * a->chunk_cap);
-    a->cnt.alloc(64);
+    a->cnt.alloc(4 * kCntWords);
     a->out_cnt.alloc(4 * 1025);
     a->out_ids.alloc(4 * z);
     a->out_p.alloc(8 * z);
@@ -453,44 +493,45 @@ void apr_run_impl(nkpr_apr *a, double alpha, double eps, const uint64_t *seeds, 
     const uint64_t z = a->z;
     a->seeds.alloc(4 * sd.size());
     NKPR_HIP(hipMemcpyAsync(a->seeds.p, sd.data(), 4 * sd.size(), hipMemcpyHostToDevice, s));
-    if (a->dirty) {
-        const unsigned gz = (unsigned)std::min<uint64_t>((z + 255) / 256, 65536);
-        hipLaunchKernelGGL(apr_clear_kernel, dim3(gz), dim3(256), 0, s, a->p.as<double>(),
-                           a->r.as<uint64_t>(), a->flags.as<uint32_t>(), z);
-    }
-    a->dirty = true;
-    hipLaunchKernelGGL(apr_seed_kernel, dim3(1), dim3(256), 0, s, a->seeds.as<uint32_t>(),
-                       (uint32_t)sd.size(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(),
-                       a->f0.as<uint32_t>(), a->cnt.as<uint32_t>());
-    NKPR_HIP(hipGetLastError());
-    // Rounds run in batches without a host read; a round whose frontier is empty returns at
-    // once, and the host reads the counters after each batch.
-    uint32_t *front[2] = {a->f0.as<uint32_t>(), a->f1.as<uint32_t>()};
+    // The rounds of a launch end by themselves when a frontier is empty.  Its blocks wait for each
+    // other, one per CU; when one of them cannot start for kMissing (other work holds its CU), the
+    // run starts again on one block.
+    constexpr uint64_t kMissing = 200000000;  // 2 s
+    uint64_t ticks = kMissing;
+    // test hook: 0 ends a wait that is not over at once
+    if (const char *e = std::getenv("NKPR_TEST_APR_WAIT"); e && *e) ticks = std::strtoull(e, nullptr, 10);
     int cus = 0;
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, a->device));
-    const unsigned grid = (unsigned)std::max(cus, 1) * 8, tgrid = 128;
-    uint32_t host_cnt[16] = {0};
-    uint64_t k_round = 0;
-    // rounds per host read of the counters (NKPR_APR_BATCH overrides)
-    int batch = kBatch;
-    if (const char *e = std::getenv("NKPR_APR_BATCH")) batch = std::max(1, std::min(256, std::atoi(e)));
-    for (;;) {
-        for (int b = 0; b < batch; ++b, ++k_round) {
-            const int k2 = (int)(k_round & 1), k3 = (int)(k_round % 3);
-            hipLaunchKernelGGL(apr_take_kernel, dim3(tgrid), dim3(256), 0, s,
-                               a->ptr.as<uint64_t>(), a->vol.as<double>(), alpha, eps,
-                               front[k2], front[k2 ^ 1], a->cnt.as<uint32_t>(), k3, k2,
-                               a->p.as<double>(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(),
-                               a->push.as<Push>(), a->chunks.as<uint2>() + (k2 ? a->chunk_cap : 0));
-            hipLaunchKernelGGL(apr_push_kernel, dim3(grid), dim3(kPushThreads), 0, s,
-                               a->dst.as<int32_t>(), a->w.as<double>(), a->vol.as<double>(), eps,
-                               a->r.as<uint64_t>(), a->flags.as<uint32_t>(), a->push.as<Push>(),
-                               a->chunks.as<uint2>() + (k2 ? a->chunk_cap : 0), front[k2 ^ 1],
-                               a->cnt.as<uint32_t>(), k3, k2);
+    unsigned grid = (unsigned)std::max(cus, 1);
+    uint32_t host_cnt[16] = {0}, round = 0;
+    auto start = [&] {
+        if (a->dirty) {
+            const unsigned gz = (unsigned)std::min<uint64_t>((z + 255) / 256, 65536);
+            hipLaunchKernelGGL(apr_clear_kernel, dim3(gz), dim3(256), 0, s, a->p.as<double>(),
+                               a->r.as<uint64_t>(), a->flags.as<uint32_t>(), z);
         }
+        a->dirty = true;
+        hipLaunchKernelGGL(apr_seed_kernel, dim3(1), dim3(256), 0, s, a->seeds.as<uint32_t>(),
+                           (uint32_t)sd.size(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(),
+                           a->f0.as<uint32_t>(), a->cnt.as<uint32_t>());
+        round = 0;
+    };
+    start();
+    for (;;) {
+        hipLaunchKernelGGL(apr_rounds_kernel, dim3(grid), dim3(kPushThreads), 0, s, a->ptr.as<uint64_t>(),
+                           a->dst.as<int32_t>(), a->w.as<double>(), a->vol.as<double>(), alpha, eps,
+                           a->f0.as<uint32_t>(), a->f1.as<uint32_t>(), a->cnt.as<uint32_t>(), round,
+                           a->p.as<double>(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(), a->push.as<Push>(),
+                           a->chunks.as<uint64_t>(), a->chunk_cap, ticks);
         NKPR_HIP(hipGetLastError());
         read_back(s, {{host_cnt, a->cnt.p, sizeof(host_cnt)}});
-        if (host_cnt[k_round % 3] == 0) break;  // the frontier of the next round is empty
+        if (host_cnt[kCntAbort]) {
+            grid = 1;
+            start();
+            continue;
+        }
+        round = host_cnt[kCntRounds];
+        if (host_cnt[round % 3] == 0) break;  // the frontier of the next round is empty
     }
     uint64_t rounds = host_cnt[kCntRounds], pushes = 0;
     std::memcpy(&pushes, host_cnt + kCntPushes, 8);
