@@ -293,8 +293,8 @@ int nkpr_csr_spmv(const nkpr_csr *a, const double *x, double *y, void *stream);
 /* One iteration of AlgebraicPageRank::run (AlgebraicPageRank.hpp:97-101) on a square matrix
  * M: y = M x + shift and *step_sq = ||y - x||_2^2 (FP64, a device pointer; summed in an order
  * fixed by the matrix).  Stream-ordered like nkpr_csr_spmv.  Like nkpr_csr_spmv it takes its
- * scratch (the list of rows longer than 32 x the lanes per row, their pieces of 4096 entries,
- * block sums: about 8 bytes per 4096 entries) from the stream's memory pool for the call. */
+ * scratch (a carry per 4096 rows and entries, block sums: about 12 bytes per 4096 of them; per
+ * 1024 below 2^22) from the stream's memory pool for the call. */
 int nkpr_csr_pagerank_step(const nkpr_csr *m, double shift, const double *x, double *y,
                            double *step_sq, void *stream);
 
