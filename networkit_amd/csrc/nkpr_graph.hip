@@ -603,6 +603,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     NKPR_CHECK(m == 0 || c->src != nullptr, "src is NULL");
     g->m = m;
     g->weighted = c->weight != nullptr;
+    g->own_degrees = c->out_wdeg == nullptr;
 
     DevBuf colptr_in_b, src_in_b, w_in_b, exists_b, wdeg_b;
     const uint64_t *colptr_in = c->colptr;
@@ -933,6 +934,7 @@ void set_weights(nkpr_graph *g, const float *w, const double *w64, const double 
     const hipStream_t s = g->stream;
     const uint64_t m = g->m, z = g->z;
     const uint32_t n = g->n;
+    g->own_degrees = out_wdeg == nullptr;
     DevBuf wb, w64b, degz, deg;
     if (!device_ptrs) {
         if (w) {

@@ -460,6 +460,7 @@ struct nkpr_graph {
     uint64_t max_in_degree = 0;
     uint64_t hub_edges = 0;  // edges from the kHubSources sources with the most out-edges
     bool weighted = false;
+    bool own_degrees = false;  // weighted out-degrees summed from the weights, not given
     double prep_ms = 0.0;
 
     nkpr::DevBuf perm;      // int32 [n]   compact id -> slot
