@@ -238,6 +238,14 @@ __global__ void segment_starts_kernel(const uint64_t *keys, uint64_t m, int vbit
     }
 }
 
+// kCap entries of padding after the last edge
+__global__ void pad_kernel(int32_t *src, float *c32, double *c64) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    src[i] = 0;
+    if (c32) c32[i] = 0.0f;
+    if (c64) c64[i] = 0.0;
+}
+
 __global__ void edge_output_kernel(const uint64_t *keys, const uint32_t *vals, uint64_t m, uint64_t vmask,
                                    const float *w_in, const double *w64_in, const int32_t *src_in,
                                    const double *wdeg, int32_t *src_out, float *coef32,
@@ -316,34 +324,46 @@ __global__ void heavy_rows_kernel(const uint32_t *ptr, uint64_t count, uint32_t 
 // Greedy work items over the rows of `lists` lists of nrows rows each (list q's in-edge offsets start
 // at ptr[q nrows]): runs of consecutive rows with at most `cap` in-edges and kRowsMax rows (a row with
 // more has an item of its own); rows longer than kCap are left out (see build_heavy).  A wave takes
-// kSegRows rows of a list and tries a step's kRowsMax ends at once.  Without `items` it only counts.
-constexpr uint32_t kSegRows = 8192;
+// seg_rows rows of a list, 64 row ends at a time in its lanes, the next 64 on their way: cuts cost no
+// memory access (a load per cut took 1.1 us, 0.29 ms for 256 rows that each fill an item).  Without
+// `items` it only counts.
 __global__ __launch_bounds__(256) void build_items_kernel(const uint32_t *ptr, uint32_t nrows, uint32_t lists,
-                                                          uint32_t segs, uint32_t cap, uint32_t *counts,
-                                                          const uint32_t *first, uint4 *items) {
+                                                          uint32_t segs, uint32_t seg_rows, uint32_t cap,
+                                                          uint32_t *counts, const uint32_t *first, uint4 *items) {
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t seg = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (seg >= lists * segs) return;
     const uint32_t *P = ptr + (uint64_t)(seg / segs) * nrows;
-    const uint32_t begin = (seg % segs) * kSegRows, end = min(nrows, begin + kSegRows);
-    uint32_t made = 0, r = begin;
-    while (r < end) {
-        const uint32_t p0 = P[r], most = min(end - r, (uint32_t)kRowsMax);
-        uint32_t fit = 0;
-        for (uint32_t c = 0; c < (uint32_t)kRowsMax; c += 64) {
-            const uint32_t k = c + lane + 1;
-            fit += (uint32_t)__popcll(__ballot(k <= most && P[r + min(k, most)] - p0 <= cap));
-        }
-        if (fit == 0) {
-            fit = 1;
-            if (P[r + 1] - p0 > (uint32_t)kCap) {
+    const uint32_t begin = (seg % segs) * seg_rows, end = min(nrows, begin + seg_rows);
+    const uint32_t at = items ? first[seg] : 0;
+    uint32_t made = 0;
+    auto put = [&](uint32_t r0, uint32_t r1, uint32_t p0, uint32_t p1) {
+        if (items && lane == 0) items[at + made] = make_uint4(r0, r1, p0, p1 - p0);
+        ++made;
+    };
+    // the item that grows: rows [r, ..) from edge p0 on; pw the first edge of the window
+    uint32_t r = begin, p0 = P[begin], pw = p0, ahead = P[min(begin + lane + 1, end)];
+    for (uint32_t w = begin; w < end; w += 64) {
+        const uint32_t e = ahead, wend = min(w + 64, end);
+        ahead = P[min(w + 64 + lane + 1, end)];
+        while (r < wend) {
+            const uint32_t j = w + lane, from = max(r, w);
+            const uint32_t next =
+                from + (uint32_t)__popcll(__ballot(j >= from && j < wend && e - p0 <= cap && j + 1 - r <= (uint32_t)kRowsMax));
+            if (next == wend && wend < end) break;  // may grow into the next window
+            if (next > r) {
+                const uint32_t p1 = next == w ? pw : __shfl(e, next - 1 - w, 64);
+                put(r, next, p0, p1);
+                r = next;
+                p0 = p1;
+            } else {
+                const uint32_t p1 = __shfl(e, r - w, 64);
+                if (p1 - p0 <= (uint32_t)kCap) put(r, r + 1, p0, p1);
                 ++r;
-                continue;
+                p0 = p1;
             }
         }
-        if (items && lane == 0) items[first[seg] + made] = make_uint4(r, r + fit, p0, P[r + fit] - p0);
-        ++made;
-        r += fit;
+        pw = __shfl(e, 63, 64);
     }
     if (!items && lane == 0) counts[seg] = made;
 }
@@ -393,8 +413,9 @@ uint32_t env_u32(const char *name, uint32_t dflt) {
 }
 
 // Splits the rows of g->colptr into direct and sliced ones, in the order in which a sweep takes
-// them; the in-edges are then sorted into that order.
-void schedule_rows(nkpr_graph *g) {
+// them; the in-edges are then sorted into that order.  sel: 32 cleared bytes for the counts of direct
+// and sliced rows and, 16 bytes on, the largest in-degree.  Reads hub_edges back along the way.
+void schedule_rows(nkpr_graph *g, uint32_t *sel, const unsigned long long *hub_edges) {
     const hipStream_t s = g->stream;
     const uint32_t n = g->n;
     // slicing pays off once the gathered vector outgrows one L2; below that everything is
@@ -418,10 +439,6 @@ void schedule_rows(nkpr_graph *g) {
     // direct and sliced rows, the direct rows' offsets and the largest in-degree, without a row's
     // length leaving the device (loops over the rows on the host and the copies they needed took
     // half of the 18 ms of a handle over 1e6 nodes)
-    DevBuf nsel;
-    nsel.alloc(32);
-    NKPR_HIP(hipMemsetAsync(nsel.p, 0, 32, s));
-    uint32_t *sel = nsel.as<uint32_t>();  // direct rows, sliced rows, -, -, largest degree
     {
         DevBuf rows, tmp, lens;
         rows.alloc(4 * std::max<size_t>(2 * (size_t)n, 1));
@@ -439,7 +456,9 @@ void schedule_rows(nkpr_graph *g) {
             NKPR_HIP(hipGetLastError());
         }
         uint32_t got[6] = {0};
-        read_back(s, {{got, sel, sizeof(got)}});
+        unsigned long long hub = 0;
+        read_back(s, {{got, sel, sizeof(got)}, {&hub, hub_edges, 8}});
+        g->hub_edges = hub;
         g->n_d = got[0];
         g->n_s = got[1];
         g->max_in_degree = (uint64_t)got[4] | ((uint64_t)got[5] << 32);
@@ -461,7 +480,6 @@ void schedule_rows(nkpr_graph *g) {
                                                   (size_t)g->n_d + 1, s));
     }
     NKPR_CHECK((uint64_t)S * g->n_s + 1 < 0xFFFFFFFFull, "too many sliced rows");
-    NKPR_HIP(hipStreamSynchronize(s));  // the temporaries go back
 }
 
 // The work items over the rows of schedule_rows, once g->src / g->coef* and g->sptr stand.
@@ -491,7 +509,11 @@ void schedule_items(nkpr_graph *g) {
     // nodes and 1.5e5 arcs ran on 40 blocks.  Such graphs take smaller items.
     uint32_t cap = kCap;
     while (S == 1 && cap > kCapMin && m < (uint64_t)cap * kItemsWanted) cap /= 2;
-    const uint32_t dsegs = (g->n_d + kSegRows - 1) / kSegRows, ssegs = (n_s + kSegRows - 1) / kSegRows;
+    // a segment of about 32 items
+    const uint64_t per_item = (uint64_t)cap * (g->n_d + ns_tot) / std::max<uint64_t>(m, 1);
+    uint32_t seg_rows = 1024;
+    while (seg_rows < 8192 && seg_rows < 32 * std::min<uint64_t>(per_item, kRowsMax)) seg_rows *= 2;
+    const uint32_t dsegs = (g->n_d + seg_rows - 1) / seg_rows, ssegs = (n_s + seg_rows - 1) / seg_rows;
     const uint32_t nseg = dsegs + S * ssegs;
     DevBuf cnt_b, first_b;
     cnt_b.alloc(4 * std::max<size_t>(nseg, 1));
@@ -500,10 +522,10 @@ void schedule_items(nkpr_graph *g) {
         uint32_t *cnt = cnt_b.as<uint32_t>();
         if (dsegs)
             hipLaunchKernelGGL(build_items_kernel, dim3((dsegs + 3) / 4), dim3(256), 0, s,
-                               (const uint32_t *)g->dptr.as<uint32_t>(), g->n_d, 1u, dsegs, cap, cnt, first, di);
+                               (const uint32_t *)g->dptr.as<uint32_t>(), g->n_d, 1u, dsegs, seg_rows, cap, cnt, first, di);
         if (ssegs)
             hipLaunchKernelGGL(build_items_kernel, dim3((S * ssegs + 3) / 4), dim3(256), 0, s,
-                               (const uint32_t *)g->sptr.as<uint32_t>(), n_s, S, ssegs, cap, cnt + dsegs,
+                               (const uint32_t *)g->sptr.as<uint32_t>(), n_s, S, ssegs, seg_rows, cap, cnt + dsegs,
                                first ? first + dsegs : nullptr, si);
         NKPR_HIP(hipGetLastError());
     };
@@ -632,49 +654,49 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         else std::memcpy(g->exists_host.data(), c->exists, z);
     }
 
-    DevBuf flags_b, outcnt_b, wdeg_own_b, counts_b;
-    flags_b.alloc(4);
-    NKPR_HIP(hipMemsetAsync(flags_b.p, 0, 4, s));
-    uint32_t *flags = flags_b.as<uint32_t>();
+    // everything that starts at zero, cleared at once: weighted out-degrees, out-degrees, then flags,
+    // counts (nodes, nodes with out-edges, hub edges), the schedule's counts and one more flag
+    const size_t own_bytes = c->out_wdeg ? 0 : 8 * (z + 1), cnt_bytes = (4 * (z + 1) + 7) / 8 * 8;
+    DevBuf zero_b;
+    zero_b.alloc(own_bytes + cnt_bytes + 128);
+    NKPR_HIP(hipMemsetAsync(zero_b.p, 0, own_bytes + cnt_bytes + 128, s));
+    uint32_t *outcnt = reinterpret_cast<uint32_t *>(zero_b.as<char>() + own_bytes);
+    char *tail = zero_b.as<char>() + own_bytes + cnt_bytes;
+    uint32_t *flags = reinterpret_cast<uint32_t *>(tail), *sel = reinterpret_cast<uint32_t *>(tail + 64);
+    uint32_t *inexact = reinterpret_cast<uint32_t *>(tail + 96);
+    auto *counts = reinterpret_cast<unsigned long long *>(tail + 8);
     if (z)
         hipLaunchKernelGGL(validate_ptr_kernel, dim3(blocks_for(z)), dim3(256), 0, s, colptr_in, z,
                            m, exists, flags);
-    outcnt_b.alloc(4 * (z + 1));
-    NKPR_HIP(hipMemsetAsync(outcnt_b.p, 0, 4 * (z + 1), s));
     const double *wdeg = nullptr;
     double *wdeg_own = nullptr;
     if (c->out_wdeg) {
         wdeg = dev ? c->out_wdeg : (const double *)h2d(wdeg_b, c->out_wdeg, 8 * z);
     } else {
-        wdeg_own_b.alloc(8 * (z + 1));
-        NKPR_HIP(hipMemsetAsync(wdeg_own_b.p, 0, 8 * (z + 1), s));
-        wdeg_own = wdeg_own_b.as<double>();
+        wdeg_own = zero_b.as<double>();
         wdeg = wdeg_own;
     }
     if (m) {
         hipLaunchKernelGGL(out_degree_kernel, dim3(agg_blocks(m)), dim3(kAggThreads), 0, s, src_in, m, z, exists, w_in,
-                           w64_in, outcnt_b.as<uint32_t>(), wdeg_own, flags);
+                           w64_in, outcnt, wdeg_own, flags);
     }
     if (c->out_wdeg && z)
         hipLaunchKernelGGL(unit_degree_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(z), 65536)),
                            dim3(256), 0, s, wdeg, z, exists, flags);
     NKPR_HIP(hipGetLastError());
+    if (z)
+        hipLaunchKernelGGL(count_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(z), 1024)), dim3(256), 0, s,
+                           outcnt, exists, z, counts, counts + 1);
+    NKPR_HIP(hipGetLastError());
     uint32_t hflags = 0;
-    read_back(s, {{&hflags, flags, 4}});
+    unsigned long long hc[2] = {0, 0};
+    read_back(s, {{&hflags, flags, 4}, {hc, counts, 16}});
     g->unit_degrees = c->out_wdeg != nullptr && !(hflags & kNotUnitDegree);
     NKPR_CHECK(!(hflags & kBadPtr), "colptr is not a non-decreasing offset array ending at m");
     NKPR_CHECK(!(hflags & kBadSrc), "an in-list names a source outside [0, z) or a deleted node");
     NKPR_CHECK(!(hflags & kBadExists), "a deleted slot has in-edges");
 
     // --- relabel: out-degree descending, deleted slots dropped ------------------------------
-    counts_b.alloc(16);
-    NKPR_HIP(hipMemsetAsync(counts_b.p, 0, 16, s));
-    auto *counts = counts_b.as<unsigned long long>();
-    if (z)
-        hipLaunchKernelGGL(count_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(z), 1024)), dim3(256), 0, s,
-                           outcnt_b.as<uint32_t>(), exists, z, counts, counts + 1);
-    unsigned long long hc[2] = {0, 0};
-    read_back(s, {{hc, counts, 16}});
     const uint32_t n = (uint32_t)hc[0];
     g->n = n;
     g->sink_begin = (uint32_t)hc[1];
@@ -706,7 +728,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
             hipLaunchKernelGGL(group_id_kernel, dim3(blocks_for(z)), dim3(256), 0, s,
                                offb.as<uint64_t>(), n_groups, z, gidb.as<uint32_t>());
             hipLaunchKernelGGL(group_keys_kernel, dim3(blocks_for(z)), dim3(256), 0, s,
-                               outcnt_b.as<uint32_t>(), exists, gidb.as<uint32_t>(), n_groups, z,
+                               outcnt, exists, gidb.as<uint32_t>(), n_groups, z,
                                k64a.as<uint64_t>(), v1.as<int32_t>(), ce.as<uint32_t>(), cn.as<uint32_t>());
             const unsigned eb = (unsigned)std::min<uint64_t>(blocks_for(z * 64), 1u << 18);
             hipLaunchKernelGGL(group_edges_kernel, dim3(eb), dim3(256), 0, s, colptr_in, src_in,
@@ -745,7 +767,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         v1.alloc(4 * z);
         v2.alloc(4 * z);
         hipLaunchKernelGGL(relabel_keys_kernel, dim3(blocks_for(z)), dim3(256), 0, s,
-                           outcnt_b.as<uint32_t>(), exists, z, k1.as<uint32_t>(), v1.as<int32_t>());
+                           outcnt, exists, z, k1.as<uint32_t>(), v1.as<int32_t>());
         hipcub::DoubleBuffer<uint32_t> kb(k1.as<uint32_t>(), k2.as<uint32_t>());
         hipcub::DoubleBuffer<int32_t> vb(v1.as<int32_t>(), v2.as<int32_t>());
         size_t tb = 0;
@@ -764,14 +786,10 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     if (n)
         hipLaunchKernelGGL(iperm_kernel, dim3(blocks_for(n)), dim3(256), 0, s, g->perm.as<int32_t>(),
                            n, iperm);
-    NKPR_HIP(hipMemsetAsync(counts, 0, 8, s));
     if (n)
         hipLaunchKernelGGL(hub_edges_kernel, dim3(1), dim3(1024), 0, s, g->perm.as<int32_t>(),
-                           std::min<uint32_t>(n, kHubSources), outcnt_b.as<uint32_t>(), counts);
+                           std::min<uint32_t>(n, kHubSources), outcnt, counts + 2);
     NKPR_HIP(hipGetLastError());
-    unsigned long long hub = 0;
-    read_back(s, {{&hub, counts, 8}});  // (the sort buffers are freed below)
-    g->hub_edges = hub;
     k1.reset(); k2.reset(); v1.reset(); v2.reset(); tmp.reset();
 
     // --- new colptr -------------------------------------------------------------------------
@@ -787,23 +805,22 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         tmp.alloc(tb);
         NKPR_HIP(hipcub::DeviceScan::ExclusiveSum(tmp.p, tb, len_b.as<uint64_t>(),
                                                   g->colptr.as<uint64_t>(), (size_t)n + 1, s));
-        NKPR_HIP(hipStreamSynchronize(s));
         tmp.reset();
     }
     len_b.reset();
 
     // --- edges: into the order of the sweep (kCap zero entries of padding after the last one) ---
-    schedule_rows(g);
+    schedule_rows(g, sel, counts + 2);
     const uint64_t ns_tot = (uint64_t)g->n_slices * g->n_s, nseg = g->n_d + ns_tot;
     g->sptr.alloc(4 * (ns_tot + 1));
     g->src.alloc(4 * (m + kCap));
-    NKPR_HIP(hipMemsetAsync(g->src.as<int32_t>() + m, 0, 4 * kCap, s));
     if (g->weighted) {
         g->coef32.alloc(4 * (m + kCap));
         g->coef64.alloc(8 * (m + kCap));
-        NKPR_HIP(hipMemsetAsync(g->coef32.as<float>() + m, 0, 4 * kCap, s));
-        NKPR_HIP(hipMemsetAsync(g->coef64.as<double>() + m, 0, 8 * kCap, s));
     }
+    hipLaunchKernelGGL(pad_kernel, dim3(kCap / 256), dim3(256), 0, s, g->src.as<int32_t>() + m,
+                       g->weighted ? g->coef32.as<float>() + m : nullptr,
+                       g->weighted ? g->coef64.as<double>() + m : nullptr);
     if (m) {
         DevBuf ka, kb2, va, vb2, place;
         ka.alloc(8 * m);
@@ -847,8 +864,6 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
             std::swap(g->emap.p, sorted.p);
             std::swap(g->emap.bytes, sorted.bytes);
         }
-        NKPR_HIP(hipStreamSynchronize(s));
-        tmp.reset();
     } else {
         NKPR_HIP(hipMemsetAsync(g->sptr.p, 0, 4 * (ns_tot + 1), s));
     }
@@ -857,7 +872,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         g->inv64.alloc(8 * std::max<uint64_t>(n, 1));
         if (n)
             hipLaunchKernelGGL(inv_degree_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
-                               g->perm.as<int32_t>(), n, outcnt_b.as<uint32_t>(), wdeg, g->inv64.as<double>(),
+                               g->perm.as<int32_t>(), n, outcnt, wdeg, g->inv64.as<double>(),
                                g->inv32.as<float>());
         NKPR_HIP(hipGetLastError());
     } else {
@@ -866,17 +881,16 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         g->invw64.alloc(8 * std::max<uint64_t>(n, 1));
         if (n)
             hipLaunchKernelGGL(inv_degree_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
-                               g->perm.as<int32_t>(), n, outcnt_b.as<uint32_t>(), wdeg, g->invw64.as<double>(),
+                               g->perm.as<int32_t>(), n, outcnt, wdeg, g->invw64.as<double>(),
                                (float *)nullptr);
         NKPR_HIP(hipGetLastError());
         g->w32_exact = true;
         if (w64_in && m) {
-            NKPR_HIP(hipMemsetAsync(flags_b.p, 0, 4, s));
             hipLaunchKernelGGL(fp32_exact_kernel, dim3((unsigned)std::min<uint64_t>(blocks_for(m), 2048)), dim3(256), 0, s,
-                               w_in, w64_in, m, flags_b.as<uint32_t>());
+                               w_in, w64_in, m, inexact);
             NKPR_HIP(hipGetLastError());
             uint32_t hf = 0;
-            read_back(s, {{&hf, flags_b.p, 4}});
+            read_back(s, {{&hf, inexact, 4}});
             g->w32_exact = hf == 0;
         }
     }
