@@ -511,7 +511,7 @@ void schedule_items(nkpr_graph *g) {
     while (S == 1 && cap > kCapMin && m < (uint64_t)cap * kItemsWanted) cap /= 2;
     // a segment of about 32 items
     const uint64_t per_item = (uint64_t)cap * (g->n_d + ns_tot) / std::max<uint64_t>(m, 1);
-    uint32_t seg_rows = 1024;
+    uint32_t seg_rows = 256;
     while (seg_rows < 8192 && seg_rows < 32 * std::min<uint64_t>(per_item, kRowsMax)) seg_rows *= 2;
     const uint32_t dsegs = (g->n_d + seg_rows - 1) / seg_rows, ssegs = (n_s + seg_rows - 1) / seg_rows;
     const uint32_t nseg = dsegs + S * ssegs;
