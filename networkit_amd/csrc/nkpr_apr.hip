@@ -230,13 +230,20 @@ __global__ __launch_bounds__(kPushThreads) void apr_rounds_kernel(
     __shared__ uint32_t list[kPushThreads + kGroups * kPushChunk];
     __shared__ uint32_t n_list, base, ok;
     __shared__ unsigned long long edges;
-    if (ld_agent(cnt + kCntAbort)) return;  // (before the first barrier: set only if this block came too late)
+    // Set already: this block came too late.  One thread asks for the whole block: the word may be set
+    // between two waves' reads, and waves that went on without the first one would find n_list, base
+    // and edges unset and pass the barriers, which do not count waves that have ended.
+    if (threadIdx.x == 0) {
+        edges = 0;
+        n_list = base = 0;
+        ok = ld_agent(cnt + kCntAbort) == 0u;
+    }
+    __syncthreads();
+    if (!ok) return;
     const uint32_t lane = threadIdx.x % kPushLanes;
     // consecutive entries go to different blocks, so that a small frontier uses every CU
     const uint32_t group = threadIdx.x / kPushLanes * gridDim.x + blockIdx.x, ngroups = gridDim.x * kGroups;
     const uint32_t thread = threadIdx.x * gridDim.x + blockIdx.x, nthreads = gridDim.x * kPushThreads;
-    if (threadIdx.x == 0) edges = 0, n_list = 0;
-    __syncthreads();
     // the block's list into the next frontier (every thread calls it)
     auto flush = [&](uint32_t *next, uint32_t *ncnt) {
         __syncthreads();

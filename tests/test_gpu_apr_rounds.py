@@ -6,6 +6,7 @@ lane groups, and the run on one block that follows when the blocks' wait for eac
 (forced with a limit of zero).  Residuals are whole numbers (2^-62 units), so the restatement in
 Python integers must agree bit for bit; p is a sum of products in round order, the same too."""
 import math
+import threading
 
 import numpy as np
 import pytest
@@ -86,3 +87,40 @@ def test_rounds_match_the_restatement(monkeypatch, z, degrees, seeds, weighted, 
         assert np.array_equal(p, want[1]) and np.array_equal(r, want[2])
         assert (st["rounds"], st["pushes"]) == want[3:]
     a.close()
+
+
+@pytest.mark.parametrize("limit", [None, "0"])
+def test_runs_of_several_threads(monkeypatch, limit):
+    """A handle per thread, whose grids share the device; with a limit of zero blocks still start
+    while others have given up, and each of them must leave or stay as a whole."""
+    if limit is not None:
+        monkeypatch.setenv("NKPR_TEST_APR_WAIT", limit)
+    cases = []
+    for k, (z, degrees, seeds) in enumerate([(300, [63, 64, 65, 128], [0, 1]), (9000, [8193, 64], [0]),
+                                             (2000, [500] * 40, list(range(1000))), (40, [0, 1], [1])]):
+        ptr, dst, w = lists(z, degrees, k, False)
+        w = np.ceil(w * 4) / 4
+        a = capi.DeviceAPR(z, ptr.astype(np.uint64), dst.astype(np.int32), w)
+        cases.append((a, seeds, rounds(z, ptr, dst, w, seeds, 0.2, 1e-4)))
+    bad = []
+
+    def work(k):
+        a, seeds, want = cases[k]
+        try:
+            for turn in range(6):
+                ids, p, r, st = a.run(seeds, 0.2, 1e-4)
+                if not (np.array_equal(ids, want[0]) and np.array_equal(p, want[1])
+                        and np.array_equal(r, want[2]) and (st["rounds"], st["pushes"]) == want[3:]):
+                    bad.append((k, turn))
+                    return
+        except Exception as e:  # the first fault ends the thread's runs
+            bad.append((k, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(k,)) for k in range(len(cases))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
+    for a, _, _ in cases:
+        a.close()
