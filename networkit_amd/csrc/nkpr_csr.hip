@@ -78,7 +78,7 @@ constexpr uint32_t kNoallocList = 1u << 21, kNoallocPieces = 1u << 22;
 constexpr uint32_t kNoallocPiece = 4096;
 
 struct CsrView {
-    uint64_t rows, nnz;
+    uint64_t rows, nnz;       // nnz: length of col_idx and values
     const uint64_t *row_idx;
     const uint64_t *col_idx;
     const double *val;
@@ -126,15 +126,26 @@ __device__ __forceinline__ double block_sum(double v) {
     return tot;
 }
 
-// Rows that have ended before merged item d: the smallest i in [max(0, d - nnz), min(d, rows)] whose
+// The entries that the offsets name: `count` of them from `first` on.  col_idx and values may hold
+// more, before them (offsets of some rows of a larger matrix) and after them (lists with room to
+// spare); the host only knows their length, so it sizes the grid and the scratch for all of them.
+struct Entries {
+    uint64_t first, count;
+};
+__device__ __forceinline__ Entries entries_of(const CsrView &A) {
+    const uint64_t first = A.row_idx[0];
+    return {first, min(A.row_idx[A.rows] - first, A.nnz)};
+}
+
+// Rows that have ended before merged item d: the smallest i in [max(0, d - count), min(d, rows)] whose
 // row end lies past entry d - i - 1.  A wave probes 64 places of the range at a time.
-__device__ __forceinline__ uint64_t rows_before(const CsrView &A, uint64_t d) {
+__device__ __forceinline__ uint64_t rows_before(const CsrView &A, const Entries &E, uint64_t d) {
     const uint32_t lane = threadIdx.x & 63;
-    uint64_t lo = d > A.nnz ? d - A.nnz : 0, hi = d < A.rows ? d : A.rows;
+    uint64_t lo = d > E.count ? d - E.count : 0, hi = d < A.rows ? d : A.rows;
     while (lo < hi) {
         const uint64_t step = (hi - lo + 63) / 64;
         const uint64_t mid = lo + (lane + 1) * step - 1;
-        const bool ended = mid < hi && A.row_idx[mid + 1] <= d - mid - 1;
+        const bool ended = mid < hi && A.row_idx[mid + 1] - E.first <= d - mid - 1;
         const uint64_t c = (uint64_t)__popcll(__ballot(ended));
         const uint64_t next = lo + (c + 1) * step - 1;
         lo += c * step;
@@ -143,7 +154,8 @@ __device__ __forceinline__ uint64_t rows_before(const CsrView &A, uint64_t d) {
     return lo;
 }
 
-// Tile t: rows [i0, i1) end in it, with entries [k0, k1).
+// Tile t: rows [i0, i1) end in it, with entries [k0, k1).  Tiles past the last merged item are empty
+// and leave no carry.
 template <typename Shape, bool STEP>
 __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
                                                                    const double *__restrict__ x,
@@ -157,12 +169,13 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
     __shared__ uint32_t n_long;
     __shared__ uint64_t s_row[2];
     const uint32_t tid = threadIdx.x, wave = tid >> 6;
+    const Entries E = entries_of(A);
     double sq = 0.0;
     for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-        const uint64_t d0 = t * kItems;
-        const uint64_t d1 = min(d0 + kItems, A.rows + A.nnz);
+        const uint64_t d0 = min(t * kItems, A.rows + E.count);
+        const uint64_t d1 = min(d0 + kItems, A.rows + E.count);
         if (wave < 2) {
-            const uint64_t i = rows_before(A, wave ? d1 : d0);
+            const uint64_t i = rows_before(A, E, wave ? d1 : d0);
             if ((tid & 63) == 0) s_row[wave] = i;
         }
         if (tid == 0) n_long = 0;
@@ -170,8 +183,8 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
         const uint64_t i0 = s_row[0], i1 = s_row[1], k0 = d0 - i0, k1 = d1 - i1;
         const uint32_t cnt = (uint32_t)(k1 - k0), whole = (uint32_t)(i1 - i0);
         // the entries, every load before the gathers that need it
-        const uint64_t *__restrict__ col = A.col_idx + k0;
-        const double *__restrict__ val = A.val + k0;
+        const uint64_t *__restrict__ col = A.col_idx + E.first + k0;
+        const double *__restrict__ val = A.val + E.first + k0;
         uint64_t c[kPer];
         double v[kPer];
 #pragma unroll
@@ -181,7 +194,7 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
             v[k] = e < cnt ? __builtin_nontemporal_load(val + e) : 0.0;
         }
         for (uint32_t j = tid; j < whole; j += kThreads)
-            ends[j + 1] = (uint16_t)(A.row_idx[i0 + j + 1] - k0);
+            ends[j + 1] = (uint16_t)(min(A.row_idx[i0 + j + 1] - E.first, k1) - k0);
         if (tid == 0) {
             ends[0] = 0;
             ends[whole + 1] = (uint16_t)cnt;
@@ -193,7 +206,7 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
         }
         __syncthreads();
         // row i0 began in an earlier tile: its sum, and its square, are finished by the fix kernel
-        const bool continued = i0 < A.rows && A.row_idx[i0] < k0;
+        const bool continued = i0 < A.rows && A.row_idx[i0] - E.first < k0;
         const uint32_t R = whole + 1;  // the last one: what is left after the last row end
         const uint32_t tail = cnt - ends[whole];
         auto put = [&](uint32_t r, double sum) {

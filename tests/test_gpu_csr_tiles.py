@@ -79,3 +79,35 @@ def test_large_tiles(rows, length):
     y2, sq2 = d.pagerank_step(x, 0.5)
     torch.cuda.synchronize()
     assert torch.equal(y, y2) and torch.equal(sq, sq2)
+
+
+# entries before the first offset and past the last one, in lists of less than a tile up to several
+@pytest.mark.parametrize("before,after", [(0, 1), (0, 5000), (1, 0), (700, 0), (2500, 3000)])
+@pytest.mark.parametrize("rows,length", [(1, 3), (700, 3), (1023, 1), (5, 2047), (40000, 110)])
+def test_lists_longer_than_the_offsets(rows, length, before, after):
+    """The offsets say which entries belong to the rows: some rows of a larger matrix, and lists with
+    room to spare.  The spare entries would change every sum (values of 1e30), and the vectors lie
+    between others that must stay as they are."""
+    import torch
+    rng = np.random.default_rng(rows + before + after)
+    nnz = rows * length
+    col, val = np.zeros(before + nnz + after, np.uint64), np.full(before + nnz + after, 1e30)
+    col[before:before + nnz] = rng.integers(0, rows, nnz)
+    val[before:before + nnz] = rng.uniform(0.1, 1.0, nnz)
+    ptr = before + length * np.arange(rows + 1, dtype=np.uint64)
+    x = rng.random(rows)
+    ref = oracle.csr_spmv(oracle.CSR(rows, rows, ptr - before, col[before:before + nnz], val[before:before + nnz]), x)
+    d = capi.DeviceCSR(rows, rows, ptr, col, val)
+    room = torch.full((3 * rows,), -7.0, dtype=torch.float64, device="cuda")
+    xd, y = torch.from_numpy(x).cuda(), room[rows:2 * rows]
+    d.spmv(xd, y)
+    torch.cuda.synchronize()
+    np.testing.assert_allclose(y.cpu().numpy(), ref, rtol=1e-12, atol=0)
+    y.fill_(-7.0)
+    sq = torch.empty(1, dtype=torch.float64, device="cuda")
+    for step in (d.pagerank_step, d.pagerank_step_noalloc):
+        step(xd, 0.25, y=y, step_sq=sq)
+        torch.cuda.synchronize()
+        np.testing.assert_allclose(y.cpu().numpy(), ref + 0.25, rtol=1e-12, atol=0)
+        assert float(sq) == pytest.approx(float(((ref + 0.25 - x) ** 2).sum()), rel=1e-12)
+    assert torch.all(room[:rows] == -7.0) and torch.all(room[2 * rows:] == -7.0)
