@@ -20,7 +20,7 @@
 //       reads its entries as one stream, puts the products into LDS and adds them row by row, lane
 //       groups for short rows and whole waves for long ones.  What is left after its last row end
 //       is the tile's carry for the row that goes on.
-//   csr_fix_kernel    adds the carries, in tile order, to the row that ended in a later tile.
+//   csr_fix_kernel    adds the carries to the row that ended in a later tile.
 //   csr_final_kernel  (steps of many tiles) adds the blocks' sums.
 // The step's (y - x)^2 is added per block of either kernel.
 //
@@ -137,11 +137,13 @@ __device__ __forceinline__ Entries entries_of(const CsrView &A) {
     return {first, min(A.row_idx[A.rows] - first, A.nnz)};
 }
 
-// Rows that have ended before merged item d: the smallest i in [max(0, d - count), min(d, rows)] whose
-// row end lies past entry d - i - 1.  A wave probes 64 places of the range at a time.
+// Rows that have ended before merged item d: the smallest i in [max(0, d - nnz), min(d, rows)] whose
+// row end lies past entry d - i - 1; all rows for an item past the last one.  A wave probes 64 places
+// of the range at a time.  The range does not depend on the extent, so that its loads and the first
+// probes are on their way together.
 __device__ __forceinline__ uint64_t rows_before(const CsrView &A, const Entries &E, uint64_t d) {
     const uint32_t lane = threadIdx.x & 63;
-    uint64_t lo = d > E.count ? d - E.count : 0, hi = d < A.rows ? d : A.rows;
+    uint64_t hi = d < A.rows ? d : A.rows, lo = d > A.nnz ? min(d - A.nnz, hi) : 0;
     while (lo < hi) {
         const uint64_t step = (hi - lo + 63) / 64;
         const uint64_t mid = lo + (lane + 1) * step - 1;
@@ -172,15 +174,15 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
     const Entries E = entries_of(A);
     double sq = 0.0;
     for (uint64_t t = blockIdx.x; t < tiles; t += gridDim.x) {
-        const uint64_t d0 = min(t * kItems, A.rows + E.count);
-        const uint64_t d1 = min(d0 + kItems, A.rows + E.count);
+        const uint64_t d0 = t * kItems, d1 = d0 + kItems;
         if (wave < 2) {
             const uint64_t i = rows_before(A, E, wave ? d1 : d0);
             if ((tid & 63) == 0) s_row[wave] = i;
         }
         if (tid == 0) n_long = 0;
         __syncthreads();
-        const uint64_t i0 = s_row[0], i1 = s_row[1], k0 = d0 - i0, k1 = d1 - i1;
+        const uint64_t i0 = s_row[0], i1 = s_row[1];
+        const uint64_t k0 = min(d0 - i0, E.count), k1 = min(d1 - i1, E.count);
         const uint32_t cnt = (uint32_t)(k1 - k0), whole = (uint32_t)(i1 - i0);
         // the entries, every load before the gathers that need it
         const uint64_t *__restrict__ col = A.col_idx + E.first + k0;
@@ -259,21 +261,69 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
     }
 }
 
-// The carries: the first of a run of tiles with the same carry row adds the run's carries, in tile
-// order, to that row.  For a step the squares of the rows finished here, after the first n_sq block
-// sums of the tile kernel, go to out[blockIdx.x].
+// The carries of row r from tile t on, added by the wave: lanes stride over kRunTurns * 64 tiles at a
+// time, then a shuffle tree.  Every lane gets the sum.
+constexpr uint32_t kRunTurns = 4;
+__device__ __forceinline__ double sum_run(const TileWork &w, uint64_t t, uint32_t r, uint64_t tiles) {
+    const uint32_t lane = threadIdx.x & 63;
+    double acc = 0.0;
+    for (uint64_t q0 = t + lane;; q0 += 64 * kRunTurns) {
+        uint32_t row[kRunTurns];
+        double c[kRunTurns];
+#pragma unroll
+        for (uint32_t k = 0; k < kRunTurns; ++k) {
+            const uint64_t q = q0 + 64 * k;
+            row[k] = q < tiles ? w.row[q] : kNoRow;
+            c[k] = q < tiles ? w.carry[q] : 0.0;
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kRunTurns; ++k)
+            if (row[k] == r) acc += c[k];
+        if (!__all(row[kRunTurns - 1] == r)) break;
+    }
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    return acc;
+}
+
+// The carries: the first of a run of tiles with the same carry row adds the run's carries, in an
+// order fixed by the matrix, to that row: in tile order up to kRunAlone of them, a wave for more.
+// For a step the squares of the rows finished here, after the first n_sq block sums of the tile
+// kernel, go to out[blockIdx.x].
+//
+// Bound by latency: two rounds of loads.  A thread that walked a run alone waited for one tile's row
+// after the other; steps with one row of 4e6, 1e7 and 1e8 entries took 594, 408 and 4040 us, now 34,
+// 59 and 433.
+constexpr uint32_t kRunAlone = 8;
 template <bool STEP>
 __global__ __launch_bounds__(kFixThreads) void csr_fix_kernel(const double *__restrict__ x, double *y,
                                                               TileWork w, uint64_t tiles,
                                                               uint32_t n_sq, double *out) {
     double sq = 0.0;
     for (uint32_t b = threadIdx.x; STEP && b < n_sq; b += kFixThreads) sq += w.partials[b];
-    for (uint64_t t = (uint64_t)blockIdx.x * kFixThreads + threadIdx.x; t < tiles;
-         t += (uint64_t)gridDim.x * kFixThreads) {
-        const uint32_t r = w.row[t];
-        if (r == kNoRow || (t > 0 && w.row[t - 1] == r)) continue;
-        double s = w.carry[t];
-        for (uint64_t q = t + 1; q < tiles && w.row[q] == r; ++q) s += w.carry[q];
+    const uint32_t lane = threadIdx.x & 63;
+    for (uint64_t t0 = (uint64_t)blockIdx.x * kFixThreads + (threadIdx.x - lane); t0 < tiles;
+         t0 += (uint64_t)gridDim.x * kFixThreads) {
+        const uint64_t t = t0 + lane;
+        // every load of the tiles at once
+        uint32_t row[kRunAlone + 1];
+        double c[kRunAlone];
+#pragma unroll
+        for (uint32_t k = 0; k <= kRunAlone; ++k) row[k] = t + k < tiles ? w.row[t + k] : kNoRow;
+#pragma unroll
+        for (uint32_t k = 0; k < kRunAlone; ++k) c[k] = t + k < tiles ? w.carry[t + k] : 0.0;
+        const uint32_t before = t > 0 && t < tiles ? w.row[t - 1] : kNoRow, r = row[0];
+        const bool first = r != kNoRow && before != r;
+        const bool many = first && row[kRunAlone] == r;
+        double s = c[0];
+#pragma unroll
+        for (uint32_t k = 1; k < kRunAlone; ++k)
+            if (row[k] == r) s += c[k];
+        for (uint64_t left = __ballot(many); left; left &= left - 1) {
+            const int l = __ffsll((long long)left) - 1;
+            const double sum = sum_run(w, t0 + l, __shfl(r, l, 64), tiles);
+            if ((int)lane == l) s = sum;
+        }
+        if (!first) continue;
         const double v = s + y[r];
         y[r] = v;
         if (STEP) {

@@ -111,3 +111,37 @@ def test_lists_longer_than_the_offsets(rows, length, before, after):
         np.testing.assert_allclose(y.cpu().numpy(), ref + 0.25, rtol=1e-12, atol=0)
         assert float(sq) == pytest.approx(float(((ref + 0.25 - x) ** 2).sum()), rel=1e-12)
     assert torch.all(room[:rows] == -7.0) and torch.all(room[2 * rows:] == -7.0)
+
+
+def test_rows_over_many_tiles():
+    """Runs of carries around what one thread adds (8 tiles of 1024 items) and around a wave's turns
+    (64 tiles a load, 256 a turn), each with an ordinary row behind it.  t positive terms in any order
+    are within t 2^-53 of their sum, relatively; torch adds them pairwise (within 1e-15)."""
+    import torch
+    tiles = [6, 7, 8, 9, 10, 63, 64, 65, 66, 255, 256, 257, 258, 320, 511, 512, 513]
+    lengths = np.array([x for k in tiles for x in (1024 * k, 3, 1024 * k + 1021)], np.int64)
+    n = len(lengths)
+    g = torch.Generator(device="cuda").manual_seed(5)
+    nnz = int(lengths.sum())
+    col = torch.randint(n, (nnz,), generator=g, device="cuda")
+    val = torch.rand(nnz, generator=g, device="cuda", dtype=torch.float64)
+    x = torch.rand(n, generator=g, device="cuda", dtype=torch.float64)
+    ref = torch.stack([(v * x[c]).sum() for v, c in zip(val.split(lengths.tolist()), col.split(lengths.tolist()))])
+    ptr = np.concatenate([[0], np.cumsum(lengths)])
+    # below 2^22 items a tile has 1024 of them: the matrix in three parts
+    for a, b in ((0, 39), (39, 45), (45, n)):
+        k0, k1 = int(ptr[a]), int(ptr[b])
+        assert k1 - k0 + b - a < 1 << 22
+        d = capi.DeviceCSR(b - a, n, ptr[a:b + 1] - k0, col[k0:k1], val[k0:k1])
+        y = d.spmv(x)
+        torch.cuda.synchronize()
+        tol = torch.from_numpy(lengths[a:b] * 2.0 ** -53 + 1e-15).cuda() * ref[a:b]
+        assert torch.all((y - ref[a:b]).abs() <= tol)
+    # the same rows in tiles of 4096 items
+    d = capi.DeviceCSR(n, n, ptr, col, val)
+    y, sq = d.pagerank_step(x, 0.5)
+    y2, sq2 = d.pagerank_step(x, 0.5)
+    torch.cuda.synchronize()
+    assert torch.all((y - 0.5 - ref).abs() <= torch.from_numpy(lengths * 2.0 ** -53 + 1e-15).cuda() * (ref + 0.5))
+    assert float(sq) == pytest.approx(float((ref + 0.5 - x).square().sum()), rel=2 * int(lengths.max()) * 2.0 ** -53)
+    assert torch.equal(y, y2) and torch.equal(sq, sq2)
