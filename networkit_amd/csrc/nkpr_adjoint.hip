@@ -149,11 +149,11 @@ __global__ void grad_factor_kernel(const double *x, uint64_t z, double score_sum
     const uint64_t v = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (v < z) deg[v] = damp * x[v] * score_sum / deg[v];
 }
-// The same from the handle's 1 / deg (compact order); slots without out-arcs are left alone.
-__global__ void grad_factor_inv_kernel(const double *x, const int32_t *perm, const double *inv, uint32_t n,
+// The same from the handle's degrees (compact order).
+__global__ void grad_factor_own_kernel(const double *x, const int32_t *perm, const double *deg, uint32_t n,
                                        double score_sum, double damp, double *factor) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
-    if (r < n) factor[perm[r]] = damp * x[perm[r]] * score_sum * inv[r];
+    if (r < n) factor[perm[r]] = damp * x[perm[r]] * score_sum / deg[r];
 }
 
 // dL/dw for every in-edge of the caller's CSC: a block per kGradTile edges, which looks its rows up
@@ -502,9 +502,8 @@ void adjoint_impl(nkpr_graph *g, const nkpr_params *p, const nkpr_csc *csc,
         if (own) {
             // the degrees that the handle has summed from these weights (summing them again took 0.38 ms
             // of atomics for 4.8e6 arcs)
-            const double *inv = g->weighted ? g->invw64.as<double>() : g->inv64.as<double>();
-            hipLaunchKernelGGL(grad_factor_inv_kernel, dim3(nblocks(n)), dim3(256), 0, s, x_z, g->perm.as<int32_t>(),
-                               inv, n, score_sum, d, deg);
+            hipLaunchKernelGGL(grad_factor_own_kernel, dim3(nblocks(n)), dim3(256), 0, s, x_z, g->perm.as<int32_t>(),
+                               (const double *)g->deg64.as<double>(), n, score_sum, d, deg);
         } else if (csc->out_wdeg) {
             const double *dz = (const double *)csc->out_wdeg;
             if (!edev) NKPR_HIP(hipMemcpyAsync(deg, dz, 8 * z, hipMemcpyHostToDevice, s));

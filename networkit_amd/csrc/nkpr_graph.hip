@@ -264,11 +264,12 @@ __global__ void edge_output_kernel(const uint64_t *keys, const uint32_t *vals, u
 }
 
 __global__ void inv_degree_kernel(const int32_t *perm, uint32_t n, const uint32_t *outcnt,
-                                  const double *wdeg, double *inv64, float *inv32) {
+                                  const double *wdeg, double *inv64, float *inv32, double *deg64) {
     const uint32_t r = blockIdx.x * blockDim.x + threadIdx.x;
     if (r >= n) return;
-    const double v = (outcnt[perm[r]] > 0) ? 1.0 / wdeg[perm[r]] : 0.0;
+    const double d = wdeg[perm[r]], v = (outcnt[perm[r]] > 0) ? 1.0 / d : 0.0;
     inv64[r] = v;
+    if (deg64) deg64[r] = d;
     if (inv32) inv32[r] = (float)v;
 }
 
@@ -867,13 +868,15 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
     } else {
         NKPR_HIP(hipMemsetAsync(g->sptr.p, 0, 4 * (ns_tot + 1), s));
     }
+    if (g->own_degrees) g->deg64.alloc(8 * std::max<uint64_t>(n, 1));
+    double *deg64 = g->own_degrees ? g->deg64.as<double>() : nullptr;
     if (!g->weighted) {
         g->inv32.alloc(4 * std::max<uint64_t>(n, 1));
         g->inv64.alloc(8 * std::max<uint64_t>(n, 1));
         if (n)
             hipLaunchKernelGGL(inv_degree_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
                                g->perm.as<int32_t>(), n, outcnt, wdeg, g->inv64.as<double>(),
-                               g->inv32.as<float>());
+                               g->inv32.as<float>(), deg64);
         NKPR_HIP(hipGetLastError());
     } else {
         // 1 / weighted out-degree, and whether every weight is an FP32 number (then the binned
@@ -882,7 +885,7 @@ void create_graph(const nkpr_csc *c, nkpr_graph *g, const uint64_t *group_off,
         if (n)
             hipLaunchKernelGGL(inv_degree_kernel, dim3(blocks_for(n)), dim3(256), 0, s,
                                g->perm.as<int32_t>(), n, outcnt, wdeg, g->invw64.as<double>(),
-                               (float *)nullptr);
+                               (float *)nullptr, deg64);
         NKPR_HIP(hipGetLastError());
         g->w32_exact = true;
         if (w64_in && m) {
@@ -948,7 +951,6 @@ void set_weights(nkpr_graph *g, const float *w, const double *w64, const double 
     const hipStream_t s = g->stream;
     const uint64_t m = g->m, z = g->z;
     const uint32_t n = g->n;
-    g->own_degrees = out_wdeg == nullptr;
     DevBuf wb, w64b, degz, deg;
     if (!device_ptrs) {
         if (w) {
@@ -1018,6 +1020,11 @@ void set_weights(nkpr_graph *g, const float *w, const double *w64, const double 
     if (exact != g->w32_exact) g->bn64.ready = false;  // the FP64 copy changes its coefficient type
     g->w32_exact = exact;
     NKPR_HIP(hipStreamSynchronize(s));
+    g->own_degrees = out_wdeg == nullptr;
+    if (g->own_degrees) {
+        std::swap(g->deg64.p, deg.p);
+        std::swap(g->deg64.bytes, deg.bytes);
+    }
     // derived copies follow the coefficients
     g->b_coef_ready = false;
     g->rowsum_ready = false;

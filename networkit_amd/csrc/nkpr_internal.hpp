@@ -471,6 +471,7 @@ struct nkpr_graph {
     nkpr::DevBuf inv32;     // float [n]   (unweighted)
     nkpr::DevBuf inv64;     // double [n]  (unweighted)
     nkpr::DevBuf invw64;    // double [n]  1 / weighted out-degree (weighted)
+    nkpr::DevBuf deg64;     // double [n]  weighted out-degree as summed here (own_degrees)
     nkpr::DevBuf rowsum64;  // double [n]  FP64 sum of each row's in-coefficients (built on use)
     bool rowsum_ready = false;
     nkpr::DevBuf flag_buf;  // uint32 [1]  device-side yes/no answers read back by the host

@@ -38,3 +38,32 @@ def test_weight_gradients(m, weighted, degrees):
     want_w, want_t, _ = dense_grads(z, ptr, src, w, np.full(z, 1.0 / z), c)
     assert np.abs(gw - want_w).max() <= 1e-9 * max(np.abs(want_w).max(), 1e-3)
     assert np.abs(gt - want_t).max() <= 1e-9 * np.abs(want_t).max()
+
+
+@pytest.mark.parametrize("degrees", ["own", "given", "set"])
+def test_sources_of_negative_weights(degrees):
+    """A source whose weights are all negative has the coefficients of one whose weights are all
+    positive, and gradients of the other sign."""
+    z, m, rng = 130, 3000, np.random.default_rng(8)
+    key = np.sort(rng.choice(z * (z - 30), m, replace=False))
+    row, src = key // z, (key % z).astype(np.int32)
+    ptr = np.concatenate([[0], np.cumsum(np.bincount(row, minlength=z))])
+    factor = np.ones(z)
+    factor[::3], factor[1] = -1.0, 1e-300
+    base = rng.uniform(0.5, 1.5, m)
+    w = base * factor[src]
+    deg = np.bincount(src, weights=w, minlength=z)
+    given = deg if degrees == "given" else None
+    if degrees == "set":
+        g = capi.DeviceGraph(z, ptr, src, base.astype(np.float32), weight64=base)
+        g.set_weights(w.astype(np.float32), w)
+    else:
+        g = capi.DeviceGraph(z, ptr, src, w.astype(np.float32), weight64=w, out_wdeg=given)
+    x = np.full(z, 1.0 / z)
+    st = g.run(x, capi.default_params(tol=1e-15, max_iterations=2000))
+    c = rng.standard_normal(z)
+    gw, _, _ = g.adjoint(ptr, src, x, st["score_sum"], c, weight=w.astype(np.float32), weight64=w, out_wdeg=given,
+                         params=capi.default_params(tol=1e-13))
+    # times the factor: the gradients of the weights without it
+    want_w, _, _ = dense_grads(z, ptr, src, base, np.full(z, 1.0 / z), c)
+    assert np.abs(gw * factor[src] - want_w).max() <= 1e-9 * np.abs(want_w).max()
