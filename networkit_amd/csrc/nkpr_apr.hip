@@ -52,6 +52,7 @@ struct nkpr_apr {
     nkpr::DevBuf p, r, flags, f0, f1, push, chunks, cnt, out_ids, out_p, out_r, out_cnt, seeds;
     uint64_t chunk_cap = 0;  // entries per heavy chunk list (two lists)
     bool dirty = true;  // p, r, flags hold a run that was not cleared
+    uint32_t apart = 0;  // runs still to be made with a launch per part (a wait of the grid expired)
     ~nkpr_apr() {
         nkpr::stream_put(stream, device);
     }
@@ -63,11 +64,18 @@ namespace {
 constexpr uint32_t kTouched = 1, kQueued = 2;
 // 512 threads: the grids of four runs (a process has four hardware queues) fit the device together, so
 // that none waits for blocks which another keeps out.  1024 took the same time alone (3.29 and 3.35 ms
-// a run); four threads share the device at 0.87 ms a run, 1.17 with two launches a round.
+// a run); four threads share the device at 0.87 ms a run, 1.17 with two launches a round.  More grids
+// than four (several processes) may keep each other's blocks out: see kMissing.
 constexpr int kPushThreads = 512;
 constexpr uint32_t kPushLanes = 32;  // lanes that push one frontier node
-// rounds per launch of the rounds kernel, after which the host looks whether the frontier is empty
-constexpr uint32_t kMaxRounds = 4096;
+// Rounds after which the host looks whether the frontier is empty: of one launch, and of launches
+// apart (NKPR_APR_BATCH, 1 to 256, overrides both).
+constexpr uint32_t kTogetherRounds = 4096, kApartRounds = 16;
+// A wait of the grid for a block that cannot start ends after kMissing (2 s, in units of 10 ns).  The
+// run, and the next kApartRuns of the handle, then launch the parts of a round apart, where no block
+// waits for another and the device stays full.
+constexpr uint64_t kMissing = 200000000;
+constexpr uint32_t kApartRuns = 64;
 constexpr double kUnit = 4611686018427387904.0;  // 2^62 fixed-point units per unit of mass
 
 // ceil(eps vol 2^62): r < thr  <=>  r 2^-62 < eps vol (the product rounded as the reference's).
@@ -160,7 +168,7 @@ template <typename T> __device__ __forceinline__ void st_agent(T *p, T v) {
 // last ones count at the top: 256 adds to one address would queue for longer than the rounds' own
 // work.  The grid has a block per CU, all of which are resident once the kernels ahead of them
 // have ended; should one still be missing after `ticks` (of 10 ns), the wait ends, every block leaves
-// (false) and the run is done again by one block, which waits for nobody.
+// (false) and the run is done again with the parts apart.
 __device__ __forceinline__ bool grid_barrier(uint32_t *cnt, uint32_t turn, uint64_t ticks, uint32_t *ok) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -200,8 +208,8 @@ __global__ void apr_seed_kernel(const uint32_t *seeds, uint32_t k, uint64_t *r, 
         for (int i = threadIdx.x; i < kCntWords; i += blockDim.x) cnt[i] = i == 0 ? k : 0u;
 }
 
-// Rounds first .. first + kMaxRounds - 1, or until a frontier is empty.  A round has two parts with
-// a grid barrier after each.
+// Rounds first .. first + rounds - 1, or until a frontier is empty.  A round has two parts with a grid
+// barrier after each; with PARTS one of the two, the launch is that part of round `first`.
 //
 // Take: a thread per frontier node u takes its residual res, adds alpha res to p[u] and leaves
 // (1 - alpha) res / 2 in r[u], queueing u again when that alone reaches its threshold; a node with
@@ -222,9 +230,11 @@ __global__ void apr_seed_kernel(const uint32_t *seeds, uint32_t k, uint64_t *r, 
 // Hyperbolic graph of 2e6 nodes, eps 1e-8, three seeds: 3.76, 2.96 and 2.73 ms a run with two launches a
 // round, 3.24, 2.46 and 2.49 now; 64 seeds on 6e6 nodes, eps 1e-9: 18.6 and 16.3 ms (1.1e10 adds
 // a second, what the atomics give).
+constexpr int kTake = 1, kPush = 2, kRound = kTake | kPush;
+template <int PARTS>
 __global__ __launch_bounds__(kPushThreads) void apr_rounds_kernel(
     const uint64_t *ptr, const int32_t *dst, const double *w, const double *vol, double alpha, double eps,
-    uint32_t *f0, uint32_t *f1, uint32_t *cnt, uint32_t first, double *p, uint64_t *r, uint32_t *flags, Push *push,
+    uint32_t *f0, uint32_t *f1, uint32_t *cnt, uint32_t first, uint32_t rounds, double *p, uint64_t *r, uint32_t *flags, Push *push,
     uint64_t *chunks, uint64_t chunk_cap, uint64_t ticks) {
     constexpr uint32_t kGroups = kPushThreads / kPushLanes;
     __shared__ uint32_t list[kPushThreads + kGroups * kPushChunk];
@@ -256,47 +266,56 @@ __global__ __launch_bounds__(kPushThreads) void apr_rounds_kernel(
         }
         __syncthreads();
     };
-    for (uint32_t round = first; round - first < kMaxRounds; ++round) {
+    for (uint32_t round = first; round - first < rounds; ++round) {
         const uint32_t k2 = round & 1, k3 = round % 3;
         const uint32_t *front = k2 ? f1 : f0;
         uint32_t *next = k2 ? f0 : f1, *ncnt = cnt + (k3 + 1) % 3, *hcnt = cnt + kCntChunks + k2;
         uint64_t *chunk = chunks + (k2 ? chunk_cap : 0);
         const uint32_t nf = ld_agent(cnt + k3);
-        if (nf == 0) break;
-        if (blockIdx.x == 0 && threadIdx.x == 0) {
-            st_agent(cnt + (k3 + 2) % 3, 0u);
-            st_agent(cnt + kCntChunks + (k2 ^ 1), 0u);
-            *reinterpret_cast<unsigned long long *>(cnt + kCntPushes) += nf;
-            cnt[kCntRounds] += 1u;
-        }
-        for (uint32_t i0 = 0; i0 < nf; i0 += nthreads) {
-            const uint32_t i = i0 + thread;
-            if (i < nf) {
-                const uint32_t u = ld_agent(front + i);
-                const uint64_t res = ld_agent(r + u), b = ptr[u], deg = ptr[u + 1] - b;
-                const double vu = vol[u], pu = ld_agent(p + u);
-                const double dres = (double)res;
-                const uint64_t keep = __double2ull_rn((1.0 - alpha) * dres / 2);
-                const bool again = keep >= threshold_of(eps, vu, true);
-                st_agent(p + u, pu + alpha * dres / kUnit);
-                st_agent(r + u, keep);
-                st_agent(flags + u, again ? (kTouched | kQueued) : kTouched);
-                Push *o = push + i;
-                st_agent(&o->first, b);
-                st_agent(&o->count_node, deg << 32 | u);
-                st_agent(&o->share, vu > 0.0 ? (1.0 - alpha) * dres / (2.0 * vu) : 0.0);
-                atomicAdd(&edges, (unsigned long long)deg);
-                if (deg > kPushChunk) {
-                    const uint32_t nc = (uint32_t)((deg + kPushChunk - 1) / kPushChunk);
-                    const uint32_t at = atomicAdd(hcnt, nc);
-                    for (uint32_t c = 0; c < nc; ++c) st_agent(chunk + at + c, (uint64_t)c << 32 | i);
+        if constexpr (PARTS & kTake) {
+            // (after the last round too: launches apart go on to the end of their batch)
+            if (blockIdx.x == 0 && threadIdx.x == 0) {
+                st_agent(cnt + (k3 + 2) % 3, 0u);
+                st_agent(cnt + kCntChunks + (k2 ^ 1), 0u);
+                if (nf) {
+                    *reinterpret_cast<unsigned long long *>(cnt + kCntPushes) += nf;
+                    cnt[kCntRounds] += 1u;
                 }
-                if (again) list[atomicAdd(&n_list, 1u)] = u;
             }
-            // (the last turn's nodes wait for those of the push)
-            if (nf - i0 > nthreads) flush(next, ncnt);
         }
-        if (!grid_barrier(cnt, 2 * round, ticks, &ok)) break;
+        if (nf == 0) break;
+        if constexpr (PARTS & kTake) {
+            for (uint32_t i0 = 0; i0 < nf; i0 += nthreads) {
+                const uint32_t i = i0 + thread;
+                if (i < nf) {
+                    const uint32_t u = ld_agent(front + i);
+                    const uint64_t res = ld_agent(r + u), b = ptr[u], deg = ptr[u + 1] - b;
+                    const double vu = vol[u], pu = ld_agent(p + u);
+                    const double dres = (double)res;
+                    const uint64_t keep = __double2ull_rn((1.0 - alpha) * dres / 2);
+                    const bool again = keep >= threshold_of(eps, vu, true);
+                    st_agent(p + u, pu + alpha * dres / kUnit);
+                    st_agent(r + u, keep);
+                    st_agent(flags + u, again ? (kTouched | kQueued) : kTouched);
+                    Push *o = push + i;
+                    st_agent(&o->first, b);
+                    st_agent(&o->count_node, deg << 32 | u);
+                    st_agent(&o->share, vu > 0.0 ? (1.0 - alpha) * dres / (2.0 * vu) : 0.0);
+                    atomicAdd(&edges, (unsigned long long)deg);
+                    if (deg > kPushChunk) {
+                        const uint32_t nc = (uint32_t)((deg + kPushChunk - 1) / kPushChunk);
+                        const uint32_t at = atomicAdd(hcnt, nc);
+                        for (uint32_t c = 0; c < nc; ++c) st_agent(chunk + at + c, (uint64_t)c << 32 | i);
+                    }
+                    if (again) list[atomicAdd(&n_list, 1u)] = u;
+                }
+                // (the last turn's nodes wait for those of the push)
+                if (PARTS == kTake || nf - i0 > nthreads) flush(next, ncnt);
+            }
+        }
+        if constexpr (PARTS == kTake) break;
+        if constexpr (PARTS == kRound)
+            if (!grid_barrier(cnt, 2 * round, ticks, &ok)) break;
         // the first turn's items are on their way beside the number of chunks
         const uint32_t nh = ld_agent(hcnt);
         uint64_t from = 0, cn = 0;
@@ -337,7 +356,9 @@ __global__ __launch_bounds__(kPushThreads) void apr_rounds_kernel(
             }
             flush(next, ncnt);
         }
-        if (!grid_barrier(cnt, 2 * round + 1, ticks, &ok)) break;
+        if constexpr (PARTS == kPush) break;
+        if constexpr (PARTS == kRound)
+            if (!grid_barrier(cnt, 2 * round + 1, ticks, &ok)) break;
     }
     __syncthreads();
     if (threadIdx.x == 0 && edges)
@@ -504,15 +525,16 @@ void apr_run_impl(nkpr_apr *a, double alpha, double eps, const uint64_t *seeds, 
     a->seeds.alloc(4 * sd.size());
     NKPR_HIP(hipMemcpyAsync(a->seeds.p, sd.data(), 4 * sd.size(), hipMemcpyHostToDevice, s));
     // The rounds of a launch end by themselves when a frontier is empty.  Its blocks wait for each
-    // other, one per CU; when one of them cannot start for kMissing (other work holds its CU), the
-    // run starts again on one block.
-    constexpr uint64_t kMissing = 200000000;  // 2 s
+    // other, one per CU.
     uint64_t ticks = kMissing;
     // test hook: 0 ends a wait that is not over at once
     if (const char *e = std::getenv("NKPR_TEST_APR_WAIT"); e && *e) ticks = std::strtoull(e, nullptr, 10);
+    uint32_t together = kTogetherRounds, batch = kApartRounds;
+    if (const char *e = std::getenv("NKPR_APR_BATCH"))
+        together = batch = (uint32_t)std::max(1, std::min(256, std::atoi(e)));
     int cus = 0;
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, a->device));
-    unsigned grid = (unsigned)std::max(cus, 1);
+    const unsigned grid = (unsigned)std::max(cus, 1);
     uint32_t host_cnt[16] = {0}, round = 0;
     auto start = [&] {
         if (a->dirty) {
@@ -526,21 +548,34 @@ void apr_run_impl(nkpr_apr *a, double alpha, double eps, const uint64_t *seeds, 
                            a->f0.as<uint32_t>(), a->cnt.as<uint32_t>());
         round = 0;
     };
-    start();
-    for (;;) {
-        hipLaunchKernelGGL(apr_rounds_kernel, dim3(grid), dim3(kPushThreads), 0, s, a->ptr.as<uint64_t>(),
+    auto launch = [&](auto kernel, unsigned blocks, uint32_t rounds) {
+        hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kPushThreads), 0, s, a->ptr.as<uint64_t>(),
                            a->dst.as<int32_t>(), a->w.as<double>(), a->vol.as<double>(), alpha, eps,
-                           a->f0.as<uint32_t>(), a->f1.as<uint32_t>(), a->cnt.as<uint32_t>(), round,
+                           a->f0.as<uint32_t>(), a->f1.as<uint32_t>(), a->cnt.as<uint32_t>(), round, rounds,
                            a->p.as<double>(), a->r.as<uint64_t>(), a->flags.as<uint32_t>(), a->push.as<Push>(),
                            a->chunks.as<uint64_t>(), a->chunk_cap, ticks);
         NKPR_HIP(hipGetLastError());
+    };
+    start();
+    bool apart = a->apart > 0;
+    if (apart) --a->apart;
+    for (;;) {
+        if (apart) {
+            for (uint32_t k = 0; k < batch; ++k, ++round) {
+                launch(apr_rounds_kernel<kTake>, 4 * grid, 1);
+                launch(apr_rounds_kernel<kPush>, 4 * grid, 1);
+            }
+        } else {
+            launch(apr_rounds_kernel<kRound>, grid, together);
+        }
         read_back(s, {{host_cnt, a->cnt.p, sizeof(host_cnt)}});
         if (host_cnt[kCntAbort]) {
-            grid = 1;
+            apart = true;
+            a->apart = kApartRuns;
             start();
             continue;
         }
-        round = host_cnt[kCntRounds];
+        if (!apart) round = host_cnt[kCntRounds];
         if (host_cnt[round % 3] == 0) break;  // the frontier of the next round is empty
     }
     uint64_t rounds = host_cnt[kCntRounds], pushes = 0;

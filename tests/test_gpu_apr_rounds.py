@@ -2,7 +2,7 @@
 
 Out-lists around the 64 edges that one lane group pushes (63, 64, 65, 128, 129), a hub whose list
 spans many chunks, self-loops, sinks as seeds, one frontier entry and more entries than the grid has
-lane groups, and the run on one block that follows when the blocks' wait for each other ends early
+lane groups, and the launches apart that follow when the blocks' wait for each other ends early
 (forced with a limit of zero).  Residuals are whole numbers (2^-62 units), so the restatement in
 Python integers must agree bit for bit; p is a sum of products in round order, the same too."""
 import math
@@ -65,7 +65,8 @@ def rounds(z, ptr, dst, w, seeds, alpha, eps):
     return ids, p[ids], np.array([float(r[u]) / UNIT for u in ids]), count, pushes
 
 
-@pytest.mark.parametrize("one_block", [False, True])
+@pytest.mark.parametrize("batch", [None, "1", "5"])  # rounds between two looks at the frontier
+@pytest.mark.parametrize("apart", [False, True])
 @pytest.mark.parametrize("weighted,self_loops", [(False, False), (True, True)])
 @pytest.mark.parametrize("z,degrees,seeds", [
     (300, [63, 64, 65, 128, 129, 0], [0, 1, 2, 3, 4]),
@@ -73,12 +74,14 @@ def rounds(z, ptr, dst, w, seeds, alpha, eps):
     (9000, [8193], range(8500)),
     (40, [0, 1], [0]),
 ])
-def test_rounds_match_the_restatement(monkeypatch, z, degrees, seeds, weighted, self_loops, one_block):
+def test_rounds_match_the_restatement(monkeypatch, z, degrees, seeds, weighted, self_loops, apart, batch):
     ptr, dst, w = lists(z, degrees, 3, self_loops)
     # weights of whole quarters: every order of adding them up gives the same volume
     w = np.ceil(w * 4) / 4 if weighted else np.ones(len(dst))
-    if one_block:
+    if apart:
         monkeypatch.setenv("NKPR_TEST_APR_WAIT", "0")
+    if batch:
+        monkeypatch.setenv("NKPR_APR_BATCH", batch)
     a = capi.DeviceAPR(z, ptr.astype(np.uint64), dst.astype(np.int32), w if weighted else None)
     want = rounds(z, ptr, dst, w, list(seeds), 0.2, 1e-4)
     for _ in range(2):
