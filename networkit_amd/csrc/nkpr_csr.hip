@@ -202,14 +202,17 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
             ends[whole + 1] = (uint16_t)cnt;
         }
 #pragma unroll
-        for (uint32_t k = 0; k < kPer; ++k)
-            if (tid + k * kThreads < cnt) v[k] *= x[c[k]];
+        for (uint32_t k = 0; k < kPer; ++k) {
+            const uint32_t e = tid + k * kThreads;
+            if (e < cnt) prod[e] = v[k] * x[c[k]];
+        }
+        __syncthreads();
         if (whole == 0) {
-            // the tile lies inside one row, and its sum is the carry: without the products' way through
-            // LDS and one wave (1000 rows of 70000 entries: 301 us a step, now 246; one row of 1e8 433 and 347)
+            // the tile lies inside one row, and its sum is the carry: added by the whole block, not by
+            // one wave (1000 rows of 70000 entries: 301 us a step, now 252; one row of 1e8 433 and 355).  From LDS:
+            // summed from the registers these take 246 and 347, and every other tile 0.6% longer
             double acc = 0.0;
-#pragma unroll
-            for (uint32_t k = 0; k < kPer; ++k) acc += v[k];
+            for (uint32_t e = tid; e < cnt; e += kThreads) acc += prod[e];
             acc = block_sum<kThreads>(acc);
             if (tid == 0) {
                 w.carry[t] = acc;
@@ -217,12 +220,6 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
             }
             continue;
         }
-#pragma unroll
-        for (uint32_t k = 0; k < kPer; ++k) {
-            const uint32_t e = tid + k * kThreads;
-            if (e < cnt) prod[e] = v[k];
-        }
-        __syncthreads();
         // row i0 began in an earlier tile: its sum, and its square, are finished by the fix kernel
         const bool continued = i0 < A.rows && A.row_idx[i0] - E.first < k0;
         const uint32_t R = whole + 1;  // the last one: what is left after the last row end
@@ -307,8 +304,8 @@ __device__ __forceinline__ double sum_run(const TileWork &w, uint64_t t, uint32_
 // kernel, go to out[blockIdx.x].
 //
 // Bound by latency: two rounds of loads.  A thread that walked a run alone waited for one tile's row
-// after the other; steps with one row of 4e6, 1e7 and 1e8 entries took 594, 408 and 4040 us, now 34, 49
-// and 347.
+// after the other; steps with one row of 4e6, 1e7 and 1e8 entries took 594, 408 and 4040 us, now 35, 50
+// and 355.
 constexpr uint32_t kRunAlone = 8;
 template <bool STEP>
 __global__ __launch_bounds__(kFixThreads) void csr_fix_kernel(const double *__restrict__ x, double *y,
