@@ -419,6 +419,13 @@ int nkpr_apr_run(nkpr_apr *a, double alpha, double eps, const uint64_t *seeds, u
 int nkpr_ranking(uint64_t z, const double *scores, const uint8_t *exists, int64_t *ids_out,
                  double *scores_out, uint64_t *count);
 
+/* Device memory of destroyed handles is kept for the next ones: at most 4 GiB per process, in
+ * blocks of at most 1 GiB (the environment's NKPR_POOL_MB sets another bound, 0 keeps nothing).
+ * Blocks unused for ten seconds are freed at the next allocation or release of this library, all
+ * of them when one of its allocations fails.  A process that stops using the library, or that
+ * needs the memory for another one, frees them with this call; it waits for the device. */
+int nkpr_release_memory(void);
+
 /* Message of the last failed call on this thread ("" if none). */
 const char *nkpr_last_error(void);
 

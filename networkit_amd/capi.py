@@ -33,7 +33,7 @@ EXPORTED = ["nkpr_params_default", "nkpr_graph_create", "nkpr_graph_create_batch
             "nkpr_csr_pagerank_step", "nkpr_algebraic_pagerank", "nkpr_nkbg_read",
             "nkpr_nkbg_free", "nkpr_nkbg_write", "nkpr_csr_pagerank_step_noalloc",
             "nkpr_apr_create", "nkpr_apr_destroy", "nkpr_apr_run", "nkpr_algebraic_create",
-            "nkpr_algebraic_run", "nkpr_algebraic_destroy"]
+            "nkpr_algebraic_run", "nkpr_algebraic_destroy", "nkpr_release_memory"]
 ABI_VERSION = 3
 
 
@@ -219,6 +219,11 @@ def _addr(a):
     if isinstance(a, np.ndarray):
         return a.ctypes.data
     return a.data_ptr()  # torch tensor
+
+
+def release_memory():
+    """Free the device memory that is kept for the next handles (nkpr_release_memory)."""
+    check(lib().nkpr_release_memory())
 
 
 class DeviceGraph:

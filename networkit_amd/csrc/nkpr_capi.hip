@@ -548,6 +548,10 @@ int nkpr_abi_version(void) { return NKPR_ABI_VERSION; }
 
 const char *nkpr_last_error(void) { return g_last_error.c_str(); }
 
+int nkpr_release_memory(void) {
+    return guarded([] { release_kept(); });
+}
+
 int nkpr_params_default(nkpr_params *p) {
     return guarded([&] {
         NKPR_CHECK(p != nullptr, "params is NULL");

@@ -456,14 +456,25 @@ struct PoolBuf {
     void *p = nullptr;
     hipStream_t s = nullptr;
     PoolBuf(size_t bytes, hipStream_t st) : s(st) {
-        const hipError_t e = hipMallocAsync(&p, bytes, st);
+        hipError_t e = hipMallocAsync(&p, bytes, st);
+        if (e != hipSuccess && !capturing(st)) {
+            // as device_alloc does
+            (void)hipGetLastError();
+            release_kept();
+            e = hipMallocAsync(&p, bytes, st);
+        }
         if (e != hipSuccess) {
+            (void)hipGetLastError();
             p = nullptr;
             throw Error(NKPR_ERR_NOMEM, std::string("hipMallocAsync failed: ") + hipGetErrorString(e));
         }
     }
     ~PoolBuf() {
         if (p) (void)hipFreeAsync(p, s);
+    }
+    static bool capturing(hipStream_t st) {
+        hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+        return hipStreamIsCapturing(st, &status) != hipSuccess || status != hipStreamCaptureStatusNone;
     }
 };
 

@@ -114,6 +114,7 @@ inline void read_back(hipStream_t s, std::initializer_list<HostCopy> copies) {
 // a released block is not handed out before the device has finished what was enqueued until then.
 void *device_alloc(size_t bytes);
 void device_free(void *p);
+void release_kept();  // frees the blocks that no handle uses
 void *pinned_alloc(size_t bytes);  // at most 4096 bytes; idle when released
 void pinned_free(void *p);
 hipStream_t stream_get();  // non-blocking, default priority

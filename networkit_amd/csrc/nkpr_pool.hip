@@ -12,8 +12,10 @@
 //               block that would pass the bound takes the place of those kept longest: blocks
 //               left by a large handle otherwise held the room that the next handles need
 //               (72 ms instead of 12.5 for the solve above, until they were old enough).
-//   given back  a block unused for kKeepSeconds is freed at the next request or release; all of
-//               them when hipMalloc fails, which is then tried again.
+//   given back  all blocks by release_kept (nkpr_release_memory), and when an allocation of this
+//               library fails, which is then tried again; a block unused for kKeepSeconds at the
+//               next request or release.  There is no timer: a process that stops calling the
+//               library keeps what it had until it asks for the release.
 //   ordering    hipFree waits for all work on the device before the memory can be used again.  The
 //               same holds here: a block is handed out only after a device synchronisation that
 //               came after its release (one for all blocks released before it).
@@ -169,6 +171,12 @@ void device_free(void *p) {
     while (P.kept_bytes + b.bytes > P.limit) P.drop_oldest();
     P.dev[b.device].kept.emplace(b.bytes, Kept{p, ++P.releases, now});
     P.kept_bytes += b.bytes;
+}
+
+void release_kept() {
+    Pool &P = pool();
+    std::lock_guard<std::mutex> lock(P.mu);
+    P.drop_all();
 }
 
 void *pinned_alloc(size_t bytes) {
