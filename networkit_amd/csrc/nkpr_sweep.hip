@@ -213,6 +213,7 @@ struct LongRows {
 };
 static_assert(kCap / (64 * kLongTurns) <= 2 * kRowsMax / kLongTurns, "long rows of an item fit");
 
+static_assert(kRowsMax <= kBlock, "a thread finishes one row of an item");
 // One stream item: rows [r0, r0+R) of a compressed list with absolute in-edge offsets `ptr`,
 // in-edges [e0, e0+cnt) (cnt <= kCap).  DIRECT rows finish with the epilogue (row ids from
 // sc.drow); sliced rows store their row sums into `out` (one slice's partial vector).
@@ -226,15 +227,11 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
     const uint32_t r0 = item.x, R = item.y - item.x, e0 = item.z, cnt = item.w;
     // issue every load that does not depend on another load first
     const uint32_t *__restrict__ pb = ptr + r0;
-    uint32_t p0 = 0, p1 = 0, p2 = 0;
+    uint32_t p0 = 0, pe = 0;
     if (tid <= R) p0 = ld_stream(pb + tid) - e0;
-    if (tid + kBlock <= R) p1 = ld_stream(pb + tid + kBlock) - e0;
-    if (tid == 0 && R == 2 * kBlock) p2 = ld_stream(pb + R) - e0;
-    uint32_t u0 = 0, u1 = 0;
-    if (DIRECT) {
-        if (tid < R) u0 = ld_stream(a.sc.drow + r0 + tid);
-        if (tid + kBlock < R) u1 = ld_stream(a.sc.drow + r0 + tid + kBlock);
-    }
+    if (tid == 0 && R == kBlock) pe = ld_stream(pb + R) - e0;
+    uint32_t u = 0;
+    if (DIRECT && tid < R) u = ld_stream(a.sc.drow + r0 + tid);
     int32_t sidx[kPer];
     T cf[kPer];
     {
@@ -251,24 +248,17 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
             }
         }
     }
-    T xo0 = 0, xo1 = 0, bv0 = 0, bv1 = 0;
-    if (DIRECT) {
+    T xo = 0, bv = 0;
+    if (DIRECT && tid < R) {
         // folded: xold is also the gathered vector, keep its lines cacheable
-        if (tid < R) {
-            xo0 = FOLDED ? a.xold[u0] : ld_stream(a.xold + u0);
-            if (BASEVEC) bv0 = ld_stream(a.base_vec + u0);
-        }
-        if (tid + kBlock < R) {
-            xo1 = FOLDED ? a.xold[u1] : ld_stream(a.xold + u1);
-            if (BASEVEC) bv1 = ld_stream(a.base_vec + u1);
-        }
+        xo = FOLDED ? a.xold[u] : ld_stream(a.xold + u);
+        if (BASEVEC) bv = ld_stream(a.base_vec + u);
     }
     T v[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) v[k] = gather(a, hub, nh, sidx[k]) * cf[k];
     if (tid <= R) s_ptr[tid] = p0;
-    if (tid + kBlock <= R) s_ptr[tid + kBlock] = p1;
-    if (tid == 0 && R == 2 * kBlock) s_ptr[R] = p2;
+    if (tid == 0 && R == kBlock) s_ptr[R] = pe;
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
         const uint32_t i = tid + k * kBlock;
@@ -314,20 +304,14 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
     }
     // one thread per row; the LDS buffers are rewritten only after the next item's first
     // barrier, which every thread reaches after this point
-    if (DIRECT) {
-        if (tid < R) {
+    if (tid < R) {
+        if (DIRECT) {
             T y = damp * s_sum[tid] + c;
-            if (BASEVEC) y += bv0;
-            epilogue_store<T, RESID>(a, u0, y, xo0, st);
+            if (BASEVEC) y += bv;
+            epilogue_store<T, RESID>(a, u, y, xo, st);
+        } else {
+            __builtin_nontemporal_store(s_sum[tid], out + r0 + tid);
         }
-        if (tid + kBlock < R) {
-            T y = damp * s_sum[tid + kBlock] + c;
-            if (BASEVEC) y += bv1;
-            epilogue_store<T, RESID>(a, u1, y, xo1, st);
-        }
-    } else {
-        if (tid < R) __builtin_nontemporal_store(s_sum[tid], out + r0 + tid);
-        if (tid + kBlock < R) __builtin_nontemporal_store(s_sum[tid + kBlock], out + r0 + tid + kBlock);
     }
 }
 
@@ -411,15 +395,15 @@ __device__ __forceinline__ void finish_sweep(const SweepArgs<T> &a, const Finali
 }
 
 // Waves a SIMD.  Six (80 VGPRs) let three blocks share a CU, as their LDS does; at five two blocks
-// share it, and the sweep of a 1.3e6-node union of graphs takes 75 instead of 67 us.  The weighted
-// FP64 sweep gains nothing from the third block: 2.40 instead of 2.28 ms per solve of an R-MAT
-// graph of 9e5 nodes.
-template <typename T, bool FOLDED> constexpr int sweep_waves() {
-    return sizeof(T) == 8 && FOLDED ? 5 : 6;
-}
+// share it, and the sweep of a 1.3e6-node union of graphs takes 75 instead of 67 us.
+constexpr int kSweepWaves = 6;
+// The weighted FP64 sweep, which streams 12 bytes an arc beside its gathers, is launched with two
+// blocks a CU all the same.  Solves of R-MAT graphs with two / three: 3e5 nodes 0.997 / 1.053 ms, 9e5
+// 2.27 / 2.38, 4e6 9.91 / 10.5; a weighted union of 1.3e6 nodes 2.33 / 2.45; equal up to 1.3e5 nodes.
+constexpr int kWeighted64Blocks = 2;
 
 template <typename T, bool FOLDED, bool BASEVEC, bool RESID>
-__global__ __launch_bounds__(kBlock, (sweep_waves<T, FOLDED>())) void sweep_kernel(SweepArgs<T> a, FinalizeArgs f) {
+__global__ __launch_bounds__(kBlock, kSweepWaves) void sweep_kernel(SweepArgs<T> a, FinalizeArgs f) {
     if (a.ctl->done) return;  // converged earlier in this batch: no-op
 
     __shared__ T s_prod[kCap];
@@ -842,6 +826,7 @@ int sweep_resident_blocks(int device, bool dbl, bool folded, int kind) {
     NKPR_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, kBlock, 0));
     int cus = 0;
     NKPR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
+    if (dbl && folded) per_cu = std::min(per_cu, kWeighted64Blocks);
     if (per_cu < 1) per_cu = 1;
     return per_cu * std::max(cus, 1);
 }
