@@ -1572,7 +1572,7 @@ bool binned64_active(nkpr_graph *g, bool one_sweep) {
 }
 
 // One FP64 sweep x' = d P x + b through the binned passes, with the epilogue, reductions and
-// stopping rule of launch_sweep<double> (the finalize kernel adds the per-bin partials in bin
+// stopping rule of launch_sweep<double> (a one-block launch adds the per-bin partials in bin
 // order).  Every kernel returns at once when the phase has stopped.
 void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArgs &f, int kind,
                     hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {

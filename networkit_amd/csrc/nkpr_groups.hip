@@ -378,7 +378,7 @@ void run_batch_impl(nkpr_graph *g, const nkpr_params *p, double *scores, uint64_
             a.sink_begin = n;
             return a;
         };
-        // the sweep's own finalize only counts sweeps; the per-graph rule stops the phase
+        // the sweep's own rule only counts sweeps; the per-graph rule stops the phase
         auto counting_rule = [&](uint64_t cap) {
             PhaseRule r{};
             r.kind = kRuleStep;

@@ -19,7 +19,7 @@ namespace nkpr {
 // of consecutive rows whose in-edges (at most kCap) are staged as products in LDS; a row
 // segment with more than kCap in-edges is a "vector" item reduced by the whole block; one
 // with more than kVectorMax in-edges is cut into kChunk-sized "split" items whose partial
-// sums the finalize kernel adds in chunk order (deterministic).
+// sums the end of the sweep adds in chunk order (deterministic).
 //
 // Source slicing.  Random gathers of the iterate are the cost of a sweep: an L2 miss moves a
 // 128-byte line for a 4- or 8-byte value.  The gathered node ids are therefore cut into
@@ -120,7 +120,6 @@ void pinned_free(void *p);
 hipStream_t stream_get();  // non-blocking, default priority
 void stream_put(hipStream_t s, int device);
 
-// Owning device allocation.
 // Row r of [lo, hi) with ptr[r] <= e < ptr[r + 1] (ptr rises; e lies in these rows).
 template <typename P>
 __device__ __forceinline__ uint64_t row_of(const P *ptr, uint64_t lo, uint64_t hi, uint64_t e) {
@@ -132,6 +131,7 @@ __device__ __forceinline__ uint64_t row_of(const P *ptr, uint64_t lo, uint64_t h
     return lo;
 }
 
+// Owning device allocation.
 struct DevBuf {
     void *p = nullptr;
     size_t bytes = 0;
@@ -154,7 +154,7 @@ struct DevBuf {
     template <typename T> T *as() const { return static_cast<T *>(p); }
 };
 
-// Device-resident control block of one sweep phase; written by the finalize kernel.
+// Device-resident control block of one sweep phase; written at the end of every sweep.
 struct PhaseCtl {
     double sink_in;   // sum of sink scores of the vector the next sweep reads
     double l1;        // ||x' - x||_1 of the last sweep
@@ -170,7 +170,7 @@ struct PhaseCtl {
     double scale;     // factor of the next sweep's product: 1, or 1 / len (kRuleNorm, rescale)
 };
 
-// Stopping rules evaluated by the finalize kernel.
+// Stopping rules evaluated at the end of a sweep.
 enum RuleKind : int32_t {
     kRuleStep = 0,       // reference: step in `norm` <= tol
     kRuleErr = 1,        // 2 d/(1-d) l1 / sum <= tol
@@ -205,7 +205,7 @@ struct Schedule {
     const uint4 *sitems;         // per slice: split chunks, vector rows, stream blocks
     uint32_t sitem_off[kSlices + 1];
     uint32_t n_s;
-    const uint8_t *split_flag;   // [n_s] 1: the finalize kernel finishes this row
+    const uint8_t *split_flag;   // [n_s] 1: finished at the end of the sweep, from its segments
     uint32_t *claim;             // [kSlices] worker claim counters (reset every sweep)
     uint32_t *arrive;            // [kArriveWords] counters of the blocks that have ended
     uint32_t workers;            // workers per slice; the sweep grid is n_slices * workers
@@ -374,7 +374,7 @@ bool binned64_active(nkpr_graph *g, bool one_sweep);
 const int32_t *slot_index(nkpr_graph *g);
 void binned_sweep64(nkpr_graph *g, const SweepArgs<double> &a, const FinalizeArgs &f, int kind,
                     hipStream_t s, hipEvent_t ev0, hipEvent_t ev1);
-// The finalize step of launch_sweep<double> alone (nkpr_sweep.hip).
+// The end of a sweep alone, as a launch of one block (nkpr_sweep.hip).
 void launch_finalize64(const SweepArgs<double> &a, const FinalizeArgs &f, hipStream_t s);
 void set_weights(nkpr_graph *g, const float *w, const double *w64, const double *out_wdeg,
                  int device_ptrs);

@@ -12,10 +12,11 @@
 //
 // The same kernel produces the convergence inputs of PageRank.cpp:34-51 (sum |x'-x| and
 // sum (x'-x)^2 in FP64), the score sum used by the normalisation at :75-80 and the sink mass
-// used at :81-92, as per-block partials.  A one-block finalize kernel then adds the
-// partials in a fixed order, finishes the rows that were split across blocks, applies the
-// stopping rule and raises a device-side `done` flag that turns later sweeps of the batch
-// into no-ops, so the host reads the state back only once per batch of sweeps.
+// used at :81-92, as per-block partials.  The block that arrives last in the sweep's last launch
+// (the sweep kernel, or the combine kernel where rows are sliced) then adds the partials in a
+// fixed order, finishes the rows that were split across blocks, applies the stopping rule and
+// raises a device-side `done` flag that turns later sweeps of the batch into no-ops, so the host
+// reads the state back only once per batch of sweeps.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -318,7 +319,10 @@ __device__ __forceinline__ void stream_item(const SweepArgs<T> &a, const uint4 i
 // One block ends a sweep: finish the rows with split segments, add all partials in a fixed order,
 // apply the stopping rule, reset the worker claim counters for the next sweep.  The block that
 // arrives last in the sweep's last launch does it (a launch of its own took 5.3 us of the 30 us
-// sweep of a 20,000-node graph).
+// sweep of a 20,000-node graph).  What it reads of other blocks' work in the same launch are the
+// partials, through agent-scope accesses.  The sums of split rows (partial, split_partial) are
+// plain stores of an earlier launch: only sliced rows are split, so with split rows this runs in
+// the combine kernel (checked in launch_pair).
 template <typename T, bool BASEVEC, bool RESID, int BLOCK>
 __device__ __forceinline__ void finish_sweep(const SweepArgs<T> &a, const FinalizeArgs &f,
                                              double (*s_red)[BLOCK / 64]) {
@@ -506,7 +510,7 @@ __global__ __launch_bounds__(kBlock, kSweepWaves) void sweep_kernel(SweepArgs<T>
 
     // per-worker partials (l1, l2, sum, sink) in FP64: indexed by the claimed worker, whose
     // rows are fixed, not by the block, whose worker depends on the order of the claims, so
-    // that the finalize kernel adds the same values in the same order on every run
+    // that finish_sweep adds the same values in the same order on every run
     if (f.n_blocks == 0) return;  // a product alone: nothing to reduce, no rule
     const Acc4 sums = block_sum4<kBlock>(st, s_red);
     if (tid == 0) put_partials(a.partials + (size_t)w * 4, sums);
@@ -516,7 +520,7 @@ __global__ __launch_bounds__(kBlock, kSweepWaves) void sweep_kernel(SweepArgs<T>
 }
 
 // Sliced rows: add the per-slice row sums in slice order and run the row epilogue.  Rows
-// with split segments are left to the finalize kernel.
+// with split segments are left to finish_sweep.
 template <typename T, bool BASEVEC, bool RESID>
 __global__ __launch_bounds__(kCombineThreads) void combine_kernel(SweepArgs<T> a, FinalizeArgs f,
                                                                   uint32_t block_base) {
@@ -764,6 +768,7 @@ template <typename T, bool FOLDED, bool BASEVEC, bool RESID>
 void launch_pair(const SweepArgs<T> &a, const FinalizeArgs &f, int combine_grid, hipStream_t s,
                  hipEvent_t ev0, hipEvent_t ev1) {
     const unsigned grid = a.sc.n_slices * a.sc.workers;
+    NKPR_CHECK(f.n_split_rows == 0 || a.sc.n_s > 0, "split rows are sliced rows");
     if (ev0) NKPR_HIP(hipEventRecord(ev0, s));
     hipLaunchKernelGGL((sweep_kernel<T, FOLDED, BASEVEC, RESID>), dim3(grid), dim3(kBlock), 0, s,
                        a, f);
