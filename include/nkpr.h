@@ -286,8 +286,9 @@ typedef struct {
 /* Replaces CSRGeneralMatrix::operator*(const Vector&) (CSRGeneralMatrix.hpp:563-578):
  * y[i] = sum over row i of values[k] * x[col_idx[k]].  x[cols] and y[rows] are distinct device
  * vectors; rows < 2^32 - 1.  Enqueued on `stream` (a hipStream_t; NULL is the null stream);
- * returns without waiting.  Its scratch comes from the stream's memory pool.  The matrix
- * structure is taken as given (see nkpr_algebraic_pagerank for a run that checks it). */
+ * returns without waiting.  Its scratch comes from the stream's memory pool.  Only the entries
+ * row_idx[0] to row_idx[rows] are read, so that the lists may hold others before and after them
+ * (nnz counts them all).  The matrix structure is taken as given (see nkpr_algebraic_pagerank for a run that checks it). */
 int nkpr_csr_spmv(const nkpr_csr *a, const double *x, double *y, void *stream);
 
 /* One iteration of AlgebraicPageRank::run (AlgebraicPageRank.hpp:97-101) on a square matrix

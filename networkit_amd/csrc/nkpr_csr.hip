@@ -27,7 +27,7 @@
 // What bounds it: the two 8-byte streams (16 bytes per entry) and the gathers of x, in flight
 // together for a whole tile.  A lane group per row with a block sum per long row kept one or two
 // entries in flight per lane and left long rows to five more launches (one of them a single
-// thread): 713 us for the step of an R-MAT matrix of 1e6 rows and 1.4e7 entries, 146 us now (the tiles
+// thread): 713 us for the step of an R-MAT matrix of 1e6 rows and 1.4e7 entries, 148 us now (the tiles
 // 129 us).
 //
 // Scratch of a product: a carry (row and sum) per tile, 12 bytes for 4096 merged items, and the
