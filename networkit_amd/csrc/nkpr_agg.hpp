@@ -13,13 +13,14 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 
 namespace nkpr {
 
 constexpr uint32_t kAggSlots = 2048;   // 32 KB: four blocks of kAggThreads a CU
 constexpr int kAggThreads = 512;
-constexpr unsigned kAggBlocks = 1024;  // persistent: a table serves m / kAggBlocks arcs
+constexpr unsigned kAggBlocks = 1024;  // persistent, at most (see agg_blocks)
 constexpr uint32_t kAggEmpty = 0xFFFFFFFFu;
 
 struct AggTable {
@@ -63,9 +64,16 @@ struct AggTable {
 };
 static_assert(kAggSlots == 1u << (32 - 21), "the hash keeps the top 11 bits");
 
+// Blocks for m arcs.  A table is emptied into memory at the end, up to kAggSlots atomics a block, so few
+// arcs a block cost more than an atomic per arc; a block per CU comes before that.  Weights of R-MAT
+// graphs in us, atomic per arc / blocks of 512 arcs / this rule: 1.4e5 arcs 38 / 43 / 27, 5.8e5
+// 115 / 142 / 74, 1.7e6 273 / 231 / 180.
+constexpr uint64_t kAggFewArcs = 1024, kAggArcs = 4096;
+constexpr uint64_t kAggFewBlocks = 256;
 inline unsigned agg_blocks(uint64_t m) {
-    const uint64_t b = (m + kAggThreads - 1) / kAggThreads;
-    return (unsigned)(b < 1 ? 1 : (b < kAggBlocks ? b : kAggBlocks));
+    uint64_t b = (m + kAggFewArcs - 1) / kAggFewArcs;
+    if (b > kAggFewBlocks) b = std::max(kAggFewBlocks, (m + kAggArcs - 1) / kAggArcs);
+    return (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(b, kAggBlocks));
 }
 
 }  // namespace nkpr
