@@ -429,6 +429,8 @@ class DeviceCSR:
         self.rows, self.cols = int(rows), int(cols)
         self.nnz = int(self.col_idx.numel())
         assert self.row_idx.numel() == self.rows + 1 and self.values.numel() == self.nnz
+        # the conversions above run on torch's stream, the calls that take no stream on their own
+        torch.cuda.current_stream(dev).synchronize()
 
     def struct(self):
         return CsrMatrix(rows=self.rows, cols=self.cols, nnz=self.nnz,

@@ -225,3 +225,25 @@ def test_csr_spmv_many_long_rows_and_pieces():
     y2, s2 = d.pagerank_step(tx, 0.1)
     torch.cuda.synchronize()
     assert torch.equal(y1, y2) and float(s1.item()) == float(s2.item())
+
+
+def test_device_arrays_converted_behind_other_work():
+    """DeviceCSR converts its arrays on torch's stream; the calls that take no stream read them on
+    their own, so they must be there when the constructor returns."""
+    import torch
+    n, m = 200000, 1600000
+    g = torch.Generator(device="cuda").manual_seed(3)
+    row = torch.sort(torch.randint(n, (m,), generator=g, device="cuda"))[0]
+    ptr = torch.zeros(n + 1, dtype=torch.int64, device="cuda")
+    ptr[1:] = torch.cumsum(torch.bincount(row, minlength=n), 0)
+    col = torch.randint(n, (m,), generator=g, device="cuda")
+    val = 0.85 / torch.bincount(col, minlength=n).double()[col]
+    torch.cuda.synchronize()
+    want, it = capi.DeviceCSR(n, n, ptr, col, val).algebraic_pagerank(tol=1e-9)
+    a = torch.rand(4096, 4096, generator=g, device="cuda")
+    for make in (lambda c: c.algebraic_pagerank(tol=1e-9), lambda c: capi.DeviceAlgebraic(c).run(tol=1e-9)):
+        for _ in range(20):
+            a @ a
+        got = make(capi.DeviceCSR(n, n, ptr.int(), col.int(), val.float().double()))
+        assert got[1] == it
+        np.testing.assert_allclose(got[0], want, rtol=1e-6, atol=0)  # FP32 values: 2^-24 / (1 - d)
