@@ -158,8 +158,9 @@ __device__ __forceinline__ uint64_t rows_before(const CsrView &A, const Entries 
 
 // Tile t: rows [i0, i1) end in it, with entries [k0, k1).  Tiles past the last merged item are empty
 // and leave no carry.
+// Six waves a SIMD: the large tile's LDS lets three blocks share a CU.
 template <typename Shape, bool STEP>
-__global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
+__global__ __launch_bounds__(Shape::kThreads, 6) void csr_tile_kernel(CsrView A,
                                                                    const double *__restrict__ x,
                                                                    double shift, double *y,
                                                                    TileWork w, uint64_t tiles) {
@@ -169,6 +170,8 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
     __shared__ uint16_t ends[kItems + 2];  // ends[j], ends[j + 1]: the tile's part of row i0 + j
     __shared__ uint16_t longs[kItems / kTurns];
     __shared__ uint32_t n_long;
+    constexpr uint32_t kSpread = kItems / kThreads;
+    __shared__ double share[kSpread][kThreads / 64];
     __shared__ uint64_t s_row[2];
     const uint32_t tid = threadIdx.x, wave = tid >> 6;
     const Entries E = entries_of(A);
@@ -207,19 +210,6 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
             if (e < cnt) prod[e] = v[k] * x[c[k]];
         }
         __syncthreads();
-        if (whole == 0) {
-            // the tile lies inside one row, and its sum is the carry: added by the whole block, not by
-            // one wave (1000 rows of 70000 entries: 301 us a step, now 252; one row of 1e8 433 and 355).  From LDS:
-            // summed from the registers these take 246 and 347, and every other tile 0.6% longer
-            double acc = 0.0;
-            for (uint32_t e = tid; e < cnt; e += kThreads) acc += prod[e];
-            acc = block_sum<kThreads>(acc);
-            if (tid == 0) {
-                w.carry[t] = acc;
-                w.row[t] = cnt ? (uint32_t)i1 : kNoRow;
-            }
-            continue;
-        }
         // row i0 began in an earlier tile: its sum, and its square, are finished by the fix kernel
         const bool continued = i0 < A.rows && A.row_idx[i0] - E.first < k0;
         const uint32_t R = whole + 1;  // the last one: what is left after the last row end
@@ -237,34 +227,57 @@ __global__ __launch_bounds__(Shape::kThreads) void csr_tile_kernel(CsrView A,
                 sq += d * d;
             }
         };
-        // G consecutive lanes a row, G ~ the average length
-        const uint32_t avg = cnt / R;
-        const int lg = avg >= 64 ? 6 : (avg >= 32 ? 5 : (avg >= 16 ? 4 : (avg >= 8 ? 3 : (avg >= 4 ? 2 : (avg >= 2 ? 1 : 0)))));
-        const uint32_t G = 1u << lg, lane = tid & (G - 1), per_pass = kThreads >> lg;
-        for (uint32_t base = 0; base < R; base += per_pass) {
-            const uint32_t r = base + (tid >> lg);
-            double acc = 0.0;
-            bool own = r < R;
-            if (own) {
-                const uint32_t b = ends[r], e = ends[r + 1];
-                if (e - b > kTurns * G) {
-                    own = false;
-                    if (lane == 0) longs[atomicAdd(&n_long, 1u)] = (uint16_t)r;
-                } else {
-                    for (uint32_t i = b + lane; i < e; i += G) acc += prod[i];
-                }
+        // n rows (at most kSpread), a share of each for every wave: rows that fill a tile or a good part of
+        // it would keep one wave each busy and the others waiting (us a step with a wave a row / so:
+        // rows of 70000 entries 301 / 252, of 1500 99 / 94; one row of 5000 in 1000 61.3 both)
+        auto spread = [&](uint32_t n, auto row) {
+            for (uint32_t k = 0; k < n; ++k) {
+                const uint32_t r = row(k), e = ends[r + 1];
+                double acc = 0.0;
+                for (uint32_t i = ends[r] + tid; i < e; i += kThreads) acc += prod[i];
+                for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+                if ((tid & 63) == 0) share[k][wave] = acc;
             }
-            for (uint32_t off = G >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-            if (own && lane == 0) put(r, acc);
-        }
-        __syncthreads();
-        const uint32_t nl = n_long;
-        for (uint32_t k = wave; k < nl; k += kThreads / 64) {
-            const uint32_t r = longs[k];
-            double acc = 0.0;
-            for (uint32_t i = ends[r] + (tid & 63); i < ends[r + 1]; i += 64) acc += prod[i];
-            for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
-            if ((tid & 63) == 0) put(r, acc);
+            __syncthreads();
+            if (tid < n) {
+                double sum = 0.0;
+                for (uint32_t k = 0; k < kThreads / 64; ++k) sum += share[tid][k];
+                put(row(tid), sum);
+            }
+        };
+        if (cnt >= kThreads * R) {  // a turn of the block or more per row
+            spread(R, [](uint32_t k) { return k; });
+        } else {
+            // G consecutive lanes a row, G ~ the average length
+            const uint32_t avg = cnt / R;
+            const int lg = avg >= 64 ? 6 : (avg >= 32 ? 5 : (avg >= 16 ? 4 : (avg >= 8 ? 3 : (avg >= 4 ? 2 : (avg >= 2 ? 1 : 0)))));
+            const uint32_t G = 1u << lg, lane = tid & (G - 1), per_pass = kThreads >> lg;
+            for (uint32_t base = 0; base < R; base += per_pass) {
+                const uint32_t r = base + (tid >> lg);
+                double acc = 0.0;
+                bool own = r < R;
+                if (own) {
+                    const uint32_t b = ends[r], e = ends[r + 1];
+                    if (e - b > kTurns * G) {
+                        own = false;
+                        if (lane == 0) longs[atomicAdd(&n_long, 1u)] = (uint16_t)r;
+                    } else {
+                        for (uint32_t i = b + lane; i < e; i += G) acc += prod[i];
+                    }
+                }
+                for (uint32_t off = G >> 1; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+                if (own && lane == 0) put(r, acc);
+            }
+            __syncthreads();
+            const uint32_t nl = n_long;
+            if (nl == 1 || nl == 2) spread(nl, [&](uint32_t k) { return (uint32_t)longs[k]; });
+            for (uint32_t k = nl > 2 ? wave : nl; k < nl; k += kThreads / 64) {
+                const uint32_t r = longs[k];
+                double acc = 0.0;
+                for (uint32_t i = ends[r] + (tid & 63); i < ends[r + 1]; i += 64) acc += prod[i];
+                for (int off = 32; off > 0; off >>= 1) acc += __shfl_xor(acc, off, 64);
+                if ((tid & 63) == 0) put(r, acc);
+            }
         }
         __syncthreads();  // the next tile rewrites the shared arrays
     }
@@ -304,8 +317,8 @@ __device__ __forceinline__ double sum_run(const TileWork &w, uint64_t t, uint32_
 // kernel, go to out[blockIdx.x].
 //
 // Bound by latency: two rounds of loads.  A thread that walked a run alone waited for one tile's row
-// after the other; steps with one row of 4e6, 1e7 and 1e8 entries took 594, 408 and 4040 us, now 35, 50
-// and 355.
+// after the other; steps with one row of 4e6, 1e7 and 1e8 entries took 594, 408 and 4040 us, now 33, 49
+// and 365.
 constexpr uint32_t kRunAlone = 8;
 template <bool STEP>
 __global__ __launch_bounds__(kFixThreads) void csr_fix_kernel(const double *__restrict__ x, double *y,
@@ -317,20 +330,15 @@ __global__ __launch_bounds__(kFixThreads) void csr_fix_kernel(const double *__re
     for (uint64_t t0 = (uint64_t)blockIdx.x * kFixThreads + (threadIdx.x - lane); t0 < tiles;
          t0 += (uint64_t)gridDim.x * kFixThreads) {
         const uint64_t t = t0 + lane;
-        // every load of the tiles at once
-        uint32_t row[kRunAlone + 1];
-        double c[kRunAlone];
-#pragma unroll
-        for (uint32_t k = 0; k <= kRunAlone; ++k) row[k] = t + k < tiles ? w.row[t + k] : kNoRow;
-#pragma unroll
-        for (uint32_t k = 0; k < kRunAlone; ++k) c[k] = t + k < tiles ? w.carry[t + k] : 0.0;
-        const uint32_t before = t > 0 && t < tiles ? w.row[t - 1] : kNoRow, r = row[0];
-        const bool first = r != kNoRow && before != r;
-        const bool many = first && row[kRunAlone] == r;
-        double s = c[0];
-#pragma unroll
-        for (uint32_t k = 1; k < kRunAlone; ++k)
-            if (row[k] == r) s += c[k];
+        const uint32_t r = t < tiles ? w.row[t] : kNoRow, last = t > 0 && t < tiles ? w.row[t - 1] : kNoRow;
+        const uint32_t next = t + 1 < tiles ? w.row[t + 1] : kNoRow;
+        const uint32_t far = t + kRunAlone < tiles ? w.row[t + kRunAlone] : kNoRow;
+        double s = t < tiles ? w.carry[t] : 0.0;
+        const bool first = r != kNoRow && last != r, many = first && far == r;
+        if (first && !many && next == r) {
+            s += w.carry[t + 1];
+            for (uint64_t q = t + 2; q < tiles && w.row[q] == r; ++q) s += w.carry[q];
+        }
         for (uint64_t left = __ballot(many); left; left &= left - 1) {
             const int l = __ffsll((long long)left) - 1;
             const double sum = sum_run(w, t0 + l, __shfl(r, l, 64), tiles);
