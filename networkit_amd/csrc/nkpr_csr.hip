@@ -18,7 +18,8 @@
 //       equal length, so that a block has as much to do whatever the rows' lengths: it finds its
 //       first row and entry by a search over row_idx (64 probes at a time, the lanes of a wave),
 //       reads its entries as one stream, puts the products into LDS and adds them row by row, lane
-//       groups for short rows and whole waves for long ones.  What is left after its last row end
+//       groups for short rows, whole waves for long ones and all waves where few rows fill the
+//       tile.  What is left after its last row end
 //       is the tile's carry for the row that goes on.
 //   csr_fix_kernel    adds the carries to the row that ended in a later tile.
 //   csr_final_kernel  (steps of many tiles) adds the blocks' sums.
